@@ -357,19 +357,22 @@ int zq3d_get_timing(zq3d_sim* sim, zq3d_timing* out);
  * kernel on interleaved storage (ty rows per workgroup, zc planes per chunk); ty == -1 is two
  * single-colour sweeps per iteration on colour-split storage; ty == -r (r = 4, 8, 16, 32) is one
  * launch per iteration on colour-split storage (r rows by zc = 8, 16, 32 planes per workgroup);
- * ty == -(100 + r) (r = 16, 32) is two iterations per launch on colour-split storage.  All produce
- * the same bits.
+ * ty == -(100 + r) (r = 16, 32) is two iterations per launch on colour-split storage;
+ * ty == -(1000 + 100 c + w) is two iterations per launch with the planes in registers (c = 2 or 4
+ * cells per lane, w waves per workgroup, up to 16 or 8; zc planes, even, at most 64).  The default,
+ * (0, 0), is the last family at the shape predicted fastest for the grid.  All produce the same bits.
  * Clobbers the projection scratch (not the fields). */
 #define ZQ3D_TUNE_MAX 32
 typedef struct zq3d_tune_report {
     int count;                       /* candidates timed */
-    int best;                        /* index of the chosen one (-1: the grid is too wide for the fused kernel) */
+    int best;                        /* index of the chosen one */
     int ty[ZQ3D_TUNE_MAX];
     int zc[ZQ3D_TUNE_MAX];
     float us_per_iter[ZQ3D_TUNE_MAX];
 } zq3d_tune_report;
 int zq3d_autotune_sor(zq3d_sim* sim, int iters, zq3d_tune_report* report);
-/* explicit shape, one of the autotuner's candidates; (0, 0) restores the default */
+/* explicit shape of any of these families (the autotuner times the ones that are fastest on some
+ * grid); (0, 0) restores the default */
 int zq3d_set_sor_shape(zq3d_sim* sim, int ty, int zc);
 /* Coarse + sub-grid projection (sub_size > 0; no reference counterpart): schedule of the coarse
  * red-black sweeps.  k == 0: one launch per colour; k > 0: k iterations per launch, each workgroup
@@ -390,8 +393,8 @@ int zq3d_get_coarse_sweep(zq3d_sim* sim, int* k, int* zc);
  * with min(sor.iters, region cells) iterations; that branch never adds the guide, so coeff and the
  * arrays' values are not read.  Host work per projection: the level map and faces cross PCIe. */
 int zq3d_set_guide(zq3d_sim* sim, float coeff, const float* gu, const float* gv, const float* gw);
-/* name of the sweep kernel the current shape runs ("k_sor_split_rb", "k_sor_split", "k_sor_fused"
- * or "k_sor_half") */
+/* name of the sweep kernel the current shape runs ("k_sor_quad", "k_sor_split_rb", "k_sor_split_rb2",
+ * "k_sor_split", "k_sor_fused" or "k_sor_half") */
 const char* zq3d_sor_kernel(zq3d_sim* sim);
 
 /* ====================== Part 4: host-side scene set-up (no GPU) ====================== */
@@ -475,8 +478,8 @@ int zq3d_adj_set_adjoint_tol(zq3d_adj* a, double rtol);
  * store is filled by the next zq3d_adj_forward and used by the zq3d_adj_backward that follows it
  * (whose controls are those of that forward); until then recomputed steps solve as without it. */
 int zq3d_adj_set_pressure_store(zq3d_adj* a, int on);
-/* sweep algorithm / tile shape of every projection of the rollout, one of zq3d_autotune_sor's
- * candidates for this grid (default (-1, 0)); all give the same bits */
+/* sweep algorithm / tile shape of every projection of the rollout, as zq3d_set_sor_shape takes it for
+ * this grid (the default is the one a simulation has); all give the same bits */
 int zq3d_adj_set_sor_shape(zq3d_adj* a, int ty, int zc);
 /* initial state: ZQ3D_FIELD_U/V/W/T/RHO (device, chosen precision), ZQ3D_FIELD_OCC (device bytes) or
  * ZQ3D_FIELD_P64 (device doubles, padded: the forward projection's warm start; default 0) */

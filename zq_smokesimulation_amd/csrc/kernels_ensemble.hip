@@ -209,7 +209,7 @@ __global__ __launch_bounds__(NT) void ke_correct(const EnsMember* __restrict__ M
     for_tiles<64, 4>(T, B, [&](int s, int, int i, int j, int k) {
         const EnsMember& m = M[s];
         float* face = AXIS == 0 ? m.u : (AXIS == 1 ? m.v : m.w);
-        st_correct<AXIS, float, float>(m.occ, m.open_mask, m.p, face, m.d, i, j, k);
+        st_correct<AXIS>(m.occ, m.open_mask, PadPressure<float>{m.p}, face, m.d, i, j, k);
     });
 }
 

@@ -14,6 +14,7 @@
 // one partial per block (wave butterfly + LDS), then one block folds the partials in index order.
 #include "zq3d_device.h"
 #include "zq3d_kernels.h"
+#include "zq3d_sor_quad.h"
 #include "zq3d_sor_split.h"
 #include "zq3d_stencils.h"
 
@@ -37,13 +38,14 @@ __global__ __launch_bounds__(BX* BY) void k_proj_setup(const float* __restrict__
                                                        const float* __restrict__ w, const uint8_t* __restrict__ occ,
                                                        int open_mask, uint8_t* __restrict__ nc,
                                                        float* __restrict__ b, float* __restrict__ p,
-                                                       double* __restrict__ part, Dims d) {
+                                                       double* __restrict__ part, Dims d,
+                                                       uint8_t* __restrict__ nq) {
     __shared__ double red[4];
     const int i = blockIdx.x * BX + threadIdx.x;
     const int j = blockIdx.y * BY + threadIdx.y;
     const int k = blockIdx.z;
     double dsum = 0.0, dcnt = 0.0;
-    st_proj_setup_plain(u, v, w, occ, open_mask, nc, b, p, d, i, j, k, dsum, dcnt);
+    st_proj_setup_plain(u, v, w, occ, open_mask, nc, b, p, d, i, j, k, dsum, dcnt, nq);
     if (part) {
         const double s = block_reduce<false>(dsum, red);
         __syncthreads();
@@ -63,7 +65,8 @@ __global__ __launch_bounds__(BX* BY) void k_proj_setup_z(const float* __restrict
                                                          const float* __restrict__ w, const uint8_t* __restrict__ occ,
                                                          int open_mask, uint8_t* __restrict__ nc,
                                                          double* __restrict__ b64, double* __restrict__ p64,
-                                                         double* __restrict__ part, Dims d) {
+                                                         double* __restrict__ part, Dims d,
+                                                         uint8_t* __restrict__ nq) {
     __shared__ double red[4];
     const int i = blockIdx.x * BX + threadIdx.x;
     const int j = blockIdx.y * BY + threadIdx.y;
@@ -92,6 +95,7 @@ __global__ __launch_bounds__(BX* BY) void k_proj_setup_z(const float* __restrict
                 n += (k < d.D - 1) ? !oa : ((open_mask & 32) != 0);
             }
             nc[o] = (uint8_t)n;
+            if (nq) st_quad_count(nq, d, i, j, k, n);
             const float u0 = u[uidx(d, i, j, k)], u1 = u[uidx(d, i + 1, j, k)];
             const float v0 = v[vidx(d, i, j, k)], v1 = v[vidx(d, i, j + 1, k)];
             const float w1 = w[widx(d, i, j, k + 1)];
@@ -417,6 +421,22 @@ __global__ __launch_bounds__(64 * NW) void k_sor_split_rb(const uint8_t* __restr
                                                   by * TY, z0, min(z0 + zc, d.D), omega, omw);
 }
 
+// K red-black iterations per launch on the quad layout (sor_quad_tile); 1-D grid of tiles, numbered so
+// each XCD (block b runs on XCD b % 8) receives a contiguous run of tiles, which share their halos
+// through that XCD's L2.  src == nullptr: the source is all zeros.
+template <int K, int CX, int NT, bool MASK>
+__global__ __launch_bounds__(NT) void k_sor_quad(const uint8_t* __restrict__ n, const float* __restrict__ b,
+                                                 const float* __restrict__ mean32, const float* __restrict__ src,
+                                                 float* __restrict__ dst, Dims d, QuadCut c, float omega, float omw) {
+    extern __shared__ float quad_lds[];
+    const int per = gridDim.x >> 3;
+    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (tile >= c.nx * c.ny * c.nz) return;  // spare block (the grid is a multiple of 8): uniform exit
+    const int rest = quad_div(tile, c.mnx), bx = tile - rest * c.nx;
+    const int bz = quad_div(rest, c.mny), by = rest - bz * c.ny;
+    sor_quad_tile<K, CX, QUAD_R, MASK, 1, NT>(n, b, *mean32, src, dst, d, c, bx, by, bz, omega, omw, quad_lds);
+}
+
 // Iteration `it` of a gated pass (k_sor_split_rb otherwise): it returns at once when the previous
 // iteration's largest update, gate[it - 1] (FP32 bits; 0 when that iteration did not run either),
 // is at most `thresh`, or, past iteration 2 GATE_K, no smaller than gate[it - 1 - GATE_K] (the
@@ -534,9 +554,9 @@ __global__ __launch_bounds__(64 * NW) void k_sor_split_rb2(const uint8_t* __rest
 // low u, v and w faces, and the cells of the last column / row / plane also the domain's high face.
 // Every face is written once, with st_correct's value, so the result equals the three per-axis
 // launches bit for bit while each pressure value is loaded once instead of three times.
-template <class P, class F>
+template <class PA, class F>
 __global__ __launch_bounds__(BX* BY) void k_correct_cells(const uint8_t* __restrict__ occ, int open_mask,
-                                                          const P* __restrict__ p, F* __restrict__ u,
+                                                          PA p, F* __restrict__ u,
                                                           F* __restrict__ v, F* __restrict__ w, Dims d) {
     const int i = blockIdx.x * BX + threadIdx.x;
     const int j = blockIdx.y * BY + threadIdx.y;
@@ -546,12 +566,12 @@ __global__ __launch_bounds__(BX* BY) void k_correct_cells(const uint8_t* __restr
     // second trip to HBM as when neighbouring planes belong to other workgroups)
     const int k1 = min((int)(blockIdx.z + 1) * RES_RZ, d.D);
     for (int k = blockIdx.z * RES_RZ; k < k1; k++) {
-        st_correct<0, P, F>(occ, open_mask, p, u, d, i, j, k);
-        if (i == d.W - 1) st_correct<0, P, F>(occ, open_mask, p, u, d, i + 1, j, k);
-        st_correct<1, P, F>(occ, open_mask, p, v, d, i, j, k);
-        if (j == d.H - 1) st_correct<1, P, F>(occ, open_mask, p, v, d, i, j + 1, k);
-        st_correct<2, P, F>(occ, open_mask, p, w, d, i, j, k);
-        if (k == d.D - 1) st_correct<2, P, F>(occ, open_mask, p, w, d, i, j, k + 1);
+        st_correct<0, PA, F>(occ, open_mask, p, u, d, i, j, k);
+        if (i == d.W - 1) st_correct<0, PA, F>(occ, open_mask, p, u, d, i + 1, j, k);
+        st_correct<1, PA, F>(occ, open_mask, p, v, d, i, j, k);
+        if (j == d.H - 1) st_correct<1, PA, F>(occ, open_mask, p, v, d, i, j + 1, k);
+        st_correct<2, PA, F>(occ, open_mask, p, w, d, i, j, k);
+        if (k == d.D - 1) st_correct<2, PA, F>(occ, open_mask, p, w, d, i, j, k + 1);
     }
 }
 
@@ -579,7 +599,8 @@ __global__ __launch_bounds__(BX* BY) void k_proj_setup_mp(const F* __restrict__ 
                                                           const F* __restrict__ w, const uint8_t* __restrict__ occ,
                                                           int open_mask, uint8_t* __restrict__ nc,
                                                           double* __restrict__ b64, double* __restrict__ p64,
-                                                          double* __restrict__ part, Dims d) {
+                                                          double* __restrict__ part, Dims d,
+                                                          uint8_t* __restrict__ nq) {
     __shared__ double red[4];
     const int i = blockIdx.x * BX + threadIdx.x;
     const int j = blockIdx.y * BY + threadIdx.y;
@@ -600,6 +621,7 @@ __global__ __launch_bounds__(BX* BY) void k_proj_setup_mp(const F* __restrict__ 
         }
         const int n = (int)c[0] + (int)c[1] + (int)c[2] + (int)c[3] + (int)c[4] + (int)c[5];
         nc[o] = (uint8_t)n;
+        if (nq) st_quad_count(nq, d, i, j, k, n);
         double u0 = (double)u[uidx(d, i, j, k)], u1 = (double)u[uidx(d, i + 1, j, k)];
         double v0 = (double)v[vidx(d, i, j, k)], v1 = (double)v[vidx(d, i, j + 1, k)];
         double w0 = (double)w[widx(d, i, j, k)], w1 = (double)w[widx(d, i, j, k + 1)];
@@ -709,10 +731,11 @@ __global__ __launch_bounds__(BX* BY) void k_residual64(const uint8_t* __restrict
     if (threadIdx.x == 0 && threadIdx.y == 0) part[block_linear()] = m;
 }
 
-// k_residual64<true> marching z: each thread owns one (i, j) column of a chunk of RES_RZ planes and
+// k_residual64 marching z (QUAD: r32 into the quad layout's right-hand side r0, else into the split ones): each thread owns one (i, j) column of a chunk of RES_RZ planes and
 // keeps the pressures of planes k-1, k, k+1 in registers, so each padded FP64 pressure is read once
 // (the per-plane kernel reads every plane for three neighbouring planes' blocks).  The same operations
 // per cell in the same order; the block maxima are over the chunk (a maximum is order-free).
+template <bool QUAD>
 __global__ __launch_bounds__(BX* BY) void k_residual64_z(const uint8_t* __restrict__ nc, const double* __restrict__ b64,
                                                          const double* __restrict__ mean64,
                                                          const double* __restrict__ p, float* __restrict__ r0,
@@ -747,7 +770,8 @@ __global__ __launch_bounds__(BX* BY) void k_residual64_z(const uint8_t* __restri
                 r = (float)rr;
                 m = fmax(m, fabs(rr));
             }
-            (((i + j + k) & 1) ? r1 : r0)[(k * d.H + j) * Wh + (i >> 1)] = r;
+            if (QUAD) r0[(k * d.H + j) * Wh + i] = r;
+            else (((i + j + k) & 1) ? r1 : r0)[(k * d.H + j) * Wh + (i >> 1)] = r;
             pm = pc;
             pc = pp;
             xl = xl2, xr = xr2, yl = yl2, yr = yr2, pp = pp2, bv = bv2, n = n2;
@@ -777,6 +801,20 @@ __global__ __launch_bounds__(BX* BY) void k_update_p64(const uint8_t* __restrict
     if (!n) return;
     p[q] = pv + (double)ev;
     if (ZERO) *ep = 0.0f;
+}
+
+// p64 += e, e in the quad layout (stride S)
+__global__ __launch_bounds__(BX* BY) void k_update_p64_quad(const uint8_t* __restrict__ nc, const float* __restrict__ e,
+                                                            double* __restrict__ p, Dims d, int S) {
+    const int i = blockIdx.x * BX + threadIdx.x;
+    const int j = blockIdx.y * BY + threadIdx.y;
+    const int k = blockIdx.z;
+    if (i >= d.W || j >= d.H) return;
+    const int q = pidx(d, i, j, k);
+    const int n = nc[cidx(d, i, j, k)];
+    const double pv = p[q];
+    const float ev = e[(k * d.H + j) * S + i];
+    if (n) p[q] = pv + (double)ev;
 }
 
 template <class F>
@@ -942,13 +980,13 @@ int reduction_partials(const Dims& d) { return 2 * cell_blocks(d); }
 
 void launch_proj_setup(const Dims& d, const float* u, const float* v, const float* w, const uint8_t* occ,
                        int open_mask, uint8_t* nc, float* b, double* b64, float* p_pad, double* p64_pad,
-                       double* part, hipStream_t s) {
+                       double* part, hipStream_t s, uint8_t* nq) {
     if (b64)
         hipLaunchKernelGGL(k_proj_setup_z, grid_z(d), dim3(BX, BY), 0, s, u, v, w, occ, open_mask, nc, b64, p64_pad,
-                           part, d);
+                           part, d, nq);
     else
         hipLaunchKernelGGL(k_proj_setup, grid_for(d.W, d.H, d.D), dim3(BX, BY), 0, s, u, v, w, occ, open_mask, nc, b,
-                           p_pad, part, d);
+                           p_pad, part, d, nq);
 }
 
 void launch_mean_finalize(const Dims& d, const double* part, float* mean32, double* mean64, int want, hipStream_t s) {
@@ -958,6 +996,98 @@ void launch_mean_finalize(const Dims& d, const double* part, float* mean32, doub
 void launch_mean_finalize_mp(const Dims& d, const double* part, double* mean64, int want, hipStream_t s) {
     const dim3 g = grid_z(d);
     hipLaunchKernelGGL(k_finish_mean, dim3(1), dim3(1024), 0, s, part, (int)(g.x * g.y * g.z), nullptr, mean64, want);
+}
+
+namespace {
+struct QuadShape {
+    int cx, nw, zc;
+};
+QuadShape quad_decode(SorShape s) {
+    const int code = -s.ty - SOR_QUAD;
+    return QuadShape{code / 100, code % 100, s.zc};
+}
+}  // namespace
+
+bool quad_shape_valid(const Dims& d, SorShape s) {
+    if (!is_quad(s)) return false;
+    const QuadShape q = quad_decode(s);
+    if ((q.cx != 2 && q.cx != 4) || q.nw < 1 || q.nw > (q.cx == 4 ? 8 : 16) || q.zc < 2 || q.zc > 64 || q.zc % 2) return false;
+    return quad_cut(d.W, d.H, d.D, 2, q.cx, q.nw, q.zc).ny > 0;
+}
+
+// The sweep shape {0, 0} stands for (computed once per handle): the cheapest cut by quad_cost, which reproduces the measured order of
+// the shapes (on 29 grids from 16^3 to 320^3 it is within 1 % of the fastest of all candidates on every
+// one).  What it gives, in microseconds per red-black iteration, beside the shape that was the default
+// (one-pass fused tiles) and the fastest of the other families (single-colour split sweeps up to 160^3,
+// one-launch split iterations above):
+//   20x24x16  3.8 (47.1, 5.3)   64^3  3.8 (49.9, 5.6)    150x97x61  6.2 (51.5, 8.7)
+//   128^3  6.3 (48.8, 10.3)     192^3  11.7 (-, 30.3)    256^3  23.8 (108, 41)
+// Small grids: a launch boundary costs 2.6 us and a chunk's serial steps 0.45 us each, so K = 2 halves
+// the launches (K = 3 and 4 measured slower: their longer pipelines cost what they save).  At 256^3 the
+// iteration moves 13 bytes a cell through the last-level cache, 26 us at the 8.4 TB/s a copy of that size
+// reaches: two iterations a pass go below it.
+QuadPlan quad_plan(const Dims& d) {
+    double t2 = 0.0, t4 = 0.0;
+    const QuadCut c2 = quad_best_cut(d.W, d.H, d.D, 2, 2, 16, &t2), c4 = quad_best_cut(d.W, d.H, d.D, 2, 4, 8, &t4);
+    const bool four = t4 < t2;
+    const QuadCut& c = four ? c4 : c2;
+    return QuadPlan{SorShape{-(SOR_QUAD + 100 * (four ? 4 : 2) + c.nw), c.zc}, quad_best_cut(d.W, d.H, d.D, 1, 2, 8)};
+}
+
+size_t quad_cells(const Dims& d) { return (size_t)quad_stride(d.W) * d.H * d.D; }
+
+namespace {
+template <int K, int CX, int NT>
+hipError_t launch_quad_one(const Dims& d, const QuadBufs& q, const QuadCut& c, const float* src, float* dst,
+                           const float* mean32, float omega, hipStream_t s) {
+    constexpr int lds = 4 * quad_lds_floats(K, CX, NT);
+    if constexpr (lds > 64 * 1024) {  // above the default limit of dynamic LDS: allowed once per process
+        static const hipError_t e0 = hipFuncSetAttribute((const void*)k_sor_quad<K, CX, NT, false>,
+                                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        static const hipError_t e1 = hipFuncSetAttribute((const void*)k_sor_quad<K, CX, NT, true>,
+                                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e0 != hipSuccess) return e0;
+        if (e1 != hipSuccess) return e1;
+    }
+    const int nb = (c.nx * c.ny * c.nz + 7) & ~7;
+    const float omw = 1.0f - omega;
+    if (c.mask)
+        hipLaunchKernelGGL((k_sor_quad<K, CX, NT, true>), dim3(nb), dim3(64 * c.nw), lds, s, q.n, q.b, mean32, src, dst,
+                           d, c, omega, omw);
+    else
+        hipLaunchKernelGGL((k_sor_quad<K, CX, NT, false>), dim3(nb), dim3(64 * c.nw), lds, s, q.n, q.b, mean32, src,
+                           dst, d, c, omega, omw);
+    return hipGetLastError();
+}
+}  // namespace
+
+// iters iterations from zero: pairs of them in one launch, an odd one on its own (first, so that the
+// launch without a source to read is the cheap one)
+int launch_quad_sweeps(const Dims& d, const QuadBufs& q, const float* mean32, float omega, int iters, SorShape shape,
+                       hipStream_t s, hipEvent_t ev0, hipEvent_t ev1, hipError_t* err) {
+    const QuadShape qs = quad_decode(shape);
+    const QuadCut c2 = quad_cut(d.W, d.H, d.D, 2, qs.cx, qs.nw, qs.zc);
+    *err = hipSuccess;
+    if (ev0) (void)hipEventRecord(ev0, s);
+    int from = 0;
+    const float* src = nullptr;
+    for (int it = 0; it < iters && *err == hipSuccess;) {
+        float* dst = q.p[1 - from];
+        if ((iters - it) & 1) {
+            *err = launch_quad_one<1, 2, 512>(d, q, q.plan.one, src, dst, mean32, omega, s);
+            it += 1;
+        } else {
+            if (qs.cx == 4) *err = launch_quad_one<2, 4, 512>(d, q, c2, src, dst, mean32, omega, s);
+            else if (c2.nw <= 8) *err = launch_quad_one<2, 2, 512>(d, q, c2, src, dst, mean32, omega, s);
+            else *err = launch_quad_one<2, 2, 1024>(d, q, c2, src, dst, mean32, omega, s);
+            it += 2;
+        }
+        src = dst;
+        from = 1 - from;
+    }
+    if (iters == 0) launch_fill_f32(q.p[0], quad_cells(d), 0.0f, s);
+    if (ev1) (void)hipEventRecord(ev1, s);
+    return from;
 }
 
 size_t split_padded_size(const Dims& d) { return (size_t)split_row((d.W + 1) / 2) * (d.H + 2) * (d.D + 2); }
@@ -1119,6 +1249,8 @@ float* launch_sor(const Dims& d, const uint8_t* nc, const float* b, const float*
 }
 
 const char* sor_kernel_name(const Dims& d, SorShape shape) {
+    if (shape.ty == 0 && shape.zc == 0) return "k_sor_quad";
+    if (is_quad(shape)) return "k_sor_quad";
     if (shape.ty == SOR_SPLIT) return "k_sor_split";
     if (shape.ty <= -SOR_TWO) return "k_sor_split_rb2";
     if (is_split(shape)) return "k_sor_split_rb";
@@ -1126,6 +1258,7 @@ const char* sor_kernel_name(const Dims& d, SorShape shape) {
 }
 
 long long sor_launches(const Dims& d, SorShape shape, int iters) {
+    if (is_quad(shape)) return (iters + 1) / 2;
     if (shape.ty == SOR_SPLIT) return 2LL * iters;
     if (shape.ty <= -SOR_TWO) return (iters + 1) / 2;
     if (is_split(shape)) return iters;
@@ -1136,41 +1269,56 @@ bool split_buffers_fit(const Dims& d) {
     return split_padded_size(d) * 4 <= 0x7FFFFFFFull && split_cell_size(d) * 4 <= 0x7FFFFFFFull;
 }
 
+bool sor_shape_valid(const Dims& d, SorShape sh) {
+    const bool zc8 = sh.zc == 8 || sh.zc == 16 || sh.zc == 32;
+    if (sh.ty == 0 && sh.zc == 0) return true;
+    if (is_quad(sh)) return quad_shape_valid(d, sh);
+    if (sh.ty > 0) return shape_supported(sh.ty) && (zc8 || sh.zc == 64) && fused_shape(d, sh).nblocks > 0;
+    if (sh.ty == SOR_SPLIT) return sh.zc == 0;
+    const int r = split_rows(sh);
+    if (sh.ty <= -SOR_TWO) return zc8 && (r == 16 || r == 32);
+    return zc8 && (r == 4 || r == 8 || r == 16 || r == 32) && split_buffers_fit(d);
+}
+
 int sor_shape_candidates(const Dims& d, SorShape* out, int max) {
-    static const int tys[] = {2, 4, 8};
-    static const int zcs[] = {8, 16, 32, 64};
     int n = 0;
-    for (int ty : tys)
-        for (int zc : zcs) {
-            const SorShape sh{ty, zc};
-            if (fused_shape(d, sh).nblocks > 0 && n < max) out[n++] = sh;
-        }
-    if (n < max) out[n++] = SorShape{SOR_SPLIT, 0};
-    static const int rb_rows[] = {4, 8, 16, 32};
-    static const int rb_zc[] = {8, 16, 32};
-    if (split_buffers_fit(d))
-        for (int ty : rb_rows)
-            for (int zc : rb_zc)
-                if (n < max) out[n++] = SorShape{-ty, zc};
-    static const int rb2_rows[] = {16, 32};
-    static const int rb2_zc[] = {8, 16, 32};
-    for (int ty : rb2_rows)
-        for (int zc : rb2_zc)
-            if (n < max) out[n++] = SorShape{-(SOR_TWO + ty), zc};
+    auto add = [&](SorShape sh) {
+        for (int i = 0; i < n; i++)
+            if (out[i].ty == sh.ty && out[i].zc == sh.zc) return;
+        if (n < max && sor_shape_valid(d, sh)) out[n++] = sh;
+    };
+    add(quad_plan(d).def);
+    static const int nws[] = {4, 8, 12, 16};
+    static const int zcs[] = {4, 8, 12, 16};
+    for (int nw : nws)
+        for (int zc : zcs) add(SorShape{-(SOR_QUAD + 200 + nw), zc});
+    for (int zc : {8, 16, 24, 32}) add(SorShape{-(SOR_QUAD + 400 + 8), zc});
+    // the older families, each at the shapes that were fastest on some grid
+    add(SorShape{SOR_SPLIT, 0});
+    add(SorShape{-16, 8});
+    add(SorShape{-16, 16});
+    add(SorShape{-32, 16});
+    add(SorShape{4, 16});
     return n;
 }
 
 void launch_correct(const Dims& d, const uint8_t* occ, int open_mask, const float* p_pad, float* u, float* v,
                     float* w, hipStream_t s) {
-    hipLaunchKernelGGL((k_correct_cells<float, float>), grid_z(d), dim3(BX, BY), 0, s, occ, open_mask, p_pad, u, v,
-                       w, d);
+    hipLaunchKernelGGL((k_correct_cells<PadPressure<float>, float>), grid_z(d), dim3(BX, BY), 0, s, occ, open_mask,
+                       PadPressure<float>{p_pad}, u, v, w, d);
+}
+
+void launch_correct_quad(const Dims& d, const uint8_t* occ, int open_mask, const float* p_quad, float* u, float* v,
+                         float* w, hipStream_t s) {
+    hipLaunchKernelGGL((k_correct_cells<QuadPressure, float>), grid_z(d), dim3(BX, BY), 0, s, occ, open_mask,
+                       QuadPressure{p_quad}, u, v, w, d);
 }
 
 template <class F>
 void launch_correct64(const Dims& d, const uint8_t* occ, int open_mask, const double* p64_pad, F* u, F* v, F* w,
                       hipStream_t s) {
-    hipLaunchKernelGGL((k_correct_cells<double, F>), grid_z(d), dim3(BX, BY), 0, s, occ, open_mask, p64_pad, u, v,
-                       w, d);
+    hipLaunchKernelGGL((k_correct_cells<PadPressure<double>, F>), grid_z(d), dim3(BX, BY), 0, s, occ, open_mask,
+                       PadPressure<double>{p64_pad}, u, v, w, d);
 }
 
 template <class F>
@@ -1182,19 +1330,20 @@ void launch_correct_all64(const Dims& d, const double* p64_pad, F* u, F* v, F* w
 
 void launch_proj_setup64(const Dims& d, const double* u, const double* v, const double* w, const uint8_t* occ,
                          int open_mask, int free_only, uint8_t* nc, double* b64, double* p64_pad, double* part,
-                         hipStream_t s) {
+                         hipStream_t s, uint8_t* nq) {
     if (free_only)
         hipLaunchKernelGGL((k_proj_setup_mp<double, true>), grid_for(d.W, d.H, d.D), dim3(BX, BY), 0, s, u, v, w, occ,
-                           open_mask, nc, b64, p64_pad, part, d);
+                           open_mask, nc, b64, p64_pad, part, d, nq);
     else
         hipLaunchKernelGGL((k_proj_setup_mp<double, false>), grid_for(d.W, d.H, d.D), dim3(BX, BY), 0, s, u, v, w,
-                           occ, open_mask, nc, b64, p64_pad, part, d);
+                           occ, open_mask, nc, b64, p64_pad, part, d, nq);
 }
 
 void launch_proj_setup_free(const Dims& d, const float* u, const float* v, const float* w, const uint8_t* occ,
-                            int open_mask, uint8_t* nc, double* b64, double* p64_pad, double* part, hipStream_t s) {
+                            int open_mask, uint8_t* nc, double* b64, double* p64_pad, double* part, hipStream_t s,
+                            uint8_t* nq) {
     hipLaunchKernelGGL((k_proj_setup_mp<float, true>), grid_for(d.W, d.H, d.D), dim3(BX, BY), 0, s, u, v, w, occ,
-                       open_mask, nc, b64, p64_pad, part, d);
+                       open_mask, nc, b64, p64_pad, part, d, nq);
 }
 
 void launch_max_abs64(const Dims& d, const uint8_t* nc, const double* b64, double* part, unsigned long long* out,
@@ -1221,8 +1370,17 @@ void launch_residual64_split(const Dims& d, const uint8_t* nc, const double* b64
                              const double* p64_pad, const SplitBufs& sp, double* part, unsigned long long* rmax,
                              hipStream_t s) {
     const dim3 g = grid_z(d);
-    hipLaunchKernelGGL(k_residual64_z, g, dim3(BX, BY), 0, s, nc, b64, mean64, p64_pad, sp.b[0], sp.b[1], part, d,
-                       (d.W + 1) / 2);
+    hipLaunchKernelGGL(k_residual64_z<false>, g, dim3(BX, BY), 0, s, nc, b64, mean64, p64_pad, sp.b[0], sp.b[1], part,
+                       d, (d.W + 1) / 2);
+    hipLaunchKernelGGL(k_finish_max, dim3(1), dim3(1024), 0, s, part, (int)(g.x * g.y * g.z), rmax);
+}
+
+void launch_residual64_quad(const Dims& d, const uint8_t* nc, const double* b64, const double* mean64,
+                            const double* p64_pad, const QuadBufs& q, double* part, unsigned long long* rmax,
+                            hipStream_t s) {
+    const dim3 g = grid_z(d);
+    hipLaunchKernelGGL(k_residual64_z<true>, g, dim3(BX, BY), 0, s, nc, b64, mean64, p64_pad, q.b, nullptr, part, d,
+                       quad_stride(d.W));
     hipLaunchKernelGGL(k_finish_max, dim3(1), dim3(1024), 0, s, part, (int)(g.x * g.y * g.z), rmax);
 }
 
@@ -1239,6 +1397,11 @@ void launch_update_p64_split(const Dims& d, const uint8_t* nc, float* const* e, 
     else
         hipLaunchKernelGGL((k_update_p64<true, false>), grid_for(d.W, d.H, d.D), dim3(BX, BY), 0, s, nc, e[0], e[1],
                            p64_pad, d, (d.W + 1) / 2);
+}
+
+void launch_update_p64_quad(const Dims& d, const uint8_t* nc, const float* e_quad, double* p64_pad, hipStream_t s) {
+    hipLaunchKernelGGL(k_update_p64_quad, grid_for(d.W, d.H, d.D), dim3(BX, BY), 0, s, nc, e_quad, p64_pad, d,
+                       quad_stride(d.W));
 }
 
 template <class F>

@@ -38,14 +38,14 @@ int project_mp(const Dims& d, F* u, F* v, F* w, const uint8_t* occ, const zq3d_s
     launch_fill_f32(&sc->zero32, 1, 0.0f, s);
     if (adjoint) {
         if constexpr (sizeof(F) == 4)
-            launch_proj_setup_free(d, u, v, w, occ, o.open_mask, B.nc, B.b64, B.p64, B.part, s);
+            launch_proj_setup_free(d, u, v, w, occ, o.open_mask, B.nc, B.b64, B.p64, B.part, s, B.quad.n);
         else
-            launch_proj_setup64(d, u, v, w, occ, o.open_mask, 1, B.nc, B.b64, B.p64, B.part, s);
+            launch_proj_setup64(d, u, v, w, occ, o.open_mask, 1, B.nc, B.b64, B.p64, B.part, s, B.quad.n);
     } else {
         if constexpr (sizeof(F) == 4)
-            launch_proj_setup(d, u, v, w, occ, o.open_mask, B.nc, nullptr, B.b64, nullptr, B.p64, B.part, s);
+            launch_proj_setup(d, u, v, w, occ, o.open_mask, B.nc, nullptr, B.b64, nullptr, B.p64, B.part, s, B.quad.n);
         else
-            launch_proj_setup64(d, u, v, w, occ, o.open_mask, 0, B.nc, B.b64, B.p64, B.part, s);
+            launch_proj_setup64(d, u, v, w, occ, o.open_mask, 0, B.nc, B.b64, B.p64, B.part, s, B.quad.n);
     }
     // the FP32-face forward set-up marches z (its own partial layout); the others run per plane
     if (sizeof(F) == 4 && !adjoint)
@@ -99,7 +99,8 @@ struct zq3d_adj {
     hipStream_t stream = nullptr;
     std::vector<float> boxes, spheres, boxes0, spheres0;  // *0: source values zeroed (adjoint)
     double rtol = 0.0;          // adjoint projection tolerance relative to max|rhs|; 0: match the forward
-    SorShape shape{SOR_SPLIT, 0};  // sweep algorithm of every projection (forward and adjoint)
+    QuadPlan plan{};
+    SorShape shape{0, 0};       // sweep algorithm of every projection (forward and adjoint)
     std::vector<double> fwd_rel;  // per step: forward tolerance / max|rhs| of its projection
     std::vector<void*> allocs;
     // state: u, v, w, T, rho, T2, rho2 (value type), vel4 (4-wide), scratch faces (Nu+Nv+Nw)
@@ -109,8 +110,8 @@ struct zq3d_adj {
     uint8_t* occ;
     // projection
     uint8_t* nc;
-    float *b, *p, *p_alt, *split_p, *split_b;
-    uint8_t* split_n;
+    float *b, *p, *p_alt, *quad, *split_p = nullptr, *split_b = nullptr;  // split_*: on need (ensure_split)
+    uint8_t* split_n = nullptr;
     double *b64, *p64, *p64_adj, *part;
     Scalars* sc;
     Readback rb;  // pinned read-back slots of the projections' reductions
@@ -147,12 +148,30 @@ int adj_alloc(zq3d_adj* a, void** p, size_t bytes) {
 
 ProjBufs proj_bufs(zq3d_adj* a, double* p64) {
     const size_t sp = split_padded_size(a->d), sc = split_cell_size(a->d);
-    const SplitBufs split{{a->split_p, a->split_p + sp},
+    SplitBufs split{};
+    if (a->split_n)
+        split = SplitBufs{{a->split_p, a->split_p + sp},
                           {a->split_b, a->split_b + sc},
                           {a->split_n, a->split_n + sc},
                           {a->split_p + 2 * sp, a->split_p + 3 * sp}};
     return ProjBufs{a->nc, a->b, a->p, a->p_alt, a->b64, p64, a->part, a->sc, a->shape, split, a->rb,
-                    {a->gate_ev[0], a->gate_ev[1]}};
+                    {a->gate_ev[0], a->gate_ev[1]}, quad_bufs(a->d, a->quad, a->plan)};
+}
+
+// The colour-split scratch, on first need (its padding slots must hold 0, which no sweep changes).
+int ensure_split(zq3d_adj* a, const char* where) {
+    if (a->split_n) return ZQ3D_OK;
+    uint8_t* n = nullptr;
+    if ((!a->split_p && adj_alloc(a, (void**)&a->split_p, 4 * split_padded_size(a->d) * 4)) ||
+        (!a->split_b && adj_alloc(a, (void**)&a->split_b, 2 * split_cell_size(a->d) * 4)) ||
+        adj_alloc(a, (void**)&n, 2 * split_cell_size(a->d))) {
+        set_err(where, "device allocation failed");
+        return ZQ3D_ERR_HIP;
+    }
+    launch_fill_f32(a->split_p, 4 * split_padded_size(a->d), 0.0f, a->stream);
+    ZQ_HIP(hipStreamSynchronize(a->stream), where);
+    a->split_n = n;
+    return ZQ3D_OK;
 }
 
 // pointers into one tape slot
@@ -426,6 +445,7 @@ extern "C" int zq3d_adj_create(const zq3d_config* cfg, int precision, int nsteps
     zq3d_adj* a = new zq3d_adj();
     a->cfg = *cfg;
     a->d = Dims{cfg->width, cfg->height, cfg->depth};
+    a->plan = quad_plan(a->d);
     a->prec = precision;
     a->nsteps = nsteps;
     a->K = std::min(checkpoint_every, nsteps);
@@ -442,9 +462,7 @@ extern "C" int zq3d_adj_create(const zq3d_config* cfg, int precision, int nsteps
     A(&a->u0, z.Nu * e); A(&a->v0, z.Nv * e); A(&a->w0, z.Nw * e); A(&a->T0, z.N * e); A(&a->R0, z.N * e);
     A((void**)&a->occ, z.N); A((void**)&a->nc, z.N);
     A((void**)&a->b, z.N * 4); A((void**)&a->p, z.Np * 4); A((void**)&a->p_alt, z.Np * 4);
-    A((void**)&a->split_p, 4 * split_padded_size(a->d) * 4);
-    A((void**)&a->split_b, 2 * split_cell_size(a->d) * 4);
-    A((void**)&a->split_n, 2 * split_cell_size(a->d));
+    A((void**)&a->quad, quad_cells(a->d) * 13);
     A((void**)&a->b64, z.N * 8); A((void**)&a->p64, z.Np * 8); A((void**)&a->p64_adj, z.Np * 8);
     A((void**)&a->p640, z.Np * 8);
     A((void**)&a->part, (size_t)reduction_partials(a->d) * 8);
@@ -466,6 +484,11 @@ extern "C" int zq3d_adj_create(const zq3d_config* cfg, int precision, int nsteps
         zq3d_adj_destroy(a);
         return ZQ3D_ERR_HIP;
     }
+    if (cfg->sor.pass_rule == 2)
+        if (int rc = ensure_split(a, where)) {
+            zq3d_adj_destroy(a);
+            return rc;
+        }
     hipStream_t s = nullptr;
     (void)hipMemsetAsync(a->u0, 0, z.Nu * e, s);
     (void)hipMemsetAsync(a->v0, 0, z.Nv * e, s);
@@ -475,7 +498,6 @@ extern "C" int zq3d_adj_create(const zq3d_config* cfg, int precision, int nsteps
     (void)hipMemsetAsync(a->occ, 0, z.N, s);
     (void)hipMemsetAsync(a->p, 0, z.Np * 4, s);
     (void)hipMemsetAsync(a->p_alt, 0, z.Np * 4, s);
-    (void)hipMemsetAsync(a->split_p, 0, 4 * split_padded_size(a->d) * 4, s);
     (void)hipMemsetAsync(a->p64, 0, z.Np * 8, s);
     (void)hipMemsetAsync(a->p64_adj, 0, z.Np * 8, s);
     (void)hipMemsetAsync(a->p640, 0, z.Np * 8, s);
@@ -542,12 +564,14 @@ extern "C" int zq3d_adj_set_pressure_store(zq3d_adj* a, int on) {
 extern "C" int zq3d_adj_set_sor_shape(zq3d_adj* a, int ty, int zc) {
     const char* where = "zq3d_adj_set_sor_shape";
     if (!a) { set_err(where, "null handle"); return ZQ3D_ERR_ARG; }
-    SorShape cand[ZQ3D_TUNE_MAX];
-    const int n = sor_shape_candidates(a->d, cand, ZQ3D_TUNE_MAX);
-    bool ok = false;
-    for (int i = 0; i < n; i++) ok = ok || (cand[i].ty == ty && cand[i].zc == zc);
-    if (!ok) { set_err(where, "shape not among the sweep candidates for this grid"); return ZQ3D_ERR_ARG; }
-    a->shape = SorShape{ty, zc};
+    const SorShape want{ty, zc};
+    if ((ty == 0 && zc == 0) || !sor_shape_valid(a->d, want)) {
+        set_err(where, "shape not among the sweep candidates for this grid");
+        return ZQ3D_ERR_ARG;
+    }
+    if (is_split(want))
+        if (int rc = ensure_split(a, where)) return rc;
+    a->shape = want;
     return ZQ3D_OK;
 }
 

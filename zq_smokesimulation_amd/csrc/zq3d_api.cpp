@@ -51,7 +51,7 @@ namespace {
 
 // ---------------- grow-only workspace for the host-pointer entry points ----------------
 enum Slot { S_U, S_V, S_W, S_OCC, S_T, S_R, S_T2, S_R2, S_VEL4, S_SCR, S_NC, S_B, S_P, S_P2, S_B64, S_P64, S_PART, S_SCAL,
-            S_BFECC, S_SPLIT, S_COUNT };
+            S_BFECC, S_SPLIT, S_QUAD, S_COUNT };
 
 struct Workspace {
     void* ptr[S_COUNT] = {};
@@ -222,7 +222,9 @@ int refine_mixed(const Dims& d, const zq3d_sor_opts& o, double tol, const ProjBu
         set_err(where, "pass_rule 2 needs colour-split arrays under 2 GiB (grids up to about 1000^3)");
         return ZQ3D_ERR_ARG;
     }
-    const bool split = gated || is_split(B.shape);
+    const SorShape shape = B.sweep_shape();
+    const bool quad = !gated && is_quad(shape);
+    const bool split = gated || is_split(shape);
     int pair = 0;  // split pressure pair holding the correction
     float* e = B.p;
     float* e_alt = B.p_alt;
@@ -230,7 +232,7 @@ int refine_mixed(const Dims& d, const zq3d_sor_opts& o, double tol, const ProjBu
         launch_split_counts(d, B.nc, B.split, s);
         launch_fill_f32(B.split.p[0], split_padded_size(d), 0.0f, s);
         launch_fill_f32(B.split.p[1], split_padded_size(d), 0.0f, s);
-    } else {
+    } else if (!quad) {  // the quad sweeps start from zero unread
         launch_fill_f32(e, z.Np, 0.0f, s);
     }
     int outer = 0, nprev = 0;
@@ -238,7 +240,9 @@ int refine_mixed(const Dims& d, const zq3d_sor_opts& o, double tol, const ProjBu
     bool count_pending = false;  // a gated pass ran; its count is read after the next wait
     double rmax = 0.0, rprev = -1.0, dmax = -1.0, dprev = -1.0;
     for (;;) {
-        if (split)
+        if (quad)
+            launch_residual64_quad(d, B.nc, B.b64, &sc->mean64, B.p64, B.quad, B.part, B.target(0, &sc->rmax), s);
+        else if (split)
             launch_residual64_split(d, B.nc, B.b64, &sc->mean64, B.p64, B.split, B.part, B.target(0, &sc->rmax), s);
         else
             launch_residual64(d, B.nc, B.b64, &sc->mean64, B.p64, B.b, B.part, B.target(0, &sc->rmax), s);
@@ -278,7 +282,15 @@ int refine_mixed(const Dims& d, const zq3d_sor_opts& o, double tol, const ProjBu
             continue;
         }
         const int n = fitted_pass_length(o.iters, o.pass_rule == 1, rmax, rprev, nprev, tol);
-        if (split) {
+        if (quad) {
+            hipEvent_t ea = nullptr, eb = nullptr;
+            if (pf) ZQ_HIP(pf->next(&ea, &eb), where);
+            hipError_t err = hipSuccess;
+            const int res = launch_quad_sweeps(d, B.quad, &sc->zero32, o.omega, n, shape, s, ea, eb, &err);
+            ZQ_HIP(err, where);
+            if (pf) ZQ_HIP(account_sweeps(d, shape, n, pf), where);
+            launch_update_p64_quad(d, B.nc, B.quad.p[res], B.p64, s);
+        } else if (split) {
             hipEvent_t ea = nullptr, eb = nullptr;
             if (pf) ZQ_HIP(pf->next(&ea, &eb), where);
             // the one-launch shapes start each pass from zero without reading the pair, so the update
@@ -329,19 +341,36 @@ int project_plain(const Dims& d, float* u, float* v, float* w, const uint8_t* oc
                   SorProf* pf) {
     const Sizes z(d);
     Scalars* sc = B.sc;
-    launch_fill_f32(B.p, z.Np, 0.0f, s);
-    launch_proj_setup(d, u, v, w, occ, o.open_mask, B.nc, B.b, nullptr, B.p, nullptr, mean_mode ? B.part : nullptr,
-                      s);
+    const SorShape shape = B.sweep_shape();
+    const bool quad = is_quad(shape);
+    if (quad) {
+        launch_proj_setup(d, u, v, w, occ, o.open_mask, B.nc, B.quad.b, nullptr, nullptr, nullptr,
+                          mean_mode ? B.part : nullptr, s, B.quad.n);
+    } else {
+        launch_fill_f32(B.p, z.Np, 0.0f, s);
+        launch_proj_setup(d, u, v, w, occ, o.open_mask, B.nc, B.b, nullptr, B.p, nullptr, mean_mode ? B.part : nullptr,
+                          s);
+    }
     if (mean_mode) {
         launch_mean_finalize(d, B.part, &sc->mean32, &sc->mean64, 1, s);
     } else {
         launch_fill_f32(&sc->mean32, 1, mean, s);
         launch_fill_f64(&sc->mean64, 1, (double)mean, s);
     }
-    float* res = nullptr;
-    ZQ_HIP(timed_sor(d, B.nc, B.b, &sc->mean32, B.p, B.p_alt, o.omega, o.iters, s, pf, &res, B.shape, &B.split),
-           "project");
-    launch_correct(d, occ, o.open_mask, res, u, v, w, s);
+    if (quad) {
+        hipEvent_t ea = nullptr, eb = nullptr;
+        if (pf) ZQ_HIP(pf->next(&ea, &eb), "project");
+        hipError_t err = hipSuccess;
+        const int res = launch_quad_sweeps(d, B.quad, &sc->mean32, o.omega, o.iters, shape, s, ea, eb, &err);
+        ZQ_HIP(err, "project");
+        if (pf) ZQ_HIP(account_sweeps(d, shape, o.iters, pf), "project");
+        launch_correct_quad(d, occ, o.open_mask, B.quad.p[res], u, v, w, s);
+    } else {
+        float* res = nullptr;
+        ZQ_HIP(timed_sor(d, B.nc, B.b, &sc->mean32, B.p, B.p_alt, o.omega, o.iters, s, pf, &res, B.shape, &B.split),
+               "project");
+        launch_correct(d, occ, o.open_mask, res, u, v, w, s);
+    }
     if (st) {
         launch_max_div64(d, u, v, w, B.nc, &sc->mean64, B.part, B.target(1, &sc->dmax), s);
         double md = 0.0, mean64 = 0.0;
@@ -365,7 +394,7 @@ int project_mixed(const Dims& d, float* u, float* v, float* w, const uint8_t* oc
                   const ProjBufs& B, zq3d_proj_stats* st, hipStream_t s, SorProf* pf) {
     Scalars* sc = B.sc;
     launch_fill_f32(&sc->zero32, 1, 0.0f, s);
-    launch_proj_setup(d, u, v, w, occ, o.open_mask, B.nc, nullptr, B.b64, nullptr, B.p64, B.part, s);
+    launch_proj_setup(d, u, v, w, occ, o.open_mask, B.nc, nullptr, B.b64, nullptr, B.p64, B.part, s, B.quad.n);
     launch_mean_finalize_mp(d, B.part, &sc->mean64, o.closed_mean, s);
     const DivCheck chk{u, v, w, occ, o.open_mask, false};
     RefineOut ro;
@@ -664,7 +693,7 @@ float solve_host(float* u, float* v, float* w, const bool* occupy, int W_, int H
     Timer t;
     Errs E;
     if (W.ensure(S_U, z.Nu * 4) || W.ensure(S_V, z.Nv * 4) || W.ensure(S_W, z.Nw * 4) || W.ensure(S_OCC, z.N) ||
-        W.ensure(S_NC, z.N) || W.ensure(S_B, z.N * 4) || W.ensure(S_P, z.Np * 4) || W.ensure(S_P2, z.Np * 4) ||
+        W.ensure(S_NC, z.N) || W.ensure(S_QUAD, quad_cells(d) * 13) ||
         W.ensure(S_PART, (size_t)reduction_partials(d) * 8) || W.ensure(S_SCAL, sizeof(Scalars)) ||
         (o.mixed_precision && (W.ensure(S_B64, z.N * 8) || W.ensure(S_P64, z.Np * 8)))) {
         set_err(where, "device allocation failed");
@@ -691,10 +720,9 @@ float solve_host(float* u, float* v, float* w, const bool* occupy, int W_, int H
         split = SplitBufs{{f, f + sp}, {f + 4 * sp, f + 4 * sp + sc}, {n8, n8 + sc}, {f + 2 * sp, f + 3 * sp}};
         launch_fill_f32(f, 4 * sp, 0.0f, 0);  // padding slots hold 0
     }
-    const ProjBufs B{(uint8_t*)W.ptr[S_NC],  (float*)W.ptr[S_B],      (float*)W.ptr[S_P],
-                     (float*)W.ptr[S_P2],    (double*)W.ptr[S_B64],   (double*)W.ptr[S_P64],
-                     (double*)W.ptr[S_PART], (Scalars*)W.ptr[S_SCAL], SorShape{0, 0}, split};
-    launch_fill_f32(B.p_alt, z.Np, 0.0f, 0);  // zero ghost layer of the second sweep buffer
+    ProjBufs B{(uint8_t*)W.ptr[S_NC],  nullptr, nullptr, nullptr, (double*)W.ptr[S_B64], (double*)W.ptr[S_P64],
+               (double*)W.ptr[S_PART], (Scalars*)W.ptr[S_SCAL], SorShape{0, 0}, split};
+    B.quad = quad_bufs(d, (float*)W.ptr[S_QUAD], quad_plan(d));
     int rc;
     if (o.mixed_precision) {
         launch_fill_f64(B.p64, z.Np, 0.0, 0);
@@ -792,7 +820,11 @@ struct zq3d_sim {
     float* p = nullptr;           // padded FP32 pressure / correction e of the mixed solve
     float* p_alt = nullptr;       // second sweep buffer (ping-pong), zero ghost layer
     double* part = nullptr;       // reduction partials
-    float* split_p = nullptr;     // colour-split pressures (2 pairs x 2 colours, padded), rhs, counts
+    float* quad = nullptr;        // quad-layout sweep scratch (quad_bufs)
+    QuadPlan plan{};
+    // colour-split pressures (2 pairs x 2 colours, padded), rhs, counts: allocated when a shape or a pass
+    // rule that sweeps there is chosen (ensure_split)
+    float* split_p = nullptr;
     float* split_b = nullptr;
     uint8_t* split_n = nullptr;
     double* b64 = nullptr;
@@ -838,12 +870,28 @@ int field_info(zq3d_sim* s, int field, void** ptr, size_t* bytes) {
 
 ProjBufs proj_bufs(zq3d_sim* s) {
     const size_t sp = split_padded_size(s->d), sc = split_cell_size(s->d);
-    const SplitBufs split{{s->split_p, s->split_p + sp},
+    SplitBufs split{};
+    if (s->split_n)
+        split = SplitBufs{{s->split_p, s->split_p + sp},
                           {s->split_b, s->split_b + sc},
                           {s->split_n, s->split_n + sc},
                           {s->split_p + 2 * sp, s->split_p + 3 * sp}};
     return ProjBufs{s->nc, s->b, s->p, s->p_alt, s->b64, s->p64, s->part, s->sc, s->shape, split, s->rb,
-                    {s->gate_ev[0], s->gate_ev[1]}};
+                    {s->gate_ev[0], s->gate_ev[1]}, quad_bufs(s->d, s->quad, s->plan)};
+}
+
+// The colour-split scratch, on first need (its padding slots must hold 0, which no sweep changes).
+int ensure_split(zq3d_sim* s, const char* where) {
+    if (s->split_n) return ZQ3D_OK;
+    const size_t sp = 4 * split_padded_size(s->d) * 4, sc = 2 * split_cell_size(s->d);
+    uint8_t* n = nullptr;
+    if (!s->split_p) ZQ_HIP(dalloc(&s->split_p, sp), where);
+    if (!s->split_b) ZQ_HIP(dalloc(&s->split_b, sc * 4), where);
+    ZQ_HIP(dalloc(&n, sc), where);
+    launch_fill_f32(s->split_p, sp / 4, 0.0f, s->stream);
+    ZQ_HIP(hipStreamSynchronize(s->stream), where);
+    s->split_n = n;
+    return ZQ3D_OK;
 }
 
 // Times one stage of a simulation with an event pair when profiling is on.
@@ -958,6 +1006,7 @@ extern "C" int zq3d_create(const zq3d_config* cfg, zq3d_sim** out) {
     zq3d_sim* s = new zq3d_sim();
     s->cfg = *cfg;
     s->d = Dims{cfg->width, cfg->height, cfg->depth};
+    s->plan = quad_plan(s->d);
     const Sizes z(s->d);
     hipError_t e = hipSuccess;
     auto A = [&](hipError_t r) { if (e == hipSuccess) e = r; };
@@ -976,9 +1025,7 @@ extern "C" int zq3d_create(const zq3d_config* cfg, zq3d_sim** out) {
     A(dalloc(&s->p, z.Np * 4));
     A(dalloc(&s->p_alt, z.Np * 4));
     A(dalloc(&s->part, (size_t)reduction_partials(s->d) * 8));
-    A(dalloc(&s->split_p, 4 * split_padded_size(s->d) * 4));
-    A(dalloc(&s->split_b, 2 * split_cell_size(s->d) * 4));
-    A(dalloc(&s->split_n, 2 * split_cell_size(s->d)));
+    A(dalloc(&s->quad, quad_cells(s->d) * 13));
     A(dalloc(&s->sc, sizeof(Scalars)));
     A(s->rb.alloc());
     A(hipEventCreateWithFlags(&s->gate_ev[0], hipEventDisableTiming));
@@ -1017,8 +1064,12 @@ extern "C" int zq3d_create(const zq3d_config* cfg, zq3d_sim** out) {
     launch_fill_u8(s->occ, z.N, 0, st);
     launch_fill_f32(s->p, z.Np, 0.0f, st);
     launch_fill_f32(s->p_alt, z.Np, 0.0f, st);
-    launch_fill_f32(s->split_p, 4 * split_padded_size(s->d), 0.0f, st);
     if (s->p64) launch_fill_f64(s->p64, z.Np, 0.0, st);
+    if (cfg->sor.pass_rule == 2)
+        if (int rc = ensure_split(s, where)) {
+            zq3d_destroy(s);
+            return rc;
+        }
     e = hipStreamSynchronize(st);
     if (e != hipSuccess) {
         set_err(where, hipGetErrorString(e));
@@ -1032,7 +1083,7 @@ extern "C" int zq3d_create(const zq3d_config* cfg, zq3d_sim** out) {
 extern "C" void zq3d_destroy(zq3d_sim* s) {
     if (!s) return;
     void* ptrs[] = {s->u, s->v, s->w, s->T, s->R, s->T2, s->R2, s->occ, s->vel4, s->scratch, s->bfecc, s->nc, s->b, s->p, s->p_alt, s->part,
-                    s->split_p, s->split_b, s->split_n,
+                    s->quad, s->split_p, s->split_b, s->split_n,
                     s->b64, s->p64, s->p64_prev, s->sc};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -1267,12 +1318,11 @@ extern "C" int zq3d_set_profiling(zq3d_sim* s, int on) {
 
 extern "C" int zq3d_set_sor_shape(zq3d_sim* s, int ty, int zc) {
     if (!s || zc < 0) { set_err("zq3d_set_sor_shape", "bad argument"); return ZQ3D_ERR_ARG; }
-    SorShape cand[32];
-    const int n = sor_shape_candidates(s->d, cand, 32);
-    bool ok = (ty == 0 && zc == 0);
-    for (int i = 0; i < n && !ok; i++) ok = cand[i].ty == ty && cand[i].zc == zc;
-    if (!ok) { set_err("zq3d_set_sor_shape", "shape not supported for this grid"); return ZQ3D_ERR_ARG; }
-    s->shape = SorShape{ty, zc};
+    const SorShape want{ty, zc};
+    if (!sor_shape_valid(s->d, want)) { set_err("zq3d_set_sor_shape", "shape not supported for this grid"); return ZQ3D_ERR_ARG; }
+    if (is_split(want))
+        if (int rc = ensure_split(s, "zq3d_set_sor_shape")) return rc;
+    s->shape = want;
     return ZQ3D_OK;
 }
 
@@ -1293,19 +1343,30 @@ extern "C" int zq3d_autotune_sor(zq3d_sim* s, int iters, zq3d_tune_report* rep) 
     hipEvent_t a = nullptr, b = nullptr;
     ZQ_HIP(hipEventCreate(&a), where);
     ZQ_HIP(hipEventCreate(&b), where);
+    if (int rc = ensure_split(s, where)) return rc;
+    const ProjBufs B = proj_bufs(s);
     launch_fill_f32(&s->sc->mean32, 1, 0.0f, s->stream);
+    launch_proj_setup(s->d, s->u, s->v, s->w, s->occ, s->cfg.sor.open_mask, s->nc, B.quad.b, nullptr, nullptr, nullptr,
+                      nullptr, s->stream, B.quad.n);
     launch_proj_setup(s->d, s->u, s->v, s->w, s->occ, s->cfg.sor.open_mask, s->nc, s->b, nullptr, s->p, nullptr,
                       nullptr, s->stream);
     int best = -1;
     float best_us = 0.0f;
     Errs E;
-    const ProjBufs B = proj_bufs(s);
+    // the events bracket the sweeps only (not the split-layout conversions)
+    auto sweeps = [&](SorShape sh, int n, hipEvent_t ea, hipEvent_t eb) {
+        if (is_quad(sh)) {
+            hipError_t err = hipSuccess;
+            launch_quad_sweeps(s->d, B.quad, &s->sc->mean32, 1.8f, n, sh, s->stream, ea, eb, &err);
+            E(err);
+        } else {
+            launch_sor(s->d, s->nc, s->b, &s->sc->mean32, s->p, s->p_alt, 1.8f, n, s->stream, sh, &B.split, ea, eb);
+        }
+    };
     for (int i = 0; i < n; i++) {
         launch_fill_f32(s->p, z.Np, 0.0f, s->stream);
-        launch_sor(s->d, s->nc, s->b, &s->sc->mean32, s->p, s->p_alt, 1.8f, 2, s->stream, cand[i], &B.split);
-        // the events bracket the sweeps only (not the split-layout conversions)
-        launch_sor(s->d, s->nc, s->b, &s->sc->mean32, s->p, s->p_alt, 1.8f, iters, s->stream, cand[i], &B.split, a,
-                   b);
+        sweeps(cand[i], 2, nullptr, nullptr);
+        sweeps(cand[i], iters, a, b);
         E(hipGetLastError());
         E(hipEventSynchronize(b));
         float ms = 0.0f;

@@ -139,13 +139,16 @@ struct ProjBufs {
     SplitBufs split; // colour-split scratch (used when shape.ty == SOR_SPLIT)
     Readback rb{};   // host read-back slots (optional)
     hipEvent_t gate_ev[2] = {nullptr, nullptr};  // progress checks of a gated pass (optional)
+    QuadBufs quad{};  // quad-layout scratch (optional; the {0, 0} shape then sweeps there)
+    // the shape the sweeps run: {0, 0} is the quad default where there is quad scratch
+    SorShape sweep_shape() const { return shape.ty == 0 && shape.zc == 0 && quad.n ? quad.plan.def : shape; }
     // where a reduction result of `slot` goes: the pinned slot, or the device scalar
     unsigned long long* target(int slot, unsigned long long* dev_scalar) const {
         return rb.dev ? rb.dev + slot : dev_scalar;
     }
     // the gate words of a gated pass; the executed count goes to pinned slot 2 when there is one
     GateBufs gate() const { return GateBufs{sc->gate, &sc->done, rb.dev ? rb.dev + 2 : &sc->done_sink}; }
-    // split storage present (the gated passes need it)
+    // split storage present (the gated passes and the split shapes need it)
     bool has_split() const { return split.p[0] && split.p[1] && split.alt[0] && split.alt[1] && split.b[0]; }
 };
 

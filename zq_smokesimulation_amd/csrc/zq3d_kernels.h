@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "zq3d_device.h"
+#include "zq3d_quad_cut.h"
 
 namespace zq3d {
 
@@ -61,18 +62,20 @@ void launch_advect_scalar(const Dims& d, const R* u, const R* v, const R* w, con
 // Doubles needed by the reduction partials of a grid (per-block sums / maxima).
 int reduction_partials(const Dims& d);
 // Neighbour counts, FP32 divergence b (or FP64 b64), zero p at uncounted cells; when part is given,
-// per-block FP64 sum/count of the divergence over fluid cells (closed-domain mean).
+// per-block FP64 sum/count of the divergence over fluid cells (closed-domain mean).  With nq the counts
+// also go to the quad layout, and the FP32 divergence goes there (b: quad layout) instead; p_pad is not written.
 void launch_proj_setup(const Dims& d, const float* u, const float* v, const float* w, const uint8_t* occ,
                        int open_mask, uint8_t* nc, float* b, double* b64, float* p_pad, double* p64_pad,
-                       double* part, hipStream_t s);
+                       double* part, hipStream_t s, uint8_t* nq = nullptr);
 // FP64 variant on FP64 faces (always b64/p64); free_only != 0 sums only the faces the correction
 // updates (between two fluid cells, and open domain faces): the right-hand side of the adjoint.
 void launch_proj_setup64(const Dims& d, const double* u, const double* v, const double* w, const uint8_t* occ,
                          int open_mask, int free_only, uint8_t* nc, double* b64, double* p64_pad, double* part,
-                         hipStream_t s);
+                         hipStream_t s, uint8_t* nq = nullptr);
 // FP32-face variant of the adjoint right-hand side (free faces only) into b64
 void launch_proj_setup_free(const Dims& d, const float* u, const float* v, const float* w, const uint8_t* occ,
-                            int open_mask, uint8_t* nc, double* b64, double* p64_pad, double* part, hipStream_t s);
+                            int open_mask, uint8_t* nc, double* b64, double* p64_pad, double* part, hipStream_t s,
+                            uint8_t* nq = nullptr);
 // mean32/mean64 = sum/count of the setup partials (0 when want == 0)
 void launch_mean_finalize(const Dims& d, const double* part, float* mean32, double* mean64, int want, hipStream_t s);
 // the same fold over the mixed-precision set-up's partials (launch_proj_setup with b64)
@@ -86,7 +89,11 @@ constexpr int SOR_TWO = 100;  // ty == -(SOR_TWO + r), r = 16 or 32: two iterati
 struct SorShape {
     int ty, zc;
 };
-inline bool is_split(SorShape s) { return s.ty <= SOR_SPLIT; }
+// ty == -(SOR_QUAD + 100 cx + nw): two iterations per launch on the quad layout (zq3d_sor_quad.h), cx (2 or 4)
+// cells a lane, tiles of nw waves (1 to 16; with cx 4 up to 8) and zc planes (even)
+constexpr int SOR_QUAD = 1000;
+inline bool is_quad(SorShape s) { return s.ty <= -SOR_QUAD; }
+inline bool is_split(SorShape s) { return s.ty <= SOR_SPLIT && !is_quad(s); }
 // the one-launch split shapes, whose first iteration can take the source pair as zeros unread
 inline bool split_zero_start(SorShape s) { return s.ty < SOR_SPLIT && s.ty > -SOR_TWO; }
 // whether the one-launch split kernels (buffer access with 32-bit offsets) can run on the grid: every
@@ -101,6 +108,38 @@ struct SplitBufs {
     uint8_t* n[2];
     float* alt[2];
 };
+// Quad-layout scratch: two pressures the sweeps ping-pong between, right-hand side, counts (quad_cells
+// values each).  The sweeps start from zero and write every value they read later, so the pressures need
+// no initialisation; the counts' padding is cleared by the projection set-up.
+// A grid's sweep plan: the shape {0, 0} stands for, and the cut of a launch of one iteration (the odd one).
+struct QuadPlan {
+    SorShape def;
+    QuadCut one;
+};
+QuadPlan quad_plan(const Dims& d);
+struct QuadBufs {
+    float* p[2];
+    float* b;
+    uint8_t* n;
+    QuadPlan plan;
+};
+size_t quad_cells(const Dims& d);
+// the arrays in one allocation of 13 quad_cells(d) bytes (null: none)
+inline QuadBufs quad_bufs(const Dims& d, float* mem, const QuadPlan& plan) {
+    const size_t n = quad_cells(d);
+    if (!mem) return QuadBufs{};
+    return QuadBufs{{mem, mem + n}, mem + 2 * n, (uint8_t*)(mem + 3 * n), plan};
+}
+bool quad_shape_valid(const Dims& d, SorShape s);
+// iters red-black iterations from zero; returns the pressure holding the result
+int launch_quad_sweeps(const Dims& d, const QuadBufs& q, const float* mean32, float omega, int iters, SorShape shape,
+                       hipStream_t s, hipEvent_t ev_begin, hipEvent_t ev_end, hipError_t* err);
+void launch_correct_quad(const Dims& d, const uint8_t* occ, int open_mask, const float* p_quad, float* u, float* v,
+                         float* w, hipStream_t s);
+void launch_residual64_quad(const Dims& d, const uint8_t* nc, const double* b64, const double* mean64,
+                            const double* p64_pad, const QuadBufs& q, double* part, unsigned long long* rmax,
+                            hipStream_t s);
+void launch_update_p64_quad(const Dims& d, const uint8_t* nc, const float* e_quad, double* p64_pad, hipStream_t s);
 // Gated passes (zq3d_sor_opts.pass_rule 2): per-iteration largest-update words, the executed
 // iteration count, and the mapped host word the count is copied to.
 constexpr int GATE_SLOTS = 8192;  // iterations per gated pass at most
@@ -144,7 +183,9 @@ void launch_split_counts(const Dims& d, const uint8_t* nc, const SplitBufs& sp, 
 const char* sor_kernel_name(const Dims& d, SorShape shape);
 // sweep-kernel launches of `iters` SOR iterations
 long long sor_launches(const Dims& d, SorShape shape, int iters);
-// fused-kernel shapes valid for this grid (LDS ring within 64 KiB); returns the count
+// whether a sweep shape can run on the grid ({0, 0} always)
+bool sor_shape_valid(const Dims& d, SorShape shape);
+// the shapes the autotuner times on this grid; returns the count
 int sor_shape_candidates(const Dims& d, SorShape* out, int max);
 void launch_correct(const Dims& d, const uint8_t* occ, int open_mask, const float* p_pad, float* u, float* v,
                     float* w, hipStream_t s);

@@ -8,6 +8,7 @@
 #pragma once
 
 #include "zq3d_device.h"
+#include "zq3d_quad_cut.h"
 
 namespace zq3d {
 
@@ -352,6 +353,17 @@ __device__ __forceinline__ float rcp_count(int n) {
                                                                                             : (1.0f / 6.0f);
 }
 
+// A cell's count in the quad layout (the byte offset 4 n of 1/n in the sweep's table; the row's last
+// cell also clears the padding) and its index there.
+__device__ __forceinline__ int st_quad_count(uint8_t* __restrict__ nq, const Dims& d, int i, int j, int k, int n) {
+    const int S = quad_stride(d.W);
+    const int o = (k * d.H + j) * S + i;
+    nq[o] = (uint8_t)(4 * n);
+    if (i == d.W - 1)
+        for (int x = d.W; x < S; x++) nq[o + x - i] = 0;
+    return o;
+}
+
 // Plain (FP32) projection set-up of one cell: neighbour count, divergence (the reference's unscaled
 // sum, ZQ_SmokeSimulationUtils3D.cpp:2403-2405, left to right), p = 0 at uncounted cells; the
 // cell's divergence and count for the closed-domain mean go to dsum/dcnt.
@@ -359,7 +371,7 @@ __device__ __forceinline__ void st_proj_setup_plain(const float* __restrict__ u,
                                                     const float* __restrict__ w, const uint8_t* __restrict__ occ,
                                                     int open_mask, uint8_t* __restrict__ nc, float* __restrict__ b,
                                                     float* __restrict__ p, const Dims& d, int i, int j, int k,
-                                                    double& dsum, double& dcnt) {
+                                                    double& dsum, double& dcnt, uint8_t* __restrict__ nq = nullptr) {
     if (i >= d.W || j >= d.H || k >= d.D) return;
     const int o = cidx(d, i, j, k);
     const int HW = d.W * d.H;
@@ -378,8 +390,12 @@ __device__ __forceinline__ void st_proj_setup_plain(const float* __restrict__ u,
     const float v0 = v[vidx(d, i, j, k)], v1 = v[vidx(d, i, j + 1, k)];
     const float w0 = w[widx(d, i, j, k)], w1 = w[widx(d, i, j, k + 1)];
     const float dv = u1 - u0 + v1 - v0 + w1 - w0;
-    b[o] = fluid ? dv : 0.0f;
-    if (!n) p[pidx(d, i, j, k)] = 0.0f;
+    if (nq) {  // counts and right-hand side in the quad layout (no pressure: its sweeps start from zero)
+        b[st_quad_count(nq, d, i, j, k, n)] = fluid ? dv : 0.0f;
+    } else {
+        b[o] = fluid ? dv : 0.0f;
+        if (!n) p[pidx(d, i, j, k)] = 0.0f;
+    }
     if (fluid) {
         dsum = (double)dv;
         dcnt = 1.0;
@@ -404,18 +420,49 @@ __device__ __forceinline__ void st_sor_half(const uint8_t* __restrict__ nc, cons
     p[q] = omw * p[q] + omega * pg;
 }
 
+// Pressures on the two sides of face (AXIS, i, j, k): the cell on the high side and the one below it
+// along the axis.  PadPressure: an array with a ghost layer (every index in range).  QuadPressure: the
+// quad layout, without ghosts (0 outside the grid).
+template <class P>
+struct PadPressure {
+    using type = P;
+    const P* p;
+    template <int AXIS>
+    __device__ __forceinline__ void sides(const Dims& d, int i, int j, int k, P& hi, P& lo) const {
+        const int pstep = AXIS == 0 ? 1 : (AXIS == 1 ? d.W + 2 : (d.W + 2) * (d.H + 2));
+        const int q = pidx(d, i, j, k);
+        hi = p[q];
+        lo = p[q - pstep];
+    }
+};
+struct QuadPressure {
+    using type = float;
+    const float* p;
+    template <int AXIS>
+    __device__ __forceinline__ void sides(const Dims& d, int i, int j, int k, float& hi, float& lo) const {
+        const int S = quad_stride(d.W);
+        const int step = AXIS == 0 ? 1 : (AXIS == 1 ? S : S * d.H);
+        const int pos = AXIS == 0 ? i : (AXIS == 1 ? j : k);
+        const int lim = AXIS == 0 ? d.W : (AXIS == 1 ? d.H : d.D);
+        const int q = (k * d.H + j) * S + i;
+        const float h = p[pos < lim ? q : q - step], l = p[pos > 0 ? q - step : q];
+        hi = pos < lim ? h : 0.0f;
+        lo = pos > 0 ? l : 0.0f;
+    }
+};
+
 // Face correction u -= p_r - p_l (ZQ_SmokeSimulationUtils3D.cpp:2815-2861 open form, :2888-2922
-// closed form).  P = float (plain) or double (mixed precision; the face is rounded once).
+// closed form).  Pressure = float (plain) or double (mixed precision; the face is rounded once).
 // st_corrected_face returns the value face (AXIS, i, j, k) holds after the correction (its own value
 // when the face is not corrected): st_correct stores it, and the mixed projection's divergence check
 // predicts the corrected field's divergence from it before anything is stored.
-template <int AXIS, class P, class F>
-__device__ __forceinline__ F st_corrected_face(const uint8_t* __restrict__ occ, int open_mask, const P* __restrict__ p,
+template <int AXIS, class PA, class F>
+__device__ __forceinline__ F st_corrected_face(const uint8_t* __restrict__ occ, int open_mask, const PA& p,
                                                const F* __restrict__ face, const Dims& d, int i, int j, int k) {
+    using P = typename PA::type;
     const int pos = AXIS == 0 ? i : (AXIS == 1 ? j : k);
     const int lim = AXIS == 0 ? d.W : (AXIS == 1 ? d.H : d.D);
     const int step = AXIS == 0 ? 1 : (AXIS == 1 ? d.W : d.W * d.H);
-    const int pstep = AXIS == 0 ? 1 : (AXIS == 1 ? d.W + 2 : (d.W + 2) * (d.H + 2));
     const int lo_bit = AXIS == 0 ? 1 : (AXIS == 1 ? 4 : 16);
     const int ci = face_cell<AXIS>(d, i, j, k);
     const int oh = occ[ci], ol = occ[(pos > 0 && pos < lim) ? ci - step : ci];  // as in st_force_face
@@ -424,19 +471,18 @@ __device__ __forceinline__ F st_corrected_face(const uint8_t* __restrict__ occ, 
     else if (pos == lim) ok = (open_mask & (lo_bit << 1)) && !oh;
     else ok = !ol && !oh;
     const F f = face[face_index<AXIS>(d, i, j, k)];
-    // padded index of the cell on the high side of the face (ghost when pos == lim); both pressures
-    // are loaded with the occupancy (every padded index is in range), not after the test
-    const int qh = pidx(d, i, j, k);
-    const P ph = p[qh], pl = p[qh - pstep];
+    // both pressures are loaded with the occupancy, not after the test
+    P ph, pl;
+    p.template sides<AXIS>(d, i, j, k, ph, pl);
     if (!ok) return f;
     return (F)((P)f - (ph - pl));
 }
 
-template <int AXIS, class P, class F>
-__device__ __forceinline__ void st_correct(const uint8_t* __restrict__ occ, int open_mask, const P* __restrict__ p,
+template <int AXIS, class PA, class F>
+__device__ __forceinline__ void st_correct(const uint8_t* __restrict__ occ, int open_mask, const PA& p,
                                            F* __restrict__ face, const Dims& d, int i, int j, int k) {
     if (!face_in<AXIS>(d, i, j, k)) return;
-    face[face_index<AXIS>(d, i, j, k)] = st_corrected_face<AXIS, P, F>(occ, open_mask, p, face, d, i, j, k);
+    face[face_index<AXIS>(d, i, j, k)] = st_corrected_face<AXIS, PA, F>(occ, open_mask, p, face, d, i, j, k);
 }
 
 // ---- sources ----
