@@ -38,20 +38,19 @@ __global__ __launch_bounds__(BX* BY) void k_advect_cells(const vec4_t<R>* __rest
 }
 
 // The three face grids from the advected cells in one launch: thread (i, j) walks a chunk of
-// APPLY_RZ planes and writes each cell's low u, v and w faces (the last column / row / plane also the
+// rz planes and writes each cell's low u, v and w faces (the last column / row / plane also the
 // domain's high face), every face with st_cells_to_face's value.  The w face below plane k reads the
 // cell of plane k-1 that the same thread read one iteration earlier.
-constexpr int APPLY_RZ = 16;
 template <class R>
 __global__ __launch_bounds__(BX* BY) void k_cells_to_faces_apply(const R* __restrict__ adv,
                                                                  const uint8_t* __restrict__ occ, R* __restrict__ u,
                                                                  R* __restrict__ v, R* __restrict__ w, Dims d,
-                                                                 int is_open) {
+                                                                 int is_open, int rz) {
     const int i = blockIdx.x * BX + threadIdx.x;
     const int j = blockIdx.y * BY + threadIdx.y;
     if (i >= d.W || j >= d.H) return;
-    const int k1 = min((int)(blockIdx.z + 1) * APPLY_RZ, d.D);
-    for (int k = blockIdx.z * APPLY_RZ; k < k1; k++) {
+    const int k1 = min((int)(blockIdx.z + 1) * rz, d.D);
+    for (int k = blockIdx.z * rz; k < k1; k++) {
         st_cells_to_face<R, 0>(adv, occ, u, d, is_open, i, j, k);
         if (i == d.W - 1) st_cells_to_face<R, 0>(adv, occ, u, d, is_open, i + 1, j, k);
         st_cells_to_face<R, 1>(adv, occ, v, d, is_open, i, j, k);
@@ -64,8 +63,9 @@ __global__ __launch_bounds__(BX* BY) void k_cells_to_faces_apply(const R* __rest
 template <class R>
 void launch_cells_to_faces_apply(const Dims& d, const R* adv, const uint8_t* occ, R* u, R* v, R* w, int is_open,
                                  hipStream_t s) {
-    hipLaunchKernelGGL(k_cells_to_faces_apply<R>, grid_for(d.W, d.H, (d.D + APPLY_RZ - 1) / APPLY_RZ), dim3(BX, BY),
-                       0, s, adv, occ, u, v, w, d, is_open);
+    const int rz = march_planes(d);
+    hipLaunchKernelGGL(k_cells_to_faces_apply<R>, grid_for(d.W, d.H, (d.D + rz - 1) / rz), dim3(BX, BY), 0, s, adv, occ,
+                       u, v, w, d, is_open, rz);
 }
 
 // Advect_Velocity_inRegular_outMAC_* (:115-230) and inMAC_outMAC_* (:232-377): backtrace from the

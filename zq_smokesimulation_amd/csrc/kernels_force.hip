@@ -34,20 +34,19 @@ __global__ __launch_bounds__(BX* BY) void k_force_cells(VI vort, R* __restrict__
                                  blockIdx.x * BX + threadIdx.x, blockIdx.y * BY + threadIdx.y, blockIdx.z);
 }
 
-// All three face grids in one launch: thread (i, j) walks a chunk of FACE_RZ planes and updates each
+// All three face grids in one launch: thread (i, j) walks a chunk of rz planes and updates each
 // cell's low u, v and w faces (the last column / row / plane also the domain's high face) with
 // st_force_face.  The w face below plane k reads the force and occupancy of plane k-1, which the
 // same thread read one iteration earlier.
-constexpr int FACE_RZ = 16;
 template <class R, bool ATTEN>
 __global__ __launch_bounds__(BX* BY) void k_force_faces(R* __restrict__ u, R* __restrict__ v, R* __restrict__ w,
                                                         const uint8_t* __restrict__ occ, const R* __restrict__ fc,
-                                                        Dims d, R dt, R dth, R aV) {
+                                                        Dims d, R dt, R dth, R aV, int rz) {
     const int i = blockIdx.x * BX + threadIdx.x;
     const int j = blockIdx.y * BY + threadIdx.y;
     if (i >= d.W || j >= d.H) return;
-    const int k1 = min((int)(blockIdx.z + 1) * FACE_RZ, d.D);
-    for (int k = blockIdx.z * FACE_RZ; k < k1; k++) {
+    const int k1 = min((int)(blockIdx.z + 1) * rz, d.D);
+    for (int k = blockIdx.z * rz; k < k1; k++) {
         st_force_face<R, 0, ATTEN>(u, occ, fc, d, dt, dth, aV, i, j, k);
         if (i == d.W - 1) st_force_face<R, 0, ATTEN>(u, occ, fc, d, dt, dth, aV, i + 1, j, k);
         st_force_face<R, 1, ATTEN>(v, occ, fc, d, dt, dth, aV, i, j, k);
@@ -91,8 +90,9 @@ inline dim3 grid_for(int nx, int ny, int nz) { return dim3((nx + BX - 1) / BX, (
 template <class R, bool ATTEN>
 void force_faces(const Dims& d, R* u, R* v, R* w, const uint8_t* occ, const R* fcell, R dt, R dth, R aV,
                  hipStream_t s) {
-    hipLaunchKernelGGL((k_force_faces<R, ATTEN>), grid_for(d.W, d.H, (d.D + FACE_RZ - 1) / FACE_RZ), dim3(BX, BY, 1),
-                       0, s, u, v, w, occ, fcell, d, dt, dth, aV);
+    const int rz = march_planes(d);
+    hipLaunchKernelGGL((k_force_faces<R, ATTEN>), grid_for(d.W, d.H, (d.D + rz - 1) / rz), dim3(BX, BY, 1), 0, s, u, v,
+                       w, occ, fcell, d, dt, dth, aV, rz);
 }
 
 }  // namespace

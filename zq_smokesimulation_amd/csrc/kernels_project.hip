@@ -23,11 +23,12 @@ namespace zq3d {
 namespace {
 
 constexpr int BX = 64, BY = 4;
-// planes per thread of the z-marching kernels (each thread owns one (i, j) column of a chunk)
-constexpr int RES_RZ = 16;
-
 inline dim3 grid_for(int nx, int ny, int nz) { return dim3((nx + BX - 1) / BX, (ny + BY - 1) / BY, nz); }
-inline dim3 grid_z(const Dims& d) { return grid_for(d.W, d.H, (d.D + RES_RZ - 1) / RES_RZ); }
+// chunks of march_planes(d) planes for the z-marching kernels (each thread owns one (i, j) column of a chunk)
+inline dim3 grid_z(const Dims& d) {
+    const int rz = march_planes(d);
+    return grid_for(d.W, d.H, (d.D + rz - 1) / rz);
+}
 
 __device__ __forceinline__ int block_linear() { return (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x; }
 
@@ -59,21 +60,21 @@ __global__ __launch_bounds__(BX* BY) void k_proj_setup(const float* __restrict__
 
 // The mixed-precision set-up: neighbour counts, FP64 divergence b64 (the same sum as the plain
 // set-up, in double), p64 = 0 where the count is 0, per-block FP64 sum/count of the divergence over
-// fluid cells.  One (i, j) column per thread up a chunk of RES_RZ planes: the occupancy of planes
+// fluid cells.  One (i, j) column per thread up a chunk of rz planes: the occupancy of planes
 // k-1, k, k+1 and the w face between planes stay in registers, so every input is read once.
 __global__ __launch_bounds__(BX* BY) void k_proj_setup_z(const float* __restrict__ u, const float* __restrict__ v,
                                                          const float* __restrict__ w, const uint8_t* __restrict__ occ,
                                                          int open_mask, uint8_t* __restrict__ nc,
                                                          double* __restrict__ b64, double* __restrict__ p64,
                                                          double* __restrict__ part, Dims d,
-                                                         uint8_t* __restrict__ nq) {
+                                                         uint8_t* __restrict__ nq, int rz) {
     __shared__ double red[4];
     const int i = blockIdx.x * BX + threadIdx.x;
     const int j = blockIdx.y * BY + threadIdx.y;
     double dsum = 0.0, dcnt = 0.0;
     if (i < d.W && j < d.H) {
         const int HW = d.W * d.H;
-        const int k0 = blockIdx.z * RES_RZ, k1 = min(k0 + RES_RZ, d.D);
+        const int k0 = blockIdx.z * rz, k1 = min(k0 + rz, d.D);
         int o = cidx(d, i, j, k0);
         int ob = k0 > 0 ? occ[o - HW] : 1;  // plane below (not read at k = 0)
         int oc = occ[o];
@@ -130,9 +131,12 @@ __global__ __launch_bounds__(1024) void k_finish_mean(const double* __restrict__
     st_fold_mean(part, nblocks, mean32, mean64, want, ss, sc);
 }
 
-// Fold per-block maxima; the result is stored as the bit pattern of a non-negative double.
+// Fold per-block maxima; the result is stored as the bit pattern of a non-negative double.  mean (nullable)
+// is passed on to mean_out: the host reads both results after one wait.
 __global__ __launch_bounds__(1024) void k_finish_max(const double* __restrict__ part, int nblocks,
-                                                     unsigned long long* __restrict__ out) {
+                                                     unsigned long long* __restrict__ out,
+                                                     const double* __restrict__ mean = nullptr,
+                                                     unsigned long long* __restrict__ mean_out = nullptr) {
     __shared__ double sm[1024];
     const int t = threadIdx.x;
     double m = 0.0;
@@ -143,7 +147,10 @@ __global__ __launch_bounds__(1024) void k_finish_max(const double* __restrict__ 
         if (t < h) sm[t] = fmax(sm[t], sm[t + h]);
         __syncthreads();
     }
-    if (t == 0) *out = (unsigned long long)__double_as_longlong(sm[0]);
+    if (t == 0) {
+        *out = (unsigned long long)__double_as_longlong(sm[0]);
+        if (mean_out) *mean_out = (unsigned long long)__double_as_longlong(*mean);
+    }
 }
 
 // One colour of a red-black SOR iteration, in place.  Thread (t, j, k) owns cell
@@ -557,15 +564,15 @@ __global__ __launch_bounds__(64 * NW) void k_sor_split_rb2(const uint8_t* __rest
 template <class PA, class F>
 __global__ __launch_bounds__(BX* BY) void k_correct_cells(const uint8_t* __restrict__ occ, int open_mask,
                                                           PA p, F* __restrict__ u,
-                                                          F* __restrict__ v, F* __restrict__ w, Dims d) {
+                                                          F* __restrict__ v, F* __restrict__ w, Dims d, int rz) {
     const int i = blockIdx.x * BX + threadIdx.x;
     const int j = blockIdx.y * BY + threadIdx.y;
     if (i >= d.W || j >= d.H) return;
     // the column marches up its chunk: the w face below plane k reads plane k-1's pressure and
     // occupancy, which this thread loaded for its u face one iteration earlier (a cache hit, not a
     // second trip to HBM as when neighbouring planes belong to other workgroups)
-    const int k1 = min((int)(blockIdx.z + 1) * RES_RZ, d.D);
-    for (int k = blockIdx.z * RES_RZ; k < k1; k++) {
+    const int k1 = min((int)(blockIdx.z + 1) * rz, d.D);
+    for (int k = blockIdx.z * rz; k < k1; k++) {
         st_correct<0, PA, F>(occ, open_mask, p, u, d, i, j, k);
         if (i == d.W - 1) st_correct<0, PA, F>(occ, open_mask, p, u, d, i + 1, j, k);
         st_correct<1, PA, F>(occ, open_mask, p, v, d, i, j, k);
@@ -731,7 +738,7 @@ __global__ __launch_bounds__(BX* BY) void k_residual64(const uint8_t* __restrict
     if (threadIdx.x == 0 && threadIdx.y == 0) part[block_linear()] = m;
 }
 
-// k_residual64 marching z (QUAD: r32 into the quad layout's right-hand side r0, else into the split ones): each thread owns one (i, j) column of a chunk of RES_RZ planes and
+// k_residual64 marching z (QUAD: r32 into the quad layout's right-hand side r0, else into the split ones): each thread owns one (i, j) column of a chunk of rz planes and
 // keeps the pressures of planes k-1, k, k+1 in registers, so each padded FP64 pressure is read once
 // (the per-plane kernel reads every plane for three neighbouring planes' blocks).  The same operations
 // per cell in the same order; the block maxima are over the chunk (a maximum is order-free).
@@ -740,11 +747,11 @@ __global__ __launch_bounds__(BX* BY) void k_residual64_z(const uint8_t* __restri
                                                          const double* __restrict__ mean64,
                                                          const double* __restrict__ p, float* __restrict__ r0,
                                                          float* __restrict__ r1, double* __restrict__ part, Dims d,
-                                                         int Wh) {
+                                                         int Wh, int rz) {
     __shared__ double red[4];
     const int i = blockIdx.x * BX + threadIdx.x;
     const int j = blockIdx.y * BY + threadIdx.y;
-    const int k0 = blockIdx.z * RES_RZ, k1 = min(k0 + RES_RZ, d.D);
+    const int k0 = blockIdx.z * rz, k1 = min(k0 + rz, d.D);
     double m = 0.0;
     if (i < d.W && j < d.H) {
         const int sy = d.W + 2, sz = (d.W + 2) * (d.H + 2);
@@ -848,7 +855,7 @@ __device__ __forceinline__ F pred_face(F f, bool ok, double ph, double pl) {
     return ok ? (F)((double)f - (ph - pl)) : f;
 }
 
-// One (i, j) column per thread up a chunk of RES_RZ planes.  Per plane a thread evaluates three
+// One (i, j) column per thread up a chunk of rz planes.  Per plane a thread evaluates three
 // faces of its cell, the low u and v faces and the high w face; the high u face comes from the
 // next lane (the lane at a block's or the grid's edge evaluates it), the high v face from the
 // next row through LDS (likewise), the low w face is the plane below's high w face.  Every face
@@ -860,14 +867,14 @@ __global__ __launch_bounds__(BX* BY) void k_max_div64_pred(const F* __restrict__
                                                            int open_mask, const uint8_t* __restrict__ nc,
                                                            const double* __restrict__ p,
                                                            const double* __restrict__ mean64,
-                                                           double* __restrict__ part, Dims d) {
+                                                           double* __restrict__ part, Dims d, int rz) {
     static_assert(BX == 64, "a block row is one wave: the high u face comes from the next lane");
     __shared__ double red[4];
     __shared__ F vrow[BY][BX];
     const int tx = threadIdx.x, ty = threadIdx.y;
     const int i = blockIdx.x * BX + tx;
     const int j = blockIdx.y * BY + ty;
-    const int k0 = blockIdx.z * RES_RZ, k1 = min(k0 + RES_RZ, d.D);
+    const int k0 = blockIdx.z * rz, k1 = min(k0 + rz, d.D);
     const bool in = i < d.W && j < d.H;
     const int sy = d.W + 2, sz = (d.W + 2) * (d.H + 2), W = d.W, HW = d.W * d.H;
     const double mean = *mean64;
@@ -983,7 +990,7 @@ void launch_proj_setup(const Dims& d, const float* u, const float* v, const floa
                        double* part, hipStream_t s, uint8_t* nq) {
     if (b64)
         hipLaunchKernelGGL(k_proj_setup_z, grid_z(d), dim3(BX, BY), 0, s, u, v, w, occ, open_mask, nc, b64, p64_pad,
-                           part, d, nq);
+                           part, d, nq, march_planes(d));
     else
         hipLaunchKernelGGL(k_proj_setup, grid_for(d.W, d.H, d.D), dim3(BX, BY), 0, s, u, v, w, occ, open_mask, nc, b,
                            p_pad, part, d, nq);
@@ -1305,20 +1312,20 @@ int sor_shape_candidates(const Dims& d, SorShape* out, int max) {
 void launch_correct(const Dims& d, const uint8_t* occ, int open_mask, const float* p_pad, float* u, float* v,
                     float* w, hipStream_t s) {
     hipLaunchKernelGGL((k_correct_cells<PadPressure<float>, float>), grid_z(d), dim3(BX, BY), 0, s, occ, open_mask,
-                       PadPressure<float>{p_pad}, u, v, w, d);
+                       PadPressure<float>{p_pad}, u, v, w, d, march_planes(d));
 }
 
 void launch_correct_quad(const Dims& d, const uint8_t* occ, int open_mask, const float* p_quad, float* u, float* v,
                          float* w, hipStream_t s) {
     hipLaunchKernelGGL((k_correct_cells<QuadPressure, float>), grid_z(d), dim3(BX, BY), 0, s, occ, open_mask,
-                       QuadPressure{p_quad}, u, v, w, d);
+                       QuadPressure{p_quad}, u, v, w, d, march_planes(d));
 }
 
 template <class F>
 void launch_correct64(const Dims& d, const uint8_t* occ, int open_mask, const double* p64_pad, F* u, F* v, F* w,
                       hipStream_t s) {
     hipLaunchKernelGGL((k_correct_cells<PadPressure<double>, F>), grid_z(d), dim3(BX, BY), 0, s, occ, open_mask,
-                       PadPressure<double>{p64_pad}, u, v, w, d);
+                       PadPressure<double>{p64_pad}, u, v, w, d, march_planes(d));
 }
 
 template <class F>
@@ -1371,7 +1378,7 @@ void launch_residual64_split(const Dims& d, const uint8_t* nc, const double* b64
                              hipStream_t s) {
     const dim3 g = grid_z(d);
     hipLaunchKernelGGL(k_residual64_z<false>, g, dim3(BX, BY), 0, s, nc, b64, mean64, p64_pad, sp.b[0], sp.b[1], part,
-                       d, (d.W + 1) / 2);
+                       d, (d.W + 1) / 2, march_planes(d));
     hipLaunchKernelGGL(k_finish_max, dim3(1), dim3(1024), 0, s, part, (int)(g.x * g.y * g.z), rmax);
 }
 
@@ -1380,7 +1387,7 @@ void launch_residual64_quad(const Dims& d, const uint8_t* nc, const double* b64,
                             hipStream_t s) {
     const dim3 g = grid_z(d);
     hipLaunchKernelGGL(k_residual64_z<true>, g, dim3(BX, BY), 0, s, nc, b64, mean64, p64_pad, q.b, nullptr, part, d,
-                       quad_stride(d.W));
+                       quad_stride(d.W), march_planes(d));
     hipLaunchKernelGGL(k_finish_max, dim3(1), dim3(1024), 0, s, part, (int)(g.x * g.y * g.z), rmax);
 }
 
@@ -1406,29 +1413,30 @@ void launch_update_p64_quad(const Dims& d, const uint8_t* nc, const float* e_qua
 
 template <class F>
 void launch_max_div64(const Dims& d, const F* u, const F* v, const F* w, const uint8_t* nc, const double* mean64,
-                      double* part, unsigned long long* dmax, hipStream_t s) {
+                      double* part, unsigned long long* dmax, hipStream_t s, unsigned long long* mean_out) {
     hipLaunchKernelGGL(k_max_div64<F>, grid_for(d.W, d.H, d.D), dim3(BX, BY), 0, s, u, v, w, nc, mean64, part, d);
-    hipLaunchKernelGGL(k_finish_max, dim3(1), dim3(1024), 0, s, part, cell_blocks(d), dmax);
+    hipLaunchKernelGGL(k_finish_max, dim3(1), dim3(1024), 0, s, part, cell_blocks(d), dmax, mean64, mean_out);
 }
 
 template <class F>
 void launch_max_div64_pred(const Dims& d, const F* u, const F* v, const F* w, const uint8_t* occ, int open_mask,
                            const uint8_t* nc, const double* p64_pad, const double* mean64, double* part,
-                           unsigned long long* dmax, hipStream_t s) {
+                           unsigned long long* dmax, hipStream_t s, unsigned long long* mean_out) {
     const dim3 g = grid_z(d);
     hipLaunchKernelGGL(k_max_div64_pred<F>, g, dim3(BX, BY), 0, s, u, v, w, occ, open_mask, nc, p64_pad, mean64, part,
-                       d);
-    hipLaunchKernelGGL(k_finish_max, dim3(1), dim3(1024), 0, s, part, (int)(g.x * g.y * g.z), dmax);
+                       d, march_planes(d));
+    hipLaunchKernelGGL(k_finish_max, dim3(1), dim3(1024), 0, s, part, (int)(g.x * g.y * g.z), dmax, mean64,
+                       mean_out);
 }
 
 #define ZQ3D_PROJ_INSTANTIATE(F)                                                                                       \
     template void launch_correct64<F>(const Dims&, const uint8_t*, int, const double*, F*, F*, F*, hipStream_t);       \
     template void launch_correct_all64<F>(const Dims&, const double*, F*, F*, F*, hipStream_t);                        \
     template void launch_max_div64<F>(const Dims&, const F*, const F*, const F*, const uint8_t*, const double*,        \
-                                      double*, unsigned long long*, hipStream_t);                                      \
+                                      double*, unsigned long long*, hipStream_t, unsigned long long*);                 \
     template void launch_max_div64_pred<F>(const Dims&, const F*, const F*, const F*, const uint8_t*, int,             \
                                            const uint8_t*, const double*, const double*, double*,                      \
-                                           unsigned long long*, hipStream_t);
+                                           unsigned long long*, hipStream_t, unsigned long long*);
 ZQ3D_PROJ_INSTANTIATE(float)
 ZQ3D_PROJ_INSTANTIATE(double)
 #undef ZQ3D_PROJ_INSTANTIATE

@@ -261,11 +261,11 @@ int refine_mixed(const Dims& d, const zq3d_sor_opts& o, double tol, const ProjBu
             if (chk->fp64)
                 launch_max_div64_pred(d, (const double*)chk->u, (const double*)chk->v, (const double*)chk->w,
                                       chk->occ, chk->open_mask, B.nc, B.p64, &sc->mean64, B.part,
-                                      B.target(1, &sc->dmax), s);
+                                      B.target(1, &sc->dmax), s, B.mean_slot());
             else
                 launch_max_div64_pred(d, (const float*)chk->u, (const float*)chk->v, (const float*)chk->w,
                                       chk->occ, chk->open_mask, B.nc, B.p64, &sc->mean64, B.part,
-                                      B.target(1, &sc->dmax), s);
+                                      B.target(1, &sc->dmax), s, B.mean_slot());
             if (int rc = read_result(B, 1, &sc->dmax, &dmax, s, where)) return rc;
             if (!(dmax > tol)) break;
             // what is left is the faces' FP32 rounding once a pass no longer shrinks it by a tenth:
@@ -326,6 +326,17 @@ int read_result(const ProjBufs& B, int slot, const unsigned long long* dev_scala
     return ZQ3D_OK;
 }
 
+int read_mean(const ProjBufs& B, double* out, hipStream_t s, const char* where) {
+    if (!B.rb.host) {
+        ZQ_HIP(hipMemcpyAsync(out, &B.sc->mean64, sizeof(*out), hipMemcpyDeviceToHost, s), where);
+        ZQ_HIP(hipStreamSynchronize(s), where);
+        return ZQ3D_OK;
+    }
+    const unsigned long long bits = ((volatile unsigned long long*)B.rb.host)[3];
+    std::memcpy(out, &bits, sizeof(*out));
+    return ZQ3D_OK;
+}
+
 int read_double_bits(const unsigned long long* dev, double* out, hipStream_t s, const char* where) {
     unsigned long long bits = 0;
     ZQ_HIP(hipMemcpyAsync(&bits, dev, sizeof(bits), hipMemcpyDeviceToHost, s), where);
@@ -372,11 +383,10 @@ int project_plain(const Dims& d, float* u, float* v, float* w, const uint8_t* oc
         launch_correct(d, occ, o.open_mask, res, u, v, w, s);
     }
     if (st) {
-        launch_max_div64(d, u, v, w, B.nc, &sc->mean64, B.part, B.target(1, &sc->dmax), s);
+        launch_max_div64(d, u, v, w, B.nc, &sc->mean64, B.part, B.target(1, &sc->dmax), s, B.mean_slot());
         double md = 0.0, mean64 = 0.0;
         if (int rc = read_result(B, 1, &sc->dmax, &md, s, "project")) return rc;
-        ZQ_HIP(hipMemcpyAsync(&mean64, &sc->mean64, sizeof(mean64), hipMemcpyDeviceToHost, s), "project");
-        ZQ_HIP(hipStreamSynchronize(s), "project");
+        if (int rc = read_mean(B, &mean64, s, "project")) return rc;
         st->outer = 0;
         st->sweeps = o.iters;
         st->max_residual = -1.0;
@@ -403,12 +413,11 @@ int project_mixed(const Dims& d, float* u, float* v, float* w, const uint8_t* oc
     launch_correct64(d, occ, o.open_mask, B.p64, u, v, w, s);
     if (!st) return ZQ3D_OK;
     if (md < 0.0) {  // the passes ran out before the residual met tol: measure the stored faces
-        launch_max_div64(d, u, v, w, B.nc, &sc->mean64, B.part, B.target(1, &sc->dmax), s);
+        launch_max_div64(d, u, v, w, B.nc, &sc->mean64, B.part, B.target(1, &sc->dmax), s, B.mean_slot());
         if (int rc = read_result(B, 1, &sc->dmax, &md, s, "project_mixed")) return rc;
     }
     double mean64 = 0.0;
-    ZQ_HIP(hipMemcpyAsync(&mean64, &sc->mean64, sizeof(mean64), hipMemcpyDeviceToHost, s), "project_mixed");
-    ZQ_HIP(hipStreamSynchronize(s), "project_mixed");
+    if (int rc = read_mean(B, &mean64, s, "project_mixed")) return rc;
     st->outer = ro.outer;
     st->sweeps = (int)ro.sweeps;
     st->max_residual = ro.rmax;

@@ -146,6 +146,8 @@ struct ProjBufs {
     unsigned long long* target(int slot, unsigned long long* dev_scalar) const {
         return rb.dev ? rb.dev + slot : dev_scalar;
     }
+    // the pinned slot a divergence check's mean goes to (null: none; read_mean then copies it)
+    unsigned long long* mean_slot() const { return rb.dev ? rb.dev + 3 : nullptr; }
     // the gate words of a gated pass; the executed count goes to pinned slot 2 when there is one
     GateBufs gate() const { return GateBufs{sc->gate, &sc->done, rb.dev ? rb.dev + 2 : &sc->done_sink}; }
     // split storage present (the gated passes and the split shapes need it)
@@ -157,6 +159,9 @@ int read_result(const ProjBufs& B, int slot, const unsigned long long* dev_scala
                 const char* where);
 
 // launch_sor, timed when pf is set (the sweeps are the only work between the two events)
+// the FP64 mean of a projection whose last divergence check (with mean_slot()) the stream has been waited for
+int read_mean(const ProjBufs& B, double* out, hipStream_t s, const char* where);
+
 hipError_t timed_sor(const Dims& d, const uint8_t* nc, const float* b, const float* mean32, float* p, float* p_alt,
                      float omega, int iters, hipStream_t s, SorProf* pf, float** result, SorShape shape,
                      const SplitBufs* split);

@@ -10,6 +10,17 @@
 
 namespace zq3d {
 
+// Planes a thread of the column-marching kernels (64 x 4 threads a block) walks: 16 reuse what neighbouring
+// planes share, but a column's planes are a serial chain of loads, so a grid with fewer than 4 blocks a CU
+// that way takes shorter columns (with 16 planes everywhere the 20x24x16 frame took 343 us, a force-face
+// pass alone 27; with this rule 271, and the 64^3 frame 907 -> 829; 256^3 keeps 16).
+inline int march_planes(const Dims& d) {
+    const long long columns = (long long)((d.W + 63) / 64) * ((d.H + 3) / 4);
+    int rz = 16;
+    while (rz > 1 && columns * ((d.D + rz - 1) / rz) < 1024) rz >>= 1;
+    return rz;
+}
+
 struct ForceParams {
     float h, dt, beta, alpha, eps, Tamb;
 };
@@ -209,16 +220,17 @@ void launch_update_p64(const Dims& d, const uint8_t* nc, float* e_pad, double* p
 // next pass starts with a zero_start sweep)
 void launch_update_p64_split(const Dims& d, const uint8_t* nc, float* const* e, double* p64_pad, hipStream_t s,
                              bool zero_e = true);
-// max |div64 - mean64| over counted cells into *dmax (bits of a non-negative double)
+// max |div64 - mean64| over counted cells into *dmax (bits of a non-negative double); mean_out (nullable)
+// receives the mean's bits
 template <class F>
 void launch_max_div64(const Dims& d, const F* u, const F* v, const F* w, const uint8_t* nc, const double* mean64,
-                      double* part, unsigned long long* dmax, hipStream_t s);
+                      double* part, unsigned long long* dmax, hipStream_t s, unsigned long long* mean_out = nullptr);
 // max |div64 - mean64| over counted cells of the faces launch_correct64 would produce from p64_pad
 // (equal bit for bit to launch_max_div64 after launch_correct64), faces left unchanged
 template <class F>
 void launch_max_div64_pred(const Dims& d, const F* u, const F* v, const F* w, const uint8_t* occ, int open_mask,
                            const uint8_t* nc, const double* p64_pad, const double* mean64, double* part,
-                           unsigned long long* dmax, hipStream_t s);
+                           unsigned long long* dmax, hipStream_t s, unsigned long long* mean_out = nullptr);
 // max |b64| over counted cells into *out (bits of a non-negative double)
 void launch_max_abs64(const Dims& d, const uint8_t* nc, const double* b64, double* part, unsigned long long* out,
                       hipStream_t s);
