@@ -1,0 +1,68 @@
+"""Which cell lists of the octree sweeps share a launch (csrc/zq3d_octree_plan.h), compiled with g++ and
+checked on the CPU over every adjacency of the four levels: each list runs once per pass in pass order,
+a launch holds only lists of levels that do not touch, and of two lists of the same or of touching
+levels the one that comes first in the one-by-one order runs in an earlier launch."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SRC = r"""
+#include "zq3d_octree_plan.h"
+#include <cstdio>
+using namespace zq3d;
+int main() {
+    const int pairs[6][2] = {{0, 1}, {1, 2}, {2, 3}, {0, 2}, {1, 3}, {0, 3}};
+    for (int adj = 0; adj < 64; adj++)
+        for (int empty = 0; empty < 256; empty++)
+            for (int iters = 0; iters <= 5; iters++) {
+                uint32_t beside[4] = {}, counts[OCT_LISTS];
+                for (int p = 0; p < 6; p++)
+                    if (adj >> p & 1) {
+                        beside[pairs[p][0]] |= 1u << pairs[p][1];
+                        beside[pairs[p][1]] |= 1u << pairs[p][0];
+                    }
+                int lists = 0;
+                for (int k = 0; k < OCT_LISTS; k++) lists += (counts[k] = empty >> k & 1 ? 0 : 5 + k) != 0;
+                const std::vector<uint8_t> plan = oct_schedule(counts, beside, iters);
+                auto tied = [&](int a, int b) { return a / 2 == b / 2 || (beside[a / 2] >> (b / 2) & 1); };
+                std::vector<int> at[OCT_LISTS];  // launch of each pass, per list
+                for (size_t i = 0; i < plan.size(); i++) {
+                    if (!plan[i]) return std::printf("empty launch: adj %d lists %d\n", adj, empty), 1;
+                    for (int k = 0; k < OCT_LISTS; k++) {
+                        if (!(plan[i] >> k & 1)) continue;
+                        at[k].push_back((int)i);
+                        for (int j = 0; j < k; j++)
+                            if ((plan[i] >> j & 1) && tied(j, k))
+                                return std::printf("touching lists share a launch: adj %d %d %d\n", adj, j, k), 1;
+                    }
+                }
+                for (int k = 0; k < OCT_LISTS; k++)
+                    if ((int)at[k].size() != (counts[k] ? iters : 0))
+                        return std::printf("passes of list %d: %d\n", k, (int)at[k].size()), 1;
+                for (int a = 0; a < OCT_LISTS; a++)
+                    for (int b = 0; b < OCT_LISTS; b++) {
+                        if (!counts[a] || !counts[b] || !tied(a, b)) continue;
+                        for (int i = 0; i < iters; i++)
+                            for (int j = 0; j < iters; j++)
+                                if (i * OCT_LISTS + a < j * OCT_LISTS + b && at[a][i] >= at[b][j])
+                                    return std::printf("order: adj %d list %d pass %d, list %d pass %d\n", adj, a, i, b, j), 1;
+                    }
+                if (!empty && iters && (int)plan.size() > OCT_LISTS * iters) return std::printf("too many\n"), 1;
+                // leaves stepping one level at a time: four launches a pass once the first has come through
+                if (!empty && adj == 7 && iters && (int)plan.size() != 4 * iters + 4)
+                    return std::printf("stepping leaves: %d launches\n", (int)plan.size()), 1;
+            }
+    std::printf("ok\n");
+    return 0;
+}
+"""
+
+
+def test_lists_keep_the_order_of_everything_they_touch(tmp_path):
+    src = tmp_path / "plan.cpp"
+    src.write_text(SRC)
+    exe = str(tmp_path / "plan")
+    inc = os.path.join(ROOT, "zq_smokesimulation_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-I", inc, str(src), "-o", exe], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True)
+    assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout

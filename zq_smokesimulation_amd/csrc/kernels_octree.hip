@@ -15,12 +15,10 @@
 // else the finer leaves square by square), and a level-m leaf's cells form one aligned run of 4^m
 // positions, skipped at once.  The sums coeff += w, sigma += w * p run in that order, so the
 // result is the lists' bit for bit.  The walks run once per projection: they fill compact
-// per-level, per-colour cell lists and, for the 2^3 to 8^3 leaves, their neighbour entries (counted,
-// scanned, written), so that each of the iters x 8 sweep launches is a gather over a short list
-// (a scene far from its obstacles is mostly 8^3 leaves, and the launches touch only those).
-#include <algorithm>
-
-#include <hipcub/hipcub.hpp>
+// per-level, per-colour cell lists with their neighbour entries and diagonals, so that each sweep
+// launch is a gather over short lists (a scene far from its obstacles is mostly 8^3 leaves, and the
+// launches touch only those).
+#include <vector>
 
 #include "zq3d_coarse.h"
 #include "zq3d_kernels.h"
@@ -228,32 +226,33 @@ __global__ __launch_bounds__(256) void k_oct_lists(OG g, const uint8_t* __restri
 }
 
 __global__ void k_oct_zero(uint32_t* count) {
-    if (threadIdx.x < 8) count[threadIdx.x] = 0u;
+    if (threadIdx.x < 4 * OCT_LISTS) count[threadIdx.x] = 0u;
 }
 
-// A neighbour entry: level in bits 30-31, the linear index at that level below; OCT_OPEN marks an
-// open domain face (its weight enters the diagonal only).
+// A neighbour entry: level in bits 30-31, the linear index at that level below.  An open domain face
+// is OCT_OPEN in a walk; it weighs in the diagonal only, so the stored entries leave it out.  OCT_NONE
+// fills a cell's unused entries.
 constexpr uint32_t OCT_OPEN = 0xFFFFFFFFu;
-constexpr int OCT_HEAD = 6;  // entries per cell kept in the transposed head (one per face)
+constexpr uint32_t OCT_NONE = 0xFFFFFFFFu;
 
 __device__ __forceinline__ uint32_t oct_entry(const OG& g, int m, int x, int y, int z) {
     return ((uint32_t)m << 30) | (uint32_t)oat(g, m, x >> m, y >> m, z >> m);
 }
 
-// The neighbour entries of the level-L cell (x, y, z), in the reference's order, handed to put(k, e);
-// returns their number.  Per face: an open domain face; else the leaf behind the face's first fine
+// The neighbour entries of the level-L cell (x, y, z), in the reference's order, handed to put(e).
+// Per face: an open domain face; else the leaf behind the face's first fine
 // cell when it is as large as this one (at level 0: the fine neighbour unless solid); else the face's
 // fine cells in interleaved order (slower axis high), one entry per leaf met (its run of 4^m
 // positions skipped), solid cells skipped.
 template <class Put>
-__device__ int oct_walk(const OG& g, const uint8_t* __restrict__ lev, int L, int x, int y, int z, Put put) {
+__device__ __forceinline__ void oct_walk(const OG& g, const uint8_t* __restrict__ lev, int L, int x, int y, int z, Put put) {
     const int S = 1 << L;
     const int cl[3] = {x, y, z}, dims[3] = {ow(g, L), oh(g, L), od(g, L)}, base[3] = {x * S, y * S, z * S};
-    int k = 0;
+#pragma unroll
     for (int f = 0; f < 6; f++) {
         const int ax = f >> 1, sd = (f & 1) ? 1 : -1;
         if ((sd < 0 && cl[ax] == 0) || (sd > 0 && cl[ax] == dims[ax] - 1)) {
-            put(k++, OCT_OPEN);
+            put(OCT_OPEN);
             continue;
         }
         const int slow = ax == 2 ? 1 : 2, fast = ax == 0 ? 1 : 0;
@@ -261,7 +260,7 @@ __device__ int oct_walk(const OG& g, const uint8_t* __restrict__ lev, int L, int
         q0[ax] = sd < 0 ? base[ax] - 1 : base[ax] + S;
         const int m0 = lev[oat(g, 0, q0[0], q0[1], q0[2])];
         if (m0 != OCT_SOLID && m0 >= L) {  // one leaf as large as this one covers the face
-            put(k++, oct_entry(g, m0, q0[0], q0[1], q0[2]));
+            put(oct_entry(g, m0, q0[0], q0[1], q0[2]));
             continue;
         }
         for (int t = 0; t < S * S;) {
@@ -278,11 +277,10 @@ __device__ int oct_walk(const OG& g, const uint8_t* __restrict__ lev, int L, int
                 t += 1;
                 continue;
             }
-            put(k++, oct_entry(g, m, q[0], q[1], q[2]));
+            put(oct_entry(g, m, q[0], q[1], q[2]));
             t += 1 << (2 * m);  // m < L here: the rest of that leaf's run on this face
         }
     }
-    return k;
 }
 
 __device__ __forceinline__ void oct_cell(const OG& g, int L, uint32_t c, int& x, int& y, int& z) {
@@ -292,127 +290,183 @@ __device__ __forceinline__ void oct_cell(const OG& g, int L, uint32_t c, int& x,
     z = (int)(c / (wl * hl));
 }
 
-// entries per listed cell (tot) and beyond the head (ovc, the scan input; ovc[n] = 0 closes it)
-__global__ __launch_bounds__(256) void k_oct_count(OG g, const uint8_t* __restrict__ lev, int L,
-                                                   const uint32_t* __restrict__ list, uint32_t n,
-                                                   uint32_t* __restrict__ tot, uint32_t* __restrict__ ovc) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i > n) return;
-    if (i == n) {
-        ovc[n] = 0;
-        return;
-    }
-    int x, y, z;
-    oct_cell(g, L, list[i], x, y, z);
-    const int k = oct_walk(g, lev, L, x, y, z, [](int, uint32_t) {});
-    tot[i] = (uint32_t)k;
-    ovc[i] = k > OCT_HEAD ? (uint32_t)(k - OCT_HEAD) : 0u;
-}
+// The lists one launch takes, one after the other over its blocks of OCT_BLOCK cells.  The set-up
+// launches take all eight, a sweep launch at most one per level.
+constexpr int OCT_BLOCK = 64;
 
-// entries: the first OCT_HEAD transposed (entry j of cell i at j * n + i, so a wave's loads of one
-// j are contiguous), the rest at the cell's scanned offset in ovf
-__global__ __launch_bounds__(256) void k_oct_fill(OG g, const uint8_t* __restrict__ lev, int L,
-                                                  const uint32_t* __restrict__ list, uint32_t n,
-                                                  uint32_t* __restrict__ head, const uint32_t* __restrict__ off,
-                                                  uint32_t* __restrict__ ovf) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    int x, y, z;
-    oct_cell(g, L, list[i], x, y, z);
-    uint32_t* ov = ovf + off[i];
-    oct_walk(g, lev, L, x, y, z, [&](int k, uint32_t e) {
-        if (k < OCT_HEAD) head[(size_t)k * n + i] = e;
-        else ov[k - OCT_HEAD] = e;
-    });
-}
-
-struct TotPtrs {
-    const uint32_t* off[8];
-    uint32_t n[8];
+struct OctSeg {
+    const uint32_t* list;
+    uint32_t* head;  // entry j of cell i at j * n + i
+    uint32_t* ovo;   // a cell's first entry in ovf, and its entries there
+    uint32_t* ovn;
+    uint32_t* ovf;
+    float* coeff;
+    float* rhs;
+    uint32_t n, first;  // cells; the launch's first block of this list
+    int k, width;       // list number 2 L + colour; entries per cell kept in the head
+    int over;           // some cell of the list has entries in ovf
+    float w0, w1, w2, w3;  // the level's weights towards a leaf of level 0..3 (open domain face: 3)
 };
 
-__global__ void k_oct_totals(TotPtrs t, uint32_t* out) {
-    const int k = threadIdx.x;
-    if (k < 8) out[k] = t.n[k] ? t.off[k][t.n[k]] : 0u;
+__device__ __forceinline__ float oct_weight(const OctSeg& q, uint32_t m) {
+    const float lo = m & 1 ? q.w1 : q.w0, hi = m & 1 ? q.w3 : q.w2;
+    return m & 2 ? hi : lo;
+}
+
+template <int N>
+struct OctSegs {
+    OctSeg s[N];
+    int count;
+};
+
+// the list of this block (every block has one: the grid is the sum of the lists' blocks)
+template <int N>
+__device__ __forceinline__ OctSeg oct_seg(const OctSegs<N>& t, uint32_t& i) {
+    OctSeg r = t.s[0];
+#pragma unroll
+    for (int j = 1; j < N; j++)
+        if (j < t.count && blockIdx.x >= t.s[j].first) r = t.s[j];
+    i = (blockIdx.x - r.first) * OCT_BLOCK + threadIdx.x;
+    return r;
+}
+
+// Per listed cell the entries beyond OCT_WIDE (ovn) and their place in ovf (ovo: order free, an
+// atomic hands out the runs); per list their sum, the largest number of entries of a cell and the
+// levels the entries name (count + 8, + 16, + 24).
+__global__ __launch_bounds__(OCT_BLOCK) void k_oct_count(OG g, const uint8_t* __restrict__ lev, OctSegs<OCT_LISTS> t,
+                                                         uint32_t* __restrict__ count) {
+    uint32_t i;
+    const OctSeg q = oct_seg(t, i);
+    uint32_t k = 0, seen = 0;
+    if (i < q.n) {
+        int x, y, z;
+        oct_cell(g, q.k >> 1, q.list[i], x, y, z);
+        oct_walk(g, lev, q.k >> 1, x, y, z, [&](uint32_t e) {
+            if (e == OCT_OPEN) return;
+            k++;
+            seen |= 1u << (e >> 30);
+        });
+        const uint32_t o = k > OCT_WIDE ? k - OCT_WIDE : 0u;
+        q.ovn[i] = o;
+        q.ovo[i] = o ? atomicAdd(count + OCT_LISTS + q.k, o) : 0u;
+    }
+    for (int d = 32; d; d >>= 1) {
+        k = max(k, (uint32_t)__shfl_xor((int)k, d, 64));
+        seen |= (uint32_t)__shfl_xor((int)seen, d, 64);
+    }
+    if (threadIdx.x == 0) {
+        // an older value read here costs at most an atomic that changes nothing
+        uint32_t *most = count + 2 * OCT_LISTS + q.k, *levels = count + 3 * OCT_LISTS + q.k;
+        if (k > __hip_atomic_load(most, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(most, k);
+        if (seen & ~__hip_atomic_load(levels, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(levels, seen);
+    }
+}
+
+// The entries, their weights' sum in walk order (open faces included) and the rest of the head row
+// filled with OCT_NONE.  A wave's stores of one entry number are contiguous.
+__global__ __launch_bounds__(OCT_BLOCK) void k_oct_fill(OG g, const uint8_t* __restrict__ lev, OctSegs<OCT_LISTS> t) {
+    uint32_t i;
+    const OctSeg q = oct_seg(t, i);
+    if (i >= q.n) return;
+    int x, y, z;
+    const int L = q.k >> 1;
+    oct_cell(g, L, q.list[i], x, y, z);
+    uint32_t* ov = q.ovf + q.ovo[i];
+    float coeff = 0.0f;
+    int k = 0;
+    oct_walk(g, lev, L, x, y, z, [&](uint32_t e) {
+        const uint32_t m = e >> 30;  // OCT_OPEN: the level-3 weight
+        coeff += oct_weight(q, m);
+        if (e == OCT_OPEN) return;
+        if (k < q.width) q.head[(size_t)k * q.n + i] = e;
+        else ov[k - q.width] = e;
+        k++;
+    });
+    for (; k < q.width; k++) q.head[(size_t)k * q.n + i] = OCT_NONE;
+    q.coeff[i] = coeff;
 }
 
 // right-hand side per listed cell in list order: the level's divergence, with `mean` the closed form
 // div - mean * 8^L
-__global__ __launch_bounds__(256) void k_oct_rhs(OG g, int L, const uint32_t* __restrict__ list, uint32_t n,
-                                                 const float* __restrict__ dl, const float* __restrict__ mean,
-                                                 float* __restrict__ rhs) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const float dd = dl[list[i]];
-    rhs[i] = mean ? dd - *mean * (float)(1 << (3 * L)) : dd;
+__global__ __launch_bounds__(OCT_BLOCK) void k_oct_rhs(LevelPtrs dl, OctSegs<OCT_LISTS> t,
+                                                       const float* __restrict__ mean) {
+    uint32_t i;
+    const OctSeg q = oct_seg(t, i);
+    if (i >= q.n) return;
+    const int L = q.k >> 1;
+    const float* d = L == 0 ? dl.p[0] : L == 1 ? dl.p[1] : L == 2 ? dl.p[2] : dl.p[3];
+    const float dd = d[q.list[i]];
+    q.rhs[i] = mean ? dd - *mean * (float)(1 << (3 * L)) : dd;
 }
 
-// One listed cell of one colour of one level: coeff += w, sigma += w * p over its entries in order,
-// then p = (sigma - rhs) / coeff (CPU_PoissonSolver3D_OpenOctreePoisson.cpp:404-425).  The head
-// entries and the right-hand side load without any dependence, then all the pressures they name.
-__device__ __forceinline__ void oct_gs_cell(const OctW& wt, const LevelPtrs& P, int L, float* pl,
-                                            const uint32_t* __restrict__ list, uint32_t n,
-                                            const uint32_t* __restrict__ head, const uint32_t* __restrict__ tot,
-                                            const uint32_t* __restrict__ off, const uint32_t* __restrict__ ovf,
-                                            const float* __restrict__ rhs, uint32_t i) {
-    const uint32_t c = list[i], nt = tot[i];
-    const float r = rhs[i];
-    uint32_t ev[OCT_HEAD];
-    float pv[OCT_HEAD];
+// The pressures of all four levels sit in one allocation: level m starts off[m] floats after p.
+struct OctP {
+    float* p;
+    uint32_t off[4];
+};
+
+__device__ __forceinline__ uint32_t oct_level_off(const OctP& P, uint32_t m) {
+    const uint32_t lo = m & 1 ? P.off[1] : P.off[0], hi = m & 1 ? P.off[3] : P.off[2];
+    return m & 2 ? hi : lo;
+}
+
+// NE entries at once: every pressure they name is in flight before the first sum.  An unused entry
+// reads cell 0 of level 0 and adds 0 (the sum is never -0, so it stays as it is).
+template <int NE>
+__device__ __forceinline__ float oct_sum(const OctP& P, const OctSeg& q, const uint32_t (&e)[NE], float sigma) {
+    float pv[NE];
 #pragma unroll
-    for (int j = 0; j < OCT_HEAD; j++) ev[j] = (uint32_t)j < nt ? head[(size_t)j * n + i] : OCT_OPEN;
-#pragma unroll
-    for (int j = 0; j < OCT_HEAD; j++)
-        pv[j] = ((uint32_t)j < nt && ev[j] != OCT_OPEN) ? P.p[ev[j] >> 30][ev[j] & 0x3FFFFFFFu] : 0.0f;
-    float coeff = 0.0f, sigma = 0.0f;
-#pragma unroll
-    for (int j = 0; j < OCT_HEAD; j++) {
-        if ((uint32_t)j >= nt) break;
-        if (ev[j] == OCT_OPEN) {
-            coeff += wt.w[L][3];  // open domain face
-        } else {
-            const float wg = wt.w[L][ev[j] >> 30];
-            coeff += wg;
-            sigma += wg * pv[j];
-        }
+    for (int j = 0; j < NE; j++) {
+        const uint32_t m = e[j] >> 30;
+        const uint32_t at = e[j] == OCT_NONE ? 0u : oct_level_off(P, m) + (e[j] & 0x3FFFFFFFu);
+        pv[j] = P.p[at];
     }
-    if (nt > OCT_HEAD) {
-        // a face with finer leaves behind it: the rest, eight at a time, in order
-        const uint32_t* ov = ovf + off[i];
-        const uint32_t no = nt - OCT_HEAD;
-        for (uint32_t k0 = 0; k0 < no; k0 += 8) {
-            uint32_t e8[8];
-            float p8[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) e8[j] = k0 + j < no ? ov[k0 + j] : OCT_OPEN;
+    for (int j = 0; j < NE; j++) {
+        const uint32_t m = e[j] >> 30;
+        const float wg = oct_weight(q, m);
+        sigma += wg * (e[j] == OCT_NONE ? 0.0f : pv[j]);
+    }
+    return sigma;
+}
+
+template <int NE>
+__device__ __forceinline__ void oct_gs_cell(const OctP& P, const OctSeg& q, uint32_t i) {
+    const uint32_t c = q.list[i];
+    const float r = q.rhs[i], coeff = q.coeff[i];
+    uint32_t ev[NE], no = 0, o0 = 0;
+    if (q.over) {
+        no = q.ovn[i];
+        o0 = q.ovo[i];
+    }
 #pragma unroll
-            for (int j = 0; j < 8; j++)
-                p8[j] = (k0 + j < no && e8[j] != OCT_OPEN) ? P.p[e8[j] >> 30][e8[j] & 0x3FFFFFFFu] : 0.0f;
+    for (int j = 0; j < NE; j++) ev[j] = q.head[(size_t)j * q.n + i];
+    float sigma = oct_sum<NE>(P, q, ev, 0.0f);
+    for (uint32_t k0 = 0; k0 < no; k0 += 8) {
+        uint32_t e8[8];
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                if (k0 + j >= no) break;
-                if (e8[j] == OCT_OPEN) {
-                    coeff += wt.w[L][3];
-                } else {
-                    const float wg = wt.w[L][e8[j] >> 30];
-                    coeff += wg;
-                    sigma += wg * p8[j];
-                }
-            }
-        }
+        for (int j = 0; j < 8; j++) e8[j] = k0 + j < no ? q.ovf[o0 + k0 + j] : OCT_NONE;
+        sigma = oct_sum<8>(P, q, e8, sigma);
     }
     sigma -= r;
-    pl[c] = sigma / coeff;
+    P.p[oct_level_off(P, (uint32_t)q.k >> 1) + c] = sigma / coeff;
 }
 
-// One colour of one level, one launch.
-__global__ __launch_bounds__(256) void k_oct_gs(OctW wt, LevelPtrs P, int L, float* __restrict__ pl,
-                                                const uint32_t* __restrict__ list, uint32_t n,
-                                                const uint32_t* __restrict__ head, const uint32_t* __restrict__ tot,
-                                                const uint32_t* __restrict__ off, const uint32_t* __restrict__ ovf,
-                                                const float* __restrict__ rhs) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) oct_gs_cell(wt, P, L, pl, list, n, head, tot, off, ovf, rhs, i);
+// One update p = (sigma - rhs) / coeff, sigma += w * p over a cell's entries in order
+// (CPU_PoissonSolver3D_OpenOctreePoisson.cpp:404-425), for every cell of the launch's lists; no two
+// of them neighbour each other.  A launch is a few microseconds of latency: every list but that of a
+// finest region is a few waves per CU at most.  So the chain of dependent loads is kept at two (the
+// list, the right-hand side, the diagonal and all head entries; then all pressures), waves spread
+// over the CUs one to a block, and a launch takes every list that may run beside the others.  256^3
+// around one sphere, thresholds 4, 8, 24 (levels step one at a time), 600 passes: 4800 launches of 7.9
+// us before, 2404 now, the frame 42.5 -> 13.9 ms.
+__global__ __launch_bounds__(OCT_BLOCK) void k_oct_gs(OctP P, OctSegs<4> t) {
+    uint32_t i;
+    const OctSeg q = oct_seg(t, i);
+    if (i >= q.n) return;
+    if (q.width <= 6) oct_gs_cell<6>(P, q, i);
+    else if (q.width <= 12) oct_gs_cell<12>(P, q, i);
+    else oct_gs_cell<OCT_WIDE>(P, q, i);
 }
 
 // ---------------------------------------------------------------------------- face correction
@@ -520,7 +574,7 @@ void octree_layout(const Dims& g, char* mem, OctreeBufs* B) {
     }
     for (int L = 0; L <= 3; L++)
         for (int c = 0; c < 2; c++) B->list[L][c] = (uint32_t*)take(4 * (level_cells(g, L) / 2 + 1));
-    B->count = (uint32_t*)take(64);
+    B->count = (uint32_t*)take(4 * 4 * OCT_LISTS);
 }
 
 void launch_octree_build(const Dims& d, const uint8_t* occ, int t1, int t2, int t3, const OctreeBufs& B,
@@ -552,109 +606,112 @@ void launch_octree_prepare(const Dims& d, const float* u, const float* v, const 
                            (const float*)B.d[L - 1], B.d[L], B.p[L]);
 }
 
+namespace {
+
+// the launch table of the lists in `mask` (bit k: list k), and its blocks
+template <int N>
+uint32_t oct_segs(const OctreeBufs& B, const OctreeLists& Ls, uint32_t mask, OctSegs<N>* t) {
+    const OctW wt = make_weights();
+    uint32_t blocks = 0;
+    t->count = 0;
+    for (int k = 0; k < OCT_LISTS; k++) {
+        const uint32_t n = Ls.counts[k];
+        if (!(mask >> k & 1) || !n) continue;
+        t->s[t->count++] = OctSeg{B.list[k / 2][k % 2], Ls.head[k], Ls.ovo[k], Ls.ovn[k], Ls.ovf[k], Ls.coeff[k],
+                                  Ls.rhs[k], n, blocks, k, Ls.width[k], Ls.over[k],
+                                  wt.w[k / 2][0], wt.w[k / 2][1], wt.w[k / 2][2], wt.w[k / 2][3]};
+        blocks += blocks_of(n, OCT_BLOCK);
+    }
+    return blocks;
+}
+
+}  // namespace
+
 hipError_t octree_build_lists(const Dims& d, const OctreeBufs& B, OctreeLists* Ls, hipStream_t s) {
     const OG g{d.W, d.H, d.D};
     hipLaunchKernelGGL(k_oct_zero, dim3(1), dim3(64), 0, s, B.count);
     hipLaunchKernelGGL(k_oct_lists, dim3(blocks_of(level_cells(d, 0), 256)), dim3(256), 0, s, g,
                        (const uint8_t*)B.lev, B.list[0][0], B.list[0][1], B.list[1][0], B.list[1][1], B.list[2][0],
                        B.list[2][1], B.list[3][0], B.list[3][1], B.count);
-    hipError_t e = hipMemcpyAsync(Ls->counts, B.count, 32, hipMemcpyDeviceToHost, s);
+    uint32_t got[4 * OCT_LISTS];
+    hipError_t e = hipMemcpyAsync(got, B.count, 4 * OCT_LISTS, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return e;
-    // per list: head (OCT_HEAD n), tot (n), ovc (n + 1), off (n + 1), rhs (n) in one buffer
-    size_t bytes = 0, nmax = 1;
-    for (int k = 0; k < 8; k++) {
-        const size_t n = Ls->counts[k];
-        bytes += up256(4 * OCT_HEAD * n) + up256(4 * n) + 2 * up256(4 * (n + 1)) + up256(4 * n);
-        nmax = std::max(nmax, n + 1);
+    size_t bytes = 0;
+    for (int k = 0; k < OCT_LISTS; k++) {
+        Ls->counts[k] = got[k];
+        bytes += 4 * up256(4 * (size_t)got[k]);
     }
     if ((e = grow(&Ls->dyn, &Ls->dyn_cap, bytes)) != hipSuccess) return e;
-    size_t scan = 0;
-    if ((e = hipcub::DeviceScan::ExclusiveSum(nullptr, scan, (const uint32_t*)nullptr, (uint32_t*)nullptr, (int)nmax,
-                                              s)) != hipSuccess)
-        return e;
-    if ((e = grow(&Ls->scan, &Ls->scan_cap, scan)) != hipSuccess) return e;
     char* p = (char*)Ls->dyn;
-    TotPtrs tp{};
-    for (int k = 0; k < 8; k++) {
-        const uint32_t n = Ls->counts[k];
-        Ls->head[k] = (uint32_t*)p;
-        p += up256(4 * OCT_HEAD * (size_t)n);
-        Ls->tot[k] = (uint32_t*)p;
-        p += up256(4 * (size_t)n);
-        Ls->ovc[k] = (uint32_t*)p;
-        p += up256(4 * ((size_t)n + 1));
-        Ls->off[k] = (uint32_t*)p;
-        p += up256(4 * ((size_t)n + 1));
-        Ls->rhs[k] = (float*)p;
-        p += up256(4 * (size_t)n);
-        tp.off[k] = Ls->off[k];
-        tp.n[k] = n;
-        if (!n) continue;
-        hipLaunchKernelGGL(k_oct_count, dim3(blocks_of((size_t)n + 1, 256)), dim3(256), 0, s, g,
-                           (const uint8_t*)B.lev, k / 2, (const uint32_t*)B.list[k / 2][k % 2], n, Ls->tot[k],
-                           Ls->ovc[k]);
-        size_t sb = Ls->scan_cap;
-        if ((e = hipcub::DeviceScan::ExclusiveSum(Ls->scan, sb, (const uint32_t*)Ls->ovc[k], Ls->off[k], (int)(n + 1),
-                                                  s)) != hipSuccess)
-            return e;
+    for (int k = 0; k < OCT_LISTS; k++) {
+        const size_t one = up256(4 * (size_t)Ls->counts[k]);
+        Ls->ovo[k] = (uint32_t*)p;
+        Ls->ovn[k] = (uint32_t*)(p + one);
+        Ls->coeff[k] = (float*)(p + 2 * one);
+        Ls->rhs[k] = (float*)(p + 3 * one);
+        Ls->head[k] = Ls->ovf[k] = nullptr;
+        Ls->width[k] = Ls->over[k] = 0;
+        p += 4 * one;
     }
-    hipLaunchKernelGGL(k_oct_totals, dim3(1), dim3(64), 0, s, tp, B.count + 8);
-    uint32_t tot[8];
-    e = hipMemcpyAsync(tot, B.count + 8, 32, hipMemcpyDeviceToHost, s);
+    OctSegs<OCT_LISTS> t{};
+    const uint32_t blocks = oct_segs(B, *Ls, 0xFF, &t);
+    if (!blocks) return hipGetLastError();
+    hipLaunchKernelGGL(k_oct_count, dim3(blocks), dim3(OCT_BLOCK), 0, s, g, (const uint8_t*)B.lev, t, B.count);
+    e = hipMemcpyAsync(got, B.count, sizeof got, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return e;
-    size_t need = 0;
-    for (int k = 0; k < 8; k++) {
-        Ls->ovf_base[k] = need;
-        need += tot[k];
+    const uint32_t *over = got + OCT_LISTS, *most = got + 2 * OCT_LISTS, *seen = got + 3 * OCT_LISTS;
+    bytes = 0;
+    for (int L = 0; L < 4; L++) Ls->beside[L] = 0;
+    for (int k = 0; k < OCT_LISTS; k++) {
+        Ls->width[k] = most[k] <= 6 ? 6 : most[k] <= 12 ? 12 : (int)OCT_WIDE;
+        Ls->over[k] = over[k] != 0;
+        bytes += up256(4 * (size_t)Ls->width[k] * Ls->counts[k]) + up256(4 * (size_t)over[k]);
+        for (int m = 0; m < 4; m++)
+            if (seen[k] >> m & 1) {
+                Ls->beside[k / 2] |= 1u << m;
+                Ls->beside[m] |= 1u << (k / 2);
+            }
     }
-    if ((e = grow((void**)&Ls->ovf, &Ls->ovf_cap, 4 * need + 4)) != hipSuccess) return e;
-    for (int k = 0; k < 8; k++) {
-        const uint32_t n = Ls->counts[k];
-        if (!n) continue;
-        hipLaunchKernelGGL(k_oct_fill, dim3(blocks_of(n, 256)), dim3(256), 0, s, g, (const uint8_t*)B.lev, k / 2,
-                           (const uint32_t*)B.list[k / 2][k % 2], n, Ls->head[k], (const uint32_t*)Ls->off[k],
-                           Ls->ovf + Ls->ovf_base[k]);
+    if ((e = grow(&Ls->ent, &Ls->ent_cap, bytes)) != hipSuccess) return e;
+    p = (char*)Ls->ent;
+    for (int k = 0; k < OCT_LISTS; k++) {
+        Ls->head[k] = (uint32_t*)p;
+        p += up256(4 * (size_t)Ls->width[k] * Ls->counts[k]);
+        Ls->ovf[k] = (uint32_t*)p;
+        p += up256(4 * (size_t)over[k]);
     }
+    oct_segs(B, *Ls, 0xFF, &t);
+    hipLaunchKernelGGL(k_oct_fill, dim3(blocks), dim3(OCT_BLOCK), 0, s, g, (const uint8_t*)B.lev, t);
     return hipGetLastError();
 }
 
 void octree_free_lists(OctreeLists* Ls) {
     if (!Ls) return;
-    for (void** p : {&Ls->dyn, (void**)&Ls->ovf, &Ls->scan})
+    for (void** p : {&Ls->dyn, &Ls->ent})
         if (*p) (void)hipFree(*p);
-    Ls->dyn = Ls->scan = nullptr;
-    Ls->ovf = nullptr;
-    Ls->dyn_cap = Ls->ovf_cap = Ls->scan_cap = 0;
+    Ls->dyn = Ls->ent = nullptr;
+    Ls->dyn_cap = Ls->ent_cap = 0;
 }
 
 int launch_octree_sweeps(const Dims& d, const OctreeBufs& B, const OctreeLists& Ls, int iters, const float* mean,
                          hipStream_t s) {
-    const OG g{d.W, d.H, d.D};
-    const OctW wt = make_weights();
-    uint32_t nmax = 0;
-    for (int k = 0; k < 8; k++) {
-        const uint32_t n = Ls.counts[k];
-        nmax = std::max(nmax, n);
-        if (n)
-            hipLaunchKernelGGL(k_oct_rhs, dim3(blocks_of(n, 256)), dim3(256), 0, s, g, k / 2,
-                               (const uint32_t*)B.list[k / 2][k % 2], n, (const float*)B.d[k / 2], mean, Ls.rhs[k]);
+    OctSegs<OCT_LISTS> all{};
+    const uint32_t blocks = oct_segs(B, Ls, 0xFF, &all);
+    if (!blocks) return 0;
+    const LevelPtrs dl{{B.d[0], B.d[1], B.d[2], B.d[3]}};
+    hipLaunchKernelGGL(k_oct_rhs, dim3(blocks), dim3(OCT_BLOCK), 0, s, dl, all, mean);
+    if (iters <= 0) return 0;
+    OctP P{B.p[0], {}};
+    for (int L = 0; L < 4; L++) P.off[L] = (uint32_t)(B.p[L] - B.p[0]);
+    const std::vector<uint8_t> plan = oct_schedule(Ls.counts, Ls.beside, iters);
+    for (uint8_t mask : plan) {
+        OctSegs<4> t{};
+        const uint32_t nb = oct_segs(B, Ls, mask, &t);
+        hipLaunchKernelGGL(k_oct_gs, dim3(nb), dim3(OCT_BLOCK), 0, s, P, t);
     }
-    if (iters <= 0 || nmax == 0) return 0;
-    const LevelPtrs P{{B.p[0], B.p[1], B.p[2], B.p[3]}};
-    int launches = 0;
-    for (int it = 0; it < iters; it++)
-        for (int k = 0; k < 8; k++) {
-            const uint32_t n = Ls.counts[k];
-            if (!n) continue;
-            hipLaunchKernelGGL(k_oct_gs, dim3(blocks_of(n, 256)), dim3(256), 0, s, wt, P, k / 2, B.p[k / 2],
-                               (const uint32_t*)B.list[k / 2][k % 2], n, (const uint32_t*)Ls.head[k],
-                               (const uint32_t*)Ls.tot[k], (const uint32_t*)Ls.off[k],
-                               (const uint32_t*)(Ls.ovf + Ls.ovf_base[k]), (const float*)Ls.rhs[k]);
-            launches++;
-        }
-    return launches;
+    return (int)plan.size();
 }
 
 void launch_octree_adjust(const Dims& d, const OctreeBufs& B, float* u, float* v, float* w, hipStream_t s) {

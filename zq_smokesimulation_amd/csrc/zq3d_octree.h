@@ -14,6 +14,7 @@
 #include <stdint.h>
 
 #include "zq3d_device.h"
+#include "zq3d_octree_plan.h"
 
 namespace zq3d {
 
@@ -27,28 +28,32 @@ struct OctreeBufs {
     float* p[4];                // pressure per level
     float* d[4];                // divergence per level
     uint32_t* list[4][2];       // per level and colour: the linear level index of every cell solved
-    uint32_t* count;            // 8 list lengths (level-major, colour-minor), then 8 overflow totals
+    uint32_t* count;            // OCT_LISTS values each (level-major, colour-minor): list lengths, entries
+                                // beyond the heads, most entries of a cell, levels the entries name
 };
 
+constexpr uint32_t OCT_WIDE = 24;  // most entries per cell kept in the transposed head
+
 // Per list k = 2 L + colour: the neighbour entries of its cells (the reference's
-// _selectInfos_for_CUDAOpenPoissonRedBlack3 lists, built on the device) and their right-hand sides,
-// rebuilt with the leaves in grow-only device buffers owned here.  head holds each cell's first six
-// entries transposed (entry j of cell i at j * n + i); the rest of a cell's entries sit in ovf at
-// ovf_base[k] + off[k][i].
+// _selectInfos_for_CUDAOpenPoissonRedBlack3 lists, built on the device), the sums of their weights
+// and their right-hand sides, rebuilt with the leaves in grow-only device buffers owned here.  head
+// holds each cell's first `width` entries transposed (entry j of cell i at j * n + i; six, twelve or
+// OCT_WIDE of them, as the list's fullest cell needs: a flat step between two levels gives nine, a
+// corner fifteen, one step on every face OCT_WIDE); the rest of a cell's entries sit in ovf.
 struct OctreeLists {
-    uint32_t counts[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // cells per level and colour
-    uint32_t* head[8] = {};
-    uint32_t* tot[8] = {};    // entries per cell
-    uint32_t* ovc[8] = {};    // entries beyond the head per cell (n + 1 values, last 0)
-    uint32_t* off[8] = {};    // exclusive sums of ovc
-    float* rhs[8] = {};       // right-hand side per cell, in list order
-    size_t ovf_base[8] = {};
-    void* dyn = nullptr;
+    uint32_t counts[OCT_LISTS] = {};  // cells per level and colour
+    uint32_t* head[OCT_LISTS] = {};
+    uint32_t* ovo[OCT_LISTS] = {};  // per cell: its first entry in ovf
+    uint32_t* ovn[OCT_LISTS] = {};  // per cell: its entries there
+    uint32_t* ovf[OCT_LISTS] = {};
+    float* coeff[OCT_LISTS] = {};  // sum of the weights, in entry order
+    float* rhs[OCT_LISTS] = {};
+    int width[OCT_LISTS] = {}, over[OCT_LISTS] = {};
+    uint32_t beside[4] = {};  // bit m of beside[L]: some level-L leaf neighbours a level-m leaf
+    void* dyn = nullptr;      // ovo, ovn, coeff, rhs
     size_t dyn_cap = 0;
-    uint32_t* ovf = nullptr;
-    size_t ovf_cap = 0;
-    void* scan = nullptr;
-    size_t scan_cap = 0;
+    void* ent = nullptr;  // head, ovf
+    size_t ent_cap = 0;
 };
 
 // bytes of one OctreeBufs allocation for the grid, and the carving of `mem` into it
@@ -69,7 +74,7 @@ void octree_free_lists(OctreeLists* Ls);
 void launch_octree_prepare(const Dims& g, const float* u, const float* v, const float* w, const OctreeBufs& B,
                            hipStream_t s);
 // the right-hand sides (mean != nullptr: the closed form div - mean * 8^L), then `iters` passes of
-// level 0 red, level 0 black, ..., level 3 black, one launch per phase.  Returns the launches made.
+// level 0 red, level 0 black, ..., level 3 black, by oct_schedule.  Returns the launches made.
 int launch_octree_sweeps(const Dims& g, const OctreeBufs& B, const OctreeLists& Ls, int iters, const float* mean,
                          hipStream_t s);
 // face correction from the level pressures
