@@ -537,8 +537,8 @@ long long zq3d_ens_cells(zq3d_ens* e);
 int zq3d_ens_stream(zq3d_ens* e, void** stream);
 /* Launch-shape autotuner: times the sweep kernels -- kind 0: single-colour half sweeps for each
  * tile shape (tbx x tby cells) and persistent launch size (blocks; 0 = one workgroup per tile);
- * kind 1: one launch per red-black iteration on colour-split storage, tiles of tbx slots x tby rows
- * x `blocks` planes (the default before any autotune is 64 x 16 x 16) -- and the cell kernels for
+ * kind 1: two red-black iterations a launch with a tile's planes in registers, tbx cells a lane x tby
+ * waves x `blocks` planes (the default before any autotune is 4 x 8 x 16) -- and the cell kernels for
  * each launch size, on the members' own grids and occupancy, and keeps the fastest.  All give the
  * same bits.  Fields are unchanged. */
 #define ZQ3D_ENS_TUNE_MAX 24
@@ -552,7 +552,8 @@ typedef struct zq3d_ens_tune {
     float probe_ms;        /* cell advection probe at that size */
 } zq3d_ens_tune;
 int zq3d_ens_autotune(zq3d_ens* e, int iters, zq3d_ens_tune* report);
-/* selects one of the autotuner's sweep candidates (kind, tbx, tby, blocks as reported) */
+/* selects one of the autotuner's sweep candidates (kind, tbx, tby, blocks as reported; the shapes of 64
+ * slots that kind 1 once reported select one near them) */
 int zq3d_ens_set_sweep(zq3d_ens* e, int kind, int tbx, int tby, int blocks);
 
 /* message of the last failed call on this thread ("" if none) */

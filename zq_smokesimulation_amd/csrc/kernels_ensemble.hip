@@ -6,10 +6,10 @@
 // workgroup takes tiles blockIdx.x, blockIdx.x + gridDim.x, ...; finds the member by binary search
 // over the table's prefix sums; and runs the same per-cell function (zq3d_stencils.h) that the
 // single-grid kernel runs for that cell.  Each member therefore steps bit for bit as a zq3d_sim
-// of the same configuration (plain FP32 projection).  The red-black sweep takes its tile shape
-// (TBX x TBY cells) as a template parameter chosen by the ensemble autotuner.
+// of the same configuration (plain FP32 projection).  The red-black sweeps take their tile shape from
+// the ensemble autotuner.
 #include "zq3d_ensemble.h"
-#include "zq3d_sor_split.h"
+#include "zq3d_sor_quad.h"
 #include "zq3d_stencils.h"
 
 namespace zq3d {
@@ -120,12 +120,13 @@ __global__ __launch_bounds__(NT) void ke_reinject(const EnsMember* __restrict__ 
 
 // set-up of the plain projection; the per-tile (sum, count) of the divergence goes to the member's
 // partials at the tile's index, as the single-grid set-up writes them per block
-__global__ __launch_bounds__(NT) void ke_proj_setup(const EnsMember* __restrict__ M, EnsTable T, int B) {
+__global__ __launch_bounds__(NT) void ke_proj_setup(const EnsMember* __restrict__ M, EnsTable T, int B, int quad) {
     __shared__ double red[4];
     for_tiles<64, 4>(T, B, [&](int s, int local, int i, int j, int k) {
         const EnsMember& m = M[s];
         double dsum = 0.0, dcnt = 0.0;
-        st_proj_setup_plain(m.u, m.v, m.w, m.occ, m.open_mask, m.nc, m.b, m.p, m.d, i, j, k, dsum, dcnt);
+        st_proj_setup_plain(m.u, m.v, m.w, m.occ, m.open_mask, m.nc, quad ? m.qb : m.b, m.p, m.d, i, j, k, dsum, dcnt,
+                            quad ? m.qn : nullptr);
         const double sm = block_reduce<false>(dsum, red);
         __syncthreads();
         const double ct = block_reduce<false>(dcnt, red);
@@ -157,59 +158,35 @@ __global__ __launch_bounds__(NT) void ke_sor_half(const EnsMember* __restrict__ 
     });
 }
 
-// every member's counts, right-hand side and pressure -> its colour-split arrays (pressure pair 0)
-__global__ __launch_bounds__(NT) void ke_split_in(const EnsMember* __restrict__ M, EnsTable T, int B) {
-    for_tiles<64, 4>(T, B, [&](int s, int, int i, int j, int k) {
-        const EnsMember& m = M[s];
-        if (i >= m.d.W || j >= m.d.H) return;
-        const int Wh = (m.d.W + 1) / 2, c = (i + j + k) & 1;
-        const int oh = (k * m.d.H + j) * Wh + (i >> 1);
-        m.sn[c][oh] = m.nc[cidx(m.d, i, j, k)];
-        m.sb[c][oh] = m.b[cidx(m.d, i, j, k)];
-        m.sp[c][split_q(Wh, m.d.H, i >> 1, j, k)] = m.p[pidx(m.d, i, j, k)];
-    });
-}
-
-// the pair holding every member's result (its own iteration count's parity) -> interleaved pressure
-__global__ __launch_bounds__(NT) void ke_split_out(const EnsMember* __restrict__ M, EnsTable T, int B) {
-    for_tiles<64, 4>(T, B, [&](int s, int, int i, int j, int k) {
-        const EnsMember& m = M[s];
-        if (i >= m.d.W || j >= m.d.H) return;
-        const int Wh = (m.d.W + 1) / 2, c = (i + j + k) & 1;
-        m.p[pidx(m.d, i, j, k)] = m.sp[2 * (m.iters & 1) + c][split_q(Wh, m.d.H, i >> 1, j, k)];
-    });
-}
-
-// iteration `it` of every member's SOR in one launch: one workgroup per tile of the table (members'
-// tiles numbered member after member, handed out so each XCD gets a contiguous run); iteration it
-// reads pair it & 1 and writes the other; members whose own iteration count is reached are left
-// alone
-// 8-wave workgroups are held to six waves per SIMD (80 VGPRs), so three share a CU: the LDS rings of
-// three fit in 160 KB and the ensemble's tiles are too small to keep a CU busy two at a time.
-template <int TX, int TY, int NW>
-__global__ __launch_bounds__(64 * NW, NW == 8 ? 6 : 1) void ke_sor_split_rb(const EnsMember* __restrict__ M,
-                                                                            EnsTable T, int B, int zc, int it) {
+// K iterations of every member's SOR in one launch (sor_quad_tile, each member cut by itself); tiles
+// are handed out so each XCD gets a contiguous run.  Members with an odd count run one iteration
+// first (K == 1, which takes only those, from zero); launch `at` of the pairs then takes every member
+// that still has two to do.
+template <int K, int CX, int NTH>
+__global__ __launch_bounds__(NTH) void ke_sor_quad(const EnsMember* __restrict__ M, EnsQuadTable T, int at) {
+    extern __shared__ float quad_lds[];
     const int per = gridDim.x >> 3;
     const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if (tile >= T.start[B]) return;  // spare block: uniform exit before any barrier
-    const int s = tile_member(T.start, B, tile);
-    const EnsMember& m = M[s];
-    if (it >= m.iters) return;
-    const int local = tile - T.start[s];
-    const int gx = T.gx[s], gy = T.gy[s];
-    const int bx = local % gx, by = (local / gx) % gy, z0 = (local / (gx * gy)) * zc;
-    const int src = it & 1;
-    sor_split_rb_tile<TX, TY, NW>(m.sn[0], m.sn[1], m.sb[0], m.sb[1], *m.mean32, m.sp[2 * src], m.sp[2 * src + 1],
-                                  m.sp[2 - 2 * src], m.sp[3 - 2 * src], m.d, (m.d.W + 1) / 2, bx * TX, by * TY, z0,
-                                  min(z0 + zc, m.d.D), m.omega, m.omw);
+    if (tile >= T.total) return;  // spare block: uniform exit before any barrier
+    const EnsQuadTile t = T.tiles[tile];
+    const EnsMember& m = M[t.member];
+    const int odd = m.iters & 1;
+    if (K == 1 ? !odd : 2 * at + 2 > m.iters - odd) return;
+    const QuadCut c = T.cuts[t.member];
+    if ((int)threadIdx.x >= 64 * c.nw) return;  // a wave that this member's tiles do not need
+    const int from = K == 1 ? 0 : (odd + at) & 1;
+    const float* src = K == 1 || (at == 0 && !odd) ? nullptr : m.qp[from];
+    sor_quad_tile<K, CX, QUAD_R, true, 1, NTH>(m.qn, m.qb, *m.mean32, src, m.qp[1 - from], m.d, c, t.bx, t.by, t.bz,
+                                              m.omega, m.omw, quad_lds);
 }
 
 template <int AXIS>
-__global__ __launch_bounds__(NT) void ke_correct(const EnsMember* __restrict__ M, EnsTable T, int B) {
+__global__ __launch_bounds__(NT) void ke_correct(const EnsMember* __restrict__ M, EnsTable T, int B, int quad) {
     for_tiles<64, 4>(T, B, [&](int s, int, int i, int j, int k) {
         const EnsMember& m = M[s];
         float* face = AXIS == 0 ? m.u : (AXIS == 1 ? m.v : m.w);
-        st_correct<AXIS>(m.occ, m.open_mask, PadPressure<float>{m.p}, face, m.d, i, j, k);
+        if (quad) st_correct<AXIS>(m.occ, m.open_mask, QuadPressure{m.qres}, face, m.d, i, j, k);
+        else st_correct<AXIS>(m.occ, m.open_mask, PadPressure<float>{m.p}, face, m.d, i, j, k);
     });
 }
 
@@ -231,10 +208,8 @@ inline unsigned grid_of(const EnsTable& T, int blocks) {
 
 // tile layouts of the sweep kernel (TBX x TBY) the autotuner may pick
 const int kEnsSweepShapes[kEnsSweepShapeCount][2] = {{64, 4}, {32, 8}, {16, 16}};
-const int kEnsRbShapes[kEnsRbShapeCount][3] = {{64, 8, 8},  {64, 8, 16},  {64, 16, 8}, {64, 16, 16},
-                                               {64, 16, 32}, {64, 32, 8}, {64, 32, 16}};
 
-void ens_launch_step(const EnsLaunch& L, hipStream_t s) {
+hipError_t ens_launch_step(const EnsLaunch& L, hipStream_t s) {
     const dim3 nt(NT);
     const EnsMember* M = L.members;
     const int B = L.count;
@@ -254,23 +229,24 @@ void ens_launch_step(const EnsLaunch& L, hipStream_t s) {
     hipLaunchKernelGGL(ke_cells_to_faces<2>, dim3(gw), nt, 0, s, M, L.wfaces, B);
     // plain projection
     ens_launch_setup(L, s);
-    if (L.sweep_rb) ens_launch_split_in(L, s);
-    ens_launch_sweeps(L, 0, L.max_iters, s);
-    if (L.sweep_rb) hipLaunchKernelGGL(ke_split_out, dim3(gc), nt, 0, s, M, L.cells, B);
-    hipLaunchKernelGGL(ke_correct<0>, dim3(gu), nt, 0, s, M, L.ufaces, B);
-    hipLaunchKernelGGL(ke_correct<1>, dim3(gv), nt, 0, s, M, L.vfaces, B);
-    hipLaunchKernelGGL(ke_correct<2>, dim3(gw), nt, 0, s, M, L.wfaces, B);
+    const hipError_t e = ens_launch_sweeps(L, L.max_iters, s);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(ke_correct<0>, dim3(gu), nt, 0, s, M, L.ufaces, B, L.sweep_quad);
+    hipLaunchKernelGGL(ke_correct<1>, dim3(gv), nt, 0, s, M, L.vfaces, B, L.sweep_quad);
+    hipLaunchKernelGGL(ke_correct<2>, dim3(gw), nt, 0, s, M, L.wfaces, B, L.sweep_quad);
     // scalar advection through the projected velocity, then the sources
     hipLaunchKernelGGL(ke_mac_to_cell4, dim3(gc), nt, 0, s, M, L.cells, B);
     hipLaunchKernelGGL(ke_advect_scalar, dim3(gc), nt, 0, s, M, L.cells, B);
     hipLaunchKernelGGL(ke_copy, dim3(2048), nt, 0, s, L.T_pool, L.T2_pool, L.cell_pool_size);
     hipLaunchKernelGGL(ke_copy, dim3(2048), nt, 0, s, L.R_pool, L.R2_pool, L.cell_pool_size);
     hipLaunchKernelGGL(ke_reinject, dim3(gc), nt, 0, s, M, L.cells, B);
+    return hipGetLastError();
 }
 
 void ens_launch_setup(const EnsLaunch& L, hipStream_t s) {
-    hipLaunchKernelGGL(ke_zero, dim3(2048), dim3(NT), 0, s, L.p_pool, L.p_pool_size);
-    hipLaunchKernelGGL(ke_proj_setup, dim3(grid_of(L.cells, L.blocks)), dim3(NT), 0, s, L.members, L.cells, L.count);
+    if (!L.sweep_quad) hipLaunchKernelGGL(ke_zero, dim3(2048), dim3(NT), 0, s, L.p_pool, L.p_pool_size);
+    hipLaunchKernelGGL(ke_proj_setup, dim3(grid_of(L.cells, L.blocks)), dim3(NT), 0, s, L.members, L.cells, L.count,
+                       L.sweep_quad);
     hipLaunchKernelGGL(ke_finish_mean, dim3(L.count), dim3(1024), 0, s, L.members, L.cells);
 }
 
@@ -280,31 +256,40 @@ void ens_launch_probe(const EnsLaunch& L, hipStream_t s) {
     hipLaunchKernelGGL(ke_advect_cells, dim3(gc), dim3(NT), 0, s, L.members, L.cells, L.count);
 }
 
-void ens_launch_split_in(const EnsLaunch& L, hipStream_t s) {
-    hipLaunchKernelGGL(ke_split_in, dim3(grid_of(L.cells, L.blocks)), dim3(NT), 0, s, L.members, L.cells, L.count);
+namespace {
+
+template <int K, int CX, int NTH>
+hipError_t launch_quad(const EnsLaunch& L, const EnsQuadTable& T, int at, hipStream_t s) {
+    constexpr int lds = 4 * quad_lds_floats(K, CX, NTH);
+    if constexpr (lds > 64 * 1024) {  // above the default limit of dynamic LDS: allowed once per process
+        static const hipError_t e = hipFuncSetAttribute((const void*)ke_sor_quad<K, CX, NTH>,
+                                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (e != hipSuccess) return e;
+    }
+    const unsigned nb = (unsigned)((T.total + 7) & ~7);  // a multiple of 8 for the XCD numbering
+    hipLaunchKernelGGL((ke_sor_quad<K, CX, NTH>), dim3(nb), dim3(NTH), lds, s, L.members, T, at);
+    return hipGetLastError();
 }
 
-void ens_launch_sweeps(const EnsLaunch& L, int it0, int it1, hipStream_t s) {
+}  // namespace
+
+hipError_t ens_launch_sweeps(const EnsLaunch& L, int iters, hipStream_t s) {
     const dim3 nt(NT);
-    if (L.sweep_rb) {
-        const int r = L.sweep_rb - 1;
-        const int ty = kEnsRbShapes[r][1], zc = kEnsRbShapes[r][2];  // tiles of 64 slots
-        const EnsTable& T = L.rb[r];
-        const unsigned nb = (unsigned)((T.total + 7) & ~7);  // a multiple of 8 for the XCD numbering
-        const EnsMember* M = L.members;
-        for (int it = it0; it < it1; it++) {
-            if (ty == 8)
-                hipLaunchKernelGGL((ke_sor_split_rb<64, 8, 8>), dim3(nb), dim3(512), 0, s, M, T, L.count, zc, it);
-            else if (ty == 16)
-                hipLaunchKernelGGL((ke_sor_split_rb<64, 16, 8>), dim3(nb), dim3(512), 0, s, M, T, L.count, zc, it);
-            else
-                hipLaunchKernelGGL((ke_sor_split_rb<64, 32, 16>), dim3(nb), dim3(1024), 0, s, M, T, L.count, zc, it);
+    if (L.sweep_quad) {
+        const int r = L.sweep_quad - 1;
+        const EnsQuadTable& T = L.quad[r];
+        hipError_t e = hipSuccess;
+        if (L.any_odd && iters > 0) e = launch_quad<1, 2, 512>(L, L.quad_one, 0, s);
+        for (int at = 0; 2 * at + 2 <= iters && e == hipSuccess; at++) {
+            if (kEnsQuadShapes[r][0] == 4) e = launch_quad<2, 4, 512>(L, T, at, s);
+            else if (kEnsQuadShapes[r][1] <= 8) e = launch_quad<2, 2, 512>(L, T, at, s);
+            else e = launch_quad<2, 2, 1024>(L, T, at, s);
         }
-        return;
+        return e;
     }
     const EnsTable& H = L.half[L.sweep_shape];
     const unsigned gh = grid_of(H, L.sweep_blocks);
-    for (int it = it0; it < it1; it++)
+    for (int it = 0; it < iters; it++)
         for (int c = 0; c < 2; c++) {
             switch (L.sweep_shape) {
             case 1: hipLaunchKernelGGL((ke_sor_half<32, 8>), dim3(gh), nt, 0, s, L.members, H, L.count, c, it); break;
@@ -312,6 +297,7 @@ void ens_launch_sweeps(const EnsLaunch& L, int it0, int it1, hipStream_t s) {
             default: hipLaunchKernelGGL((ke_sor_half<64, 4>), dim3(gh), nt, 0, s, L.members, H, L.count, c, it); break;
             }
         }
+    return hipGetLastError();
 }
 
 }  // namespace zq3d

@@ -26,15 +26,17 @@ struct zq3d_ens {
     hipStream_t stream = nullptr;
     EnsLaunch L{};
     // pool offsets per member (elements)
-    std::vector<size_t> off_u, off_v, off_w, off_c, off_p, off_part, off_sc, off_sp;
+    std::vector<size_t> off_u, off_v, off_w, off_c, off_p, off_part, off_q;
     float *u = nullptr, *v = nullptr, *w = nullptr, *T = nullptr, *R = nullptr, *T2 = nullptr, *R2 = nullptr;
     uint8_t *occ = nullptr, *nc = nullptr;
     float4* vel4 = nullptr;
     float *scratch = nullptr, *b = nullptr, *p = nullptr, *mean32 = nullptr;
     double* part = nullptr;
-    uint8_t* split_n = nullptr;  // colour-split counts (2 per member), right-hand sides, pressures (4)
-    float *split_b = nullptr, *split_p = nullptr;
-    size_t Nu = 0, Nv = 0, Nw = 0, Nc = 0, Np = 0, Nparts = 0, Nsc = 0, Nsp = 0;
+    uint8_t* quad_n = nullptr;  // quad-layout counts, right-hand sides, pressures (two)
+    float *quad_b = nullptr, *quad_p[2] = {nullptr, nullptr};
+    EnsQuadTile* dev_tiles = nullptr;
+    QuadCut* dev_cuts = nullptr;
+    size_t Nu = 0, Nv = 0, Nw = 0, Nc = 0, Np = 0, Nparts = 0, Nq = 0;
     long long cells = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -44,13 +46,6 @@ struct zq3d_ens {
 namespace {
 
 int cdiv(int a, int b) { return (a + b - 1) / b; }
-
-// whether the one-launch split sweeps can serve every member (split_buffers_fit)
-bool rb_fits(const zq3d_ens* e) {
-    for (const Dims& d : e->dims)
-        if (!split_buffers_fit(d)) return false;
-    return true;
-}
 
 void drop_graph(zq3d_ens* e) {
     if (e->exec) (void)hipGraphExecDestroy(e->exec);
@@ -113,11 +108,18 @@ void build_tables(zq3d_ens* e, std::vector<int>& flat, std::vector<size_t>& at) 
         const int tbx = kEnsSweepShapes[sh][0], tby = kEnsSweepShapes[sh][1];
         add([tbx, tby](const Dims& d, int& x, int& y, int& z) { x = cdiv((d.W + 1) / 2, tbx), y = cdiv(d.H, tby), z = d.D; });
     }
-    for (int r = 0; r < kEnsRbShapeCount; r++) {
-        const int tx = kEnsRbShapes[r][0], ty = kEnsRbShapes[r][1], zc = kEnsRbShapes[r][2];
-        add([tx, ty, zc](const Dims& d, int& x, int& y, int& z) {
-            x = cdiv((d.W + 1) / 2, tx), y = cdiv(d.H, ty), z = cdiv(d.D, zc);
-        });
+}
+
+// the tiles of every member under shape {cells a lane, waves, planes} for K iterations a launch
+void quad_table(const zq3d_ens* e, int K, const int shape[3], std::vector<EnsQuadTile>& tiles,
+                std::vector<QuadCut>& cuts) {
+    for (int s = 0; s < e->count; s++) {
+        const Dims& d = e->dims[s];
+        const QuadCut c = quad_cut(d.W, d.H, d.D, K, shape[0], shape[1], shape[2]);
+        cuts.push_back(c);
+        for (int z = 0; z < c.nz; z++)
+            for (int y = 0; y < c.ny; y++)
+                for (int x = 0; x < c.nx; x++) tiles.push_back(EnsQuadTile{s, x, y, z});
     }
 }
 
@@ -168,10 +170,8 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
         e->off_c.push_back(e->Nc);
         e->off_p.push_back(e->Np);
         e->off_part.push_back(e->Nparts);
-        e->off_sc.push_back(e->Nsc);
-        e->off_sp.push_back(e->Nsp);
-        e->Nsc += 2 * split_cell_size(d);
-        e->Nsp += 4 * split_padded_size(d);
+        e->off_q.push_back(e->Nq);
+        e->Nq += quad_cells(d);
         e->Nu += z.Nu;
         e->Nv += z.Nv;
         e->Nw += z.Nw;
@@ -183,6 +183,14 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
     std::vector<int> flat;
     std::vector<size_t> at;
     build_tables(e, flat, at);
+    std::vector<EnsQuadTile> tiles;
+    std::vector<QuadCut> cuts;
+    size_t tile_at[kEnsQuadShapeCount + 1];
+    for (int r = 0; r <= kEnsQuadShapeCount; r++) {
+        tile_at[r] = tiles.size();
+        if (r < kEnsQuadShapeCount) quad_table(e, 2, kEnsQuadShapes[r], tiles, cuts);
+        else quad_table(e, 1, kEnsQuadOne, tiles, cuts);
+    }
     int bad = 0;
     bad |= ens_alloc(e, &e->u, e->Nu * 4) | ens_alloc(e, &e->v, e->Nv * 4) | ens_alloc(e, &e->w, e->Nw * 4);
     bad |= ens_alloc(e, &e->T, e->Nc * 4) | ens_alloc(e, &e->R, e->Nc * 4) | ens_alloc(e, &e->T2, e->Nc * 4) |
@@ -191,8 +199,10 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
     bad |= ens_alloc(e, &e->scratch, (e->Nu + e->Nv + e->Nw) * 4) | ens_alloc(e, &e->b, e->Nc * 4) |
            ens_alloc(e, &e->p, e->Np * 4);
     bad |= ens_alloc(e, &e->part, e->Nparts * 8) | ens_alloc(e, &e->mean32, (size_t)count * 4);
-    bad |= ens_alloc(e, &e->split_n, e->Nsc) | ens_alloc(e, &e->split_b, e->Nsc * 4) |
-           ens_alloc(e, &e->split_p, e->Nsp * 4);
+    bad |= ens_alloc(e, &e->quad_n, e->Nq) | ens_alloc(e, &e->quad_b, e->Nq * 4) |
+           ens_alloc(e, &e->quad_p[0], e->Nq * 4) | ens_alloc(e, &e->quad_p[1], e->Nq * 4);
+    bad |= ens_alloc(e, &e->dev_tiles, tiles.size() * sizeof(EnsQuadTile)) |
+           ens_alloc(e, &e->dev_cuts, cuts.size() * sizeof(QuadCut));
     bad |= ens_alloc(e, &e->dev_members, sizeof(EnsMember) * count) | ens_alloc(e, &e->dev_tables, flat.size() * 4);
     if (bad || hipStreamCreate(&e->stream) != hipSuccess) {
         set_err(where, "device allocation failed");
@@ -223,12 +233,11 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
         m.p = e->p + e->off_p[s];
         m.part = e->part + e->off_part[s];
         m.mean32 = e->mean32 + s;
-        const size_t sc = split_cell_size(d), sp = split_padded_size(d);
-        for (int c = 0; c < 2; c++) {
-            m.sn[c] = e->split_n + e->off_sc[s] + c * sc;
-            m.sb[c] = e->split_b + e->off_sc[s] + c * sc;
-        }
-        for (int q = 0; q < 4; q++) m.sp[q] = e->split_p + e->off_sp[s] + q * sp;
+        m.qn = e->quad_n + e->off_q[s];
+        m.qb = e->quad_b + e->off_q[s];
+        for (int q = 0; q < 2; q++) m.qp[q] = e->quad_p[q] + e->off_q[s];
+        // launches that write this member's pressure: the odd iteration and the pairs
+        m.qres = m.qp[(c.sor.iters + 1) / 2 & 1];
         // the single-grid launchers' host arithmetic (launch_force_atten, launch_advect_*, launch_sor)
         m.h = c.voxel_size;
         m.inv_h = step_scale<float>(c.voxel_size).inv;
@@ -251,9 +260,12 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
         m.omw = 1.0f - c.sor.omega;
         e->host.push_back(m);
         e->L.max_iters = std::max(e->L.max_iters, c.sor.iters);
+        e->L.any_odd |= c.sor.iters & 1;
     }
     Errs E;
     E(hipMemcpy(e->dev_tables, flat.data(), flat.size() * 4, hipMemcpyHostToDevice));
+    E(hipMemcpy(e->dev_tiles, tiles.data(), tiles.size() * sizeof(EnsQuadTile), hipMemcpyHostToDevice));
+    E(hipMemcpy(e->dev_cuts, cuts.data(), cuts.size() * sizeof(QuadCut), hipMemcpyHostToDevice));
     E(hipMemsetAsync(e->u, 0, e->Nu * 4, e->stream));
     E(hipMemsetAsync(e->v, 0, e->Nv * 4, e->stream));
     E(hipMemsetAsync(e->w, 0, e->Nw * 4, e->stream));
@@ -263,10 +275,8 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
     E(hipMemsetAsync(e->p, 0, e->Np * 4, e->stream));
     E(hipMemsetAsync(e->nc, 0, e->Nc, e->stream));
     E(hipMemsetAsync(e->b, 0, e->Nc * 4, e->stream));
-    // slots past a row's end and the padding of the split arrays stay 0 from here on
-    E(hipMemsetAsync(e->split_n, 0, e->Nsc, e->stream));
-    E(hipMemsetAsync(e->split_b, 0, e->Nsc * 4, e->stream));
-    E(hipMemsetAsync(e->split_p, 0, e->Nsp * 4, e->stream));
+    // a member of no iterations keeps this pressure
+    E(hipMemsetAsync(e->quad_p[0], 0, e->Nq * 4, e->stream));
     if (E.e != hipSuccess) {
         set_err(where, hipGetErrorString(E.e));
         zq3d_ens_destroy(e);
@@ -284,11 +294,13 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
     L.vfaces = table_at(e, flat, at[2]);
     L.wfaces = table_at(e, flat, at[3]);
     for (int sh = 0; sh < kEnsSweepShapeCount; sh++) L.half[sh] = table_at(e, flat, at[4 + sh]);
-    for (int r = 0; r < kEnsRbShapeCount; r++) L.rb[r] = table_at(e, flat, at[4 + kEnsSweepShapeCount + r]);
+    for (int r = 0; r <= kEnsQuadShapeCount; r++) {
+        const size_t end = r < kEnsQuadShapeCount ? tile_at[r + 1] : tiles.size();
+        (r < kEnsQuadShapeCount ? L.quad[r] : L.quad_one) =
+            EnsQuadTable{e->dev_tiles + tile_at[r], e->dev_cuts + (size_t)r * count, (int)(end - tile_at[r])};
+    }
     L.sweep_shape = 0;
-    // one-launch iterations, 64 slots x 16 rows x 16 planes per workgroup, when every member's split
-    // arrays are small enough for them; else the half sweeps
-    L.sweep_rb = rb_fits(e) ? 4 : 0;
+    L.sweep_quad = kEnsQuadDefault;
     L.blocks = 0;
     L.sweep_blocks = 0;
     L.p_pool = e->p;
@@ -366,15 +378,13 @@ extern "C" int zq3d_ens_step(zq3d_ens* e, int steps, int use_graph) {
     const char* where = "zq3d_ens_step";
     if (!e || steps < 0) { set_err(where, "bad argument"); return ZQ3D_ERR_ARG; }
     if (!use_graph) {
-        for (int n = 0; n < steps; n++) ens_launch_step(e->L, e->stream);
-        ZQ_HIP(hipGetLastError(), where);
+        for (int n = 0; n < steps; n++) ZQ_HIP(ens_launch_step(e->L, e->stream), where);
         return ZQ3D_OK;
     }
     if (e->graph_stale) {
         drop_graph(e);
         ZQ_HIP(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal), where);
-        ens_launch_step(e->L, e->stream);
-        const hipError_t cap = hipGetLastError();
+        const hipError_t cap = ens_launch_step(e->L, e->stream);
         const hipError_t end = hipStreamEndCapture(e->stream, &e->graph);
         ZQ_HIP(cap, where);
         ZQ_HIP(end, where);
@@ -407,15 +417,22 @@ extern "C" int zq3d_ens_set_sweep(zq3d_ens* e, int kind, int tbx, int tby, int b
     if (kind == 0) {
         for (int sh = 0; sh < kEnsSweepShapeCount; sh++)
             if (kEnsSweepShapes[sh][0] == tbx && kEnsSweepShapes[sh][1] == tby && blocks >= 0) {
-                L.sweep_rb = 0;
+                L.sweep_quad = 0;
                 L.sweep_shape = sh;
                 L.sweep_blocks = blocks;
                 ok = true;
             }
-    } else if (kind == 1 && rb_fits(e)) {
-        for (int r = 0; r < kEnsRbShapeCount; r++)
-            if (kEnsRbShapes[r][0] == tbx && kEnsRbShapes[r][1] == tby && kEnsRbShapes[r][2] == blocks) {
-                L.sweep_rb = r + 1;
+                L.sweep_quad = 0;
+    } else if (kind == 1) {
+        // the 64-slot shapes of the one-iteration launches that these sweeps replaced: same bits
+        static const int old[][2] = {{8, 8}, {8, 16}, {16, 8}, {16, 16}, {16, 32}, {32, 8}, {32, 16}};
+        if (tbx == 64)
+            for (const auto& o : old)
+                if (o[0] == tby && o[1] == blocks) tbx = 2;
+        if (tbx == 2 && tby == 32) tby = 16;
+        for (int r = 0; r < kEnsQuadShapeCount; r++)
+            if (kEnsQuadShapes[r][0] == tbx && kEnsQuadShapes[r][1] == tby && kEnsQuadShapes[r][2] == blocks) {
+                L.sweep_quad = r + 1;
                 ok = true;
             }
     }
@@ -449,15 +466,17 @@ extern "C" int zq3d_ens_autotune(zq3d_ens* e, int iters, zq3d_ens_tune* rep) {
         E(hipEventElapsedTime(&ms, a, b));
         return ms;
     };
-    // the sweeps run on the live counts and right-hand sides (interleaved and colour-split)
-    ens_launch_setup(e->L, e->stream);
-    ens_launch_split_in(e->L, e->stream);
-    int best_sh = 0, best_sb = 0, best_rb = 0;
+    // the sweeps run on the live counts and right-hand sides (interleaved and quad layout)
+    for (int q = 0; q < 2; q++) {
+        L.sweep_quad = q;
+        ens_launch_setup(L, e->stream);
+    }
+    int best_sh = 0, best_sb = 0, best_quad = 0;
     float best = -1.0f;
     int n = 0;
-    auto consider = [&](int tbx, int tby, int blk, float us, int sh, int sb, int rb) {
+    auto consider = [&](int tbx, int tby, int blk, float us, int sh, int sb, int quad) {
         if (rep && n < ZQ3D_ENS_TUNE_MAX) {
-            rep->kind[n] = rb ? 1 : 0;
+            rep->kind[n] = quad ? 1 : 0;
             rep->tbx[n] = tbx;
             rep->tby[n] = tby;
             rep->blocks[n] = blk;
@@ -468,25 +487,26 @@ extern "C" int zq3d_ens_autotune(zq3d_ens* e, int iters, zq3d_ens_tune* rep) {
             best = us;
             best_sh = sh;
             best_sb = sb;
-            best_rb = rb;
+            best_quad = quad;
         }
     };
-    L.sweep_rb = 0;
+    L.sweep_quad = 0;
     for (int sh = 0; sh < kEnsSweepShapeCount; sh++)
         for (int bi = 0; bi < nb; bi++) {
             L.sweep_shape = sh;
             L.sweep_blocks = blocks[bi];
-            const float ms = time_it([&] { ens_launch_sweeps(L, 0, iters, e->stream); });
+            const float ms = time_it([&] { E(ens_launch_sweeps(L, iters, e->stream)); });
             consider(kEnsSweepShapes[sh][0], kEnsSweepShapes[sh][1], blocks[bi], 1e3f * ms / iters, sh, blocks[bi], 0);
         }
-    for (int r = 0; r < kEnsRbShapeCount && rb_fits(e); r++) {
-        L.sweep_rb = r + 1;
-        const float ms = time_it([&] { ens_launch_sweeps(L, 0, iters, e->stream); });
-        consider(kEnsRbShapes[r][0], kEnsRbShapes[r][1], kEnsRbShapes[r][2], 1e3f * ms / iters, 0, 0, r + 1);
+    const int even = (iters + 1) & ~1;  // two iterations a launch
+    for (int r = 0; r < kEnsQuadShapeCount; r++) {
+        L.sweep_quad = r + 1;
+        const float ms = time_it([&] { E(ens_launch_sweeps(L, even, e->stream)); });
+        consider(kEnsQuadShapes[r][0], kEnsQuadShapes[r][1], kEnsQuadShapes[r][2], 1e3f * ms / even, 0, 0, r + 1);
     }
     L.sweep_shape = best_sh;
     L.sweep_blocks = best_sb;
-    L.sweep_rb = best_rb;
+    L.sweep_quad = best_quad;
     int best_b = 0;
     float best_cell = -1.0f;
     for (int bi = 0; bi < nb; bi++) {
@@ -505,10 +525,10 @@ extern "C" int zq3d_ens_autotune(zq3d_ens* e, int iters, zq3d_ens_tune* rep) {
     e->graph_stale = true;
     if (rep) {
         rep->count = n;
-        rep->best_kind = best_rb ? 1 : 0;
-        rep->best_tbx = best_rb ? kEnsRbShapes[best_rb - 1][0] : kEnsSweepShapes[best_sh][0];
-        rep->best_tby = best_rb ? kEnsRbShapes[best_rb - 1][1] : kEnsSweepShapes[best_sh][1];
-        rep->best_sweep_blocks = best_rb ? kEnsRbShapes[best_rb - 1][2] : best_sb;
+        rep->best_kind = best_quad ? 1 : 0;
+        rep->best_tbx = best_quad ? kEnsQuadShapes[best_quad - 1][0] : kEnsSweepShapes[best_sh][0];
+        rep->best_tby = best_quad ? kEnsQuadShapes[best_quad - 1][1] : kEnsSweepShapes[best_sh][1];
+        rep->best_sweep_blocks = best_quad ? kEnsQuadShapes[best_quad - 1][2] : best_sb;
         rep->best_us_per_iter = best;
         rep->best_blocks = best_b;
         rep->probe_ms = best_cell;

@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include "zq3d_device.h"
+#include "zq3d_quad_cut.h"
 
 namespace zq3d {
 
@@ -21,11 +22,10 @@ struct EnsMember {
     float4* vel4;    // cell velocity; also the vorticity scratch of the force stage
     float* scratch;  // 3N: cell force, then advected cell velocity
     float *b, *p;    // divergence, padded pressure
-    // colour-split SOR storage: counts and right-hand side per colour, padded pressure per
-    // (pair, colour) at sp[2 * pair + colour]; the one-launch iteration ping-pongs between pairs
-    uint8_t* sn[2];
-    float* sb[2];
-    float* sp[4];
+    // quad-layout SOR storage (zq3d_sor_quad.h): counts, right-hand side, the two pressures the sweeps
+    // ping-pong between and the one that ends up with the result
+    uint8_t* qn;
+    float *qb, *qp[2], *qres;
     double* part;    // (sum, count) per set-up tile
     float* mean32;
     float h, dt, dth, two_h, ch, dtt;
@@ -50,9 +50,27 @@ struct EnsTable {
 
 constexpr int kEnsSweepShapeCount = 3;
 extern const int kEnsSweepShapes[kEnsSweepShapeCount][2];  // TBX x TBY of the sweep kernel
-// slots x rows x planes per workgroup of the one-launch red-black iteration on colour-split storage
-constexpr int kEnsRbShapeCount = 7;
-extern const int kEnsRbShapes[kEnsRbShapeCount][3];
+// cells a lane x waves x planes of the sweeps that run two red-black iterations a launch.  64 members
+// of 32 to 96 cells an axis (17.5 M cells), us per iteration: 43.4, 36.6, 37.6 / 41.9, 37.5, 41.2 with
+// two cells a lane, 28.7 with four and 16 planes (the one-iteration launches on colour-split storage
+// that these replace took 83.9, the half sweeps at best 175): with thousands of tiles it is issue
+// that counts, and four cells a lane share the row's neighbours best.
+constexpr int kEnsQuadShapeCount = 9;
+constexpr int kEnsQuadShapes[kEnsQuadShapeCount][3] = {{2, 8, 8},   {2, 8, 16}, {2, 8, 32}, {2, 16, 8}, {2, 16, 16},
+                                                       {2, 16, 32}, {4, 8, 12}, {4, 8, 16}, {4, 8, 24}};
+constexpr int kEnsQuadDefault = 8;  // sweep_quad of a new ensemble
+constexpr int kEnsQuadOne[3] = {2, 8, 8};  // the shape of the launch of one iteration
+
+struct EnsQuadTile {
+    int member, bx, by, bz;
+};
+
+// Every member's tiles, member after member, and how each member is cut.
+struct EnsQuadTable {
+    const EnsQuadTile* tiles;
+    const QuadCut* cuts;
+    int total;
+};
 
 struct EnsLaunch {
     const EnsMember* members;  // device array
@@ -60,8 +78,9 @@ struct EnsLaunch {
     EnsTable cells, ufaces, vfaces, wfaces;
     EnsTable half[kEnsSweepShapeCount];  // half-row grids of the sweep, one per tile shape
     int sweep_shape;                     // index into kEnsSweepShapes
-    EnsTable rb[kEnsRbShapeCount];       // tile tables of the one-launch iteration, one per shape
-    int sweep_rb;                        // 0: half sweeps of sweep_shape; r > 0: kEnsRbShapes[r - 1]
+    EnsQuadTable quad[kEnsQuadShapeCount], quad_one;
+    int sweep_quad;                      // 0: half sweeps of sweep_shape; r > 0: kEnsQuadShapes[r - 1]
+    int any_odd;                         // some member's iteration count is odd
     int blocks;                          // workgroups of the persistent launches (<= 0: one per tile)
     int sweep_blocks;
     int max_iters;
@@ -70,15 +89,13 @@ struct EnsLaunch {
 };
 
 // all stages of one step of every member
-void ens_launch_step(const EnsLaunch& L, hipStream_t s);
-// projection set-up of every member (pressure zeroed, counts, divergence, mean)
+hipError_t ens_launch_step(const EnsLaunch& L, hipStream_t s);
+// projection set-up of every member: counts, divergence and mean, for the selected sweep
 void ens_launch_setup(const EnsLaunch& L, hipStream_t s);
 // mac -> cell velocity and cell advection of every member: writes only scratch, so it can be
 // repeated to time launch shapes
 void ens_launch_probe(const EnsLaunch& L, hipStream_t s);
-// red-black iterations [it0, it1) of every member's SOR (on colour-split storage when sweep_rb)
-void ens_launch_sweeps(const EnsLaunch& L, int it0, int it1, hipStream_t s);
-// interleaved counts, right-hand side and pressure -> colour-split storage (pair 0)
-void ens_launch_split_in(const EnsLaunch& L, hipStream_t s);
+// `iters` red-black iterations of every member's SOR, no more than the member's own count
+hipError_t ens_launch_sweeps(const EnsLaunch& L, int iters, hipStream_t s);
 
 }  // namespace zq3d
