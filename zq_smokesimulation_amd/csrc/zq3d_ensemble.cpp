@@ -21,7 +21,7 @@ struct zq3d_ens {
     std::vector<Dims> dims;
     std::vector<EnsMember> host;  // descriptors as uploaded
     EnsMember* dev_members = nullptr;
-    int* dev_tables = nullptr;
+    EnsTile* dev_tables = nullptr;
     std::vector<void*> allocs;
     hipStream_t stream = nullptr;
     EnsLaunch L{};
@@ -80,34 +80,28 @@ int ens_alloc(zq3d_ens* e, T** p, size_t bytes) {
     return 0;
 }
 
-// tables: cells, u/v/w faces, and the half-row grid per sweep shape; each as start[count+1], gx, gy
-void build_tables(zq3d_ens* e, std::vector<int>& flat, std::vector<size_t>& at) {
-    const int B = e->count;
-    auto add = [&](auto grid_of) {
-        at.push_back(flat.size());
-        std::vector<int> start(B + 1), gx(B), gy(B);
-        int total = 0;
-        for (int s = 0; s < B; s++) {
-            int x, y, z;
-            grid_of(e->dims[s], x, y, z);
-            start[s] = total;
-            gx[s] = x;
-            gy[s] = y;
-            total += x * y * z;
-        }
-        start[B] = total;
-        flat.insert(flat.end(), start.begin(), start.end());
-        flat.insert(flat.end(), gx.begin(), gx.end());
-        flat.insert(flat.end(), gy.begin(), gy.end());
-    };
-    add([](const Dims& d, int& x, int& y, int& z) { x = cdiv(d.W, 64), y = cdiv(d.H, 4), z = d.D; });
-    add([](const Dims& d, int& x, int& y, int& z) { x = cdiv(d.W + 1, 64), y = cdiv(d.H, 4), z = d.D; });
-    add([](const Dims& d, int& x, int& y, int& z) { x = cdiv(d.W, 64), y = cdiv(d.H + 1, 4), z = d.D; });
-    add([](const Dims& d, int& x, int& y, int& z) { x = cdiv(d.W, 64), y = cdiv(d.H, 4), z = d.D + 1; });
-    for (int sh = 0; sh < kEnsSweepShapeCount; sh++) {
-        const int tbx = kEnsSweepShapes[sh][0], tby = kEnsSweepShapes[sh][1];
-        add([tbx, tby](const Dims& d, int& x, int& y, int& z) { x = cdiv((d.W + 1) / 2, tbx), y = cdiv(d.H, tby), z = d.D; });
+// blocks of tbx x tby cells (half: of half rows) of every member
+std::vector<EnsTile> block_tiles(const zq3d_ens* e, int tbx, int tby, bool half) {
+    std::vector<EnsTile> t;
+    for (int s = 0; s < e->count; s++) {
+        const Dims& d = e->dims[s];
+        const int gx = cdiv(half ? (d.W + 1) / 2 : d.W, tbx), gy = cdiv(d.H, tby);
+        int n = 0;
+        for (int z = 0; z < d.D; z++)
+            for (int b = 0; b < gx * gy; b++) t.push_back(EnsTile{s, b, n++, z});
     }
+    return t;
+}
+
+// 256 cells of a plane x kEnsPlanes planes of every member
+std::vector<EnsTile> cell_tiles(const zq3d_ens* e) {
+    std::vector<EnsTile> t;
+    for (int s = 0; s < e->count; s++) {
+        const Dims& d = e->dims[s];
+        for (int z = 0; z < d.D; z += kEnsPlanes)
+            for (int c = 0; c < d.W * d.H; c += 256) t.push_back(EnsTile{s, c, z, std::min(z + kEnsPlanes, d.D)});
+    }
+    return t;
 }
 
 // the tiles of every member under shape {cells a lane, waves, planes} for K iterations a launch
@@ -121,11 +115,6 @@ void quad_table(const zq3d_ens* e, int K, const int shape[3], std::vector<EnsQua
             for (int y = 0; y < c.ny; y++)
                 for (int x = 0; x < c.nx; x++) tiles.push_back(EnsQuadTile{s, x, y, z});
     }
-}
-
-EnsTable table_at(const zq3d_ens* e, const std::vector<int>& flat, size_t at) {
-    const int B = e->count;
-    return EnsTable{e->dev_tables + at, e->dev_tables + at + B + 1, e->dev_tables + at + 2 * B + 1, flat[at + B]};
 }
 
 int field_span(zq3d_ens* e, int s, int field, void** p, size_t* bytes) {
@@ -180,9 +169,17 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
         e->Nparts += 2 * (size_t)cdiv(d.W, 64) * cdiv(d.H, 4) * d.D;
         e->cells += (long long)z.N;
     }
-    std::vector<int> flat;
+    // tile tables: cells, set-up blocks, half-row blocks per sweep shape
+    std::vector<EnsTile> flat;
     std::vector<size_t> at;
-    build_tables(e, flat, at);
+    for (int t = 0; t < 2 + kEnsSweepShapeCount; t++) {
+        const std::vector<EnsTile> one = t == 0   ? cell_tiles(e)
+                                         : t == 1 ? block_tiles(e, 64, 4, false)
+                                                  : block_tiles(e, kEnsSweepShapes[t - 2][0], kEnsSweepShapes[t - 2][1], true);
+        at.push_back(flat.size());
+        flat.insert(flat.end(), one.begin(), one.end());
+    }
+    at.push_back(flat.size());
     std::vector<EnsQuadTile> tiles;
     std::vector<QuadCut> cuts;
     size_t tile_at[kEnsQuadShapeCount + 1];
@@ -203,7 +200,7 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
            ens_alloc(e, &e->quad_p[0], e->Nq * 4) | ens_alloc(e, &e->quad_p[1], e->Nq * 4);
     bad |= ens_alloc(e, &e->dev_tiles, tiles.size() * sizeof(EnsQuadTile)) |
            ens_alloc(e, &e->dev_cuts, cuts.size() * sizeof(QuadCut));
-    bad |= ens_alloc(e, &e->dev_members, sizeof(EnsMember) * count) | ens_alloc(e, &e->dev_tables, flat.size() * 4);
+    bad |= ens_alloc(e, &e->dev_members, sizeof(EnsMember) * count) | ens_alloc(e, &e->dev_tables, flat.size() * sizeof(EnsTile));
     if (bad || hipStreamCreate(&e->stream) != hipSuccess) {
         set_err(where, "device allocation failed");
         zq3d_ens_destroy(e);
@@ -232,6 +229,7 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
         m.b = e->b + e->off_c[s];
         m.p = e->p + e->off_p[s];
         m.part = e->part + e->off_part[s];
+        m.tiles = cdiv(d.W, 64) * cdiv(d.H, 4) * d.D;
         m.mean32 = e->mean32 + s;
         m.qn = e->quad_n + e->off_q[s];
         m.qb = e->quad_b + e->off_q[s];
@@ -263,7 +261,7 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
         e->L.any_odd |= c.sor.iters & 1;
     }
     Errs E;
-    E(hipMemcpy(e->dev_tables, flat.data(), flat.size() * 4, hipMemcpyHostToDevice));
+    E(hipMemcpy(e->dev_tables, flat.data(), flat.size() * sizeof(EnsTile), hipMemcpyHostToDevice));
     E(hipMemcpy(e->dev_tiles, tiles.data(), tiles.size() * sizeof(EnsQuadTile), hipMemcpyHostToDevice));
     E(hipMemcpy(e->dev_cuts, cuts.data(), cuts.size() * sizeof(QuadCut), hipMemcpyHostToDevice));
     E(hipMemsetAsync(e->u, 0, e->Nu * 4, e->stream));
@@ -289,11 +287,10 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
     EnsLaunch& L = e->L;
     L.members = e->dev_members;
     L.count = count;
-    L.cells = table_at(e, flat, at[0]);
-    L.ufaces = table_at(e, flat, at[1]);
-    L.vfaces = table_at(e, flat, at[2]);
-    L.wfaces = table_at(e, flat, at[3]);
-    for (int sh = 0; sh < kEnsSweepShapeCount; sh++) L.half[sh] = table_at(e, flat, at[4 + sh]);
+    auto table = [&](int t) { return EnsTable{e->dev_tables + at[t], (int)(at[t + 1] - at[t])}; };
+    L.cells = table(0);
+    L.setup = table(1);
+    for (int sh = 0; sh < kEnsSweepShapeCount; sh++) L.half[sh] = table(2 + sh);
     for (int r = 0; r <= kEnsQuadShapeCount; r++) {
         const size_t end = r < kEnsQuadShapeCount ? tile_at[r + 1] : tiles.size();
         (r < kEnsQuadShapeCount ? L.quad[r] : L.quad_one) =
@@ -305,11 +302,6 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
     L.sweep_blocks = 0;
     L.p_pool = e->p;
     L.p_pool_size = e->Np;
-    L.T_pool = e->T;
-    L.T2_pool = e->T2;
-    L.R_pool = e->R;
-    L.R2_pool = e->R2;
-    L.cell_pool_size = e->Nc;
     *out = e;
     return ZQ3D_OK;
 }

@@ -27,6 +27,7 @@ struct EnsMember {
     uint8_t* qn;
     float *qb, *qp[2], *qres;
     double* part;    // (sum, count) per set-up tile
+    int tiles;       // set-up tiles
     float* mean32;
     float h, dt, dth, two_h, ch, dtt;
     float inv_h;     // 1/h when h is a power of two (backtrace steps multiply), else 0 (they divide)
@@ -39,12 +40,17 @@ struct EnsMember {
     float sph[kEnsMaxSources][6];  // x0, y0, z0 (cells), r^2 (cells^2), rho, T
 };
 
-// Packed tile table of one grid kind: member s owns tiles [start[s], start[s+1]), a gx x gy x gz
-// grid of tiles.
+// One tile of a cell table: cells first .. first + 255 (x fastest) of a plane, planes k0 .. k1 - 1.
+// Of a block table (TBX x TBY cells of one plane): first = the block's number in the plane, k0 = in the
+// member, k1 = the plane.
+struct EnsTile {
+    int member, first, k0, k1;
+};
+constexpr int kEnsPlanes = 4;  // planes of a cell tile
+
+// Every member's tiles, member after member.
 struct EnsTable {
-    const int* start;  // count + 1
-    const int* gx;
-    const int* gy;
+    const EnsTile* tiles;
     int total;
 };
 
@@ -75,7 +81,7 @@ struct EnsQuadTable {
 struct EnsLaunch {
     const EnsMember* members;  // device array
     int count;
-    EnsTable cells, ufaces, vfaces, wfaces;
+    EnsTable cells, setup;               // cell tiles; 64 x 4 blocks of the projection set-up
     EnsTable half[kEnsSweepShapeCount];  // half-row grids of the sweep, one per tile shape
     int sweep_shape;                     // index into kEnsSweepShapes
     EnsQuadTable quad[kEnsQuadShapeCount], quad_one;
@@ -84,8 +90,8 @@ struct EnsLaunch {
     int blocks;                          // workgroups of the persistent launches (<= 0: one per tile)
     int sweep_blocks;
     int max_iters;
-    float *p_pool, *T_pool, *T2_pool, *R_pool, *R2_pool;
-    size_t p_pool_size, cell_pool_size;
+    float* p_pool;
+    size_t p_pool_size;
 };
 
 // all stages of one step of every member
