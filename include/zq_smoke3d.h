@@ -359,8 +359,11 @@ int zq3d_get_timing(zq3d_sim* sim, zq3d_timing* out);
  * launch per iteration on colour-split storage (r rows by zc = 8, 16, 32 planes per workgroup);
  * ty == -(100 + r) (r = 16, 32) is two iterations per launch on colour-split storage;
  * ty == -(1000 + 100 c + w) is two iterations per launch with the planes in registers (c = 2 or 4
- * cells per lane, w waves per workgroup, up to 16 or 8; zc planes, even, at most 64).  The default,
- * (0, 0), is the last family at the shape predicted fastest for the grid.  All produce the same bits.
+ * cells per lane, w waves per workgroup, up to 16 or 8; zc planes, even, at most 64);
+ * ty == -(100000 + 10000 log2(lx) + 100 y + z) is zc iterations (up to 8) per launch on boxes of
+ * lx x y x z threads (lx a power of two up to 64, 1024 threads at most) that hold 2 x 2 x 4 cells each
+ * in registers; a grid of one box takes all iterations at once.  The default, (0, 0), is the shape of
+ * the last two families predicted fastest for the grid.  All produce the same bits.
  * Clobbers the projection scratch (not the fields). */
 #define ZQ3D_TUNE_MAX 32
 typedef struct zq3d_tune_report {

@@ -1,4 +1,4 @@
-"""GPU: the quad-layout sweeps (several red-black iterations per launch, planes in registers) against the
+"""GPU: the quad-layout sweeps (several red-black iterations per launch, planes or boxes in registers) against the
 oracle's SOR bit for bit, at the sizes where tiles, row groups, lanes and chunks end."""
 import numpy as np
 import pytest
@@ -17,9 +17,10 @@ def project(W, H, D, shapes, iters, mask, closed, seed=3):
     sim = z.SmokeSim3D(W, H, D, sor_open_mask=mask, sor_closed_mean=0, sor_omega=1.7, sor_iters=iters)
     ref = [a.copy() for a in (u, v, w)]
     O.project(*ref, occ, mask, 0.0, 1.7, iters)
-    assert sim.sor_kernel() == "k_sor_quad"
     for shape in shapes:
         sim.set_sor_shape(*shape)
+        if shape[0]:
+            assert sim.sor_kernel() == ("k_sor_block" if shape[0] <= -100000 else "k_sor_quad")
         sim.set_state(u=u, v=v, w=w, occ=occ)
         sim.project()
         g = sim.get_state()
@@ -35,7 +36,7 @@ def project(W, H, D, shapes, iters, mask, closed, seed=3):
                                   (521, 7, 5)])
 @pytest.mark.parametrize("iters", [0, 1, 2, 5])
 def test_default_shape_at_tile_edges(dims, iters):
-    project(*dims, [(0, 0)], iters, O.OPEN_YHI | O.OPEN_XLO, False)
+    project(*dims, [(0, 0), (-1216, 4), (-1408, 8)], iters, O.OPEN_YHI | O.OPEN_XLO, False)
 
 
 # (code, grid): few and many waves, both lane widths, each on a grid that it cuts along several axes (at 140
@@ -49,10 +50,26 @@ def test_every_width_and_wave_count(code, dims):
     project(*dims, shapes, 4, O.ALL_FACES, False)
 
 
+# boxes of lx x ty x tz threads (code: log2 lx, ty, tz), one box and several along each axis, odd sizes, a
+# last box of a few cells, iteration counts that the launches do not divide
+@pytest.mark.parametrize("code,ks,dims", [((3, 8, 4), (1, 2, 3), (20, 24, 16)), ((3, 8, 4), (2,), (33, 17, 19)),
+                                          ((4, 12, 4), (1,), (20, 24, 16)), ((4, 12, 4), (1,), (3, 2, 2)),
+                                          ((2, 5, 3), (1,), (29, 23, 26)), ((6, 4, 4), (1,), (128, 9, 21)),
+                                          ((6, 6, 2), (1,), (131, 13, 13)), ((5, 6, 5), (1, 2), (65, 40, 37)),
+                                          ((1, 5, 5), (1,), (4, 21, 30)), ((4, 10, 6), (2, 3), (70, 31, 40))])
+def test_boxes_held_in_registers(code, ks, dims):
+    ty = -(100000 + 10000 * code[0] + 100 * code[1] + code[2])
+    shapes = [(ty, k) for k in ks]
+    project(*dims, shapes, 7, 0, True)
+    project(*dims, shapes, 4, O.ALL_FACES, False)
+    project(*dims, shapes, 1, O.OPEN_ZHI, False)
+
+
 def test_shapes_outside_the_range_are_refused():
     import zq_smokesimulation_amd as z
     sim = z.SmokeSim3D(40, 40, 40)
-    for s in ((-1200, 4), (-1217, 4), (-1409, 4), (-1308, 4), (-1208, 3), (-1208, 0), (-1208, 66), (-1201, 4)):
+    for s in ((-1200, 4), (-1217, 4), (-1409, 4), (-1308, 4), (-1208, 3), (-1208, 0), (-1208, 66), (-1201, 4),
+              (-130804, 0), (-130804, 9), (-130800, 2), (-100804, 2), (-170804, 1), (-161610, 1), (-120404, 2)):
         with pytest.raises(z._lib.ZQ3DError):
             sim.set_sor_shape(*s)
     sim.close()

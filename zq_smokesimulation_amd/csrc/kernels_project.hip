@@ -14,6 +14,7 @@
 // one partial per block (wave butterfly + LDS), then one block folds the partials in index order.
 #include "zq3d_device.h"
 #include "zq3d_kernels.h"
+#include "zq3d_sor_block.h"
 #include "zq3d_sor_quad.h"
 #include "zq3d_sor_split.h"
 #include "zq3d_stencils.h"
@@ -442,6 +443,21 @@ __global__ __launch_bounds__(NT) void k_sor_quad(const uint8_t* __restrict__ n, 
     const int rest = quad_div(tile, c.mnx), bx = tile - rest * c.nx;
     const int bz = quad_div(rest, c.mny), by = rest - bz * c.ny;
     sor_quad_tile<K, CX, QUAD_R, MASK, 1, NT>(n, b, *mean32, src, dst, d, c, bx, by, bz, omega, omw, quad_lds);
+}
+
+// `iters` red-black iterations of a box per workgroup (sor_block_tile), tiles numbered as k_sor_quad's.
+template <int NT>
+__global__ __launch_bounds__(NT) void k_sor_block(const uint8_t* __restrict__ n, const float* __restrict__ b,
+                                                  const float* __restrict__ mean32, const float* __restrict__ src,
+                                                  float* __restrict__ dst, Dims d, BlockCut c, int iters, float omega,
+                                                  float omw) {
+    extern __shared__ float block_lds[];
+    const int per = gridDim.x >> 3;
+    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (tile >= c.nx * c.ny * c.nz) return;  // spare block (the grid is a multiple of 8): uniform exit
+    const int rest = quad_div(tile, c.mnx), bx = tile - rest * c.nx;
+    const int bz = quad_div(rest, c.mny), by = rest - bz * c.ny;
+    sor_block_tile<false>(n, BlockWeights{}, b, *mean32, src, dst, d, c, bx, by, bz, iters, omega, omw, block_lds);
 }
 
 // Iteration `it` of a gated pass (k_sor_split_rb otherwise): it returns at once when the previous
@@ -1013,31 +1029,52 @@ QuadShape quad_decode(SorShape s) {
     const int code = -s.ty - SOR_QUAD;
     return QuadShape{code / 100, code % 100, s.zc};
 }
+SorShape block_shape(const BlockCut& c) {
+    int lg = 0;
+    while ((1 << lg) < c.lx) lg++;
+    return SorShape{-(SOR_BLOCK + 10000 * lg + 100 * c.ty + c.tz), c.K};
+}
+BlockCut block_decode(const Dims& d, SorShape s) {
+    const int code = -s.ty - SOR_BLOCK;
+    if (code / 10000 > 6 || code / 100 % 100 < 1 || code % 100 < 1) return BlockCut{};
+    return block_cut(d.W, d.H, d.D, 1 << (code / 10000), code / 100 % 100, code % 100, s.zc);
+}
 }  // namespace
 
 bool quad_shape_valid(const Dims& d, SorShape s) {
     if (!is_quad(s)) return false;
+    if (is_block(s)) {
+        const BlockCut c = block_decode(d, s);
+        // (boxes address the whole grid with 32-bit offsets)
+        return c.lx >= 2 && c.lx <= 64 && c.ty >= 1 && c.tz >= 1 && c.K >= 1 && c.K <= 8 && c.nx > 0 &&
+               quad_cells(d) < (1u << 29);
+    }
     const QuadShape q = quad_decode(s);
     if ((q.cx != 2 && q.cx != 4) || q.nw < 1 || q.nw > (q.cx == 4 ? 8 : 16) || q.zc < 2 || q.zc > 64 || q.zc % 2) return false;
     return quad_cut(d.W, d.H, d.D, 2, q.cx, q.nw, q.zc).ny > 0;
 }
 
-// The sweep shape {0, 0} stands for (computed once per handle): the cheapest cut by quad_cost, which reproduces the measured order of
-// the shapes (on 29 grids from 16^3 to 320^3 it is within 1 % of the fastest of all candidates on every
-// one).  What it gives, in microseconds per red-black iteration, beside the shape that was the default
-// (one-pass fused tiles) and the fastest of the other families (single-colour split sweeps up to 160^3,
-// one-launch split iterations above):
-//   20x24x16  3.8 (47.1, 5.3)   64^3  3.8 (49.9, 5.6)    150x97x61  6.2 (51.5, 8.7)
-//   128^3  6.3 (48.8, 10.3)     192^3  11.7 (-, 30.3)    256^3  23.8 (108, 41)
-// Small grids: a launch boundary costs 2.6 us and a chunk's serial steps 0.45 us each, so K = 2 halves
-// the launches (K = 3 and 4 measured slower: their longer pipelines cost what they save).  At 256^3 the
-// iteration moves 13 bytes a cell through the last-level cache, 26 us at the 8.4 TB/s a copy of that size
-// reaches: two iterations a pass go below it.
+// The sweep shape {0, 0} stands for (computed once per handle): the cheapest marching cut by quad_cost, or
+// the cheapest boxes where block_cost is below it.  What it gives, in microseconds per red-black
+// iteration, beside the shape that was the default (one-pass fused tiles) and the fastest of the older
+// families (single-colour split sweeps up to 160^3, one-launch split iterations above):
+//   marching:  128^3  6.3 (48.8, 10.3)   150x97x61  6.2 (51.5, 8.7)   192^3  11.7 (-, 30.3)   256^3  23.8 (108, 41)
+//   boxes (marching): 20x24x16  1.3 (3.8)   32^3  2.2 (3.6)   64^3  3.3 (3.8)   96^3  5.1 (5.9)   128^3  9.0 (5.9)
+// Marching: K = 2 halves the launches and passes; K = 3 and 4 measured slower, their longer pipelines cost
+// what they save.  At 256^3 the iteration moves 13 bytes a cell through the last-level cache, 26 us at the
+// 8.4 TB/s a copy of that size reaches: two iterations a pass go below it.  Boxes have no pipeline and one
+// round trip of loads, so three iterations a launch pay until their halo outgrows them (about 110^3).
 QuadPlan quad_plan(const Dims& d) {
     double t2 = 0.0, t4 = 0.0;
     const QuadCut c2 = quad_best_cut(d.W, d.H, d.D, 2, 2, 16, &t2), c4 = quad_best_cut(d.W, d.H, d.D, 2, 4, 8, &t4);
     const bool four = t4 < t2;
     const QuadCut& c = four ? c4 : c2;
+    double tb = 0.0;
+    const BlockCut cb = block_best_cut(d.W, d.H, d.D, 40, BLOCK_THREADS, &tb);
+    // (predictions that close are in favour of the marching cuts, which lose less when wrong: at 64x64x256
+    // both are 4.8, measured 5.8 against 5.1)
+    if (cb.nx && 2.0 * tb < 0.9 * std::min(t2, t4) && quad_cells(d) < (1u << 29))
+        return QuadPlan{block_shape(cb), quad_best_cut(d.W, d.H, d.D, 1, 2, 8)};
     return QuadPlan{SorShape{-(SOR_QUAD + 100 * (four ? 4 : 2) + c.nw), c.zc}, quad_best_cut(d.W, d.H, d.D, 1, 2, 8)};
 }
 
@@ -1068,17 +1105,54 @@ hipError_t launch_quad_one(const Dims& d, const QuadBufs& q, const QuadCut& c, c
 }
 }  // namespace
 
+namespace {
+template <int NT>
+hipError_t launch_block_one(const Dims& d, const QuadBufs& q, const BlockCut& c, const float* src, float* dst,
+                            const float* mean32, int iters, float omega, hipStream_t s) {
+    const int lds = block_lds_bytes(c);
+    static const hipError_t e = hipFuncSetAttribute((const void*)k_sor_block<NT>,
+                                                    hipFuncAttributeMaxDynamicSharedMemorySize, 32 + 96 * (NT + 1));
+    if (e != hipSuccess) return e;
+    const int nb = (c.nx * c.ny * c.nz + 7) & ~7;
+    hipLaunchKernelGGL(k_sor_block<NT>, dim3(nb), dim3((block_threads(c) + 63) & ~63), lds, s, q.n, q.b, mean32, src,
+                       dst, d, c, iters, omega, 1.0f - omega);
+    return hipGetLastError();
+}
+
+// c.K iterations a launch; a grid of one box (no halo) runs them all in one, up to a bound that keeps a
+// launch within milliseconds
+int launch_block_sweeps(const Dims& d, const QuadBufs& q, const float* mean32, float omega, int iters, SorShape shape,
+                        hipStream_t s, hipError_t* err) {
+    const BlockCut c = block_decode(d, shape);
+    const int most = c.halo ? c.K : BLOCK_MOST;
+    int from = 0;
+    const float* src = nullptr;
+    for (int it = 0; it < iters && *err == hipSuccess;) {
+        const int k = std::min(most, iters - it);
+        float* dst = q.p[1 - from];
+        if (block_threads(c) <= 512) *err = launch_block_one<512>(d, q, c, src, dst, mean32, k, omega, s);
+        else *err = launch_block_one<1024>(d, q, c, src, dst, mean32, k, omega, s);
+        it += k;
+        src = dst;
+        from = 1 - from;
+    }
+    return from;
+}
+}  // namespace
+
 // iters iterations from zero: pairs of them in one launch, an odd one on its own (first, so that the
 // launch without a source to read is the cheap one)
 int launch_quad_sweeps(const Dims& d, const QuadBufs& q, const float* mean32, float omega, int iters, SorShape shape,
                        hipStream_t s, hipEvent_t ev0, hipEvent_t ev1, hipError_t* err) {
-    const QuadShape qs = quad_decode(shape);
-    const QuadCut c2 = quad_cut(d.W, d.H, d.D, 2, qs.cx, qs.nw, qs.zc);
     *err = hipSuccess;
     if (ev0) (void)hipEventRecord(ev0, s);
     int from = 0;
     const float* src = nullptr;
-    for (int it = 0; it < iters && *err == hipSuccess;) {
+    const bool block = is_block(shape);
+    if (block) from = launch_block_sweeps(d, q, mean32, omega, iters, shape, s, err);
+    const QuadShape qs = quad_decode(shape);
+    const QuadCut c2 = block ? QuadCut{} : quad_cut(d.W, d.H, d.D, 2, qs.cx, qs.nw, qs.zc);
+    for (int it = block ? iters : 0; it < iters && *err == hipSuccess;) {
         float* dst = q.p[1 - from];
         if ((iters - it) & 1) {
             *err = launch_quad_one<1, 2, 512>(d, q, q.plan.one, src, dst, mean32, omega, s);
@@ -1256,8 +1330,8 @@ float* launch_sor(const Dims& d, const uint8_t* nc, const float* b, const float*
 }
 
 const char* sor_kernel_name(const Dims& d, SorShape shape) {
-    if (shape.ty == 0 && shape.zc == 0) return "k_sor_quad";
-    if (is_quad(shape)) return "k_sor_quad";
+    if (shape.ty == 0 && shape.zc == 0) return is_block(quad_plan(d).def) ? "k_sor_block" : "k_sor_quad";
+    if (is_quad(shape)) return is_block(shape) ? "k_sor_block" : "k_sor_quad";
     if (shape.ty == SOR_SPLIT) return "k_sor_split";
     if (shape.ty <= -SOR_TWO) return "k_sor_split_rb2";
     if (is_split(shape)) return "k_sor_split_rb";
@@ -1265,6 +1339,11 @@ const char* sor_kernel_name(const Dims& d, SorShape shape) {
 }
 
 long long sor_launches(const Dims& d, SorShape shape, int iters) {
+    if (is_block(shape)) {
+        const BlockCut c = block_decode(d, shape);
+        const int most = c.halo ? c.K : BLOCK_MOST;
+        return (iters + most - 1) / most;
+    }
     if (is_quad(shape)) return (iters + 1) / 2;
     if (shape.ty == SOR_SPLIT) return 2LL * iters;
     if (shape.ty <= -SOR_TWO) return (iters + 1) / 2;
@@ -1295,6 +1374,7 @@ int sor_shape_candidates(const Dims& d, SorShape* out, int max) {
         if (n < max && sor_shape_valid(d, sh)) out[n++] = sh;
     };
     add(quad_plan(d).def);
+    add(block_shape(block_best_cut(d.W, d.H, d.D, 40, BLOCK_THREADS)));
     static const int nws[] = {4, 8, 12, 16};
     static const int zcs[] = {4, 8, 12, 16};
     for (int nw : nws)

@@ -103,7 +103,11 @@ struct SorShape {
 // ty == -(SOR_QUAD + 100 cx + nw): two iterations per launch on the quad layout (zq3d_sor_quad.h), cx (2 or 4)
 // cells a lane, tiles of nw waves (1 to 16; with cx 4 up to 8) and zc planes (even)
 constexpr int SOR_QUAD = 1000;
-inline bool is_quad(SorShape s) { return s.ty <= -SOR_QUAD; }
+// ty == -(SOR_BLOCK + 10000 log2(lx) + 100 ty + tz): zc iterations per launch on the quad layout, boxes of
+// lx x ty x tz threads of 2 x 2 x 4 cells (zq3d_sor_block.h); a grid of one box takes a whole pass at once
+constexpr int SOR_BLOCK = 100000;
+inline bool is_block(SorShape s) { return s.ty <= -SOR_BLOCK; }
+inline bool is_quad(SorShape s) { return s.ty <= -SOR_QUAD; }  // the quad layout: either kind
 inline bool is_split(SorShape s) { return s.ty <= SOR_SPLIT && !is_quad(s); }
 // the one-launch split shapes, whose first iteration can take the source pair as zeros unread
 inline bool split_zero_start(SorShape s) { return s.ty < SOR_SPLIT && s.ty > -SOR_TWO; }
