@@ -336,7 +336,9 @@ def coarse_leg(args):
     rec, tm, sweep = scene_leg(FINE256, args.coarse_steps, args.warmup,
                                "expsimu3D/fine256.txt: 256^3, COARSE_OPEN_POISSON_SOR, subSize 8 (32^3 coarse "
                                "grid), maxIter 600, internal sphere, box source")
-    rec["coarse_sweep_schedule"] = {"iterations_per_launch": sweep[0], "planes_per_workgroup": sweep[1]}
+    # zc < 0: boxes held in registers, coded -(10000 log2(lx) + 100 ty + tz) threads
+    rec["coarse_sweep_schedule"] = {"iterations_per_launch": sweep[0],
+                                    "box" if sweep[1] < 0 else "planes_per_workgroup": sweep[1]}
     rec["coarse_sweep_launches_per_step"] = tm["sor_launches"] / max(tm["steps"], 1)
     return rec
 

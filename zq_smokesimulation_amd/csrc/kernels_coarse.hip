@@ -17,6 +17,7 @@
 
 #include "zq3d_coarse.h"
 #include "zq3d_kernels.h"
+#include "zq3d_sor_block.h"
 
 namespace zq3d {
 namespace {
@@ -358,6 +359,45 @@ __global__ __launch_bounds__(1024) void k_coarse_slab(CG g, const float* __restr
     const int zend = min(z0 + zc, g.Dc);
     for (int e = threadIdx.x; e < (zend - z0) * PS; e += blockDim.x)
         dst[(size_t)(z0 + 1) * PS + e] = P[(z0 - L.zlo) * PS + e];
+}
+
+// The operator in the quad layout for the boxes below: weights of every cell's low faces, 1/diagonal and
+// divergence, zeros in a row's padding.
+__global__ __launch_bounds__(256) void k_coarse_pack(CG g, CoarseBufs B) {
+    const int S = quad_stride(g.Wc);
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (size_t)S * g.Hc * g.Dc) return;
+    const int i = (int)(t % S), j = (int)((t / S) % g.Hc), k = (int)(t / ((size_t)S * g.Hc));
+    const bool in = i < g.Wc;
+    B.qx[t] = in ? B.rU[c_u(g, i, j, k)] : 0.0f;
+    B.qy[t] = in ? B.rV[c_v(g, i, j, k)] : 0.0f;
+    B.qz[t] = in ? B.rW[c_w(g, i, j, k)] : 0.0f;
+    B.qi[t] = in ? B.inv[c_c(g, i, j, k)] : 0.0f;
+    B.qd[t] = in ? B.div[c_c(g, i, j, k)] : 0.0f;
+}
+
+// quad layout -> padded pressure (the ghosts stay 0)
+__global__ __launch_bounds__(256) void k_coarse_unpack(CG g, const float* __restrict__ q, float* __restrict__ p) {
+    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (size_t)g.Wc * g.Hc * g.Dc) return;
+    const int i = (int)(t % g.Wc), j = (int)((t / g.Wc) % g.Hc), k = (int)(t / ((size_t)g.Wc * g.Hc));
+    p[c_p(g, i, j, k)] = q[((size_t)k * g.Hc + j) * quad_stride(g.Wc) + i];
+}
+
+// `iters` iterations of a box per workgroup (sor_block_tile with the face weights).  The slabs above
+// spend a launch on staging seven arrays through LDS and read every operand of an update from it; here
+// the operands are registers: at 32^3 coarse cells an iteration takes
+// 2.45 us (slabs 5.8, a launch a colour 6.4), at 128^3 4.3 (6.6).
+__global__ __launch_bounds__(512) void k_coarse_block(CG g, BlockWeights w, const float* __restrict__ div,
+                                                      const float* __restrict__ src, float* __restrict__ dst, BlockCut c,
+                                                      int iters, float omega, float omw) {
+    extern __shared__ float lds[];
+    const int per = gridDim.x >> 3;
+    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (tile >= c.nx * c.ny * c.nz) return;  // spare block (the grid is a multiple of 8): uniform exit
+    const int rest = quad_div(tile, c.mnx), bx = tile - rest * c.nx;
+    const int bz = quad_div(rest, c.mny), by = rest - bz * c.ny;
+    sor_block_tile<true>(nullptr, w, div, 0.0f, src, dst, Dims{g.Wc, g.Hc, g.Dc}, c, bx, by, bz, iters, omega, omw, lds);
 }
 
 // ------------------------------------------------------------------------------ coarse delta
@@ -976,11 +1016,29 @@ bool slab_lds_enabled() {
     return ok;
 }
 
+BlockCut coarse_block(const CoarseDims& cd, CoarseSweep sw) {
+    const int code = -sw.zc;
+    if (code / 10000 < 1 || code / 10000 > 6 || code / 100 % 100 < 1 || code % 100 < 1) return BlockCut{};
+    return block_cut(cd.Wc, cd.Hc, cd.Dc, 1 << (code / 10000), code / 100 % 100, code % 100, sw.k);
+}
+
 bool coarse_sweep_valid(const CoarseDims& cd, CoarseSweep sw) {
     if (sw.k == 0) return true;
+    if (sw.zc < 0) {
+        if (sw.k < 0 || sw.k > 8) return false;
+        const BlockCut c = coarse_block(cd, sw);
+        // (boxes address the whole grid with 32-bit offsets)
+        return c.nx > 0 && block_threads(c) <= 512 && (size_t)quad_stride(cd.Wc) * cd.Hc * cd.Dc < (1u << 29);
+    }
     if (sw.k < 0 || sw.zc <= 0) return false;
     const size_t lds = coarse_slab_lds(cd, sw);
     return lds <= kSlabMaxLds && (lds <= 64 * 1024 || slab_lds_enabled());
+}
+
+long long coarse_sweep_launches(const CoarseDims& cd, CoarseSweep sw, int iters) {
+    if (sw.k <= 0) return 2LL * iters;
+    const int most = sw.zc < 0 && !coarse_block(cd, sw).halo ? BLOCK_MOST : sw.k;
+    return (iters + most - 1) / most;
 }
 
 const float* launch_coarse_sor(const CoarseDims& cd, const CoarseBufs& B, float omega, int iters, CoarseSweep sw,
@@ -994,6 +1052,27 @@ const float* launch_coarse_sor(const CoarseDims& cd, const CoarseBufs& B, float 
                 hipLaunchKernelGGL(k_coarse_sweep, dim3(blocks_for(n, 256)), dim3(256), 0, s, g, (const float*)B.rU,
                                    (const float*)B.rV, (const float*)B.rW, (const float*)B.inv, (const float*)B.div,
                                    B.p, c, omega, omw);
+        return B.p;
+    }
+    if (sw.zc < 0) {
+        const BlockCut c = coarse_block(cd, sw);
+        const int most = c.halo ? c.K : BLOCK_MOST, lds = block_lds_bytes(c);  // (512 threads: under 64 KiB)
+        const unsigned nb = (unsigned)((c.nx * c.ny * c.nz + 7) & ~7);
+        const float* from = nullptr;
+        int to = 0;
+        hipLaunchKernelGGL(k_coarse_pack, dim3(blocks_for((size_t)quad_stride(cd.Wc) * cd.Hc * cd.Dc, 256)), dim3(256),
+                           0, s, g, B);
+        for (int done = 0; done < iters;) {
+            const int k = std::min(most, iters - done);
+            hipLaunchKernelGGL(k_coarse_block, dim3(nb), dim3((block_threads(c) + 63) & ~63), lds, s, g,
+                               BlockWeights{B.qx, B.qy, B.qz, B.qi}, (const float*)B.qd, from, B.qp[to], c, k, omega,
+                               omw);
+            from = B.qp[to];
+            to = 1 - to;
+            done += k;
+        }
+        if (from)
+            hipLaunchKernelGGL(k_coarse_unpack, dim3(blocks_for(cd.Nc(), 256)), dim3(256), 0, s, g, from, B.p);
         return B.p;
     }
     float* src = B.p;
@@ -1017,6 +1096,14 @@ int coarse_sweep_candidates(const CoarseDims& cd, CoarseSweep* out, int max) {
     int n = 0;
     for (const CoarseSweep& c : all)
         if (n < max && coarse_sweep_valid(cd, c)) out[n++] = c;
+    // boxes: the plain solver's choice and the shapes that were fastest on some coarse grid of 32^3 to 128^3
+    const BlockCut c = block_best_cut(cd.Wc, cd.Hc, cd.Dc, 40, 512);
+    int lg = 0;
+    while ((1 << lg) < c.lx) lg++;
+    const CoarseSweep boxes[] = {{c.K, -(10000 * lg + 100 * c.ty + c.tz)}, {3, -30804}, {2, -30503}, {2, -30805},
+                                 {3, -40804}, {2, -31004}, {2, -40605}};
+    for (const CoarseSweep& b : boxes)
+        if (n < max && coarse_sweep_valid(cd, b)) out[n++] = b;
     return n;
 }
 

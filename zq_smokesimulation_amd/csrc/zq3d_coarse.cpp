@@ -37,6 +37,8 @@ size_t coarse_layout(const CoarseDims& cd, char* base, CoarseBufs* B) {
     f(&o->div, cd.Nc());
     f(&o->p, cd.Np());
     f(&o->p2, cd.Np());
+    const size_t nq = (size_t)quad_stride(cd.Wc) * cd.Hc * cd.Dc;
+    for (float** q : {&o->qx, &o->qy, &o->qz, &o->qi, &o->qd, &o->qp[0], &o->qp[1]}) f(q, nq);
     f(&o->vol, cd.Nc());
     if (base) o->mean = (double*)(base + off);
     off += 256;
@@ -65,8 +67,8 @@ int check_block(const Dims& d, int s, const char* where) {
 // Times every valid sweep schedule (iters iterations each, HIP events on the null stream) on the
 // coarse arrays as they stand and keeps the fastest; all schedules give the same bits.
 int tune_coarse_sweep(CoarseState* c, int iters, const char* where) {
-    CoarseSweep cand[16];
-    const int n = coarse_sweep_candidates(c->cd, cand, 16);
+    CoarseSweep cand[20];
+    const int n = coarse_sweep_candidates(c->cd, cand, 20);
     hipEvent_t a = nullptr, b = nullptr;
     ZQ_HIP(hipEventCreate(&a), where);
     ZQ_HIP(hipEventCreate(&b), where);
@@ -149,7 +151,7 @@ int project_coarse(const CoarseState& c, float* u, float* v, float* w, const uin
     const float* p = launch_coarse_sor(c.cd, c.B, o.omega, o.iters, c.sweep, s);
     if (pf) {
         ZQ_HIP(hipEventRecord(eb, s), where);
-        pf->launches += c.sweep.k > 0 ? (o.iters + c.sweep.k - 1) / c.sweep.k : 2LL * o.iters;
+        pf->launches += coarse_sweep_launches(c.cd, c.sweep, o.iters);
     }
     launch_coarse_prolong(c.cd, c.B, p, o.open_mask, occ, u, v, w, s, c.guide, c.guide_coeff);
     if (c.cd.s > 1) launch_sub_project(c.cd, c.B, occ, u, v, w, s);

@@ -38,6 +38,8 @@ struct CoarseBufs {
     float* div;              // coarse divergence
     float* p;                // padded coarse pressure (zero ghost layer)
     float* p2;               // second pressure the multi-iteration sweep ping-pongs with
+    // quad layout (zq3d_sor_block.h): weights of the low x, y, z faces, 1/diagonal, divergence, two pressures
+    float *qx, *qy, *qz, *qi, *qd, *qp[2];
     uint8_t* cocc;           // coarse occupancy
     uint8_t* regular;        // 1: the block holds no solid fine cell
     float *gU, *gV, *gW;     // guide faces (guiding control)
@@ -53,7 +55,9 @@ void launch_coarse_setup(const CoarseDims& g, const uint8_t* occ, int open_mask,
 void launch_coarse_restrict(const CoarseDims& g, const float* u, const float* v, const float* w, const CoarseBufs& B,
                             hipStream_t s);
 // Sweep schedule of the coarse SOR: k == 0 launches each colour separately; k > 0 runs k red-black
-// iterations per launch on slabs of zc z-planes (halo planes recomputed).  All give the same bits.
+// iterations per launch on slabs of zc z-planes (halo planes recomputed) or, with zc < 0, on boxes held
+// in registers (zq3d_sor_block.h), zc == -(10000 log2(lx) + 100 ty + tz) with lx x ty x tz threads a box
+// (at most 512; a grid of one box takes all iterations in one launch).  All give the same bits.
 struct CoarseSweep {
     int k, zc;
 };
@@ -63,7 +67,8 @@ int coarse_sweep_candidates(const CoarseDims& g, CoarseSweep* out, int max);
 // closed domains: div -= mean * vol on every non-solid coarse cell, mean = sum(div) / sum(vol) over
 // them in FP64 (one workgroup, fixed summation order, so repeatable)
 void launch_coarse_remove_mean(const CoarseDims& g, const CoarseBufs& B, hipStream_t s);
-// `iters` red-black iterations from B.p (colour 0 first); returns B.p or B.p2, whichever holds the result
+long long coarse_sweep_launches(const CoarseDims& g, CoarseSweep sw, int iters);
+// `iters` red-black iterations from B.p = 0 (colour 0 first); returns B.p or B.p2, whichever holds the result
 const float* launch_coarse_sor(const CoarseDims& g, const CoarseBufs& B, float omega, int iters, CoarseSweep sw,
                                hipStream_t s);
 // adds the coarse correction (pressure p; with guide != 0 also guide_coeff * (guide - coarse face))
