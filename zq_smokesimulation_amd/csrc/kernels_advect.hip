@@ -246,13 +246,13 @@ void advect_velocity_bfecc(const Dims& d, R* u, R* v, R* w, const uint8_t* occ, 
     if (mode == 3) {  // inMAC_outMAC: F1 = adv(u; u); F2 = adv(F1; -u); keep u, u = u~; adv(u~; kept) -> F1
         R* F2 = bf;
         R* K = bf + NF;
-        const MacVel<R> Vf{u, v, w, d};
-        faces_in<R>(d, Vf, Vf, occ, ou, ov, ow, ap, s);
-        faces_in<R>(d, NegVel<R, MacVel<R>>{Vf}, MacVel<R>{ou, ov, ow, d}, occ, F2, F2 + Nu, F2 + Nu + Nv, ap, s);
+        const MacVelCached<R> Vf{u, v, w, d, {}, {}, {}};
+        faces_in<R>(d, Vf, MacVel<R>{u, v, w, d}, occ, ou, ov, ow, ap, s);
+        faces_in<R>(d, NegVel<R, MacVelCached<R>>{Vf}, MacVel<R>{ou, ov, ow, d}, occ, F2, F2 + Nu, F2 + Nu + Nv, ap, s);
         increment<R>(u, F2, K, u, Nu, s);
         increment<R>(v, F2 + Nu, K + Nu, v, Nv, s);
         increment<R>(w, F2 + Nu + Nv, K + Nu + Nv, w, Nw, s);
-        faces_in<R>(d, MacVel<R>{K, K + Nu, K + Nu + Nv, d}, MacVel<R>{u, v, w, d}, occ, ou, ov, ow, ap, s);
+        faces_in<R>(d, MacVelCached<R>{K, K + Nu, K + Nu + Nv, d, {}, {}, {}}, MacVel<R>{u, v, w, d}, occ, ou, ov, ow, ap, s);
     } else {  // mode 5, inReg_outMAC: F = adv(phi; v); C = cells(F); F = adv(C; -v); C = cells(F); C = phi~; F = adv(C; v)
         V4* C = (V4*)bf;
         launch_mac_to_cell4<R>(d, u, v, w, vel4, s, occ);
@@ -302,12 +302,12 @@ void launch_advect_velocity(const Dims& d, R* u, R* v, R* w, const uint8_t* occ,
         hipLaunchKernelGGL((k_advect_faces<R, 2, RegularVelCached<R>>), grid_for(d.W, d.H, d.D + 1), blk, 0, s, V, occ,
                            ow, d, h, ap.steps, dtt);
     } else {  // mode 2: inMAC_outMAC
-        const MacVel<R> V{u, v, w, d};
-        hipLaunchKernelGGL((k_advect_faces<R, 0, MacVel<R>>), grid_for(d.W + 1, d.H, d.D), blk, 0, s, V, occ, ou, d,
+        const MacVelCached<R> V{u, v, w, d, {}, {}, {}};
+        hipLaunchKernelGGL((k_advect_faces<R, 0, MacVelCached<R>>), grid_for(d.W + 1, d.H, d.D), blk, 0, s, V, occ, ou, d,
                            h, ap.steps, dtt);
-        hipLaunchKernelGGL((k_advect_faces<R, 1, MacVel<R>>), grid_for(d.W, d.H + 1, d.D), blk, 0, s, V, occ, ov, d,
+        hipLaunchKernelGGL((k_advect_faces<R, 1, MacVelCached<R>>), grid_for(d.W, d.H + 1, d.D), blk, 0, s, V, occ, ov, d,
                            h, ap.steps, dtt);
-        hipLaunchKernelGGL((k_advect_faces<R, 2, MacVel<R>>), grid_for(d.W, d.H, d.D + 1), blk, 0, s, V, occ, ow, d,
+        hipLaunchKernelGGL((k_advect_faces<R, 2, MacVelCached<R>>), grid_for(d.W, d.H, d.D + 1), blk, 0, s, V, occ, ow, d,
                            h, ap.steps, dtt);
     }
     hipLaunchKernelGGL((k_apply_faces<R, 0>), grid_for(d.W + 1, d.H, d.D), blk, 0, s, ou, occ, u, d, is_open);
@@ -323,8 +323,8 @@ void launch_advect_scalar(const Dims& d, const R* u, const R* v, const R* w, con
     const StepScale<R> h = step_scale<R>(ap.h);
     const R dtt = (R)ap.dtt;
     if (mac) {
-        const MacVel<R> V{u, v, w, d};
-        hipLaunchKernelGGL((k_advect_scalar<R, MacVel<R>>), grid_for(d.W, d.H, d.D), blk, 0, s, V, occ, Tin, Rin, Tout,
+        const MacVelCached<R> V{u, v, w, d, {}, {}, {}};
+        hipLaunchKernelGGL((k_advect_scalar<R, MacVelCached<R>>), grid_for(d.W, d.H, d.D), blk, 0, s, V, occ, Tin, Rin, Tout,
                            Rout, d, h, ap.steps, dtt);
     } else {
         launch_mac_to_cell4<R>(d, u, v, w, vel4, s, occ);
