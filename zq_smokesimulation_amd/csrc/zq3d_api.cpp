@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "zq3d_device.h"
+#include "zq3d_hostcopy.h"
 #include "zq3d_internal.h"
 #include "zq3d_kernels.h"
 #include "zq_smoke3d.h"
@@ -57,6 +58,7 @@ struct Workspace {
     void* ptr[S_COUNT] = {};
     size_t cap[S_COUNT] = {};
     std::mutex mu;
+    HostCopy copy;
     hipError_t ensure(int slot, size_t bytes) {
         if (cap[slot] >= bytes) return hipSuccess;
         if (ptr[slot]) (void)hipFree(ptr[slot]);
@@ -72,6 +74,7 @@ struct Workspace {
             ptr[i] = nullptr;
             cap[i] = 0;
         }
+        copy.release();
     }
 };
 
@@ -498,16 +501,11 @@ extern "C" float Advect_Velocity(float* u, float* v, float* w, const bool* occup
     float* dv = (float*)W.ptr[S_V];
     float* dw = (float*)W.ptr[S_W];
     uint8_t* docc = (uint8_t*)W.ptr[S_OCC];
-    E(hipMemcpy(du, u, z.Nu * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(dv, v, z.Nv * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(dw, w, z.Nw * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(docc, occupy, z.N, hipMemcpyHostToDevice));
+    E(W.copy.to_device({{du, u, z.Nu * 4}, {dv, v, z.Nv * 4}, {dw, w, z.Nw * 4}, {docc, occupy, z.N}}));
     const AdvParams ap{g_adv.h, g_adv.dtt, (int)g_adv.steps};
     launch_advect_velocity(d, du, dv, dw, docc, is_open ? 1 : 0, mode, ap, (float4*)W.ptr[S_VEL4],
                            (float*)W.ptr[S_SCR], 0, bfecc ? (float*)W.ptr[S_BFECC] : nullptr);
-    E(hipMemcpy(u, du, z.Nu * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(v, dv, z.Nv * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(w, dw, z.Nw * 4, hipMemcpyDeviceToHost));
+    E(W.copy.to_host({{du, u, z.Nu * 4}, {dv, v, z.Nv * 4}, {dw, w, z.Nw * 4}}));
     E(hipGetLastError());
     const hipError_t e = E.e;
     const float ms = t.stop();
@@ -545,18 +543,14 @@ extern "C" float Advect_Scalar(const float* u, const float* v, const float* w, c
         set_err(where, "device allocation failed");
         return -1.0f;
     }
-    E(hipMemcpy(W.ptr[S_U], u, z.Nu * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_V], v, z.Nv * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_W], w, z.Nw * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_OCC], occupy, z.N, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_T], input_temperature, z.N * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_R], input_density, z.N * 4, hipMemcpyHostToDevice));
+    E(W.copy.to_device({{W.ptr[S_U], u, z.Nu * 4}, {W.ptr[S_V], v, z.Nv * 4}, {W.ptr[S_W], w, z.Nw * 4},
+                        {W.ptr[S_OCC], occupy, z.N}, {W.ptr[S_T], input_temperature, z.N * 4},
+                        {W.ptr[S_R], input_density, z.N * 4}}));
     const AdvParams ap{g_adv.h, g_adv.dtt, (int)g_adv.steps};
     launch_advect_scalar(d, (float*)W.ptr[S_U], (float*)W.ptr[S_V], (float*)W.ptr[S_W], (uint8_t*)W.ptr[S_OCC],
                          (float*)W.ptr[S_T], (float*)W.ptr[S_R], (float*)W.ptr[S_T2], (float*)W.ptr[S_R2],
                          mode == 0 ? 1 : 0, ap, (float4*)W.ptr[S_VEL4], 0);
-    E(hipMemcpy(output_temperature, W.ptr[S_T2], z.N * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(output_density, W.ptr[S_R2], z.N * 4, hipMemcpyDeviceToHost));
+    E(W.copy.to_host({{W.ptr[S_T2], output_temperature, z.N * 4}, {W.ptr[S_R2], output_density, z.N * 4}}));
     E(hipGetLastError());
     const hipError_t e = E.e;
     const float ms = t.stop();
@@ -583,18 +577,13 @@ extern "C" float AddForce3D(float* mac_u, float* mac_v, float* mac_w, const bool
         set_err(where, "device allocation failed");
         return -1.0f;
     }
-    E(hipMemcpy(W.ptr[S_U], mac_u, z.Nu * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_V], mac_v, z.Nv * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_W], mac_w, z.Nw * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_OCC], occupy, z.N, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_T], temperature, z.N * 4, hipMemcpyHostToDevice));
+    E(W.copy.to_device({{W.ptr[S_U], mac_u, z.Nu * 4}, {W.ptr[S_V], mac_v, z.Nv * 4}, {W.ptr[S_W], mac_w, z.Nw * 4},
+                        {W.ptr[S_OCC], occupy, z.N}, {W.ptr[S_T], temperature, z.N * 4}}));
     const ForceParams fp{deltah, deltat, buoyCoeff, 0.0f, confineCoeff, Tamb};
     launch_force_atten<float>(d, (float*)W.ptr[S_U], (float*)W.ptr[S_V], (float*)W.ptr[S_W], (float*)W.ptr[S_T],
                               nullptr, (uint8_t*)W.ptr[S_OCC], nullptr, fp, 0, 1.0f, 1.0f, 1.0f,
                               (float4*)W.ptr[S_VEL4], (float*)W.ptr[S_SCR], 0);
-    E(hipMemcpy(mac_u, W.ptr[S_U], z.Nu * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(mac_v, W.ptr[S_V], z.Nv * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(mac_w, W.ptr[S_W], z.Nw * 4, hipMemcpyDeviceToHost));
+    E(W.copy.to_host({{W.ptr[S_U], mac_u, z.Nu * 4}, {W.ptr[S_V], mac_v, z.Nv * 4}, {W.ptr[S_W], mac_w, z.Nw * 4}}));
     E(hipGetLastError());
     const hipError_t e = E.e;
     const float ms = t.stop();
@@ -625,21 +614,16 @@ extern "C" float ZQ3D_AddForce3D_ex(float* mac_u, float* mac_v, float* mac_w, co
         set_err(where, "device allocation failed");
         return -1.0f;
     }
-    E(hipMemcpy(W.ptr[S_U], mac_u, z.Nu * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_V], mac_v, z.Nv * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_W], mac_w, z.Nw * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_OCC], occupy, z.N, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_T], temperature, z.N * 4, hipMemcpyHostToDevice));
-    if (density) E(hipMemcpy(W.ptr[S_R], density, z.N * 4, hipMemcpyHostToDevice));
-    if (extra_force) E(hipMemcpy(W.ptr[S_T2], extra_force, z.N * 12, hipMemcpyHostToDevice));
+    E(W.copy.to_device({{W.ptr[S_U], mac_u, z.Nu * 4}, {W.ptr[S_V], mac_v, z.Nv * 4}, {W.ptr[S_W], mac_w, z.Nw * 4},
+                        {W.ptr[S_OCC], occupy, z.N}, {W.ptr[S_T], temperature, z.N * 4},
+                        {W.ptr[S_R], density, density ? z.N * 4 : 0},
+                        {W.ptr[S_T2], extra_force, extra_force ? z.N * 12 : 0}}));
     const ForceParams fp{deltah, deltat, buoyCoeff, gravityCoeff, confineCoeff, Tamb};
     launch_force_atten<float>(d, (float*)W.ptr[S_U], (float*)W.ptr[S_V], (float*)W.ptr[S_W], (float*)W.ptr[S_T],
                        density ? (float*)W.ptr[S_R] : nullptr, (uint8_t*)W.ptr[S_OCC],
                        extra_force ? (float*)W.ptr[S_T2] : nullptr, fp, 0, 1.0f, 1.0f, 1.0f, (float4*)W.ptr[S_VEL4],
                        (float*)W.ptr[S_SCR], 0);
-    E(hipMemcpy(mac_u, W.ptr[S_U], z.Nu * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(mac_v, W.ptr[S_V], z.Nv * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(mac_w, W.ptr[S_W], z.Nw * 4, hipMemcpyDeviceToHost));
+    E(W.copy.to_host({{W.ptr[S_U], mac_u, z.Nu * 4}, {W.ptr[S_V], mac_v, z.Nv * 4}, {W.ptr[S_W], mac_w, z.Nw * 4}}));
     E(hipGetLastError());
     const float ms = t.stop();
     if (E.e != hipSuccess) { set_err(where, hipGetErrorString(E.e)); return -1.0f; }
@@ -666,19 +650,13 @@ extern "C" float Attenuation3D(float* mac_u, float* mac_v, float* mac_w, float* 
         set_err(where, "device allocation failed");
         return -1.0f;
     }
-    E(hipMemcpy(W.ptr[S_U], mac_u, z.Nu * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_V], mac_v, z.Nv * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_W], mac_w, z.Nw * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_OCC], occupy, z.N, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_T], temperature, z.N * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_R], density, z.N * 4, hipMemcpyHostToDevice));
+    E(W.copy.to_device({{W.ptr[S_U], mac_u, z.Nu * 4}, {W.ptr[S_V], mac_v, z.Nv * 4}, {W.ptr[S_W], mac_w, z.Nw * 4},
+                        {W.ptr[S_OCC], occupy, z.N}, {W.ptr[S_T], temperature, z.N * 4},
+                        {W.ptr[S_R], density, z.N * 4}}));
     launch_attenuation(d, (float*)W.ptr[S_U], (float*)W.ptr[S_V], (float*)W.ptr[S_W], (float*)W.ptr[S_T],
                        (float*)W.ptr[S_R], (uint8_t*)W.ptr[S_OCC], velAtten, tempAtten, densityAtten, 0);
-    E(hipMemcpy(mac_u, W.ptr[S_U], z.Nu * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(mac_v, W.ptr[S_V], z.Nv * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(mac_w, W.ptr[S_W], z.Nw * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(temperature, W.ptr[S_T], z.N * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(density, W.ptr[S_R], z.N * 4, hipMemcpyDeviceToHost));
+    E(W.copy.to_host({{W.ptr[S_U], mac_u, z.Nu * 4}, {W.ptr[S_V], mac_v, z.Nv * 4}, {W.ptr[S_W], mac_w, z.Nw * 4},
+                      {W.ptr[S_T], temperature, z.N * 4}, {W.ptr[S_R], density, z.N * 4}}));
     E(hipGetLastError());
     const hipError_t e = E.e;
     const float ms = t.stop();
@@ -712,10 +690,7 @@ float solve_host(float* u, float* v, float* w, const bool* occupy, int W_, int H
     float* dv = (float*)W.ptr[S_V];
     float* dw = (float*)W.ptr[S_W];
     uint8_t* docc = (uint8_t*)W.ptr[S_OCC];
-    E(hipMemcpy(du, u, z.Nu * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(dv, v, z.Nv * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(dw, w, z.Nw * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(docc, occupy, z.N, hipMemcpyHostToDevice));
+    E(W.copy.to_device({{du, u, z.Nu * 4}, {dv, v, z.Nv * 4}, {dw, w, z.Nw * 4}, {docc, occupy, z.N}}));
     // gated passes run on colour-split storage: pressure pairs, right-hand sides, counts
     SplitBufs split{};
     if (o.mixed_precision && o.pass_rule == 2) {
@@ -740,9 +715,7 @@ float solve_host(float* u, float* v, float* w, const bool* occupy, int W_, int H
         rc = project_plain(d, du, dv, dw, docc, o, given_mean, o.closed_mean ? 1 : 0, B, st, 0);
     }
     if (rc) return -1.0f;
-    E(hipMemcpy(u, du, z.Nu * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(v, dv, z.Nv * 4, hipMemcpyDeviceToHost));
-    E(hipMemcpy(w, dw, z.Nw * 4, hipMemcpyDeviceToHost));
+    E(W.copy.to_host({{du, u, z.Nu * 4}, {dv, v, z.Nv * 4}, {dw, w, z.Nw * 4}}));
     E(hipGetLastError());
     const hipError_t e = E.e;
     const float ms = t.stop();
@@ -800,11 +773,9 @@ extern "C" float ZQ3D_MACtoRegular4(const float* mac_u, const float* mac_v, cons
         set_err(where, "device allocation failed");
         return -1.0f;
     }
-    E(hipMemcpy(W.ptr[S_U], mac_u, z.Nu * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_V], mac_v, z.Nv * 4, hipMemcpyHostToDevice));
-    E(hipMemcpy(W.ptr[S_W], mac_w, z.Nw * 4, hipMemcpyHostToDevice));
+    E(W.copy.to_device({{W.ptr[S_U], mac_u, z.Nu * 4}, {W.ptr[S_V], mac_v, z.Nv * 4}, {W.ptr[S_W], mac_w, z.Nw * 4}}));
     launch_mac_to_cell4(d, (float*)W.ptr[S_U], (float*)W.ptr[S_V], (float*)W.ptr[S_W], (float4*)W.ptr[S_VEL4], 0);
-    E(hipMemcpy(vel4, W.ptr[S_VEL4], z.N * 16, hipMemcpyDeviceToHost));
+    E(W.copy.to_host({{W.ptr[S_VEL4], vel4, z.N * 16}}));
     E(hipGetLastError());
     const hipError_t e = E.e;
     const float ms = t.stop();
@@ -1235,7 +1206,7 @@ extern "C" int zq3d_set_coarse_sweep(zq3d_sim* s, int k, int zc) {
     if (s->cfg.sub_size <= 0) { set_err(where, "the simulation has no coarse grid (sub_size == 0)"); return ZQ3D_ERR_STATE; }
     const CoarseSweep sw{k, zc};
     if (k < 0 || (k > 0 && !coarse_sweep_valid(s->coarse.cd, sw))) {
-        set_err(where, "k must be 0, or k > 0 and zc > 0 with the slab's planes within 160 KiB of LDS");
+        set_err(where, "k must be 0, or k > 0 and zc > 0 with the slab's planes within 160 KiB of LDS, or zc < 0 a valid box");
         return ZQ3D_ERR_ARG;
     }
     s->coarse.sweep = k == 0 ? CoarseSweep{0, 0} : sw;
