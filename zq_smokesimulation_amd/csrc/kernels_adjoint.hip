@@ -157,7 +157,7 @@ struct MacVelAdj {
 template <class R, class Vel>
 __device__ __forceinline__ int trace_path(const Vel& V, const uint8_t* __restrict__ occ, const Dims& d, R h,
                                           int steps, R dtt, R px, R py, R pz, R3<R>* q) {
-    OccCache oc;
+    OccCache<R> oc;
     bool open = trace_open_cached(occ, d, px, py, pz, oc);
     R3<R> vel = V(px, py, pz);
     int n = 0;
@@ -294,6 +294,7 @@ struct RevTile {
     R3<R> g;
     Cell4Taps<R> cc;
     R acc[8][3];
+    CellFloor<R> at;  // the cell of cc
     __device__ __forceinline__ void flush() {
         if (cc.i0 < 0) return;
         const int ti[8] = {cc.i0, cc.i1, cc.i0, cc.i1, cc.i0, cc.i1, cc.i0, cc.i1};
@@ -306,12 +307,17 @@ struct RevTile {
                 if (acc[t][a] != R(0)) w->add(a, ti[t], tj[t], tk[t], acc[t][a]);
     }
     __device__ __forceinline__ void step(const R3<R>& p) {
-        const Tri<R> t = cell_tri<R>(d, p);
-        if (!cc.same(t.i0, t.i1, t.j0, t.j1, t.k0, t.k1)) {
-            flush();
-            cc.fetch(vel4, d.W, d.H, t.i0, t.i1, t.j0, t.j1, t.k0, t.k1);
+        const R x = p.x - R(0.5), y = p.y - R(0.5), z = p.z - R(0.5);
+        Tri<R> t{cc.i0, cc.i1, cc.j0, cc.j1, cc.k0, cc.k1, x - at.x, y - at.y, z - at.z};
+        if (!all_of(unit_weight(t.ax), unit_weight(t.ay), unit_weight(t.az))) {
+            t = cell_tri<R>(d, p);
+            at = cell_floor<R>(x, y, z, d.W, d.H, d.D);
+            if (!cc.same(t.i0, t.i1, t.j0, t.j1, t.k0, t.k1)) {
+                flush();
+                cc.fetch(vel4, d.W, d.H, t.i0, t.i1, t.j0, t.j1, t.k0, t.k1);
 #pragma unroll
-            for (int x = 0; x < 8; x++) acc[x][0] = acc[x][1] = acc[x][2] = R(0);
+                for (int x = 0; x < 8; x++) acc[x][0] = acc[x][1] = acc[x][2] = R(0);
+            }
         }
         // put -c g at p: weights of the 8 taps (order t000 t100 t010 t110 t001 t101 t011 t111)
         const R bx = R(1) - t.ax, by = R(1) - t.ay, bz = R(1) - t.az;
@@ -338,18 +344,23 @@ struct RevTile {
 template <class R, class Vel>
 __device__ __forceinline__ int trace_box(const Vel& V, const uint8_t* __restrict__ occ, const Dims& d, R h,
                                          int steps, R dtt, R px, R py, R pz, R3<R>* q, R3<R>* last, int* box) {
-    OccCache oc;
+    OccCache<R> oc;
     bool open = trace_open_cached(occ, d, px, py, pz, oc);
     R3<R> vel = V(px, py, pz);
     int n = 0;
     int istep = 0;
     *last = R3<R>{px, py, pz};
+    CellFloor<R> at;  // the cell that went into the box last
     do {
         if (!open) break;
         const R3<R> p{px, py, pz};
         q[n++] = p;
-        const Tri<R> t = cell_tri<R>(d, p);
-        box_grow(box, t.i0, t.i1, t.j0, t.j1, t.k0, t.k1);
+        const R x = px - R(0.5), y = py - R(0.5), z = pz - R(0.5);
+        if (!all_of(unit_weight(x - at.x), unit_weight(y - at.y), unit_weight(z - at.z))) {
+            const Tri<R> t = cell_tri<R>(d, p);
+            at = cell_floor<R>(x, y, z, d.W, d.H, d.D);
+            box_grow(box, t.i0, t.i1, t.j0, t.j1, t.k0, t.k1);
+        }
         *last = p;
         px = px - (vel.x * dtt) / h;
         py = py - (vel.y * dtt) / h;

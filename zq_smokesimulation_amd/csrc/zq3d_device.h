@@ -175,21 +175,49 @@ __device__ __forceinline__ int axis_floor(R x, int n, R& a) {
     return (int)fx;
 }
 
+// The floors of a cached cell's filter coordinates.  x lies in the same cell as the cached position exactly
+// when 0 <= x - floor < 1 (the subtraction is exact there, or rounds to 1 just below a floor of -1,
+// which reads as another cell and is then looked up in full), and the difference is the weight, so a
+// step inside a cell takes one subtraction and one comparison an axis instead of the limits, the floor
+// and the conversion.  NaN, also the initial state, is no unit weight.
+template <class R>
+struct CellFloor {
+    R x = (R)NAN, y = (R)NAN, z = (R)NAN;
+};
+// The floors of a cell looked up in full (coordinates limited to [-1, n]: a floor of n stands for
+// everything above too and is looked up each time).
+template <class R>
+__device__ __forceinline__ CellFloor<R> cell_floor(int x, int y, int z, int nx, int ny, int nz) {
+    return CellFloor<R>{x < nx ? (R)x : (R)NAN, y < ny ? (R)y : (R)NAN, z < nz ? (R)z : (R)NAN};
+}
+// the same from the filter coordinates
+template <class R>
+__device__ __forceinline__ CellFloor<R> cell_floor(R x, R y, R z, int nx, int ny, int nz) {
+    R a;
+    return cell_floor<R>(axis_floor(x, nx, a), axis_floor(y, ny, a), axis_floor(z, nz, a), nx, ny, nz);
+}
+// all three, without a branch between them
+__device__ __forceinline__ bool all_of(bool a, bool b, bool c) { return ((int)a & (int)b & (int)c) != 0; }
+__device__ __forceinline__ bool unit_weight(float a) { return __builtin_bit_cast(unsigned, a) < 0x3f800000u; }
+__device__ __forceinline__ bool unit_weight(double a) { return a >= 0.0 && a < 1.0; }
+// 0 <= p <= n for a coordinate that is not -0 (n >= 0)
+__device__ __forceinline__ bool within(float p, float n) {
+    return __builtin_bit_cast(unsigned, p) <= __builtin_bit_cast(unsigned, n);
+}
+__device__ __forceinline__ bool within(double p, double n) { return p >= 0.0 && p <= n; }
+
 // The 8 taps of one trilinear cell of a 4-wide grid in the form the x-lerps use: for each x pair
 // the low tap lo and the difference hi - lo, so that lerp(lo, hi, ax) = lo + ax*(hi - lo) takes its
 // subtraction once per cell instead of once per sample (the same operations on the same values:
-// identical results).  The cell is keyed by the floors (kx, ky, kz) of the filter coordinates.
+// identical results).  (x, y, z): the floors of the filter coordinates.
 // The fourth component of a tap holds its cell's occupancy (nonzero = solid) in the grids the forward
 // backtrace samples (st_mac_to_cell4 with occupancy): bit t of `solid` is tap t's, t = x + 2y + 4z
 // over the taps 000, 100, 010, 110, 001, 101, 011, 111.
 template <class R>
 struct Cell4Lerp {
-    int kx = INT_MIN, ky = INT_MIN, kz = INT_MIN;
     unsigned solid = 0;
     R3<R> a00, d00, a10, d10, a01, d01, a11, d11;  // pairs (i0,j0,k0)-(i1,..), (i0,j1,k0), (i0,j0,k1), (i0,j1,k1)
     __device__ __forceinline__ void fetch(const vec4_t<R>* __restrict__ g, const Dims& d, int x, int y, int z) {
-        if (x == kx && y == ky && z == kz) return;
-        kx = x, ky = y, kz = z;
         const int i0 = clampi(x, 0, d.W - 1), i1 = clampi(x + 1, 0, d.W - 1);
         const int j0 = clampi(y, 0, d.H - 1), j1 = clampi(y + 1, 0, d.H - 1);
         const int k0 = clampi(z, 0, d.D - 1), k1 = clampi(z + 1, 0, d.D - 1);
@@ -219,18 +247,22 @@ struct RegularVelCached {
     Dims d;
     mutable Cell4Lerp<R> c;
     mutable R ax = R(0), ay = R(0), az = R(0);  // weights of the last prepared position
+    mutable CellFloor<R> at;                    // the cell whose taps c holds
     // taps and weights of the trilinear cell around (px, py, pz)
     __device__ __forceinline__ void prepare(R px, R py, R pz) const {
-        const int x = axis_floor(px - R(0.5), d.W, ax);
-        const int y = axis_floor(py - R(0.5), d.H, ay);
-        const int z = axis_floor(pz - R(0.5), d.D, az);
-        c.fetch(vel4, d, x, y, z);
+        const R x = px - R(0.5), y = py - R(0.5), z = pz - R(0.5);
+        ax = x - at.x, ay = y - at.y, az = z - at.z;
+        if (all_of(unit_weight(ax), unit_weight(ay), unit_weight(az))) return;
+        const int kx = axis_floor(x, d.W, ax), ky = axis_floor(y, d.H, ay), kz = axis_floor(z, d.D, az);
+        c.fetch(vel4, d, kx, ky, kz);
+        at = cell_floor<R>(kx, ky, kz, d.W, d.H, d.D);
     }
     // Whether the cell containing the prepared position is solid.  For a position inside
     // [0,W]x[0,H]x[0,D], clamp(floor(p), 0, n-1) along an axis is the high tap exactly when the
     // weight is at least 1/2 (p - 1/2 and its fraction are exact in FP32 below 2^23), so the cell
     // the reference point-samples is one of the 8 taps.
     __device__ __forceinline__ bool solid_prepared() const {
+        if (!c.solid) return false;
         const int t = (ax >= R(0.5) ? 1 : 0) | (ay >= R(0.5) ? 2 : 0) | (az >= R(0.5) ? 4 : 0);
         return (c.solid >> t) & 1u;
     }
@@ -311,14 +343,20 @@ struct MacVelCached {
     const R* w;
     Dims d;
     mutable Cell1Lerp<R> cu, cv, cw;
+    mutable CellFloor<R> at, half;  // of the faces and of the half-shifted cell centres
     __device__ __forceinline__ R3<R> operator()(R px, R py, R pz) const {
-        R fx, fy, fz, hx, hy, hz;  // weights at the faces and at the half-shifted cell centres
-        const int x = axis_floor(px, d.W + 1, fx), xh = axis_floor(px - R(0.5), d.W, hx);
-        const int y = axis_floor(py, d.H + 1, fy), yh = axis_floor(py - R(0.5), d.H, hy);
-        const int z = axis_floor(pz, d.D + 1, fz), zh = axis_floor(pz - R(0.5), d.D, hz);
-        cu.fetch(u, d.W + 1, d.H, d.D, x, yh, zh);
-        cv.fetch(v, d.W, d.H + 1, d.D, xh, y, zh);
-        cw.fetch(w, d.W, d.H, d.D + 1, xh, yh, z);
+        const R qx = px - R(0.5), qy = py - R(0.5), qz = pz - R(0.5);
+        R fx = px - at.x, fy = py - at.y, fz = pz - at.z, hx = qx - half.x, hy = qy - half.y, hz = qz - half.z;
+        if (!all_of(all_of(unit_weight(fx), unit_weight(fy), unit_weight(fz)), all_of(unit_weight(hx), unit_weight(hy), unit_weight(hz)), true)) {
+            const int x = axis_floor(px, d.W + 1, fx), xh = axis_floor(qx, d.W, hx);
+            const int y = axis_floor(py, d.H + 1, fy), yh = axis_floor(qy, d.H, hy);
+            const int z = axis_floor(pz, d.D + 1, fz), zh = axis_floor(qz, d.D, hz);
+            cu.fetch(u, d.W + 1, d.H, d.D, x, yh, zh);
+            cv.fetch(v, d.W, d.H + 1, d.D, xh, y, zh);
+            cw.fetch(w, d.W, d.H, d.D + 1, xh, yh, z);
+            at = cell_floor<R>(x, y, z, d.W + 1, d.H + 1, d.D + 1);
+            half = cell_floor<R>(xh, yh, zh, d.W, d.H, d.D);
+        }
         return R3<R>{cu.value(fx, hy, hz), cv.value(hx, fy, hz), cw.value(hx, hy, fz)};
     }
 };
@@ -337,18 +375,23 @@ struct NegVel {
 // True while the backtrace may take another step from (px,py,pz): inside [0,W]x[0,H]x[0,D] and
 // not in a solid cell (point sample, clamp).  The occupancy byte of the cell last tested is kept:
 // consecutive backtrace points usually share a cell, so most tests load nothing.
+template <class R>
 struct OccCache {
     int o = -1;
     bool open = false;
+    CellFloor<R> at;
 };
 
 template <class R>
 __device__ __forceinline__ bool trace_open_cached(const uint8_t* __restrict__ occ, const Dims& d, R px, R py, R pz,
-                                                  OccCache& c) {
-    if (!(px >= R(0) && px <= (R)d.W && py >= R(0) && py <= (R)d.H && pz >= R(0) && pz <= (R)d.D)) return false;
-    const int oi = clampi((int)zfloor(px), 0, d.W - 1);
-    const int oj = clampi((int)zfloor(py), 0, d.H - 1);
-    const int ok = clampi((int)zfloor(pz), 0, d.D - 1);
+                                                  OccCache<R>& c) {
+    if (!all_of(within(px, (R)d.W), within(py, (R)d.H), within(pz, (R)d.D))) return false;
+    if (all_of(unit_weight(px - c.at.x), unit_weight(py - c.at.y), unit_weight(pz - c.at.z))) return c.open;
+    const R fx = zfloor(px), fy = zfloor(py), fz = zfloor(pz);
+    c.at = CellFloor<R>{fx, fy, fz};
+    const int oi = clampi((int)fx, 0, d.W - 1);
+    const int oj = clampi((int)fy, 0, d.H - 1);
+    const int ok = clampi((int)fz, 0, d.D - 1);
     const int o = cidx(d, oi, oj, ok);
     if (o != c.o) {
         c.o = o;
@@ -394,7 +437,7 @@ template <class R>
 __device__ __forceinline__ R3<R> backtrace_taps(const RegularVelCached<R>& V, const Dims& d, const StepScale<R>& sc,
                                                 int steps, R dtt, R px, R py, R pz) {
     auto open_at = [&](R x, R y, R z) {
-        if (!(x >= R(0) && x <= (R)d.W && y >= R(0) && y <= (R)d.H && z >= R(0) && z <= (R)d.D)) return false;
+        if (!all_of(within(x, (R)d.W), within(y, (R)d.H), within(z, (R)d.D))) return false;
         V.prepare(x, y, z);
         return !V.solid_prepared();
     };
@@ -419,7 +462,7 @@ __device__ __forceinline__ R3<R> backtrace(const Vel& V, const uint8_t* __restri
     if constexpr (std::is_same<Vel, RegularVelCached<R>>::value)
         return backtrace_taps<R>(V, d, sc, steps, dtt, px, py, pz);
     R3<R> last{px, py, pz};
-    OccCache oc;
+    OccCache<R> oc;
     bool open = trace_open_cached(occ, d, px, py, pz, oc);
     for (int istep = 0; istep < steps; istep++) {
         if (!open) break;
