@@ -63,42 +63,67 @@ struct LevelPtrs {
 };
 
 // ---------------------------------------------------------------------------- distance field
-// x lines: one thread per (y, z) row
+// x lines: one wave per (y, z) row, 64 cells at a time; a ballot of the solid cells gives every lane the
+// nearest one at or below it (forward pass) and above it (backward pass), with the last one met carried
+// from chunk to chunk.  (One thread a row walked the row with a load a step: 345 us at 256^3.)
 __global__ __launch_bounds__(256) void k_oct_dist_x(OG g, const uint8_t* __restrict__ occ, int32_t* __restrict__ dist) {
-    const size_t line = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t line = (size_t)blockIdx.x * 4 + threadIdx.x / 64;
     if (line >= (size_t)g.H * g.D) return;
+    const int lane = threadIdx.x & 63;
     const size_t base = line * g.W;
-    int d = OCT_INF;
-    for (int i = 0; i < g.W; i++) {
-        d = occ[base + i] ? 0 : min(d + 1, OCT_INF);
-        dist[base + i] = d;
+    const unsigned long long below = ~0ull >> (63 - lane), above = ~0ull << lane;
+    int last = -1;  // the nearest solid cell before the chunk
+    for (int x0 = 0; x0 < g.W; x0 += 64) {
+        const int i = x0 + lane;
+        const unsigned long long solid = __ballot(i < g.W && occ[base + i] != 0), m = solid & below;
+        const int at = m ? x0 + 63 - __clzll((long long)m) : last;
+        if (i < g.W) dist[base + i] = at >= 0 ? i - at : OCT_INF;
+        if (solid) last = x0 + 63 - __clzll((long long)solid);
     }
-    d = OCT_INF;
-    for (int i = g.W - 1; i >= 0; i--) {
-        d = min(dist[base + i], min(d + 1, OCT_INF));
-        dist[base + i] = d;
+    int next = -1;
+    for (int x0 = (g.W - 1) / 64 * 64; x0 >= 0; x0 -= 64) {
+        const int i = x0 + lane;
+        const unsigned long long solid = __ballot(i < g.W && occ[base + i] != 0), m = solid & above;
+        const int at = m ? x0 + __ffsll(m) - 1 : next;
+        if (i < g.W && at >= 0) dist[base + i] = min(dist[base + i], at - i);
+        if (solid) next = x0 + __ffsll(solid) - 1;
     }
 }
 
-// lines along y (axis 1) or z (axis 2): one thread per (x, other) pair, x fastest across lanes
-__global__ __launch_bounds__(256) void k_oct_dist_yz(OG g, int axis, int32_t* __restrict__ dist, int finish) {
+// lines along y (axis 1) or z (axis 2): one thread per (x, other) pair, x fastest across lanes; the
+// values of OCT_AHEAD steps are in flight together (a load a step left each of the few waves waiting
+// out the memory's latency 2 n times)
+constexpr int OCT_AHEAD = 16;
+__global__ __launch_bounds__(64) void k_oct_dist_yz(OG g, int axis, int32_t* __restrict__ dist, int finish) {
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int n = axis == 1 ? g.H : g.D;
     const int other = axis == 1 ? g.D : g.H;
     if (t >= (size_t)g.W * other) return;
     const int x = (int)(t % g.W), o = (int)(t / g.W);
     const size_t stride = axis == 1 ? (size_t)g.W : (size_t)g.W * g.H;
-    const size_t base = axis == 1 ? (size_t)o * g.H * g.W + x : (size_t)o * g.W + x;
+    int32_t* const p = dist + (axis == 1 ? (size_t)o * g.H * g.W + x : (size_t)o * g.W + x);
     int d = OCT_INF;
-    for (int i = 0; i < n; i++) {
-        d = min(dist[base + i * stride], min(d + 1, OCT_INF));
-        dist[base + i * stride] = d;
+    for (int i0 = 0; i0 < n; i0 += OCT_AHEAD) {
+        int v[OCT_AHEAD];
+#pragma unroll
+        for (int q = 0; q < OCT_AHEAD; q++) v[q] = i0 + q < n ? p[(i0 + q) * stride] : OCT_INF;
+#pragma unroll
+        for (int q = 0; q < OCT_AHEAD; q++) {
+            d = min(v[q], min(d + 1, OCT_INF));
+            if (i0 + q < n) p[(i0 + q) * stride] = d;
+        }
     }
     d = OCT_INF;
-    for (int i = n - 1; i >= 0; i--) {
-        d = min(dist[base + i * stride], min(d + 1, OCT_INF));
-        // no solid cell anywhere: every distance is W + H + D (_buildOctreeInfo, :5365-5373)
-        dist[base + i * stride] = (finish && d >= OCT_INF) ? g.W + g.H + g.D : d;
+    for (int i0 = (n - 1) / OCT_AHEAD * OCT_AHEAD; i0 >= 0; i0 -= OCT_AHEAD) {
+        int v[OCT_AHEAD];
+#pragma unroll
+        for (int q = 0; q < OCT_AHEAD; q++) v[q] = i0 + q < n ? p[(i0 + q) * stride] : OCT_INF;
+#pragma unroll
+        for (int q = OCT_AHEAD - 1; q >= 0; q--) {
+            d = min(v[q], min(d + 1, OCT_INF));
+            // no solid cell anywhere: every distance is W + H + D (_buildOctreeInfo, :5365-5373)
+            if (i0 + q < n) p[(i0 + q) * stride] = (finish && d >= OCT_INF) ? g.W + g.H + g.D : d;
+        }
     }
 }
 
@@ -182,47 +207,46 @@ __global__ __launch_bounds__(256) void k_oct_restrict(OG g, int L, const float* 
 }
 
 // ---------------------------------------------------------------------------- Gauss-Seidel
-// Wave-aggregated append of `idx` to `list` where `pred` holds: one atomic per wave and list.
-__device__ __forceinline__ void wave_append(bool pred, uint32_t idx, uint32_t* list, uint32_t* count) {
-    const unsigned long long mask = __ballot(pred);
-    if (!mask) return;
-    const int lane = __lane_id();
-    const int leader = __ffsll((long long)mask) - 1;
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(count, (uint32_t)__popcll(mask));
-    base = __shfl(base, leader, 64);
-    if (pred) list[base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] = idx;
-}
-
 // The cells each sweep updates, per level and colour (red: even x + y + z at the level): every
 // level-0..2 leaf, and every level-3 leaf whose column's block at z = 0 is a leaf (the reference's
 // level-3 list test, ZQ_SmokeOctreeGrid3D.cpp:8416; the blocks that test takes that are no leaf are
 // never read, so they are left out).  Within a list the order is free: cells of one colour and level
 // never neighbour each other.
+// A workgroup counts its cells per list in LDS, takes its places with one atomic a list and writes (an
+// atomic a wave and list had all of the fine grid's waves queue at eight addresses: 170 us at 256^3).
+constexpr int OCT_LIST_CELLS = 8;  // cells a thread
 __global__ __launch_bounds__(256) void k_oct_lists(OG g, const uint8_t* __restrict__ lev, uint32_t* l00, uint32_t* l01,
                                                    uint32_t* l10, uint32_t* l11, uint32_t* l20, uint32_t* l21,
                                                    uint32_t* l30, uint32_t* l31, uint32_t* count) {
-    const size_t c = (size_t)blockIdx.x * 256 + threadIdx.x;
+    __shared__ uint32_t n[OCT_LISTS], base[OCT_LISTS];
+    if (threadIdx.x < OCT_LISTS) n[threadIdx.x] = 0u;
+    __syncthreads();
     const size_t N = (size_t)g.W * g.H * g.D;
-    const bool valid = c < N;
-    int x = 0, y = 0, z = 0, m = -1;
-    if (valid) {
-        x = (int)(c % g.W);
-        y = (int)((c / g.W) % g.H);
-        z = (int)(c / ((size_t)g.W * g.H));
-        m = lev[c];
-    }
-    uint32_t* lists[4][2] = {{l00, l01}, {l10, l11}, {l20, l21}, {l30, l31}};
+    int list[OCT_LIST_CELLS];  // -1: in none
+    uint32_t idx[OCT_LIST_CELLS], pos[OCT_LIST_CELLS];
 #pragma unroll
-    for (int L = 0; L < 4; L++) {
-        const int mask = (1 << L) - 1;
-        bool take = valid && m == L && ((x | y | z) & mask) == 0;
-        if (L == 3 && take) take = lev[oat(g, 0, x, y, 0)] == 3;
-        const int col = ((x >> L) + (y >> L) + (z >> L)) & 1;
-        const uint32_t idx = (uint32_t)oat(g, L, x >> L, y >> L, z >> L);
-        wave_append(take && col == 0, idx, lists[L][0], count + 2 * L);
-        wave_append(take && col == 1, idx, lists[L][1], count + 2 * L + 1);
+    for (int q = 0; q < OCT_LIST_CELLS; q++) {
+        const size_t c = ((size_t)blockIdx.x * OCT_LIST_CELLS + q) * 256 + threadIdx.x;
+        list[q] = -1;
+        if (c >= N) continue;
+        const int L = lev[c];
+        if (L == OCT_SOLID) continue;
+        const int x = (int)(c % g.W), y = (int)((c / g.W) % g.H), z = (int)(c / ((size_t)g.W * g.H));
+        if ((x | y | z) & ((1 << L) - 1)) continue;
+        if (L == 3 && lev[oat(g, 0, x, y, 0)] != 3) continue;
+        list[q] = 2 * L + (((x >> L) + (y >> L) + (z >> L)) & 1);
+        idx[q] = (uint32_t)oat(g, L, x >> L, y >> L, z >> L);
+        pos[q] = atomicAdd(&n[list[q]], 1u);
     }
+    __syncthreads();
+    if (threadIdx.x < OCT_LISTS && n[threadIdx.x]) base[threadIdx.x] = atomicAdd(count + threadIdx.x, n[threadIdx.x]);
+    __syncthreads();
+    uint32_t* const lists[OCT_LISTS] = {l00, l01, l10, l11, l20, l21, l30, l31};
+#pragma unroll
+    for (int q = 0; q < OCT_LIST_CELLS; q++)
+#pragma unroll
+        for (int k = 0; k < OCT_LISTS; k++)
+            if (list[q] == k) lists[k][base[k] + pos[q]] = idx[q];
 }
 
 __global__ void k_oct_zero(uint32_t* count) {
@@ -470,61 +494,55 @@ __global__ __launch_bounds__(OCT_BLOCK) void k_oct_gs(OctP P, OctSegs<4> t) {
 }
 
 // ---------------------------------------------------------------------------- face correction
-// the leaf beside a face at coordinate f holding fine cell c: the cell itself (level 0) or a coarser
-// leaf whose block the face bounds
-__device__ __forceinline__ bool oct_side(const OG& g, const uint8_t* lev, const LevelPtrs& P, int f, int x, int y,
-                                         int z, float& len, float& pv) {
-    const int m = lev[oat(g, 0, x, y, z)];
-    if (m == OCT_SOLID) return false;
-    if (m > 0 && (f & ((1 << m) - 1)) != 0) return false;
-    len = 0.5f * (float)(1 << m);
-    pv = P.p[m][oat(g, m, x >> m, y >> m, z >> m)];
-    return true;
+// half the size of the level-m leaf holding fine cell (x, y, z), and its pressure
+__device__ __forceinline__ float oct_half(int m) { return 0.5f * (float)(1 << m); }
+__device__ __forceinline__ float oct_pressure(const OG& g, const LevelPtrs& P, int m, int x, int y, int z) {
+    const float* p = m & 2 ? (m & 1 ? P.p[3] : P.p[2]) : (m & 1 ? P.p[1] : P.p[0]);
+    return p[oat(g, m, x >> m, y >> m, z >> m)];
 }
 
-// face -= (p2 - p1) / (len1 + len2) between two leaves; domain faces against a ghost 4 cells out
-// (Adjust_MAC_{u,v,w}_OpenOctreePoisson_Kernel, CPU_PoissonSolver3D_OpenOctreePoisson.cpp:6-373)
-__global__ __launch_bounds__(256) void k_oct_adjust(OG g, LevelPtrs P, const uint8_t* __restrict__ lev, float* u,
-                                                    float* v, float* w) {
-    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t nu = (size_t)(g.W + 1) * g.H * g.D, nv = (size_t)g.W * (g.H + 1) * g.D;
-    const size_t nw = (size_t)g.W * g.H * (g.D + 1);
-    int ax, i, j, k, ex[3];
-    float* face;
-    if (t < nu) {
-        ax = 0;
-        ex[0] = g.W + 1, ex[1] = g.H, ex[2] = g.D;
-        face = u + t;
-    } else if ((t -= nu) < nv) {
-        ax = 1;
-        ex[0] = g.W, ex[1] = g.H + 1, ex[2] = g.D;
-        face = v + t;
-    } else if ((t -= nv) < nw) {
-        ax = 2;
-        ex[0] = g.W, ex[1] = g.H, ex[2] = g.D + 1;
-        face = w + t;
-    } else {
-        return;
+// face -= (p2 - p1) / (len1 + len2) between two leaves (no face inside a leaf or beside a solid cell);
+// domain faces against a ghost 4 cells out
+// (Adjust_MAC_{u,v,w}_OpenOctreePoisson_Kernel, CPU_PoissonSolver3D_OpenOctreePoisson.cpp:6-373).
+// A thread does its cell's low faces, beside the last cell of an axis also the domain's high face: the
+// cell's level and pressure serve all of them.  (A thread a face: 240 us at 256^3; now 115.)
+__global__ __launch_bounds__(256) void k_oct_adjust(OG g, LevelPtrs P, const uint8_t* __restrict__ lev,
+                                                    float* __restrict__ u, float* __restrict__ v,
+                                                    float* __restrict__ w) {
+    const int x = blockIdx.x * 64 + threadIdx.x, y = blockIdx.y * 4 + threadIdx.y, z = blockIdx.z;
+    if (x >= g.W || y >= g.H) return;
+    const size_t c = oat(g, 0, x, y, z), plane = (size_t)g.W * g.H;
+    const int m = lev[c];
+    if (m == OCT_SOLID) return;
+    const int mx = x ? lev[c - 1] : 0, my = y ? lev[c - g.W] : 0, mz = z ? lev[c - plane] : 0;
+    const int low = (1 << m) - 1;
+    const float len = oct_half(m);
+    const size_t cu = ((size_t)z * g.H + y) * (g.W + 1) + x, cv = ((size_t)z * (g.H + 1) + y) * g.W + x, cw = c;
+    // this leaf's side of the low faces, and whether the neighbour's block also ends there
+    const bool fx = (x & low) == 0, fy = (y & low) == 0, fz = (z & low) == 0;
+    const bool hx = x == g.W - 1, hy = y == g.H - 1, hz = z == g.D - 1;
+    if (!(fx || fy || fz || hx || hy || hz)) return;
+    const float pc = oct_pressure(g, P, m, x, y, z);
+    auto between = [&](float* face, int n, int f, float pn) {
+        if (f & ((1 << n) - 1)) return;
+        *face = *face - (pc - pn) / (oct_half(n) + len);
+    };
+    if (fx) {
+        if (x == 0) u[cu] = u[cu] - (pc - 0.0f) / (4.0f + len);
+        else if (mx != OCT_SOLID) between(u + cu, mx, x, oct_pressure(g, P, mx, x - 1, y, z));
     }
-    i = (int)(t % ex[0]);
-    j = (int)((t / ex[0]) % ex[1]);
-    k = (int)(t / ((size_t)ex[0] * ex[1]));
-    const int fc[3] = {i, j, k};
-    const int f = fc[ax], n = ax == 0 ? g.W : ax == 1 ? g.H : g.D;
-    int lo[3] = {i, j, k};
-    lo[ax] -= 1;
-    float len1, len2, pa, pb;
-    if (f == 0) {
-        if (!oct_side(g, lev, P, 0, i, j, k, len2, pb)) return;
-        *face = *face - (pb - 0.0f) / (4.0f + len2);
-    } else if (f == n) {
-        if (!oct_side(g, lev, P, f, lo[0], lo[1], lo[2], len1, pa)) return;
-        *face = *face - (0.0f - pa) / (4.0f + len1);
-    } else {
-        if (!oct_side(g, lev, P, f, lo[0], lo[1], lo[2], len1, pa)) return;
-        if (!oct_side(g, lev, P, f, i, j, k, len2, pb)) return;
-        *face = *face - (pb - pa) / (len1 + len2);
+    if (fy) {
+        if (y == 0) v[cv] = v[cv] - (pc - 0.0f) / (4.0f + len);
+        else if (my != OCT_SOLID) between(v + cv, my, y, oct_pressure(g, P, my, x, y - 1, z));
     }
+    if (fz) {
+        if (z == 0) w[cw] = w[cw] - (pc - 0.0f) / (4.0f + len);
+        else if (mz != OCT_SOLID) between(w + cw, mz, z, oct_pressure(g, P, mz, x, y, z - 1));
+    }
+    // (the dimensions are multiples of 8: a leaf always ends at the domain's high side)
+    if (hx) u[cu + 1] = u[cu + 1] - (0.0f - pc) / (4.0f + len);
+    if (hy) v[cv + g.W] = v[cv + g.W] - (0.0f - pc) / (4.0f + len);
+    if (hz) w[cw + plane] = w[cw + plane] - (0.0f - pc) / (4.0f + len);
 }
 
 unsigned blocks_of(size_t n, int b) { return (unsigned)((n + b - 1) / b); }
@@ -580,9 +598,9 @@ void octree_layout(const Dims& g, char* mem, OctreeBufs* B) {
 void launch_octree_build(const Dims& d, const uint8_t* occ, int t1, int t2, int t3, const OctreeBufs& B,
                          hipStream_t s) {
     const OG g{d.W, d.H, d.D};
-    hipLaunchKernelGGL(k_oct_dist_x, dim3(blocks_of((size_t)d.H * d.D, 256)), dim3(256), 0, s, g, occ, B.dist);
-    hipLaunchKernelGGL(k_oct_dist_yz, dim3(blocks_of((size_t)d.W * d.D, 256)), dim3(256), 0, s, g, 1, B.dist, 0);
-    hipLaunchKernelGGL(k_oct_dist_yz, dim3(blocks_of((size_t)d.W * d.H, 256)), dim3(256), 0, s, g, 2, B.dist, 1);
+    hipLaunchKernelGGL(k_oct_dist_x, dim3(blocks_of((size_t)d.H * d.D, 4)), dim3(256), 0, s, g, occ, B.dist);
+    hipLaunchKernelGGL(k_oct_dist_yz, dim3(blocks_of((size_t)d.W * d.D, 64)), dim3(64), 0, s, g, 1, B.dist, 0);
+    hipLaunchKernelGGL(k_oct_dist_yz, dim3(blocks_of((size_t)d.W * d.H, 64)), dim3(64), 0, s, g, 2, B.dist, 1);
     for (int L = 1; L <= 3; L++)
         hipLaunchKernelGGL(k_oct_min, dim3(blocks_of(level_cells(d, L), 256)), dim3(256), 0, s, g, L,
                            (const int32_t*)B.mn[L - 1], B.mn[L]);
@@ -630,7 +648,7 @@ uint32_t oct_segs(const OctreeBufs& B, const OctreeLists& Ls, uint32_t mask, Oct
 hipError_t octree_build_lists(const Dims& d, const OctreeBufs& B, OctreeLists* Ls, hipStream_t s) {
     const OG g{d.W, d.H, d.D};
     hipLaunchKernelGGL(k_oct_zero, dim3(1), dim3(64), 0, s, B.count);
-    hipLaunchKernelGGL(k_oct_lists, dim3(blocks_of(level_cells(d, 0), 256)), dim3(256), 0, s, g,
+    hipLaunchKernelGGL(k_oct_lists, dim3(blocks_of(level_cells(d, 0), 256 * OCT_LIST_CELLS)), dim3(256), 0, s, g,
                        (const uint8_t*)B.lev, B.list[0][0], B.list[0][1], B.list[1][0], B.list[1][1], B.list[2][0],
                        B.list[2][1], B.list[3][0], B.list[3][1], B.count);
     uint32_t got[4 * OCT_LISTS];
@@ -717,8 +735,7 @@ int launch_octree_sweeps(const Dims& d, const OctreeBufs& B, const OctreeLists& 
 void launch_octree_adjust(const Dims& d, const OctreeBufs& B, float* u, float* v, float* w, hipStream_t s) {
     const OG g{d.W, d.H, d.D};
     const LevelPtrs P{{B.p[0], B.p[1], B.p[2], B.p[3]}};
-    const size_t nf = (size_t)(d.W + 1) * d.H * d.D + (size_t)d.W * (d.H + 1) * d.D + (size_t)d.W * d.H * (d.D + 1);
-    hipLaunchKernelGGL(k_oct_adjust, dim3(blocks_of(nf, 256)), dim3(256), 0, s, g, P, (const uint8_t*)B.lev, u, v, w);
+    hipLaunchKernelGGL(k_oct_adjust, fine_grid(d), dim3(64, 4), 0, s, g, P, (const uint8_t*)B.lev, u, v, w);
 }
 
 void launch_octree_sub_project(const Dims& d, const OctreeBufs& B, float* u, float* v, float* w, hipStream_t s) {
