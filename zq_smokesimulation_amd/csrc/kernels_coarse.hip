@@ -387,7 +387,7 @@ __global__ __launch_bounds__(256) void k_coarse_unpack(CG g, const float* __rest
 // `iters` iterations of a box per workgroup (sor_block_tile with the face weights).  The slabs above
 // spend a launch on staging seven arrays through LDS and read every operand of an update from it; here
 // the operands are registers: at 32^3 coarse cells an iteration takes
-// 2.45 us (slabs 5.8, a launch a colour 6.4), at 128^3 4.3 (6.6).
+// 2.45 us (slabs 5.8, a launch a colour 6.4), at 64^3 4.3 (6.5).
 __global__ __launch_bounds__(512) void k_coarse_block(CG g, BlockWeights w, const float* __restrict__ div,
                                                       const float* __restrict__ src, float* __restrict__ dst, BlockCut c,
                                                       int iters, float omega, float omw) {
@@ -743,6 +743,45 @@ __device__ __forceinline__ double block_sum(double x, double* red) {
     __syncthreads();
     return a;
 }
+// x plus the value OFF lanes away (lane ^ OFF), without a trip through LDS
+template <int OFF>
+__device__ __forceinline__ unsigned lane_xor(unsigned x) {
+    if constexpr (OFF == 1) return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, true);  // quad [1,0,3,2]
+    if constexpr (OFF == 2) return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, true);  // quad [2,3,0,1]
+    if constexpr (OFF == 4) {  // lanes 0-3, 8-11 of a row from four above, the others from four below
+        const int up = __builtin_amdgcn_update_dpp(0, (int)x, 0x104, 0xf, 0x5, true);
+        return (unsigned)__builtin_amdgcn_update_dpp(up, (int)x, 0x114, 0xf, 0xa, true);
+    }
+    return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, true);  // 8: rotated by half a row
+}
+template <int OFF>
+__device__ __forceinline__ double add_xor(double x) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+    unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+    if constexpr (OFF >= 16) {
+        // the swap leaves the lower halves' values everywhere in one result, the upper halves' in the other
+        const auto l = OFF == 32 ? __builtin_amdgcn_permlane32_swap(lo, lo, false, false)
+                                 : __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = OFF == 32 ? __builtin_amdgcn_permlane32_swap(hi, hi, false, false)
+                                 : __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        return __builtin_bit_cast(double, (unsigned long long)h[0] << 32 | l[0]) +
+               __builtin_bit_cast(double, (unsigned long long)h[1] << 32 | l[1]);
+    } else {
+        lo = lane_xor<OFF>(lo), hi = lane_xor<OFF>(hi);
+        return x + __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+    }
+}
+// block_sum's sum, in its order, with one barrier: red must not be written again before another barrier
+template <int NT>
+__device__ __forceinline__ double block_sum1(double x, double* red) {
+    x = add_xor<1>(add_xor<2>(add_xor<4>(add_xor<8>(add_xor<16>(add_xor<32>(x))))));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = x;
+    __syncthreads();
+    double a = 0.0;
+#pragma unroll
+    for (int i = 0; i < NT / 64; i++) a += red[i];
+    return a;
+}
 template <int NT>
 __device__ __forceinline__ int block_min(int x, int* redi) {
     for (int off = 32; off > 0; off >>= 1) x = min(x, __shfl_xor(x, off, 64));
@@ -777,10 +816,10 @@ __global__ __launch_bounds__(((S * S * S + 63) / 64) * 64) void k_sub_solids(CG 
     __shared__ float Vs[S][S + 1][S];
     __shared__ float Ws[S + 1][S][S];
     __shared__ uint8_t fl[N];
-    __shared__ int lab[N];
-    __shared__ double dsh[N];
+    __shared__ int lab[N + 1];
+    __shared__ double dsh[N + 1];
     __shared__ float p32[N];
-    __shared__ double red[NT / 64];
+    __shared__ double red[NT / 64], red2[NT / 64];
     __shared__ int redi[NT / 64];
     const int t = threadIdx.x;
     const int x0 = bi * S, y0 = bj * S, z0 = bk * S;
@@ -810,16 +849,23 @@ __global__ __launch_bounds__(((S * S * S + 63) / 64) * 64) void k_sub_solids(CG 
     if (t < N) fl[t] = me;
     const int nfl = __syncthreads_count(me);
     if (nfl < 2) return;
-    // fluid neighbours inside the block
+    // fluid neighbours inside the block; the slot past the cells (label INT_MAX, value 0) stands for the
+    // missing ones, so that the six are registers and every load is unconditional
     int nbr[6];
     int nn = 0;
-    if (me) {
-        if (ci > 0 && fl[t - 1]) nbr[nn++] = t - 1;
-        if (ci < S - 1 && fl[t + 1]) nbr[nn++] = t + 1;
-        if (cj > 0 && fl[t - S]) nbr[nn++] = t - S;
-        if (cj < S - 1 && fl[t + S]) nbr[nn++] = t + S;
-        if (ck > 0 && fl[t - S * S]) nbr[nn++] = t - S * S;
-        if (ck < S - 1 && fl[t + S * S]) nbr[nn++] = t + S * S;
+    {
+        const bool in[6] = {ci > 0, ci < S - 1, cj > 0, cj < S - 1, ck > 0, ck < S - 1};
+        const int at[6] = {t - 1, t + 1, t - S, t + S, t - S * S, t + S * S};
+#pragma unroll
+        for (int n = 0; n < 6; n++) {
+            const bool has = me && in[n] && fl[at[n]];
+            nbr[n] = has ? at[n] : N;
+            nn += has;
+        }
+    }
+    if (t == 0) {
+        lab[N] = INT_MAX;
+        dsh[N] = 0.0;
     }
     // divergence (left to right, as ZQ_SolveClosedPressure3D, :2569-2571)
     double b = 0.0;
@@ -832,7 +878,8 @@ __global__ __launch_bounds__(((S * S * S + 63) / 64) * 64) void k_sub_solids(CG 
     __syncthreads();
     for (;;) {
         int m = mylab;
-        for (int n = 0; n < nn; n++) m = min(m, lab[nbr[n]]);
+#pragma unroll
+        for (int n = 0; n < 6; n++) m = min(m, lab[nbr[n]]);
         __syncthreads();
         const int ch = me && m < mylab;
         if (ch) {
@@ -857,7 +904,11 @@ __global__ __launch_bounds__(((S * S * S + 63) / 64) * 64) void k_sub_solids(CG 
             }
         }
     }
-    // CG on A = -L (cnt p - sum of fluid neighbours), A x = -b, from x = 0
+    // CG on A = -L (cnt p - sum of fluid neighbours), A x = -b, from x = 0.  An iteration is a chain of
+    // latencies (two sums over the workgroup), so each sum has its own array and needs one barrier, and
+    // its wave part moves lanes with DPP.  Around a sphere at 256^3 in
+    // 8^3 blocks the stage takes 145 us (334 with two barriers and shuffles through LDS a sum, and the
+    // neighbours in an indexed list).
     double x = 0.0, r = -b, d = r;
     double rr = block_sum<NT>(r * r, red);
     const double stop = rr * 1e-24;
@@ -868,15 +919,16 @@ __global__ __launch_bounds__(((S * S * S + 63) / 64) * 64) void k_sub_solids(CG 
         double q = 0.0;
         if (me) {
             double sn = 0.0;
-            for (int n = 0; n < nn; n++) sn += dsh[nbr[n]];
+#pragma unroll
+            for (int n = 0; n < 6; n++) sn += dsh[nbr[n]];
             q = (double)nn * d - sn;
         }
-        const double dq = block_sum<NT>(d * q, red);
+        const double dq = block_sum1<NT>(d * q, red);
         if (!(dq > 0.0)) break;
         const double alpha = rr / dq;
         x += alpha * d;
         r -= alpha * q;
-        const double rn = block_sum<NT>(r * r, red);
+        const double rn = block_sum1<NT>(r * r, red2);
         d = r + (rn / rr) * d;
         rr = rn;
     }
@@ -1091,19 +1143,21 @@ const float* launch_coarse_sor(const CoarseDims& cd, const CoarseBufs& B, float 
 }
 
 int coarse_sweep_candidates(const CoarseDims& cd, CoarseSweep* out, int max) {
-    static const CoarseSweep all[] = {{0, 0}, {1, 1}, {1, 2}, {2, 1}, {2, 2}, {2, 4}, {3, 1}, {3, 2}, {4, 1}, {4, 2},
-                                      {4, 4}, {6, 1}, {8, 1}};
+    // a launch a colour for grids too large for boxes (slabs are slower than boxes on every grid whose
+    // planes fit LDS: 5.8 against 2.45 us an iteration at 32^3, 6.5 against 4.3 at 64^3; they stay selectable)
     int n = 0;
-    for (const CoarseSweep& c : all)
-        if (n < max && coarse_sweep_valid(cd, c)) out[n++] = c;
+    if (n < max) out[n++] = CoarseSweep{0, 0};
     // boxes: the plain solver's choice and the shapes that were fastest on some coarse grid of 32^3 to 128^3
     const BlockCut c = block_best_cut(cd.Wc, cd.Hc, cd.Dc, 40, 512);
     int lg = 0;
     while ((1 << lg) < c.lx) lg++;
     const CoarseSweep boxes[] = {{c.K, -(10000 * lg + 100 * c.ty + c.tz)}, {3, -30804}, {2, -30503}, {2, -30805},
                                  {3, -40804}, {2, -31004}, {2, -40605}};
-    for (const CoarseSweep& b : boxes)
-        if (n < max && coarse_sweep_valid(cd, b)) out[n++] = b;
+    for (const CoarseSweep& b : boxes) {
+        bool had = !coarse_sweep_valid(cd, b);
+        for (int i = 0; i < n; i++) had = had || (out[i].k == b.k && out[i].zc == b.zc);
+        if (n < max && !had) out[n++] = b;
+    }
     return n;
 }
 

@@ -64,8 +64,8 @@ int check_block(const Dims& d, int s, const char* where) {
 
 }  // namespace
 
-// Times every valid sweep schedule (iters iterations each, HIP events on the null stream) on the
-// coarse arrays as they stand and keeps the fastest; all schedules give the same bits.
+// Times the candidate schedules (iters iterations each, the better of two runs, HIP events on the null
+// stream) on the coarse arrays as they stand and keeps the fastest; all schedules give the same bits.
 int tune_coarse_sweep(CoarseState* c, int iters, const char* where) {
     CoarseSweep cand[20];
     const int n = coarse_sweep_candidates(c->cd, cand, 20);
@@ -76,15 +76,17 @@ int tune_coarse_sweep(CoarseState* c, int iters, const char* where) {
     int bi = 0;
     for (int i = 0; i < n; i++) {
         (void)launch_coarse_sor(c->cd, c->B, 1.0f, 2, cand[i], nullptr);  // first-launch costs
-        (void)hipEventRecord(a, nullptr);
-        (void)launch_coarse_sor(c->cd, c->B, 1.0f, iters, cand[i], nullptr);
-        (void)hipEventRecord(b, nullptr);
-        (void)hipEventSynchronize(b);
-        float ms = 0.0f;
-        (void)hipEventElapsedTime(&ms, a, b);
-        if (i == 0 || ms < best) {
-            best = ms;
-            bi = i;
+        for (int run = 0; run < 2; run++) {
+            (void)hipEventRecord(a, nullptr);
+            (void)launch_coarse_sor(c->cd, c->B, 1.0f, iters, cand[i], nullptr);
+            (void)hipEventRecord(b, nullptr);
+            (void)hipEventSynchronize(b);
+            float ms = 0.0f;
+            (void)hipEventElapsedTime(&ms, a, b);
+            if ((i == 0 && run == 0) || ms < best) {
+                best = ms;
+                bi = i;
+            }
         }
     }
     (void)hipEventDestroy(a);
@@ -109,7 +111,7 @@ int coarse_create(const Dims& d, int s, CoarseState* out, const char* where) {
     launch_fill_f32(out->B.p, out->cd.Np(), 0.0f, nullptr);
     launch_fill_f32(out->B.p2, out->cd.Np(), 0.0f, nullptr);
     ZQ_HIP(hipStreamSynchronize(nullptr), where);
-    return tune_coarse_sweep(out, 20, where);
+    return tune_coarse_sweep(out, 24, where);
 }
 
 int coarse_set_guide(CoarseState* c, float coeff, const float* gu, const float* gv, const float* gw, hipStream_t s,
@@ -158,9 +160,7 @@ int project_coarse(const CoarseState& c, float* u, float* v, float* w, const uin
     ZQ_HIP(hipGetLastError(), where);
     if (st) {
         Scalars* sc = B.sc;
-        launch_fill_f64(&sc->mean64, 1, 0.0, s);
-        launch_proj_setup(c.cd.f, u, v, w, occ, o.open_mask, B.nc, B.b, nullptr, B.p, nullptr, nullptr, s);
-        launch_max_div64(c.cd.f, u, v, w, B.nc, &sc->mean64, B.part, B.target(1, &sc->dmax), s);
+        launch_max_div64_occ(c.cd.f, u, v, w, occ, o.open_mask, B.part, B.target(1, &sc->dmax), s);
         double md = 0.0;
         if (int rc = read_result(B, 1, &sc->dmax, &md, s, where)) return rc;
         st->outer = 0;

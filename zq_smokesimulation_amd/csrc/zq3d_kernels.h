@@ -229,6 +229,9 @@ void launch_update_p64_split(const Dims& d, const uint8_t* nc, float* const* e, 
 template <class F>
 void launch_max_div64(const Dims& d, const F* u, const F* v, const F* w, const uint8_t* nc, const double* mean64,
                       double* part, unsigned long long* dmax, hipStream_t s, unsigned long long* mean_out = nullptr);
+// max |div64| over the cells projection set-up would count (fluid, with a fluid or open side)
+void launch_max_div64_occ(const Dims& d, const float* u, const float* v, const float* w, const uint8_t* occ,
+                          int open_mask, double* part, unsigned long long* dmax, hipStream_t s);
 // max |div64 - mean64| over counted cells of the faces launch_correct64 would produce from p64_pad
 // (equal bit for bit to launch_max_div64 after launch_correct64), faces left unchanged
 template <class F>
