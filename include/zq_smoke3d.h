@@ -542,8 +542,8 @@ int zq3d_ens_stream(zq3d_ens* e, void** stream);
 /* Launch-shape autotuner: times the sweep kernels -- kind 0: single-colour half sweeps for each
  * tile shape (tbx x tby cells) and persistent launch size (blocks; 0 = one workgroup per tile);
  * kind 1: two red-black iterations a launch with a tile's planes in registers, tbx cells a lane x tby
- * waves x `blocks` planes (the default before any autotune is 4 x 8 x 16) -- and the cell kernels for
- * each launch size, on the members' own grids and occupancy, and keeps the fastest.  All give the
+ * waves x `blocks` planes, seven fixed shapes and the five depths predicted fastest for the members
+ * (the default before any autotune is the one predicted fastest) -- and the cell kernels for each launch size, on the members' own grids and occupancy, and keeps the fastest.  All give the
  * same bits.  Fields are unchanged. */
 #define ZQ3D_ENS_TUNE_MAX 24
 typedef struct zq3d_ens_tune {

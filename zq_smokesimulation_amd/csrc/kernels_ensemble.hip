@@ -173,17 +173,13 @@ __global__ __launch_bounds__(NT) void ke_sor_half(const EnsMember* __restrict__ 
     });
 }
 
-// K iterations of every member's SOR in one launch (sor_quad_tile, each member cut by itself); tiles
-// are handed out so each XCD gets a contiguous run.  Members with an odd count run one iteration
+// K iterations of every member's SOR in one launch (sor_quad_tile, each member cut by itself).  Members with an odd count run one iteration
 // first (K == 1, which takes only those, from zero); launch `at` of the pairs then takes every member
 // that still has two to do.
 template <int K, int CX, int NTH>
 __global__ __launch_bounds__(NTH) void ke_sor_quad(const EnsMember* __restrict__ M, EnsQuadTable T, int at) {
     extern __shared__ float quad_lds[];
-    const int per = gridDim.x >> 3;
-    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if (tile >= T.total) return;  // spare block: uniform exit before any barrier
-    const EnsQuadTile t = T.tiles[tile];
+    const EnsQuadTile t = T.tiles[blockIdx.x];
     const EnsMember& m = M[t.member];
     const int odd = m.iters & 1;
     if (K == 1 ? !odd : 2 * at + 2 > m.iters - odd) return;
@@ -270,8 +266,7 @@ hipError_t launch_quad(const EnsLaunch& L, const EnsQuadTable& T, int at, hipStr
                                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds);
         if (e != hipSuccess) return e;
     }
-    const unsigned nb = (unsigned)((T.total + 7) & ~7);  // a multiple of 8 for the XCD numbering
-    hipLaunchKernelGGL((ke_sor_quad<K, CX, NTH>), dim3(nb), dim3(NTH), lds, s, L.members, T, at);
+    hipLaunchKernelGGL((ke_sor_quad<K, CX, NTH>), dim3((unsigned)T.total), dim3(NTH), lds, s, L.members, T, at);
     return hipGetLastError();
 }
 
@@ -285,8 +280,8 @@ hipError_t ens_launch_sweeps(const EnsLaunch& L, int iters, hipStream_t s) {
         hipError_t e = hipSuccess;
         if (L.any_odd && iters > 0) e = launch_quad<1, 2, 512>(L, L.quad_one, 0, s);
         for (int at = 0; 2 * at + 2 <= iters && e == hipSuccess; at++) {
-            if (kEnsQuadShapes[r][0] == 4) e = launch_quad<2, 4, 512>(L, T, at, s);
-            else if (kEnsQuadShapes[r][1] <= 8) e = launch_quad<2, 2, 512>(L, T, at, s);
+            if (L.quad_shape[r][0] == 4) e = launch_quad<2, 4, 512>(L, T, at, s);
+            else if (L.quad_shape[r][1] <= 8) e = launch_quad<2, 2, 512>(L, T, at, s);
             else e = launch_quad<2, 2, 1024>(L, T, at, s);
         }
         return e;

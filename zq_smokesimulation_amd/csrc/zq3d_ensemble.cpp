@@ -5,6 +5,8 @@
 
 #include <algorithm>
 #include <cstring>
+#include <functional>
+#include <queue>
 #include <vector>
 
 #include "zq3d_ensemble.h"
@@ -104,17 +106,72 @@ std::vector<EnsTile> cell_tiles(const zq3d_ens* e) {
     return t;
 }
 
-// the tiles of every member under shape {cells a lane, waves, planes} for K iterations a launch
-void quad_table(const zq3d_ens* e, int K, const int shape[3], std::vector<EnsQuadTile>& tiles,
-                std::vector<QuadCut>& cuts) {
+// The tiles of every member under shape {cells a lane, waves, planes} for K iterations a launch, the longest
+// first, and the members' cuts (either null: not wanted); returns the microseconds a launch is predicted
+// to take: tiles start in this order, XCD b % 8 takes block b, a CU one tile at a time, and a tile costs
+// its plane steps by quad_cost's latency and issue time.
+double quad_table(const zq3d_ens* e, int K, const int shape[3], std::vector<EnsQuadTile>* tiles,
+                  std::vector<QuadCut>* cuts) {
+    struct Timed {
+        double us;
+        EnsQuadTile t;
+    };
+    std::vector<Timed> all;
     for (int s = 0; s < e->count; s++) {
         const Dims& d = e->dims[s];
         const QuadCut c = quad_cut(d.W, d.H, d.D, K, shape[0], shape[1], shape[2]);
-        cuts.push_back(c);
-        for (int z = 0; z < c.nz; z++)
+        if (cuts) cuts->push_back(c);
+        for (int z = 0; z < c.nz; z++) {
+            const int steps = quad_z_begin(c, K, z + 1, d.D) - quad_z_begin(c, K, z, d.D) + (z ? 4 * K - 2 : 2 * K - 1);
+            const double us = 1.5 + steps * quad_step_us(K, shape[0], c.nw);
             for (int y = 0; y < c.ny; y++)
-                for (int x = 0; x < c.nx; x++) tiles.push_back(EnsQuadTile{s, x, y, z});
+                for (int x = 0; x < c.nx; x++) all.push_back(Timed{us, EnsQuadTile{s, x, y, z}});
+        }
     }
+    std::stable_sort(all.begin(), all.end(), [](const Timed& a, const Timed& b) { return a.us > b.us; });
+    std::priority_queue<double, std::vector<double>, std::greater<double>> xcd[8];
+    for (auto& q : xcd)
+        for (int cu = 0; cu < 32; cu++) q.push(0.0);
+    double last = 0.0;
+    for (size_t i = 0; i < all.size(); i++) {
+        if (tiles) tiles->push_back(all[i].t);
+        auto& q = xcd[i % 8];
+        const double end = q.top() + all[i].us;
+        q.pop();
+        q.push(end);
+        last = std::max(last, end);
+    }
+    return last;
+}
+
+// The shapes of an ensemble: the fixed ones, then the depths of four cells a lane predicted fastest;
+// returns the shape predicted fastest of all.
+int quad_shapes(const zq3d_ens* e, int (*shapes)[3]) {
+    struct Depth {
+        double us;
+        int zc;
+    };
+    std::vector<Depth> depths;
+    double best_us = 0.0;
+    int n = 0, best = 0;
+    auto add = [&](int cx, int nw, int zc, double us) {
+        shapes[n][0] = cx, shapes[n][1] = nw, shapes[n][2] = zc;
+        if (n == 0 || us < best_us) {
+            best_us = us;
+            best = n;
+        }
+        n++;
+    };
+    for (const auto& f : kEnsQuadShapes) add(f[0], f[1], f[2], quad_table(e, 2, f, nullptr, nullptr));
+    for (int zc = 2; zc <= 64; zc += 2) {
+        bool had = false;
+        for (const auto& f : kEnsQuadShapes) had = had || (f[0] == 4 && f[2] == zc);
+        const int shape[3] = {4, 8, zc};
+        if (!had) depths.push_back(Depth{quad_table(e, 2, shape, nullptr, nullptr), zc});
+    }
+    std::stable_sort(depths.begin(), depths.end(), [](const Depth& a, const Depth& b) { return a.us < b.us; });
+    for (int i = 0; n < kEnsQuadShapeCount; i++) add(4, 8, depths[i].zc, depths[i].us);
+    return best;
 }
 
 int field_span(zq3d_ens* e, int s, int field, void** p, size_t* bytes) {
@@ -183,10 +240,11 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
     std::vector<EnsQuadTile> tiles;
     std::vector<QuadCut> cuts;
     size_t tile_at[kEnsQuadShapeCount + 1];
+    const int quad_best = quad_shapes(e, e->L.quad_shape);
     for (int r = 0; r <= kEnsQuadShapeCount; r++) {
         tile_at[r] = tiles.size();
-        if (r < kEnsQuadShapeCount) quad_table(e, 2, kEnsQuadShapes[r], tiles, cuts);
-        else quad_table(e, 1, kEnsQuadOne, tiles, cuts);
+        if (r < kEnsQuadShapeCount) quad_table(e, 2, e->L.quad_shape[r], &tiles, &cuts);
+        else quad_table(e, 1, kEnsQuadOne, &tiles, &cuts);
     }
     int bad = 0;
     bad |= ens_alloc(e, &e->u, e->Nu * 4) | ens_alloc(e, &e->v, e->Nv * 4) | ens_alloc(e, &e->w, e->Nw * 4);
@@ -297,7 +355,7 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
             EnsQuadTable{e->dev_tiles + tile_at[r], e->dev_cuts + (size_t)r * count, (int)(end - tile_at[r])};
     }
     L.sweep_shape = 0;
-    L.sweep_quad = kEnsQuadDefault;
+    L.sweep_quad = quad_best + 1;
     L.blocks = 0;
     L.sweep_blocks = 0;
     L.p_pool = e->p;
@@ -420,10 +478,14 @@ extern "C" int zq3d_ens_set_sweep(zq3d_ens* e, int kind, int tbx, int tby, int b
         static const int old[][2] = {{8, 8}, {8, 16}, {16, 8}, {16, 16}, {16, 32}, {32, 8}, {32, 16}};
         if (tbx == 64)
             for (const auto& o : old)
-                if (o[0] == tby && o[1] == blocks) tbx = 2;
-        if (tbx == 2 && tby == 32) tby = 16;
+                if (o[0] == tby && o[1] == blocks) {
+                    tbx = 2;
+                    tby = tby == 8 ? 8 : 16;
+                    blocks = blocks == 8 ? 8 : 16;
+                    break;
+                }
         for (int r = 0; r < kEnsQuadShapeCount; r++)
-            if (kEnsQuadShapes[r][0] == tbx && kEnsQuadShapes[r][1] == tby && kEnsQuadShapes[r][2] == blocks) {
+            if (L.quad_shape[r][0] == tbx && L.quad_shape[r][1] == tby && L.quad_shape[r][2] == blocks) {
                 L.sweep_quad = r + 1;
                 ok = true;
             }
@@ -494,7 +556,7 @@ extern "C" int zq3d_ens_autotune(zq3d_ens* e, int iters, zq3d_ens_tune* rep) {
     for (int r = 0; r < kEnsQuadShapeCount; r++) {
         L.sweep_quad = r + 1;
         const float ms = time_it([&] { E(ens_launch_sweeps(L, even, e->stream)); });
-        consider(kEnsQuadShapes[r][0], kEnsQuadShapes[r][1], kEnsQuadShapes[r][2], 1e3f * ms / even, 0, 0, r + 1);
+        consider(L.quad_shape[r][0], L.quad_shape[r][1], L.quad_shape[r][2], 1e3f * ms / even, 0, 0, r + 1);
     }
     L.sweep_shape = best_sh;
     L.sweep_blocks = best_sb;
@@ -518,9 +580,9 @@ extern "C" int zq3d_ens_autotune(zq3d_ens* e, int iters, zq3d_ens_tune* rep) {
     if (rep) {
         rep->count = n;
         rep->best_kind = best_quad ? 1 : 0;
-        rep->best_tbx = best_quad ? kEnsQuadShapes[best_quad - 1][0] : kEnsSweepShapes[best_sh][0];
-        rep->best_tby = best_quad ? kEnsQuadShapes[best_quad - 1][1] : kEnsSweepShapes[best_sh][1];
-        rep->best_sweep_blocks = best_quad ? kEnsQuadShapes[best_quad - 1][2] : best_sb;
+        rep->best_tbx = best_quad ? L.quad_shape[best_quad - 1][0] : kEnsSweepShapes[best_sh][0];
+        rep->best_tby = best_quad ? L.quad_shape[best_quad - 1][1] : kEnsSweepShapes[best_sh][1];
+        rep->best_sweep_blocks = best_quad ? L.quad_shape[best_quad - 1][2] : best_sb;
         rep->best_us_per_iter = best;
         rep->best_blocks = best_b;
         rep->probe_ms = best_cell;

@@ -56,22 +56,25 @@ struct EnsTable {
 
 constexpr int kEnsSweepShapeCount = 3;
 extern const int kEnsSweepShapes[kEnsSweepShapeCount][2];  // TBX x TBY of the sweep kernel
-// cells a lane x waves x planes of the sweeps that run two red-black iterations a launch.  64 members
-// of 32 to 96 cells an axis (17.5 M cells), us per iteration: 43.4, 36.6, 37.6 / 41.9, 37.5, 41.2 with
-// two cells a lane, 28.7 with four and 16 planes (the one-iteration launches on colour-split storage
-// that these replace took 83.9, the half sweeps at best 175): with thousands of tiles it is issue
-// that counts, and four cells a lane share the row's neighbours best.
-constexpr int kEnsQuadShapeCount = 9;
-constexpr int kEnsQuadShapes[kEnsQuadShapeCount][3] = {{2, 8, 8},   {2, 8, 16}, {2, 8, 32}, {2, 16, 8}, {2, 16, 16},
-                                                       {2, 16, 32}, {4, 8, 12}, {4, 8, 16}, {4, 8, 24}};
-constexpr int kEnsQuadDefault = 8;  // sweep_quad of a new ensemble
+// cells a lane x waves x planes of the sweeps that run two red-black iterations a launch.  With thousands
+// of tiles it is issue that counts, and four cells a lane share the row's neighbours best; then how
+// evenly the tiles fill the CUs (one tile of four cells a lane a CU), which depends on the members.  64
+// members of 32 to 96 cells an axis (17.5 M cells), us per iteration: 34.5 to 45.6 with two cells a lane;
+// with four 37.2 at 8 planes, 28.9 at 16, 24.5 at 32 (the one-iteration launches on colour-split storage that these replace took 83.9, the half
+// sweeps at best 175).
+constexpr int kEnsQuadShapeCount = 12;
+constexpr int kEnsQuadFixed = 7;  // shapes every ensemble has; the rest are the depths of four cells a lane
+                                  // that are predicted fastest for its members
+constexpr int kEnsQuadShapes[kEnsQuadFixed][3] = {{2, 8, 8}, {2, 8, 16}, {2, 16, 8}, {2, 16, 16},
+                                                  {4, 8, 8}, {4, 8, 16}, {4, 8, 32}};
 constexpr int kEnsQuadOne[3] = {2, 8, 8};  // the shape of the launch of one iteration
 
 struct EnsQuadTile {
     int member, bx, by, bz;
 };
 
-// Every member's tiles, member after member, and how each member is cut.
+// Every member's tiles, the longest first (workgroups start in this order, so the short ones fill the
+// end), and how each member is cut.
 struct EnsQuadTable {
     const EnsQuadTile* tiles;
     const QuadCut* cuts;
@@ -85,7 +88,8 @@ struct EnsLaunch {
     EnsTable half[kEnsSweepShapeCount];  // half-row grids of the sweep, one per tile shape
     int sweep_shape;                     // index into kEnsSweepShapes
     EnsQuadTable quad[kEnsQuadShapeCount], quad_one;
-    int sweep_quad;                      // 0: half sweeps of sweep_shape; r > 0: kEnsQuadShapes[r - 1]
+    int quad_shape[kEnsQuadShapeCount][3];
+    int sweep_quad;                      // 0: half sweeps of sweep_shape; r > 0: quad_shape[r - 1]
     int any_odd;                         // some member's iteration count is odd
     int blocks;                          // workgroups of the persistent launches (<= 0: one per tile)
     int sweep_blocks;

@@ -91,15 +91,20 @@ inline QuadCut quad_cut(int W, int H, int D, int K, int cx, int nw, int zc) {
     return c;
 }
 
-// Predicted microseconds of one launch: a fixed cost, then every workgroup's steps, a step costing a
-// latency and an issue time per wave a SIMD runs (CUs beyond one round of workgroups share them).
+// Predicted microseconds of a plane step: a latency and the issue time per wave a SIMD runs.
+inline double quad_step_us(int K, int cx, int nw) {
+    const double issue = (cx / 2) * (K == 2 ? 0.21 : 0.12);
+    return 0.24 + issue * std::max(1.0, nw / 4.0);
+}
+
+// Predicted microseconds of one launch: a fixed cost, then every workgroup's steps (CUs beyond one round of
+// workgroups share them).
 inline double quad_cost(const QuadCut& c, int K, int cx) {
     const double tiles = (double)c.nx * c.ny * c.nz, steps = c.zc + 4 * K - 2;
-    const double waves = std::max(1.0, c.nw / 4.0), rounds = std::max(1.0, tiles / 256.0);
-    const double lat = 0.24, issue = (cx / 2) * (K == 2 ? 0.21 : 0.12);
+    const double rounds = std::max(1.0, tiles / 256.0);
     // beyond one round the last one may be nearly empty
     const double full = tiles <= 256.0 ? 1.0 : 0.5 * (rounds + (double)((int)((tiles + 255.0) / 256.0)));
-    return 4.0 + steps * (lat + issue * waves) * full;
+    return 4.0 + steps * quad_step_us(K, cx, c.nw) * full;
 }
 
 // The cheapest cut of up to `most` waves by quad_cost.
