@@ -121,12 +121,27 @@ private:
         }
     }
 
+    // without a slot (no pinned memory to be had): the batch by plain copies
+    hipError_t plain(size_t b) {
+        (void)hipGetLastError();
+        hipError_t e = hipSuccess;
+        for (size_t k = batches_[b].first; k < batches_[b].first + batches_[b].count && e == hipSuccess; k++) {
+            const Piece& q = pieces_[k];
+            e = to_dev_ ? hipMemcpy(q.dev, q.host, q.bytes, hipMemcpyHostToDevice)
+                        : hipMemcpy(q.host, q.dev, q.bytes, hipMemcpyDeviceToHost);
+        }
+        return e;
+    }
+
     hipError_t push(Lane& l) {
         hipError_t e = hipSuccess;
         for (int i = 0; e == hipSuccess; i ^= 1) {
             const size_t b = next_.fetch_add(1);
             if (b >= batches_.size()) break;
-            if ((e = ready(l, i)) != hipSuccess) break;
+            if (ready(l, i) != hipSuccess) {
+                e = plain(b);
+                continue;
+            }
             if (l.used[i] && (e = hipEventSynchronize(l.ev[i])) != hipSuccess) break;
             l.used[i] = false;
             for (size_t k = batches_[b].first; k < batches_[b].first + batches_[b].count && e == hipSuccess; k++) {
@@ -150,9 +165,12 @@ private:
         for (int i = 0;; i ^= 1) {
             size_t b = none;
             if (e == hipSuccess && (b = next_.fetch_add(1)) >= batches_.size()) b = none;
-            if (b != none) {
-                e = ready(l, i);
-                if (e == hipSuccess && l.used[i]) e = hipEventSynchronize(l.ev[i]);
+            bool copied = false;
+            if (b != none && ready(l, i) != hipSuccess) {
+                e = plain(b);
+                copied = true;
+            } else if (b != none) {
+                if (l.used[i]) e = hipEventSynchronize(l.ev[i]);
                 for (size_t k = batches_[b].first; k < batches_[b].first + batches_[b].count && e == hipSuccess; k++) {
                     const Piece& q = pieces_[k];
                     e = hipMemcpyAsync(l.slot[i] + q.at, q.dev, q.bytes, hipMemcpyDeviceToHost, 0);
@@ -170,7 +188,7 @@ private:
                         std::memcpy(pieces_[k].host, l.slot[o] + pieces_[k].at, pieces_[k].bytes);
                 else if (e == hipSuccess) e = r;
                 in_slot[o] = none;
-            } else if (in_slot[i] == none) {
+            } else if (in_slot[i] == none && !copied) {
                 return e;
             }
         }
