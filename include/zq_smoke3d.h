@@ -543,8 +543,9 @@ int zq3d_ens_stream(zq3d_ens* e, void** stream);
  * tile shape (tbx x tby cells) and persistent launch size (blocks; 0 = one workgroup per tile);
  * kind 1: two red-black iterations a launch with a tile's planes in registers, tbx cells a lane x tby
  * waves x `blocks` planes, seven fixed shapes and the five depths predicted fastest for the members
- * (the default before any autotune is the one predicted fastest) -- and the cell kernels for each launch size, on the members' own grids and occupancy, and keeps the fastest.  All give the
- * same bits.  Fields are unchanged. */
+ * (the default before any autotune is the one predicted fastest) -- and the cell kernels for each launch
+ * size, on the members' own grids and occupancy, and keeps the fastest.  All give the same bits.  Fields
+ * are unchanged. */
 #define ZQ3D_ENS_TUNE_MAX 24
 typedef struct zq3d_ens_tune {
     int count;
@@ -562,7 +563,8 @@ int zq3d_ens_set_sweep(zq3d_ens* e, int kind, int tbx, int tby, int blocks);
 
 /* message of the last failed call on this thread ("" if none) */
 const char* zq3d_last_error(void);
-/* frees the device workspace cached by the Part 1/2 host-pointer functions */
+/* frees the device workspace and the pinned copy slots cached by the Part 1/2 host-pointer functions, and
+ * ends the threads that fill the slots */
 void zq3d_release_workspace(void);
 
 #ifdef __cplusplus

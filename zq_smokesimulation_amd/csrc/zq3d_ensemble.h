@@ -60,8 +60,8 @@ extern const int kEnsSweepShapes[kEnsSweepShapeCount][2];  // TBX x TBY of the s
 // of tiles it is issue that counts, and four cells a lane share the row's neighbours best; then how
 // evenly the tiles fill the CUs (one tile of four cells a lane a CU), which depends on the members.  64
 // members of 32 to 96 cells an axis (17.5 M cells), us per iteration: 34.5 to 45.6 with two cells a lane;
-// with four 37.2 at 8 planes, 28.9 at 16, 24.5 at 32 (the one-iteration launches on colour-split storage that these replace took 83.9, the half
-// sweeps at best 175).
+// with four 37.2 at 8 planes, 28.9 at 16, 24.5 at 32 (the one-iteration launches on colour-split storage
+// that these replace took 83.9, the half sweeps at best 175).
 constexpr int kEnsQuadShapeCount = 12;
 constexpr int kEnsQuadFixed = 7;  // shapes every ensemble has; the rest are the depths of four cells a lane
                                   // that are predicted fastest for its members

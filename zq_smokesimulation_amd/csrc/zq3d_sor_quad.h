@@ -2,9 +2,9 @@
 // planes in registers; shared by the single-grid kernel (kernels_project.hip) and the ensemble
 // kernel (kernels_ensemble.hip).
 //
-// Storage ("quad" layout): interleaved rows of S = quad_stride(W) values, no ghosts: cell (x, y, z) at (z*H + y)*S + x.  b holds the right-hand side, n the byte offset 4*count
-// of 1/count in the tile's table (0: not updated); cells W..S-1 have n = 0 and, in every pressure a
-// sweep writes, p = 0.
+// Storage ("quad" layout): interleaved rows of S = quad_stride(W) values, no ghosts: cell (x, y, z) at
+// (z*H + y)*S + x.  b holds the right-hand side, n the byte offset 4*count of 1/count in the tile's
+// table (0: not updated); cells W..S-1 have n = 0 and, in every pressure a sweep writes, p = 0.
 //
 // A thread owns CX neighbouring cells (both colours) of R rows and marches z.  With V_0 the old black
 // values and V_s the values after single-colour sweep s = 1..2K (odd red, even black), step t
@@ -22,7 +22,7 @@
 // What bounds it: at one sweep pair per pass (the colour-split tile of zq3d_sor_split.h) a step's
 // instructions are mostly indexing, LDS and selects (47 VALU a cell update); here an update takes
 // about 14, so K = 2 pays although it updates the halos twice.  Measured figures stand at
-// quad_shape_default (kernels_project.hip).
+// quad_plan (kernels_project.hip).
 #pragma once
 
 #include "zq3d_device.h"

@@ -1,6 +1,5 @@
 // zq3d_sor_split.h -- colour-split storage of the SOR and the one-pass red-black iteration of one
-// tile, shared by the single-grid kernel (kernels_project.hip) and the ensemble kernel
-// (kernels_ensemble.hip).
+// tile (the kernels are in kernels_project.hip).
 #pragma once
 
 #include "zq3d_device.h"
