@@ -36,8 +36,8 @@ hipGraph after the launch-shape autotuner; value = all members' voxels * steps /
 
 Prints one JSON line.  value = voxels * steps / wall time (Mvoxel-steps/s).  roofline: the
 red-black SOR sweep kernel the autotuner picked (the dominant kernel), algorithmic bytes 13 B/voxel
-per red+black iteration (6.5 B/voxel per single-colour launch) over its event-timed mean launch
-time; step_frac: the whole step's algorithmic bytes over the step time.  cpu_baseline: the
+per launch (a kernel that runs two iterations a launch reads and writes the grid once for both;
+6.5 B/voxel for a single-colour launch) over its event-timed mean launch time; step_frac: the whole step's algorithmic bytes over the step time.  cpu_baseline: the
 CPU oracle on a bounded sample of the same step (see --help).
 """
 import argparse
@@ -51,7 +51,7 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 METRIC = "Mvoxel-steps/s at 256³ fwd & fwd+adjoint; HBM GB/s vs peak; divergence"
 HBM_PEAK_GBS = 8000.0
-SOR_BYTES_PER_VOXEL_ITER = 13.0
+SOR_BYTES_PER_VOXEL = 13.0  # of one pass of the sweeps over the grid
 FULL_RUN = 500  # steps of the 256^3 workload
 # SOR relaxation of the 256^3 workload: the best of 1.93, 1.95, 1.96, 1.965, 1.968, 1.97, 1.972, 1.98,
 # 1.985, 1.99 over the 500-step run (sweeps per step 467, 334, 268, 235, 233, 237, 240, 325, 434, 635;
@@ -449,12 +449,12 @@ def optimal_omega(n):
     return 2.0 / (1.0 + math.sin(math.pi / n))
 
 
-def step_bytes(N, sweeps, residuals):
+def step_bytes(N, passes, residuals):
     """Algorithmic bytes of one forward step (compulsory reads and writes per stage, FP32 = 4 B,
     occupancy 1 B): force + attenuation 41, velocity advection 25, divergence 17, gradient correction
-    29, scalar advection 29 (141 B/voxel), 13 B/voxel per red+black SOR iteration and 9 B/voxel per
-    FP64 residual evaluation."""
-    return N * (141.0 + SOR_BYTES_PER_VOXEL_ITER * sweeps + 9.0 * residuals)
+    29, scalar advection 29 (141 B/voxel), 13 B/voxel per pass of the SOR over the grid (one or
+    more iterations) and 9 B/voxel per FP64 residual evaluation."""
+    return N * (141.0 + SOR_BYTES_PER_VOXEL * passes + 9.0 * residuals)
 
 
 def main():
@@ -555,14 +555,14 @@ def main():
     max_div = float(max(s["max_div"] for s in stats))
     converged = all(s["converged"] == 1 for s in stats)
 
-    # every SOR iteration is one fused launch (or two single-colour launches on grids too wide for
-    # the fused kernel's LDS ring); bytes per launch follow from iterations / launches
+    # a launch runs two iterations in one pass over the grid, or one, or one colour of one
     iters = float(sum(s["sweeps"] for s in stats))
     launches = max(tm["sor_launches"], 1)
     launch_ms = tm["ms_sor"] / launches
-    bytes_per_launch = SOR_BYTES_PER_VOXEL_ITER * N * iters / launches
+    grid_passes = min(1.0, launches / max(iters, 1.0))  # per iteration
+    bytes_per_launch = SOR_BYTES_PER_VOXEL * N * grid_passes * iters / launches
     achieved = bytes_per_launch / (launch_ms * 1e-3) / 1e9
-    step_gbs = step_bytes(N, sweeps_mean, outer_mean + 1.0) / (ms_per_step * 1e-3) / 1e9
+    step_gbs = step_bytes(N, grid_passes * sweeps_mean, outer_mean + 1.0) / (ms_per_step * 1e-3) / 1e9
     traffic = None
     tr = read_traffic(args.traffic or os.path.join(ROOT, "profiles", "%s_%d_traffic.txt" % (sor_kernel, W)))
     if tr and int(tr["size"]) == W and tr["kernel"] == sor_kernel:
@@ -582,7 +582,7 @@ def main():
                                    for q in (0, 50, 90, 100)},
         "max_div": float(max(s["max_div"] for s in full_stats)),
         "every_step_within_tol": all(s["converged"] == 1 and s["max_div"] <= args.tol for s in full_stats),
-        "step_frac": round(step_bytes(N, full_sweeps, full_passes + 1.0) / (full_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
+        "step_frac": round(step_bytes(N, grid_passes * full_sweeps, full_passes + 1.0) / (full_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
         "note": "steps 0..%d of the workload from rest on one clock (the timed steps included)" % (nfull - 1),
     }
     out = {
@@ -626,7 +626,8 @@ def main():
             "mean_launch_us": round(launch_ms * 1e3, 3),
             "step_achieved": round(step_gbs, 1),
             "step_frac": round(step_gbs / HBM_PEAK_GBS, 4),
-            "step_bytes": "N*(141 + 13*sweeps + 9*(passes + 1)) per step, means over the timed steps",
+            "step_bytes": "N*(141 + 13*launch passes over the grid + 9*(refinement passes + 1)) per step, "
+                          "means over the timed steps",
         },
         "projection": {
             "sor_sweeps_per_step": sweeps_mean,
