@@ -178,40 +178,45 @@ __device__ __forceinline__ void st_force_cell(const vec4_t<R>* __restrict__ vort
 // so the face becomes (face + dt*avg f) * aV in one read-modify-write.  AXIS 0/1/2 = u/v/w.
 // The reference's AddForce_w_Kernel also runs its interior formula at z = 0 reading cell z-1
 // (:380-384, out of bounds); this follows the slice variant (:400-419).
+// st_forced_face returns the face's new value and whether the face takes it (both are formed before
+// anything is stored, so that a kernel can have the operands of several faces in flight).
+template <class R>
+struct FaceUpdate {
+    R value;
+    bool ok;
+};
+
+template <class R, int AXIS, bool ATTEN>
+__device__ __forceinline__ FaceUpdate<R> st_forced_face(const R* __restrict__ face, const uint8_t* __restrict__ occ,
+                                                        const R* __restrict__ fc, const Dims& d, R dt, R dth, R aV,
+                                                        int i, int j, int k) {
+    const int pos = AXIS == 0 ? i : (AXIS == 1 ? j : k);
+    const int lim = AXIS == 0 ? d.W : (AXIS == 1 ? d.H : d.D);
+    const int step = AXIS == 0 ? 1 : (AXIS == 1 ? d.W : d.W * d.H);
+    const int ci = face_cell<AXIS>(d, i, j, k);
+    const R* f = fc + (size_t)AXIS * d.W * d.H * d.D;
+    // both cells' occupancy and force load together (on a domain face the low index is the face's
+    // own cell and its values are not used; ci points at the last cell where pos == lim)
+    const int cl = (pos > 0 && pos < lim) ? ci - step : ci;
+    const int oh = occ[ci], ol = occ[cl];
+    const R fh = f[ci], fl = f[cl];
+    const R f0 = face[face_index<AXIS>(d, i, j, k)];  // loaded with the occupancy, not after it
+    const bool domain = pos == 0 || pos == lim;
+    const R add = domain ? dt * fh : dth * (fh + fl);
+    FaceUpdate<R> r;
+    r.value = f0 + add;
+    if (ATTEN) r.value = r.value * aV;
+    r.ok = !oh && (domain || !ol);
+    return r;
+}
+
 template <class R, int AXIS, bool ATTEN>
 __device__ __forceinline__ void st_force_face(R* __restrict__ face, const uint8_t* __restrict__ occ,
                                               const R* __restrict__ fc, const Dims& d, R dt, R dth, R aV, int i, int j,
                                               int k) {
     if (!face_in<AXIS>(d, i, j, k)) return;
-    const int pos = AXIS == 0 ? i : (AXIS == 1 ? j : k);
-    const int lim = AXIS == 0 ? d.W : (AXIS == 1 ? d.H : d.D);
-    const int step = AXIS == 0 ? 1 : (AXIS == 1 ? d.W : d.W * d.H);
-    const int ci = face_cell<AXIS>(d, i, j, k);
-    const int fi = face_index<AXIS>(d, i, j, k);
-    const R* f = fc + (size_t)AXIS * d.W * d.H * d.D;
-    // both cells' occupancy and force load together (on a domain face the low index is the face's
-    // own cell and its values are not used)
-    const int cl = (pos > 0 && pos < lim) ? ci - step : ci;
-    const int oh = occ[ci], ol = occ[cl];
-    const R fh = f[ci], fl = f[cl];
-    bool ok;
-    R add;
-    if (pos == 0) {
-        ok = !oh;
-        add = dt * fh;
-    } else if (pos == lim) {
-        ok = !oh;  // ci already points at the last cell
-        add = dt * fh;
-    } else {
-        ok = !ol && !oh;
-        add = dth * (fh + fl);
-    }
-    const R f0 = face[fi];  // loaded with the occupancy, not after it
-    if (ok) {
-        R x = f0 + add;
-        if (ATTEN) x = x * aV;
-        face[fi] = x;
-    }
+    const FaceUpdate<R> r = st_forced_face<R, AXIS, ATTEN>(face, occ, fc, d, dt, dth, aV, i, j, k);
+    if (r.ok) face[face_index<AXIS>(d, i, j, k)] = r.value;
 }
 
 // ---- advection (ZQ_CUDA_Advection3D.cu, ZQ_CUDA_MACtoRegular.cu) ----
@@ -255,29 +260,32 @@ __device__ __forceinline__ void st_advect_cell(const vec4_t<R>* __restrict__ vel
 // Apply_Advect_Velocity_Result_{Open,Closed}_* (ZQ_CUDA_Advection3D.cu:471-650): the face value is
 // the average of the two advected cells (a domain face copies its inside cell) and is stored only
 // where the face's cells are fluid.
+// st_face_of_cells returns that value and whether it is stored.
 template <class R, int AXIS>
-__device__ __forceinline__ void st_cells_to_face(const R* __restrict__ adv, const uint8_t* __restrict__ occ,
-                                                 R* __restrict__ face, const Dims& d, int is_open, int i, int j,
-                                                 int k) {
-    if (!face_in<AXIS>(d, i, j, k)) return;
+__device__ __forceinline__ FaceUpdate<R> st_face_of_cells(const R* __restrict__ adv, const uint8_t* __restrict__ occ,
+                                                          const Dims& d, int is_open, int i, int j, int k) {
     const int pos = AXIS == 0 ? i : (AXIS == 1 ? j : k);
     const int lim = AXIS == 0 ? d.W : (AXIS == 1 ? d.H : d.D);
     const int step = AXIS == 0 ? 1 : (AXIS == 1 ? d.W : d.W * d.H);
     const int ci = face_cell<AXIS>(d, i, j, k);
     const R* a = adv + (size_t)AXIS * d.W * d.H * d.D;
-    const int cl = (pos > 0 && pos < lim) ? ci - step : ci;  // as in st_force_face
+    const int cl = (pos > 0 && pos < lim) ? ci - step : ci;  // as in st_forced_face
     const int oh = occ[ci], ol = occ[cl];
     const R ah = a[ci], al = a[cl];
-    bool ok;
-    R val;
-    if (pos == 0 || pos == lim) {
-        ok = is_open && !oh;
-        val = ah;
-    } else {
-        ok = !oh && !ol;
-        val = R(0.5) * (ah + al);
-    }
-    if (ok) face[face_index<AXIS>(d, i, j, k)] = val;
+    const bool domain = pos == 0 || pos == lim;
+    FaceUpdate<R> r;
+    r.value = domain ? ah : R(0.5) * (ah + al);
+    r.ok = !oh && (domain ? is_open != 0 : !ol);
+    return r;
+}
+
+template <class R, int AXIS>
+__device__ __forceinline__ void st_cells_to_face(const R* __restrict__ adv, const uint8_t* __restrict__ occ,
+                                                 R* __restrict__ face, const Dims& d, int is_open, int i, int j,
+                                                 int k) {
+    if (!face_in<AXIS>(d, i, j, k)) return;
+    const FaceUpdate<R> r = st_face_of_cells<R, AXIS>(adv, occ, d, is_open, i, j, k);
+    if (r.ok) face[face_index<AXIS>(d, i, j, k)] = r.value;
 }
 
 // Advect_Scalar_{Regular,MAC}_Velocity_Kernel (:379-469): backtrace from the cell centre, sample T
@@ -465,7 +473,7 @@ __device__ __forceinline__ F st_corrected_face(const uint8_t* __restrict__ occ, 
     const int step = AXIS == 0 ? 1 : (AXIS == 1 ? d.W : d.W * d.H);
     const int lo_bit = AXIS == 0 ? 1 : (AXIS == 1 ? 4 : 16);
     const int ci = face_cell<AXIS>(d, i, j, k);
-    const int oh = occ[ci], ol = occ[(pos > 0 && pos < lim) ? ci - step : ci];  // as in st_force_face
+    const int oh = occ[ci], ol = occ[(pos > 0 && pos < lim) ? ci - step : ci];  // as in st_forced_face
     bool ok;
     if (pos == 0) ok = (open_mask & lo_bit) && !oh;
     else if (pos == lim) ok = (open_mask & (lo_bit << 1)) && !oh;
