@@ -758,8 +758,8 @@ __global__ __launch_bounds__(BX* BY) void k_residual64(const uint8_t* __restrict
     if (threadIdx.x == 0 && threadIdx.y == 0) part[block_linear()] = m;
 }
 
-// k_residual64 marching z (QUAD: r32 into the quad layout's right-hand side r0, else into the split ones): each thread owns one (i, j) column of a chunk of rz planes and
-// keeps the pressures of planes k-1, k, k+1 in registers, so each padded FP64 pressure is read once
+// k_residual64 marching z (QUAD: r32 into the quad layout's right-hand side r0, else into the split
+// ones): each thread owns one (i, j) column of a chunk of rz planes and keeps the pressures of planes k-1, k, k+1 in registers, so each padded FP64 pressure is read once
 // (the per-plane kernel reads every plane for three neighbouring planes' blocks).  The same operations
 // per cell in the same order; the block maxima are over the chunk (a maximum is order-free).
 template <bool QUAD>
@@ -911,7 +911,9 @@ __device__ __forceinline__ F pred_face(F f, bool ok, double ph, double pl) {
 // next lane (the lane at a block's or the grid's edge evaluates it), the high v face from the
 // next row through LDS (likewise), the low w face is the plane below's high w face.  Every face
 // is evaluated once, and six times fewer loads are issued than with a cell per thread evaluating
-// all six.
+// all six.  Bound by memory latency: a plane's loads are all unconditional (an index outside the grid is
+// the cell's own, and its value is not used) and one barrier a plane suffices with two row buffers
+// (256^3: 127 us; with a load behind each occupancy test and two barriers 174).
 template <class F>
 __global__ __launch_bounds__(BX* BY) void k_max_div64_pred(const F* __restrict__ u, const F* __restrict__ v,
                                                            const F* __restrict__ w, const uint8_t* __restrict__ occ,
@@ -921,7 +923,7 @@ __global__ __launch_bounds__(BX* BY) void k_max_div64_pred(const F* __restrict__
                                                            double* __restrict__ part, Dims d, int rz) {
     static_assert(BX == 64, "a block row is one wave: the high u face comes from the next lane");
     __shared__ double red[4];
-    __shared__ F vrow[BY][BX];
+    __shared__ F vrow[2][BY][BX];
     const int tx = threadIdx.x, ty = threadIdx.y;
     const int i = blockIdx.x * BX + tx;
     const int j = blockIdx.y * BY + ty;
@@ -952,34 +954,30 @@ __global__ __launch_bounds__(BX* BY) void k_max_div64_pred(const F* __restrict__
         if (in) {
             n = nc[o];
             pu = p[q + sz];
-            ou = k + 1 < d.D ? occ[o + HW] : 1;
-            {  // low u face
-                const bool ok = i == 0 ? ((open_mask & 1) && !oc) : (!occ[o - 1] && !oc);
-                ul = pred_face(u[uidx(d, i, j, k)], ok, pc, p[q - 1]);
-            }
-            {  // low v face
-                const bool ok = j == 0 ? ((open_mask & 4) && !oc) : (!occ[o - W] && !oc);
-                vb = pred_face(v[vidx(d, i, j, k)], ok, pc, p[q - sy]);
-            }
-            {  // high w face
-                const bool ok = k + 1 == d.D ? ((open_mask & 32) && !oc) : (!oc && !ou);
-                wt = pred_face(w[widx(d, i, j, k + 1)], ok, pu, pc);
-            }
+            const double pl = p[q - 1], pb = p[q - sy];
+            const F fu = u[uidx(d, i, j, k)], fv = v[vidx(d, i, j, k)], fw = w[widx(d, i, j, k + 1)];
+            const int ol = occ[i > 0 ? o - 1 : o], ob = occ[j > 0 ? o - W : o], oh = occ[k + 1 < d.D ? o + HW : o];
+            ou = k + 1 < d.D ? oh : 1;
+            // low u, low v and high w face
+            ul = pred_face(fu, !oc & (i == 0 ? (open_mask & 1) != 0 : !ol), pc, pl);
+            vb = pred_face(fv, !oc & (j == 0 ? (open_mask & 4) != 0 : !ob), pc, pb);
+            wt = pred_face(fw, !oc & (k + 1 == d.D ? (open_mask & 32) != 0 : !ou), pu, pc);
             if (right_here) {
-                const bool ok = i + 1 == d.W ? ((open_mask & 2) && !oc) : (!occ[o + 1] && !oc);
-                ur = pred_face(u[uidx(d, i + 1, j, k)], ok, p[q + 1], pc);
+                const int orr = occ[i + 1 < W ? o + 1 : o];
+                ur = pred_face(u[uidx(d, i + 1, j, k)], !oc & (i + 1 == W ? (open_mask & 2) != 0 : !orr), p[q + 1],
+                               pc);
             }
             if (top_here) {
-                const bool ok = j + 1 == d.H ? ((open_mask & 8) && !oc) : (!occ[o + W] && !oc);
-                vt = pred_face(v[vidx(d, i, j + 1, k)], ok, p[q + sy], pc);
+                const int ot = occ[j + 1 < d.H ? o + W : o];
+                vt = pred_face(v[vidx(d, i, j + 1, k)], !oc & (j + 1 == d.H ? (open_mask & 8) != 0 : !ot), p[q + sy],
+                               pc);
             }
         }
         const F ul_next = __shfl_down(ul, 1, BX);
-        vrow[ty][tx] = vb;
+        vrow[k & 1][ty][tx] = vb;
         __syncthreads();
         if (!right_here) ur = ul_next;
-        if (!top_here) vt = vrow[ty + 1][tx];
-        __syncthreads();  // vrow is rewritten at the next plane
+        if (!top_here) vt = vrow[k & 1][ty + 1][tx];  // rewritten two planes on, past the next barrier
         if (in && n) {
             const double du = (double)ur - (double)ul;
             const double dv = (double)vt - (double)vb;
