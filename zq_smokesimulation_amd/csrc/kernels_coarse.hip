@@ -1143,10 +1143,7 @@ const float* launch_coarse_sor(const CoarseDims& cd, const CoarseBufs& B, float 
 }
 
 int coarse_sweep_candidates(const CoarseDims& cd, CoarseSweep* out, int max) {
-    // a launch a colour for grids too large for boxes (slabs are slower than boxes on every grid whose
-    // planes fit LDS: 5.8 against 2.45 us an iteration at 32^3, 6.5 against 4.3 at 64^3; they stay selectable)
     int n = 0;
-    if (n < max) out[n++] = CoarseSweep{0, 0};
     // boxes: the plain solver's choice and the shapes that were fastest on some coarse grid of 32^3 to 128^3
     const BlockCut c = block_best_cut(cd.Wc, cd.Hc, cd.Dc, 40, 512);
     int lg = 0;
@@ -1158,6 +1155,9 @@ int coarse_sweep_candidates(const CoarseDims& cd, CoarseSweep* out, int max) {
         for (int i = 0; i < n; i++) had = had || (out[i].k == b.k && out[i].zc == b.zc);
         if (n < max && !had) out[n++] = b;
     }
+    // a launch a colour for grids too large for boxes (slabs are slower than boxes on every grid whose
+    // planes fit LDS: 5.8 against 2.45 us an iteration at 32^3, 6.5 against 4.3 at 64^3; they stay selectable)
+    if (n < max) out[n++] = CoarseSweep{0, 0};
     return n;
 }
 
