@@ -38,7 +38,7 @@ __global__ __launch_bounds__(BX* BY) void k_force_cells(VI vort, R* __restrict__
 // cell's low u, v and w faces (the last column / row / plane also the domain's high face) with
 // st_force_face.  The w face below plane k reads the force and occupancy of plane k-1, which the
 // same thread read one iteration earlier.  Bound by memory latency: the three faces' operands load
-// together, before anything is stored (256^3: 135 us, 4.6 TB/s; one face after another 175).
+// together, before anything is stored (256^3: 135-142 us, 4.5 TB/s; one face after another 175).
 template <class R, bool ATTEN>
 __global__ __launch_bounds__(BX* BY) void k_force_faces(R* __restrict__ u, R* __restrict__ v, R* __restrict__ w,
                                                         const uint8_t* __restrict__ occ, const R* __restrict__ fc,
