@@ -6,7 +6,9 @@
 // are cut into batches of up to a slot, and each thread copies a batch between the caller's memory and
 // its own pinned slots (two, so that the link works on one while the thread works on the other) and
 // enqueues the device copy on the null stream, in whose order the kernels follow.  A call of one batch
-// (small grids) stays on the calling thread: its arrays share a slot and a single wait.
+// (small grids) stays on the calling thread: its arrays share a slot and a single wait.  Memory that the
+// runtime knows (pinned by the caller: the link reads it without a slot; or device memory, which the host
+// may not be able to read) is left to hipMemcpy.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -194,12 +196,30 @@ private:
         }
     }
 
-    // the arrays as batches of a slot each, small arrays sharing one
+    // whether the host array is ordinary memory (a query is about a microsecond)
+    static bool pageable(const void* p) {
+        hipPointerAttribute_t a{};
+        if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+        (void)hipGetLastError();  // (runtimes that report such memory as an error)
+        return true;
+    }
+
+    static hipError_t copy(const HostSpan& s, bool to_dev) {
+        return to_dev ? hipMemcpy(s.dev, s.host, s.bytes, hipMemcpyHostToDevice)
+                      : hipMemcpy(const_cast<void*>(s.host), s.dev, s.bytes, hipMemcpyDeviceToHost);
+    }
+
+    // the ordinary arrays as batches of a slot each, small arrays sharing one
     void plan(std::initializer_list<HostSpan> a) {
         pieces_.clear();
         batches_.clear();
+        direct_.clear();
         size_t at = kSlot;
-        for (const HostSpan& s : a)
+        for (const HostSpan& s : a) {
+            if (s.bytes && !pageable(s.host)) {
+                direct_.push_back(s);
+                continue;
+            }
             for (size_t o = 0; o < s.bytes;) {
                 if (at >= kSlot) {
                     batches_.push_back(Batch{pieces_.size(), 0});
@@ -211,6 +231,7 @@ private:
                 o += n;
                 at = (at + n + 255) & ~(size_t)255;
             }
+        }
     }
 
     void start() {
@@ -238,16 +259,16 @@ private:
         } catch (...) {  // no memory for the plan: the plain copies
             hipError_t e = hipSuccess;
             for (const HostSpan& s : a)
-                if (s.bytes && e == hipSuccess)
-                    e = to_dev ? hipMemcpy(s.dev, s.host, s.bytes, hipMemcpyHostToDevice)
-                               : hipMemcpy(const_cast<void*>(s.host), s.dev, s.bytes, hipMemcpyDeviceToHost);
+                if (s.bytes && e == hipSuccess) e = copy(s, to_dev);
             return e;
         }
-        if (batches_.empty()) return hipSuccess;
+        hipError_t e = hipSuccess;
+        for (size_t k = 0; k < direct_.size() && e == hipSuccess; k++) e = copy(direct_[k], to_dev);
+        if (e != hipSuccess || batches_.empty()) return e;
         to_dev_ = to_dev;
         next_ = 0;
         err_.store(hipSuccess);
-        hipError_t e = hipGetDevice(&device_);
+        e = hipGetDevice(&device_);
         if (e != hipSuccess) return e;
         const bool many = batches_.size() > 1 && pool_;
         if (many) {
@@ -267,6 +288,7 @@ private:
 
     std::vector<Piece> pieces_;
     std::vector<Batch> batches_;
+    std::vector<HostSpan> direct_;  // arrays that hipMemcpy takes
     std::atomic<size_t> next_{0};
     std::atomic<hipError_t> err_{hipSuccess};
     bool to_dev_ = false;
