@@ -132,6 +132,16 @@ OPAQUE = r"""
     CHECK(h.to_host({{db.data(), p, N}, {da.data(), b.data(), N}}) == hipSuccess);
     CHECK(hidden == b0 && b == a);
 """
+# two results for one array (a caller with one scalar field passes it twice): the later one stays, also where
+# the earlier one's copies are slow to arrive
+SHARED = r"""
+    std::vector<char> host(2 * N), first = array(5), second = array(6);
+    fake.slow = first.data(), fake.slow_n = 64;
+    CHECK(h.to_host({{first.data(), host.data(), N}, {second.data(), host.data(), N}}) == hipSuccess);
+    CHECK(std::memcmp(host.data(), second.data(), N) == 0);
+    CHECK(h.to_host({{first.data(), host.data() + N / 2, N}, {second.data(), host.data(), N}}) == hipSuccess);
+    CHECK(std::memcmp(host.data(), second.data(), N) == 0 && std::memcmp(host.data() + N, first.data() + N / 2, N / 2) == 0);
+"""
 
 
 def run(tmp_path, body):
@@ -150,3 +160,7 @@ def run(tmp_path, body):
 @pytest.mark.parametrize("body", [PINNED, OPAQUE], ids=["pinned", "opaque"])
 def test_memory_the_runtime_knows_goes_to_hipmemcpy(tmp_path, body):
     run(tmp_path, body)
+
+
+def test_results_for_one_array_keep_their_order(tmp_path):
+    run(tmp_path, SHARED)

@@ -12,6 +12,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 #include <unistd.h>
 
 #include <algorithm>
@@ -252,15 +253,32 @@ private:
         }
     }
 
+    // the arrays one after the other
+    static hipError_t in_turn(std::initializer_list<HostSpan> a, bool to_dev) {
+        hipError_t e = hipSuccess;
+        for (const HostSpan& s : a)
+            if (s.bytes && e == hipSuccess) e = copy(s, to_dev);
+        return e;
+    }
+
+    // whether two of the host arrays share memory
+    static bool overlap(std::initializer_list<HostSpan> a) {
+        for (const HostSpan* s = a.begin(); s != a.end(); s++)
+            for (const HostSpan* t = a.begin(); t != s; t++) {
+                const uintptr_t x = (uintptr_t)s->host, y = (uintptr_t)t->host;
+                if (s->bytes && t->bytes && x < y + t->bytes && y < x + s->bytes) return true;
+            }
+        return false;
+    }
+
     hipError_t run(std::initializer_list<HostSpan> a, bool to_dev) {
+        // results for one array (a caller's single scalar field as temperature and density): the last one stays
+        if (!to_dev && overlap(a)) return in_turn(a, to_dev);
         try {
             plan(a);
             if (batches_.size() > 1) start();
         } catch (...) {  // no memory for the plan: the plain copies
-            hipError_t e = hipSuccess;
-            for (const HostSpan& s : a)
-                if (s.bytes && e == hipSuccess) e = copy(s, to_dev);
-            return e;
+            return in_turn(a, to_dev);
         }
         hipError_t e = hipSuccess;
         for (size_t k = 0; k < direct_.size() && e == hipSuccess; k++) e = copy(direct_[k], to_dev);
