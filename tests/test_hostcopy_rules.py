@@ -142,6 +142,17 @@ SHARED = r"""
     CHECK(h.to_host({{first.data(), host.data() + N / 2, N}, {second.data(), host.data(), N}}) == hipSuccess);
     CHECK(std::memcmp(host.data(), second.data(), N) == 0 && std::memcmp(host.data() + N, first.data() + N / 2, N / 2) == 0);
 """
+# a kernel launch that failed before the copies is still reported when they find no pinned memory
+FAILED_LAUNCH = r"""
+    std::vector<char> host(N), dev = array(7);
+    fake.no_pinned = true;
+    fake_last = hipErrorLaunchFailure;
+    hipError_t e = h.to_host({{dev.data(), host.data(), N}});
+    if (e == hipSuccess) e = hipGetLastError();
+    CHECK(e == hipErrorLaunchFailure && host == dev);
+    fake_last = hipSuccess;
+    CHECK(h.to_device({{dev.data(), host.data(), N}}) == hipSuccess && hipGetLastError() == hipSuccess);
+"""
 
 
 def run(tmp_path, body):
@@ -164,3 +175,7 @@ def test_memory_the_runtime_knows_goes_to_hipmemcpy(tmp_path, body):
 
 def test_results_for_one_array_keep_their_order(tmp_path):
     run(tmp_path, SHARED)
+
+
+def test_an_earlier_error_is_not_lost(tmp_path):
+    run(tmp_path, FAILED_LAUNCH)

@@ -272,6 +272,13 @@ private:
     }
 
     hipError_t run(std::initializer_list<HostSpan> a, bool to_dev) {
+        // an error of earlier work on this thread (a launch that failed): the copies may clear it
+        const hipError_t before = hipPeekAtLastError();
+        const hipError_t e = copy_all(a, to_dev);
+        return e != hipSuccess ? e : before;
+    }
+
+    hipError_t copy_all(std::initializer_list<HostSpan> a, bool to_dev) {
         // results for one array (a caller's single scalar field as temperature and density): the last one stays
         if (!to_dev && overlap(a)) return in_turn(a, to_dev);
         try {
