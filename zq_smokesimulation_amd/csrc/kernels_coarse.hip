@@ -17,6 +17,7 @@
 
 #include "zq3d_coarse.h"
 #include "zq3d_kernels.h"
+#include "zq3d_lds.h"
 #include "zq3d_sor_block.h"
 
 namespace zq3d {
@@ -1062,10 +1063,8 @@ size_t coarse_slab_lds(const CoarseDims& cd, CoarseSweep sw) {
 }
 
 bool slab_lds_enabled() {
-    static const bool ok =
-        hipFuncSetAttribute((const void*)k_coarse_slab, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSlabMaxLds) ==
-        hipSuccess;
-    return ok;
+    static LdsLimit limit;
+    return limit.raise((const void*)k_coarse_slab, (int)kSlabMaxLds) == hipSuccess;
 }
 
 BlockCut coarse_block(const CoarseDims& cd, CoarseSweep sw) {

@@ -14,6 +14,7 @@
 // MAC to cells 292, 94; set-up 417, 300; cell force 274, 191; vorticity 197, 165; force faces 460, 247;
 // face apply 446, 189; correction 468, 152.  All bound by memory or, the advections, by their gathers.
 #include "zq3d_ensemble.h"
+#include "zq3d_lds.h"
 #include "zq3d_sor_quad.h"
 #include "zq3d_stencils.h"
 
@@ -261,9 +262,9 @@ namespace {
 template <int K, int CX, int NTH>
 hipError_t launch_quad(const EnsLaunch& L, const EnsQuadTable& T, int at, hipStream_t s) {
     constexpr int lds = 4 * quad_lds_floats(K, CX, NTH);
-    if constexpr (lds > 64 * 1024) {  // above the default limit of dynamic LDS: allowed once per process
-        static const hipError_t e = hipFuncSetAttribute((const void*)ke_sor_quad<K, CX, NTH>,
-                                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if constexpr (lds > 64 * 1024) {
+        static LdsLimit limit;
+        const hipError_t e = limit.raise((const void*)ke_sor_quad<K, CX, NTH>, lds);
         if (e != hipSuccess) return e;
     }
     hipLaunchKernelGGL((ke_sor_quad<K, CX, NTH>), dim3((unsigned)T.total), dim3(NTH), lds, s, L.members, T, at);

@@ -14,6 +14,7 @@
 // one partial per block (wave butterfly + LDS), then one block folds the partials in index order.
 #include "zq3d_device.h"
 #include "zq3d_kernels.h"
+#include "zq3d_lds.h"
 #include "zq3d_sor_block.h"
 #include "zq3d_sor_quad.h"
 #include "zq3d_sor_split.h"
@@ -1118,13 +1119,11 @@ template <int K, int CX, int NT>
 hipError_t launch_quad_one(const Dims& d, const QuadBufs& q, const QuadCut& c, const float* src, float* dst,
                            const float* mean32, float omega, hipStream_t s) {
     constexpr int lds = 4 * quad_lds_floats(K, CX, NT);
-    if constexpr (lds > 64 * 1024) {  // above the default limit of dynamic LDS: allowed once per process
-        static const hipError_t e0 = hipFuncSetAttribute((const void*)k_sor_quad<K, CX, NT, false>,
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        static const hipError_t e1 = hipFuncSetAttribute((const void*)k_sor_quad<K, CX, NT, true>,
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if (e0 != hipSuccess) return e0;
-        if (e1 != hipSuccess) return e1;
+    if constexpr (lds > 64 * 1024) {
+        static LdsLimit plain, masked;
+        const hipError_t e = c.mask ? masked.raise((const void*)k_sor_quad<K, CX, NT, true>, lds)
+                                    : plain.raise((const void*)k_sor_quad<K, CX, NT, false>, lds);
+        if (e != hipSuccess) return e;
     }
     const int nb = (c.nx * c.ny * c.nz + 7) & ~7;
     const float omw = 1.0f - omega;
@@ -1143,9 +1142,11 @@ template <int NT>
 hipError_t launch_block_one(const Dims& d, const QuadBufs& q, const BlockCut& c, const float* src, float* dst,
                             const float* mean32, int iters, float omega, hipStream_t s) {
     const int lds = block_lds_bytes(c);
-    static const hipError_t e = hipFuncSetAttribute((const void*)k_sor_block<NT>,
-                                                    hipFuncAttributeMaxDynamicSharedMemorySize, 32 + 96 * (NT + 1));
-    if (e != hipSuccess) return e;
+    if constexpr (32 + 96 * (NT + 1) > 64 * 1024) {
+        static LdsLimit limit;
+        const hipError_t e = limit.raise((const void*)k_sor_block<NT>, 32 + 96 * (NT + 1));
+        if (e != hipSuccess) return e;
+    }
     const int nb = (c.nx * c.ny * c.nz + 7) & ~7;
     hipLaunchKernelGGL(k_sor_block<NT>, dim3(nb), dim3((block_threads(c) + 63) & ~63), lds, s, q.n, q.b, mean32, src,
                        dst, d, c, iters, omega, 1.0f - omega);
