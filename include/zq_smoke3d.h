@@ -483,7 +483,8 @@ int zq3d_adj_set_adjoint_tol(zq3d_adj* a, double rtol);
  * (whose controls are those of that forward); until then recomputed steps solve as without it. */
 int zq3d_adj_set_pressure_store(zq3d_adj* a, int on);
 /* sweep algorithm / tile shape of every projection of the rollout, as zq3d_set_sor_shape takes it for
- * this grid (the default is the one a simulation has); all give the same bits */
+ * this grid (a rollout begins with a simulation's default, and (0, 0) restores it); all give the same
+ * bits */
 int zq3d_adj_set_sor_shape(zq3d_adj* a, int ty, int zc);
 /* initial state: ZQ3D_FIELD_U/V/W/T/RHO (device, chosen precision), ZQ3D_FIELD_OCC (device bytes) or
  * ZQ3D_FIELD_P64 (device doubles, padded: the forward projection's warm start; default 0) */

@@ -253,6 +253,24 @@ def test_sweep_shape_does_not_change_rollout_or_gradient(dtype):
         np.testing.assert_allclose(g, out[0][1], rtol=0, atol=tol * gmax)
 
 
+def test_the_default_sweeps_can_be_restored():
+    """set_sor_shape(0, 0) puts a rollout back to the sweeps it was created with; what no grid supports is
+    still refused and leaves the shape as it was."""
+    import zq_smokesimulation_amd as z
+    W, H, D, nsteps = 40, 36, 28, 2
+    eng, _ = make_engine(W, H, D, nsteps, 2, torch.float32, closed=True, obstacle=True)
+    ctrl = torch.zeros(eng.controls_shape(), device=DEV)
+    want = eng.forward(ctrl).cpu().numpy()
+    for shape in ((-16, 16), (0, 0)):
+        print("shape", shape, flush=True)
+        eng.set_sor_shape(*shape)
+        np.testing.assert_array_equal(eng.forward(ctrl).cpu().numpy(), want)
+    with pytest.raises(z.ZQ3DError):
+        eng.set_sor_shape(-3, 8)
+    np.testing.assert_array_equal(eng.forward(ctrl).cpu().numpy(), want)
+    eng.close()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_pressure_store_gives_the_same_rollout_and_gradient(dtype):
     """With the forward's pressures stored, the backward's recomputed steps apply them instead of

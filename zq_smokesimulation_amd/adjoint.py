@@ -106,7 +106,8 @@ class SmokeRollout:
         check(_lib.lib().zq3d_adj_set_pressure_store(self._h, int(bool(on))), "zq3d_adj_set_pressure_store")
 
     def set_sor_shape(self, ty, zc):
-        """Sweep algorithm of every projection (a SmokeSim3D.autotune_sor candidate); same bits."""
+        """Sweep algorithm of every projection (a SmokeSim3D.autotune_sor candidate; (0, 0): the
+        default); same bits."""
         check(_lib.lib().zq3d_adj_set_sor_shape(self._h, int(ty), int(zc)), "zq3d_adj_set_sor_shape")
 
     # ---- rollout -------------------------------------------------------------------

@@ -565,8 +565,8 @@ extern "C" int zq3d_adj_set_sor_shape(zq3d_adj* a, int ty, int zc) {
     const char* where = "zq3d_adj_set_sor_shape";
     if (!a) { set_err(where, "null handle"); return ZQ3D_ERR_ARG; }
     const SorShape want{ty, zc};
-    if ((ty == 0 && zc == 0) || !sor_shape_valid(a->d, want)) {
-        set_err(where, "shape not among the sweep candidates for this grid");
+    if (!sor_shape_valid(a->d, want)) {
+        set_err(where, "shape not supported for this grid");
         return ZQ3D_ERR_ARG;
     }
     if (is_split(want))
