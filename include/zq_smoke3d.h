@@ -381,7 +381,8 @@ int zq3d_set_sor_shape(zq3d_sim* sim, int ty, int zc);
  * red-black sweeps.  k == 0: one launch per colour; k > 0: k iterations per launch, each workgroup
  * owning zc z-planes of the coarse grid and recomputing a halo of 2k planes in LDS, or, with
  * zc == -(10000 log2(lx) + 100 ty + tz), boxes of lx x ty x tz threads (lx a power of two up to 64, 512
- * threads at most) that hold 2 x 2 x 4 cells each in registers (k up to 8).  zq3d_create times the valid schedules and keeps the fastest; all produce the same bits. */
+ * threads at most) that hold 2 x 2 x 4 cells each in registers (k up to 8).  zq3d_create takes the
+ * schedule predicted fastest for the coarse grid; all produce the same bits. */
 int zq3d_set_coarse_sweep(zq3d_sim* sim, int k, int zc);
 int zq3d_get_coarse_sweep(zq3d_sim* sim, int* k, int* zc);
 /* Guiding control of the coarse + sub-grid projection (ZQ_ApplyGuidingVelocity3D,

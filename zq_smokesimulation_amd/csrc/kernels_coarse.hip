@@ -1141,23 +1141,21 @@ const float* launch_coarse_sor(const CoarseDims& cd, const CoarseBufs& B, float 
     return src;
 }
 
-int coarse_sweep_candidates(const CoarseDims& cd, CoarseSweep* out, int max) {
-    int n = 0;
-    // boxes: the plain solver's choice and the shapes that were fastest on some coarse grid of 32^3 to 128^3
-    const BlockCut c = block_best_cut(cd.Wc, cd.Hc, cd.Dc, 40, 512);
+// Boxes where they are predicted faster than a launch a colour (6.4 us an iteration and 11.5 ps a cell:
+// 6.7 us at 64^3, 199 at 256^3).  They were on every grid measured; what the rule gives, in microseconds an
+// iteration, beside the fastest of all boxes and a launch a colour:
+//   32^3  2.64, 2.64, 6.5   64^3  4.54, 4.54, 7.1   100x60x40  4.4, 4.2, 8.0   96^3  8.6, 8.6, 15.7
+//   128^3  21.1, 18.6, 25.4   256^3  158, 156, 200   worst of 35 grids: 64x64x256  12.7, 9.7, 12.5
+// (Slabs take 3.8 to 13 where their planes fit LDS; they stay selectable.)  No schedule is timed at creation:
+// that cost 1.7 ms at 64^3 and 6.9 at 128^3.
+CoarseSweep coarse_sweep_default(const CoarseDims& cd) {
+    const size_t cells = (size_t)quad_stride(cd.Wc) * cd.Hc * cd.Dc;
+    double us = 0.0;
+    const BlockCut c = block_best_cut(cd.Wc, cd.Hc, cd.Dc, 40, 512, &us, block_cost_weighted);
     int lg = 0;
     while ((1 << lg) < c.lx) lg++;
-    const CoarseSweep boxes[] = {{c.K, -(10000 * lg + 100 * c.ty + c.tz)}, {3, -30804}, {2, -30503}, {2, -30805},
-                                 {3, -40804}, {2, -31004}, {2, -40605}};
-    for (const CoarseSweep& b : boxes) {
-        bool had = !coarse_sweep_valid(cd, b);
-        for (int i = 0; i < n; i++) had = had || (out[i].k == b.k && out[i].zc == b.zc);
-        if (n < max && !had) out[n++] = b;
-    }
-    // a launch a colour for grids too large for boxes (slabs are slower than boxes on every grid whose
-    // planes fit LDS: 5.8 against 2.45 us an iteration at 32^3, 6.5 against 4.3 at 64^3; they stay selectable)
-    if (n < max) out[n++] = CoarseSweep{0, 0};
-    return n;
+    const CoarseSweep box{c.K, -(10000 * lg + 100 * c.ty + c.tz)};
+    return c.nx && us <= 6.4 + 11.5e-6 * cells && coarse_sweep_valid(cd, box) ? box : CoarseSweep{0, 0};
 }
 
 void launch_coarse_prolong(const CoarseDims& cd, const CoarseBufs& B, const float* p, int open_mask, const uint8_t* occ,

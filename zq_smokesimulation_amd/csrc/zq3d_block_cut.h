@@ -61,9 +61,22 @@ inline double block_cost(const BlockCut& c, int k) {
     return 3.65 + rounds * (0.96 + 0.35 * simd + 2.0 * k * 0.26 * simd);
 }
 
+// The same of the weighted operator (the coarse grid's sweeps), whose weights fill the registers: a CU holds 8
+// waves, and all boxes' loads (six arrays of short rows) count, 0.67 ps a cell and 8.7 a row of the box.
+// (Fitted to 3700 launches on 17 grids from 8^3 to 256^3, profiles/coarse_box_shapes.txt.)
+inline double block_cost_weighted(const BlockCut& c, int k) {
+    const int waves = (block_threads(c) + 63) / 64, boxes = c.nx * c.ny * c.nz;
+    const int per = (boxes + 255) / 256, holds = std::max(1, 8 / waves);
+    const int rounds = (per + holds - 1) / holds;
+    const double simd = std::max(1.0, waves * std::min(per, holds) / 4.0);
+    const double rows = (double)boxes * (BLOCK_Y * c.ty) * (BLOCK_Z * c.tz);
+    return 2.0 + rounds * (2.2 + 0.55 * simd + 2.0 * k * (0.26 + 0.2 * simd)) + 1e-6 * rows * (0.67 * BLOCK_X * c.lx + 8.7);
+}
+
 // The cheapest cut per iteration of at most `most` threads (iters: of a pass; a single box runs all of
 // them in one launch).
-inline BlockCut block_best_cut(int W, int H, int D, int iters, int most, double* cost = nullptr) {
+inline BlockCut block_best_cut(int W, int H, int D, int iters, int most, double* cost = nullptr,
+                               double (*price)(const BlockCut&, int) = block_cost) {
     static const int tys[] = {4, 5, 6, 7, 8, 9, 10, 12, 14, 16, 20, 24, 32};
     static const int tzs[] = {1, 2, 3, 4, 5, 6, 7, 8};
     BlockCut best{};
@@ -75,7 +88,7 @@ inline BlockCut block_best_cut(int W, int H, int D, int iters, int most, double*
                     const BlockCut c = block_cut(W, H, D, lx, ty, tz, K);
                     if (!c.nx || (c.halo == 0 && K > 1) || block_threads(c) > most) continue;
                     const int k = c.halo ? K : std::max(iters, 1);
-                    const double t = block_cost(c, k) / k;
+                    const double t = price(c, k) / k;
                     if (best.nx == 0 || t < least) {
                         best = c;
                         least = t;

@@ -64,57 +64,17 @@ int check_block(const Dims& d, int s, const char* where) {
 
 }  // namespace
 
-// Times the candidate schedules (iters iterations each, HIP events on the null stream; a second run for one
-// within a quarter of the best so far) on the coarse arrays as they stand and keeps the fastest; all
-// schedules give the same bits.
-int tune_coarse_sweep(CoarseState* c, int iters, const char* where) {
-    CoarseSweep cand[20];
-    const int n = coarse_sweep_candidates(c->cd, cand, 20);
-    hipEvent_t a = nullptr, b = nullptr;
-    ZQ_HIP(hipEventCreate(&a), where);
-    ZQ_HIP(hipEventCreate(&b), where);
-    float best = 0.0f;
-    int bi = -1;
-    for (int i = 0; i < n; i++) {
-        (void)launch_coarse_sor(c->cd, c->B, 1.0f, 2, cand[i], nullptr);  // first-launch costs
-        for (int run = 0; run < 2; run++) {
-            (void)hipEventRecord(a, nullptr);
-            (void)launch_coarse_sor(c->cd, c->B, 1.0f, iters, cand[i], nullptr);
-            (void)hipEventRecord(b, nullptr);
-            (void)hipEventSynchronize(b);
-            float ms = 0.0f;
-            (void)hipEventElapsedTime(&ms, a, b);
-            if (bi >= 0 && ms > 1.25f * best) break;
-            if (bi < 0 || ms < best) {
-                best = ms;
-                bi = i;
-            }
-        }
-    }
-    (void)hipEventDestroy(a);
-    (void)hipEventDestroy(b);
-    ZQ_HIP(hipGetLastError(), where);
-    c->sweep = cand[bi];
-    return ZQ3D_OK;
-}
-
 int coarse_create(const Dims& d, int s, CoarseState* out, const char* where) {
     if (int rc = check_block(d, s, where)) return rc;
     out->cd = coarse_dims(d, s);
     const size_t bytes = coarse_layout(out->cd, nullptr, nullptr);
     ZQ_HIP(hipMalloc(&out->mem, bytes), where);
     coarse_layout(out->cd, (char*)out->mem, &out->B);
-    // a fluid coarse grid with unit fractions to time the schedules on
-    launch_fill_f32(out->B.rU, out->cd.Nu(), 1.0f, nullptr);
-    launch_fill_f32(out->B.rV, out->cd.Nv(), 1.0f, nullptr);
-    launch_fill_f32(out->B.rW, out->cd.Nw(), 1.0f, nullptr);
-    launch_fill_f32(out->B.inv, out->cd.Nc(), 1.0f / 6.0f, nullptr);
-    launch_fill_f32(out->B.div, out->cd.Nc(), 0.0f, nullptr);
     launch_fill_f32(out->B.p, out->cd.Np(), 0.0f, nullptr);
     launch_fill_f32(out->B.p2, out->cd.Np(), 0.0f, nullptr);
     ZQ_HIP(hipStreamSynchronize(nullptr), where);
-    // multiples of every box depth; fewer where an iteration is long enough to be told apart
-    return tune_coarse_sweep(out, out->cd.Nc() > (size_t)64 * 64 * 64 ? 12 : 24, where);
+    out->sweep = coarse_sweep_default(out->cd);
+    return ZQ3D_OK;
 }
 
 int coarse_set_guide(CoarseState* c, float coeff, const float* gu, const float* gv, const float* gw, hipStream_t s,

@@ -62,8 +62,8 @@ struct CoarseSweep {
     int k, zc;
 };
 bool coarse_sweep_valid(const CoarseDims& g, CoarseSweep sw);
-// schedules valid for the grid (LDS of a slab within 160 KiB); returns the count
-int coarse_sweep_candidates(const CoarseDims& g, CoarseSweep* out, int max);
+// the schedule predicted fastest for the grid
+CoarseSweep coarse_sweep_default(const CoarseDims& g);
 // closed domains: div -= mean * vol on every non-solid coarse cell, mean = sum(div) / sum(vol) over
 // them in FP64 (one workgroup, fixed summation order, so repeatable)
 void launch_coarse_remove_mean(const CoarseDims& g, const CoarseBufs& B, hipStream_t s);
