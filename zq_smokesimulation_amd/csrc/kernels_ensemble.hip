@@ -24,6 +24,23 @@ namespace {
 
 constexpr int NT = 256;
 
+// the tiles of a table, one a thread; the member by binary search over the members' first tiles
+__global__ __launch_bounds__(NT) void ke_tiles(const EnsMember* __restrict__ M, int count, const int* __restrict__ first,
+                                               int total, EnsTiling t, EnsTile* __restrict__ out) {
+    const int tile = blockIdx.x * NT + threadIdx.x;
+    if (tile >= total) return;
+    int lo = 0, hi = count - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (first[mid] <= tile) lo = mid;
+        else hi = mid - 1;
+    }
+    const Dims d = M[lo].d;
+    const int local = tile - first[lo], per = ens_plane_tiles(d, t), z = local / per, b = local - z * per;
+    out[tile] = t.tbx ? EnsTile{lo, b, local, z}
+                      : EnsTile{lo, 256 * b, z * kEnsPlanes, min((z + 1) * kEnsPlanes, d.D)};
+}
+
 // Runs f(member, i, j, k) over the tiles of table T: cells first .. first + 255 of the plane, planes
 // k0 .. k1 - 1.
 template <class F>
@@ -220,6 +237,13 @@ inline unsigned grid_of(const EnsTable& T, int blocks) {
 
 // tile layouts of the sweep kernel (TBX x TBY) the autotuner may pick
 const int kEnsSweepShapes[kEnsSweepShapeCount][2] = {{64, 4}, {32, 8}, {16, 16}};
+
+hipError_t ens_launch_tiles(const EnsMember* members, int count, const int* first, int total, EnsTiling t, EnsTile* out,
+                            hipStream_t s) {
+    hipLaunchKernelGGL(ke_tiles, dim3((unsigned)((total + NT - 1) / NT)), dim3(NT), 0, s, members, count, first, total, t,
+                       out);
+    return hipGetLastError();
+}
 
 hipError_t ens_launch_step(const EnsLaunch& L, hipStream_t s) {
     const dim3 nt(NT), gc(grid_of(L.cells, L.blocks));

@@ -5,10 +5,9 @@
 
 #include <algorithm>
 #include <cstring>
-#include <functional>
-#include <queue>
 #include <vector>
 
+#include "zq3d_ens_plan.h"
 #include "zq3d_ensemble.h"
 #include "zq3d_internal.h"
 #include "zq3d_kernels.h"
@@ -23,7 +22,6 @@ struct zq3d_ens {
     std::vector<Dims> dims;
     std::vector<EnsMember> host;  // descriptors as uploaded
     EnsMember* dev_members = nullptr;
-    EnsTile* dev_tables = nullptr;
     std::vector<void*> allocs;
     hipStream_t stream = nullptr;
     EnsLaunch L{};
@@ -36,8 +34,6 @@ struct zq3d_ens {
     double* part = nullptr;
     uint8_t* quad_n = nullptr;  // quad-layout counts, right-hand sides, pressures (two)
     float *quad_b = nullptr, *quad_p[2] = {nullptr, nullptr};
-    EnsQuadTile* dev_tiles = nullptr;
-    QuadCut* dev_cuts = nullptr;
     size_t Nu = 0, Nv = 0, Nw = 0, Nc = 0, Np = 0, Nparts = 0, Nq = 0;
     long long cells = 0;
     hipGraph_t graph = nullptr;
@@ -82,66 +78,53 @@ int ens_alloc(zq3d_ens* e, T** p, size_t bytes) {
     return 0;
 }
 
-// blocks of tbx x tby cells (half: of half rows) of every member
-std::vector<EnsTile> block_tiles(const zq3d_ens* e, int tbx, int tby, bool half) {
-    std::vector<EnsTile> t;
-    for (int s = 0; s < e->count; s++) {
-        const Dims& d = e->dims[s];
-        const int gx = cdiv(half ? (d.W + 1) / 2 : d.W, tbx), gy = cdiv(d.H, tby);
-        int n = 0;
-        for (int z = 0; z < d.D; z++)
-            for (int b = 0; b < gx * gy; b++) t.push_back(EnsTile{s, b, n++, z});
-    }
-    return t;
-}
+// Columns of tiles of the same waves and planes.
+struct QuadColumns {
+    int nw, D;
+    long long n;
+};
 
-// 256 cells of a plane x kEnsPlanes planes of every member
-std::vector<EnsTile> cell_tiles(const zq3d_ens* e) {
-    std::vector<EnsTile> t;
+// The members' tile columns under shapes of cx cells a lane and nw waves.
+std::vector<QuadColumns> quad_columns(const zq3d_ens* e, int cx, int nw) {
+    std::vector<QuadColumns> all;
     for (int s = 0; s < e->count; s++) {
         const Dims& d = e->dims[s];
-        for (int z = 0; z < d.D; z += kEnsPlanes)
-            for (int c = 0; c < d.W * d.H; c += 256) t.push_back(EnsTile{s, c, z, std::min(z + kEnsPlanes, d.D)});
-    }
-    return t;
-}
-
-// The tiles of every member under shape {cells a lane, waves, planes} for K iterations a launch, the longest
-// first, and the members' cuts (either null: not wanted); returns the microseconds a launch is predicted
-// to take: tiles start in this order, XCD b % 8 takes block b, a CU one tile at a time, and a tile costs
-// its plane steps by quad_cost's latency and issue time.
-double quad_table(const zq3d_ens* e, int K, const int shape[3], std::vector<EnsQuadTile>* tiles,
-                  std::vector<QuadCut>* cuts) {
-    struct Timed {
-        double us;
-        EnsQuadTile t;
-    };
-    std::vector<Timed> all;
-    for (int s = 0; s < e->count; s++) {
-        const Dims& d = e->dims[s];
-        const QuadCut c = quad_cut(d.W, d.H, d.D, K, shape[0], shape[1], shape[2]);
-        if (cuts) cuts->push_back(c);
-        for (int z = 0; z < c.nz; z++) {
-            const int steps = quad_z_begin(c, K, z + 1, d.D) - quad_z_begin(c, K, z, d.D) + (z ? 4 * K - 2 : 2 * K - 1);
-            const double us = 1.5 + steps * quad_step_us(K, shape[0], c.nw);
-            for (int y = 0; y < c.ny; y++)
-                for (int x = 0; x < c.nx; x++) all.push_back(Timed{us, EnsQuadTile{s, x, y, z}});
+        const Dims* last = s ? &e->dims[s - 1] : nullptr;
+        if (last && last->W == d.W && last->H == d.H && last->D == d.D) {
+            all.push_back(all.back());
+            continue;
         }
+        const QuadCut c = quad_cut(d.W, d.H, d.D, 2, cx, nw, 2);
+        all.push_back(QuadColumns{c.nw, d.D, (long long)c.nx * c.ny});
     }
-    std::stable_sort(all.begin(), all.end(), [](const Timed& a, const Timed& b) { return a.us > b.us; });
-    std::priority_queue<double, std::vector<double>, std::greater<double>> xcd[8];
-    for (auto& q : xcd)
-        for (int cu = 0; cu < 32; cu++) q.push(0.0);
-    double last = 0.0;
-    for (size_t i = 0; i < all.size(); i++) {
-        if (tiles) tiles->push_back(all[i].t);
-        auto& q = xcd[i % 8];
-        const double end = q.top() + all[i].us;
-        q.pop();
-        q.push(end);
-        last = std::max(last, end);
+    std::sort(all.begin(), all.end(),
+              [](const QuadColumns& x, const QuadColumns& y) { return x.nw != y.nw ? x.nw < y.nw : x.D < y.D; });
+    size_t n = 0;
+    for (const QuadColumns& c : all)
+        if (n && all[n - 1].nw == c.nw && all[n - 1].D == c.D) all[n - 1].n += c.n;
+        else all[n++] = c;
+    all.resize(n);
+    return all;
+}
+
+// Microseconds that a launch of two iterations with chunks of zc planes is predicted to take.
+double quad_us(const std::vector<QuadColumns>& columns, int cx, int zc) {
+    // tiles by their steps and waves, which set their time
+    constexpr int MOST = 17;
+    std::vector<long long> tiles((size_t)(zc + 8) * MOST, 0);
+    for (const QuadColumns& q : columns) {
+        QuadCut c{};
+        c.zc = zc;
+        c.nz = quad_chunks(q.D, 2, zc);
+        // (all chunks but the last take the same steps)
+        tiles[(size_t)ens_chunk_steps(c, 2, 0, q.D) * MOST + q.nw] += q.n * (c.nz - 1);
+        tiles[(size_t)ens_chunk_steps(c, 2, c.nz - 1, q.D) * MOST + q.nw] += q.n;
     }
-    return last;
+    std::vector<EnsRun> runs;
+    for (size_t k = 0; k < tiles.size(); k++)
+        if (tiles[k]) runs.push_back(EnsRun{ens_tile_us((int)(k / MOST), 2, cx, (int)(k % MOST)), tiles[k]});
+    std::sort(runs.begin(), runs.end(), [](const EnsRun& x, const EnsRun& y) { return x.us > y.us; });
+    return ens_fill_us(runs);
 }
 
 // The shapes of an ensemble: the fixed ones, then the depths of four cells a lane predicted fastest;
@@ -162,16 +145,87 @@ int quad_shapes(const zq3d_ens* e, int (*shapes)[3]) {
         }
         n++;
     };
-    for (const auto& f : kEnsQuadShapes) add(f[0], f[1], f[2], quad_table(e, 2, f, nullptr, nullptr));
+    std::vector<QuadColumns> columns;
+    for (int k = 0; k < kEnsQuadFixed; k++) {
+        const auto& f = kEnsQuadShapes[k];
+        if (!k || f[0] != kEnsQuadShapes[k - 1][0] || f[1] != kEnsQuadShapes[k - 1][1]) columns = quad_columns(e, f[0], f[1]);
+        add(f[0], f[1], f[2], quad_us(columns, f[0], f[2]));
+    }
+    columns = quad_columns(e, 4, 8);
     for (int zc = 2; zc <= 64; zc += 2) {
         bool had = false;
         for (const auto& f : kEnsQuadShapes) had = had || (f[0] == 4 && f[2] == zc);
-        const int shape[3] = {4, 8, zc};
-        if (!had) depths.push_back(Depth{quad_table(e, 2, shape, nullptr, nullptr), zc});
+        if (!had) depths.push_back(Depth{quad_us(columns, 4, zc), zc});
     }
     std::stable_sort(depths.begin(), depths.end(), [](const Depth& a, const Depth& b) { return a.us < b.us; });
     for (int i = 0; n < kEnsQuadShapeCount; i++) add(4, 8, depths[i].zc, depths[i].us);
     return best;
+}
+
+// The table of a shape: every member's cut, and the tiles, the longest first.  Made when the shape is first
+// selected (most ensembles run one).
+int make_quad_table(zq3d_ens* e, int K, const int shape[3], EnsQuadTable* table, const char* where) {
+    if (table->total) return ZQ3D_OK;
+    struct Chunk {
+        double us;
+        int s, z, nx, ny;
+    };
+    std::vector<Chunk> chunks;
+    std::vector<QuadCut> cuts;
+    size_t total = 0;
+    for (int s = 0; s < e->count; s++) {
+        const Dims& d = e->dims[s];
+        const QuadCut c = quad_cut(d.W, d.H, d.D, K, shape[0], shape[1], shape[2]);
+        cuts.push_back(c);
+        for (int z = 0; z < c.nz; z++)
+            chunks.push_back(Chunk{ens_tile_us(ens_chunk_steps(c, K, z, d.D), K, shape[0], c.nw), s, z, c.nx, c.ny});
+        total += (size_t)c.nx * c.ny * c.nz;
+    }
+    std::stable_sort(chunks.begin(), chunks.end(), [](const Chunk& a, const Chunk& b) { return a.us > b.us; });
+    std::vector<EnsQuadTile> tiles;
+    tiles.reserve(total);
+    for (const Chunk& c : chunks)
+        for (int y = 0; y < c.ny; y++)
+            for (int x = 0; x < c.nx; x++) tiles.push_back(EnsQuadTile{c.s, x, y, c.z});
+    EnsQuadTile* dt = nullptr;
+    QuadCut* dc = nullptr;
+    if (ens_alloc(e, &dt, tiles.size() * sizeof(EnsQuadTile)) || ens_alloc(e, &dc, cuts.size() * sizeof(QuadCut))) {
+        set_err(where, "device allocation failed");
+        return ZQ3D_ERR_HIP;
+    }
+    ZQ_HIP(hipMemcpy(dt, tiles.data(), tiles.size() * sizeof(EnsQuadTile), hipMemcpyHostToDevice), where);
+    ZQ_HIP(hipMemcpy(dc, cuts.data(), cuts.size() * sizeof(QuadCut), hipMemcpyHostToDevice), where);
+    *table = EnsQuadTable{dt, dc, (int)tiles.size()};
+    return ZQ3D_OK;
+}
+
+// The table of a cell or block stage, written on the device from the members' first tiles.
+int make_table(zq3d_ens* e, EnsTiling t, EnsTable* table, const char* where) {
+    if (table->total) return ZQ3D_OK;
+    std::vector<int> first(1, 0);
+    for (const Dims& d : e->dims) first.push_back(first.back() + ens_tiles_of(d, t));
+    EnsTile* tiles = nullptr;
+    int* dev = nullptr;
+    if (ens_alloc(e, &tiles, (size_t)first.back() * sizeof(EnsTile)) || ens_alloc(e, &dev, first.size() * sizeof(int))) {
+        set_err(where, "device allocation failed");
+        return ZQ3D_ERR_HIP;
+    }
+    ZQ_HIP(hipMemcpyAsync(dev, first.data(), first.size() * sizeof(int), hipMemcpyHostToDevice, e->stream), where);
+    ZQ_HIP(ens_launch_tiles(e->dev_members, e->count, dev, first.back(), t, tiles, e->stream), where);
+    ZQ_HIP(hipStreamSynchronize(e->stream), where);
+    *table = EnsTable{tiles, first.back()};
+    return ZQ3D_OK;
+}
+
+// The tables of the sweeps that L selects.
+int make_sweep_tables(zq3d_ens* e, EnsLaunch* L, const char* where) {
+    if (!L->sweep_quad) {
+        const int* shape = kEnsSweepShapes[L->sweep_shape];
+        return make_table(e, EnsTiling{shape[0], shape[1], true}, &L->half[L->sweep_shape], where);
+    }
+    if (L->any_odd)
+        if (int rc = make_quad_table(e, 1, kEnsQuadOne, &L->quad_one, where)) return rc;
+    return make_quad_table(e, 2, L->quad_shape[L->sweep_quad - 1], &L->quad[L->sweep_quad - 1], where);
 }
 
 int field_span(zq3d_ens* e, int s, int field, void** p, size_t* bytes) {
@@ -226,26 +280,6 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
         e->Nparts += 2 * (size_t)cdiv(d.W, 64) * cdiv(d.H, 4) * d.D;
         e->cells += (long long)z.N;
     }
-    // tile tables: cells, set-up blocks, half-row blocks per sweep shape
-    std::vector<EnsTile> flat;
-    std::vector<size_t> at;
-    for (int t = 0; t < 2 + kEnsSweepShapeCount; t++) {
-        const std::vector<EnsTile> one = t == 0   ? cell_tiles(e)
-                                         : t == 1 ? block_tiles(e, 64, 4, false)
-                                                  : block_tiles(e, kEnsSweepShapes[t - 2][0], kEnsSweepShapes[t - 2][1], true);
-        at.push_back(flat.size());
-        flat.insert(flat.end(), one.begin(), one.end());
-    }
-    at.push_back(flat.size());
-    std::vector<EnsQuadTile> tiles;
-    std::vector<QuadCut> cuts;
-    size_t tile_at[kEnsQuadShapeCount + 1];
-    const int quad_best = quad_shapes(e, e->L.quad_shape);
-    for (int r = 0; r <= kEnsQuadShapeCount; r++) {
-        tile_at[r] = tiles.size();
-        if (r < kEnsQuadShapeCount) quad_table(e, 2, e->L.quad_shape[r], &tiles, &cuts);
-        else quad_table(e, 1, kEnsQuadOne, &tiles, &cuts);
-    }
     int bad = 0;
     bad |= ens_alloc(e, &e->u, e->Nu * 4) | ens_alloc(e, &e->v, e->Nv * 4) | ens_alloc(e, &e->w, e->Nw * 4);
     bad |= ens_alloc(e, &e->T, e->Nc * 4) | ens_alloc(e, &e->R, e->Nc * 4) | ens_alloc(e, &e->T2, e->Nc * 4) |
@@ -256,9 +290,7 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
     bad |= ens_alloc(e, &e->part, e->Nparts * 8) | ens_alloc(e, &e->mean32, (size_t)count * 4);
     bad |= ens_alloc(e, &e->quad_n, e->Nq) | ens_alloc(e, &e->quad_b, e->Nq * 4) |
            ens_alloc(e, &e->quad_p[0], e->Nq * 4) | ens_alloc(e, &e->quad_p[1], e->Nq * 4);
-    bad |= ens_alloc(e, &e->dev_tiles, tiles.size() * sizeof(EnsQuadTile)) |
-           ens_alloc(e, &e->dev_cuts, cuts.size() * sizeof(QuadCut));
-    bad |= ens_alloc(e, &e->dev_members, sizeof(EnsMember) * count) | ens_alloc(e, &e->dev_tables, flat.size() * sizeof(EnsTile));
+    bad |= ens_alloc(e, &e->dev_members, sizeof(EnsMember) * count);
     if (bad || hipStreamCreate(&e->stream) != hipSuccess) {
         set_err(where, "device allocation failed");
         zq3d_ens_destroy(e);
@@ -319,9 +351,6 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
         e->L.any_odd |= c.sor.iters & 1;
     }
     Errs E;
-    E(hipMemcpy(e->dev_tables, flat.data(), flat.size() * sizeof(EnsTile), hipMemcpyHostToDevice));
-    E(hipMemcpy(e->dev_tiles, tiles.data(), tiles.size() * sizeof(EnsQuadTile), hipMemcpyHostToDevice));
-    E(hipMemcpy(e->dev_cuts, cuts.data(), cuts.size() * sizeof(QuadCut), hipMemcpyHostToDevice));
     E(hipMemsetAsync(e->u, 0, e->Nu * 4, e->stream));
     E(hipMemsetAsync(e->v, 0, e->Nv * 4, e->stream));
     E(hipMemsetAsync(e->w, 0, e->Nw * 4, e->stream));
@@ -338,28 +367,23 @@ extern "C" int zq3d_ens_create(int count, const zq3d_config* cfgs, zq3d_ens** ou
         zq3d_ens_destroy(e);
         return ZQ3D_ERR_HIP;
     }
-    if (int rc = upload_members(e, where)) {
-        zq3d_ens_destroy(e);
-        return rc;
-    }
     EnsLaunch& L = e->L;
     L.members = e->dev_members;
     L.count = count;
-    auto table = [&](int t) { return EnsTable{e->dev_tables + at[t], (int)(at[t + 1] - at[t])}; };
-    L.cells = table(0);
-    L.setup = table(1);
-    for (int sh = 0; sh < kEnsSweepShapeCount; sh++) L.half[sh] = table(2 + sh);
-    for (int r = 0; r <= kEnsQuadShapeCount; r++) {
-        const size_t end = r < kEnsQuadShapeCount ? tile_at[r + 1] : tiles.size();
-        (r < kEnsQuadShapeCount ? L.quad[r] : L.quad_one) =
-            EnsQuadTable{e->dev_tiles + tile_at[r], e->dev_cuts + (size_t)r * count, (int)(end - tile_at[r])};
-    }
     L.sweep_shape = 0;
-    L.sweep_quad = quad_best + 1;
+    L.sweep_quad = quad_shapes(e, L.quad_shape) + 1;
     L.blocks = 0;
     L.sweep_blocks = 0;
     L.p_pool = e->p;
     L.p_pool_size = e->Np;
+    int rc = upload_members(e, where);
+    if (!rc) rc = make_table(e, EnsTiling{0, 0, false}, &L.cells, where);
+    if (!rc) rc = make_table(e, EnsTiling{64, 4, false}, &L.setup, where);
+    if (!rc) rc = make_sweep_tables(e, &L, where);
+    if (rc) {
+        zq3d_ens_destroy(e);
+        return rc;
+    }
     *out = e;
     return ZQ3D_OK;
 }
@@ -491,6 +515,7 @@ extern "C" int zq3d_ens_set_sweep(zq3d_ens* e, int kind, int tbx, int tby, int b
             }
     }
     if (!ok) { set_err(where, "not a sweep candidate (see zq3d_ens_autotune)"); return ZQ3D_ERR_ARG; }
+    if (int rc = make_sweep_tables(e, &L, where)) return rc;
     e->L = L;
     e->graph_stale = true;
     return ZQ3D_OK;
@@ -504,6 +529,14 @@ extern "C" int zq3d_ens_autotune(zq3d_ens* e, int iters, zq3d_ens_tune* rep) {
     if (!e || iters < 1) { set_err(where, "bad argument"); return ZQ3D_ERR_ARG; }
     static const int blocks[] = {0, 256, 1024, 4096};
     const int nb = (int)(sizeof(blocks) / sizeof(blocks[0]));
+    // (kept also where tuning fails later on)
+    for (int sh = 0; sh < kEnsSweepShapeCount; sh++)
+        if (int rc = make_table(e, EnsTiling{kEnsSweepShapes[sh][0], kEnsSweepShapes[sh][1], true}, &e->L.half[sh], where))
+            return rc;
+    for (int r = 0; r < kEnsQuadShapeCount; r++)
+        if (int rc = make_quad_table(e, 2, e->L.quad_shape[r], &e->L.quad[r], where)) return rc;
+    if (e->L.any_odd)
+        if (int rc = make_quad_table(e, 1, kEnsQuadOne, &e->L.quad_one, where)) return rc;
     hipEvent_t a = nullptr, b = nullptr;
     ZQ_HIP(hipEventCreate(&a), where);
     ZQ_HIP(hipEventCreate(&b), where);

@@ -48,6 +48,19 @@ struct EnsTile {
 };
 constexpr int kEnsPlanes = 4;  // planes of a cell tile
 
+// How a stage cuts a plane: blocks of tbx x tby cells (half: of half rows), or, with tbx == 0, the cell tiles.
+struct EnsTiling {
+    int tbx, tby;
+    bool half;
+};
+__host__ __device__ inline int ens_plane_tiles(const Dims& d, EnsTiling t) {
+    if (!t.tbx) return (d.W * d.H + 255) / 256;
+    return ((t.half ? (d.W + 1) / 2 : d.W) + t.tbx - 1) / t.tbx * ((d.H + t.tby - 1) / t.tby);
+}
+__host__ __device__ inline int ens_tiles_of(const Dims& d, EnsTiling t) {
+    return ens_plane_tiles(d, t) * (t.tbx ? d.D : (d.D + kEnsPlanes - 1) / kEnsPlanes);
+}
+
 // Every member's tiles, member after member.
 struct EnsTable {
     const EnsTile* tiles;
@@ -85,9 +98,9 @@ struct EnsLaunch {
     const EnsMember* members;  // device array
     int count;
     EnsTable cells, setup;               // cell tiles; 64 x 4 blocks of the projection set-up
-    EnsTable half[kEnsSweepShapeCount];  // half-row grids of the sweep, one per tile shape
+    EnsTable half[kEnsSweepShapeCount];  // half-row grids of the sweep, one per tile shape (made on need)
     int sweep_shape;                     // index into kEnsSweepShapes
-    EnsQuadTable quad[kEnsQuadShapeCount], quad_one;
+    EnsQuadTable quad[kEnsQuadShapeCount], quad_one;  // (made on need)
     int quad_shape[kEnsQuadShapeCount][3];
     int sweep_quad;                      // 0: half sweeps of sweep_shape; r > 0: quad_shape[r - 1]
     int any_odd;                         // some member's iteration count is odd
@@ -98,6 +111,9 @@ struct EnsLaunch {
     size_t p_pool_size;
 };
 
+// fills a table of `total` tiles of the tiling: member s begins at tile first[s]
+hipError_t ens_launch_tiles(const EnsMember* members, int count, const int* first, int total, EnsTiling t, EnsTile* out,
+                            hipStream_t s);
 // all stages of one step of every member
 hipError_t ens_launch_step(const EnsLaunch& L, hipStream_t s);
 // projection set-up of every member: counts, divergence and mean, for the selected sweep

@@ -55,6 +55,12 @@ ZQ_HD inline int quad_z_begin(const QuadCut& c, int K, int bz, int D) {
     return bz == c.nz || z > D ? D : z;
 }
 
+// chunks of zc planes that D planes make (the first holds 2K - 1 more)
+ZQ_HD inline int quad_chunks(int D, int K, int zc) {
+    const int first = zc + 2 * K - 1;
+    return 1 + (D > first ? (D - first + zc - 1) / zc : 0);
+}
+
 // The cut of a W x H x D grid for K iterations a pass, cx cells a lane, nw waves and zc planes (even).
 // ny == 0: a tile of these waves would own no row.
 inline QuadCut quad_cut(int W, int H, int D, int K, int cx, int nw, int zc) {
@@ -83,8 +89,7 @@ inline QuadCut quad_cut(int W, int H, int D, int K, int cx, int nw, int zc) {
         c.ny = 2 + (left > 0 ? (left + mid - 1) / mid : 0);
     }
     c.zc = zc;
-    const int first = zc + J - 1;
-    c.nz = 1 + (D > first ? (D - first + zc - 1) / zc : 0);
+    c.nz = quad_chunks(D, K, zc);
     c.mlx = quad_magic(c.lx);
     c.mnx = quad_magic(c.nx);
     c.mny = quad_magic(std::max(c.ny, 1));
