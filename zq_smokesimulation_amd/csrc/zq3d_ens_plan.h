@@ -27,7 +27,8 @@ struct EnsRun {
 // its i-th tile is as long as any other's i-th, and it has as many.  A tile goes to the CU that is free
 // first; the CUs' free times stay sorted in two queues, those from before the run and those that a tile
 // of the run set, and whole rounds of a run are added at once, so a run of any length costs a few dozen
-// steps (one by one with a heap, 512 members of 64^3 took 9 ms for all shapes; now 0.2).
+// steps.  (One by one with a heap, and with every shape's tables made at once, creating 512 members of
+// 64^3 took 20 ms and two of 512^3 44; now 2.3 and 2.7.)
 inline double ens_fill_us(const std::vector<EnsRun>& runs) {
     constexpr int CUS = 32;
     double cu[CUS] = {}, set[CUS], merged[CUS];
