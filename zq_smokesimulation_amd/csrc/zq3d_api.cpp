@@ -5,6 +5,7 @@
 // (e.g. ZQ_CUDA_AddForce3D.cu:616-651).  Part 3 keeps all fields resident in HBM.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -874,6 +875,13 @@ int ensure_split(zq3d_sim* s, const char* where) {
     return ZQ3D_OK;
 }
 
+void free_split(zq3d_sim* s) {
+    for (void* p : {(void*)s->split_p, (void*)s->split_b, (void*)s->split_n})
+        if (p) (void)hipFree(p);
+    s->split_p = s->split_b = nullptr;
+    s->split_n = nullptr;
+}
+
 // Times one stage of a simulation with an event pair when profiling is on.
 struct StageTimer {
     zq3d_sim* s;
@@ -1313,17 +1321,21 @@ extern "C" int zq3d_autotune_sor(zq3d_sim* s, int iters, zq3d_tune_report* rep) 
     if (!s || iters < 1) { set_err(where, "bad argument"); return ZQ3D_ERR_ARG; }
     const Sizes z(s->d);
     SorShape cand[ZQ3D_TUNE_MAX];
-    const int n = sor_shape_candidates(s->d, cand, ZQ3D_TUNE_MAX);
+    int n = sor_shape_candidates(s->d, cand, ZQ3D_TUNE_MAX);  // (the default is always one of them)
     if (rep) std::memset(rep, 0, sizeof(*rep));
-    if (n == 0) {
-        s->shape = SorShape{0, 0};
-        if (rep) rep->best = -1;
-        return ZQ3D_OK;
+    // without room for the colour-split arrays (over 20 bytes a cell) the other shapes are timed
+    if (ensure_split(s, where) != ZQ3D_OK) {
+        (void)hipGetLastError();
+        free_split(s);
+        n = (int)(std::remove_if(cand, cand + n, is_split) - cand);
     }
     hipEvent_t a = nullptr, b = nullptr;
     ZQ_HIP(hipEventCreate(&a), where);
-    ZQ_HIP(hipEventCreate(&b), where);
-    if (int rc = ensure_split(s, where)) return rc;
+    if (hipEventCreate(&b) != hipSuccess) {
+        (void)hipEventDestroy(a);
+        set_err(where, "event creation failed");
+        return ZQ3D_ERR_HIP;
+    }
     const ProjBufs B = proj_bufs(s);
     launch_fill_f32(&s->sc->mean32, 1, 0.0f, s->stream);
     launch_proj_setup(s->d, s->u, s->v, s->w, s->occ, s->cfg.sor.open_mask, s->nc, B.quad.b, nullptr, nullptr, nullptr,
@@ -1365,8 +1377,9 @@ extern "C" int zq3d_autotune_sor(zq3d_sim* s, int iters, zq3d_tune_report* rep) 
     (void)hipEventDestroy(a);
     (void)hipEventDestroy(b);
     launch_fill_f32(s->p, z.Np, 0.0f, s->stream);
+    if (E.e == hipSuccess) s->shape = cand[best];
+    if (!is_split(s->shape) && s->cfg.sor.pass_rule != 2) free_split(s);  // (waits for the sweeps)
     if (E.e != hipSuccess) { set_err(where, hipGetErrorString(E.e)); return ZQ3D_ERR_HIP; }
-    s->shape = cand[best];
     if (rep) {
         rep->count = n;
         rep->best = best;
