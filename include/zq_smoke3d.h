@@ -559,9 +559,12 @@ typedef struct zq3d_ens_tune {
     float probe_ms;        /* cell advection probe at that size */
 } zq3d_ens_tune;
 int zq3d_ens_autotune(zq3d_ens* e, int iters, zq3d_ens_tune* report);
-/* selects one of the autotuner's sweep candidates (kind, tbx, tby, blocks as reported; the shapes of 64
- * slots that kind 1 once reported select one near them) */
+/* selects one of the autotuner's sweep candidates (kind, tbx, tby, blocks as reported).  Results saved
+ * when kind 1 had shapes of 64 slots (64 x 8, 16 or 32 rows x 8, 16 or 32 planes) are still taken: those
+ * sweeps are gone, and the shape of two cells a lane next to them runs instead.  zq3d_ens_get_sweep says
+ * which shape runs. */
 int zq3d_ens_set_sweep(zq3d_ens* e, int kind, int tbx, int tby, int blocks);
+int zq3d_ens_get_sweep(zq3d_ens* e, int* kind, int* tbx, int* tby, int* blocks);
 
 /* message of the last failed call on this thread ("" if none) */
 const char* zq3d_last_error(void);

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 MEMBERS = [((3, 2, 2), False, 2), ((300, 11, 9), True, 7), ((24, 90, 20), False, 0), ((40, 9, 70), True, 1),
            ((67, 35, 33), True, 12)]
-SHAPES = [(2, 8, 8), (2, 16, 8), (2, 16, 16), (4, 8, 8), (4, 8, 16), (4, 8, 32), (64, 16, 32), (64, 32, 8)]
+SHAPES = [(2, 8, 8), (2, 16, 8), (2, 16, 16), (4, 8, 8), (4, 8, 16), (4, 8, 32)]
 
 
 @pytest.mark.parametrize("which", [[0, 1, 2, 3, 4], [2], [0, 4]], ids=str)
@@ -39,6 +39,7 @@ def test_members_of_any_iteration_count_and_size(which):
             print("ensemble", which, shape, flush=True)
             if shape:
                 ens.set_sweep(1, *shape)
+                assert ens.sweep() == ("split_one_launch",) + shape
             ens.step(1, graph=shape != (4, 8, 16))
             ens.synchronize()
             for m, sim in enumerate(sims):
@@ -52,4 +53,26 @@ def test_members_of_any_iteration_count_and_size(which):
     finally:
         for sim in sims:
             sim.close()
+        ens.close()
+
+
+def test_the_sweep_that_runs_is_reported():
+    """A saved shape of the sweeps on 64 slots selects the nearest one and is reported as that; a refused shape
+    changes nothing."""
+    import zq_smokesimulation_amd as z
+    from zq_smokesimulation_amd.ensemble import SmokeEnsemble, member_config
+    ens = SmokeEnsemble([member_config(24, 20, 18, **member_args(True, 0.0, 0.5, 3, 24))])
+    try:
+        for rows, planes, want in ((8, 8, (2, 8, 8)), (8, 16, (2, 8, 16)), (16, 8, (2, 16, 8)), (16, 32, (2, 16, 16)),
+                                   (32, 8, (2, 16, 8)), (32, 16, (2, 16, 16))):
+            print("saved shape", rows, planes, flush=True)
+            ens.set_sweep("split_one_launch", 64, rows, planes)
+            assert ens.sweep() == ("split_one_launch",) + want
+        for bad in ((1, 64, 16, 12), (1, 2, 8, 7), (0, 64, 5, 0), (0, 64, 4, -1), (2, 64, 4, 0)):
+            with pytest.raises(z.ZQ3DError):
+                ens.set_sweep(*bad)
+            assert ens.sweep() == ("split_one_launch", 2, 16, 16)
+        ens.set_sweep("half_sweeps", 32, 8, 256)
+        assert ens.sweep() == ("half_sweeps", 32, 8, 256)
+    finally:
         ens.close()

@@ -294,6 +294,9 @@ def _bind_adjoint(L):
 
 
 ENS_TUNE_MAX = 24
+# The names of the sweep kinds 0 and 1 in reports.  Kind 1 runs two iterations a launch with a tile's planes in
+# registers; its name is that of the sweeps it replaced, which programs compare with.
+ENS_SWEEP_KINDS = ("half_sweeps", "split_one_launch")
 
 
 class EnsTune(C.Structure):
@@ -310,7 +313,7 @@ class EnsTune(C.Structure):
 
     def as_dict(self):
         n = self.count
-        kinds = ("half_sweeps", "split_one_launch")
+        kinds = ENS_SWEEP_KINDS
         return {"candidates": [{"kind": kinds[self.kind[i]], "tbx": self.tbx[i], "tby": self.tby[i],
                                 "blocks": self.blocks[i], "us_per_iter": round(self.us_per_iter[i], 3)}
                                for i in range(n)],
@@ -335,4 +338,5 @@ def _bind_ensemble(L):
     L.zq3d_ens_stream.argtypes = [vp, C.POINTER(C.c_void_p)]
     L.zq3d_ens_autotune.argtypes = [vp, C.c_int, C.POINTER(EnsTune)]
     L.zq3d_ens_set_sweep.argtypes = [vp, C.c_int, C.c_int, C.c_int, C.c_int]
+    L.zq3d_ens_get_sweep.argtypes = [vp] + [C.POINTER(C.c_int)] * 4
     return L

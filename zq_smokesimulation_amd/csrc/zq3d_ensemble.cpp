@@ -496,9 +496,8 @@ extern "C" int zq3d_ens_set_sweep(zq3d_ens* e, int kind, int tbx, int tby, int b
                 L.sweep_blocks = blocks;
                 ok = true;
             }
-                L.sweep_quad = 0;
     } else if (kind == 1) {
-        // the 64-slot shapes of the one-iteration launches that these sweeps replaced: same bits
+        // saved shapes of the sweeps on 64 slots that these replaced: the nearest one here (same bits)
         static const int old[][2] = {{8, 8}, {8, 16}, {16, 8}, {16, 16}, {16, 32}, {32, 8}, {32, 16}};
         if (tbx == 64)
             for (const auto& o : old)
@@ -518,6 +517,17 @@ extern "C" int zq3d_ens_set_sweep(zq3d_ens* e, int kind, int tbx, int tby, int b
     if (int rc = make_sweep_tables(e, &L, where)) return rc;
     e->L = L;
     e->graph_stale = true;
+    return ZQ3D_OK;
+}
+
+extern "C" int zq3d_ens_get_sweep(zq3d_ens* e, int* kind, int* tbx, int* tby, int* blocks) {
+    if (!e || !kind || !tbx || !tby || !blocks) { set_err("zq3d_ens_get_sweep", "null argument"); return ZQ3D_ERR_ARG; }
+    const EnsLaunch& L = e->L;
+    const int* quad = L.sweep_quad ? L.quad_shape[L.sweep_quad - 1] : nullptr;
+    *kind = quad ? 1 : 0;
+    *tbx = quad ? quad[0] : kEnsSweepShapes[L.sweep_shape][0];
+    *tby = quad ? quad[1] : kEnsSweepShapes[L.sweep_shape][1];
+    *blocks = quad ? quad[2] : L.sweep_blocks;
     return ZQ3D_OK;
 }
 

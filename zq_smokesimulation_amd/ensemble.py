@@ -103,6 +103,14 @@ class SmokeEnsemble:
         return rep.as_dict()
 
     def set_sweep(self, kind, tbx, tby, blocks):
-        """Selects an autotuner candidate: kind "half_sweeps" (0) or "split_one_launch" (1)."""
-        k = {"half_sweeps": 0, "split_one_launch": 1}.get(kind, kind)
+        """Selects an autotuner candidate: kind "half_sweeps" (0: tbx x tby cells a tile, `blocks` workgroups)
+        or "split_one_launch" (1: two iterations a launch, tbx cells a lane, tby waves, `blocks` planes).  The
+        64-slot shapes that kind 1 once had select the nearest one (see sweep())."""
+        k = {n: i for i, n in enumerate(_lib.ENS_SWEEP_KINDS)}.get(kind, kind)
         check(_lib.lib().zq3d_ens_set_sweep(self._h, int(k), int(tbx), int(tby), int(blocks)), "zq3d_ens_set_sweep")
+
+    def sweep(self):
+        """The sweeps that run: (kind, tbx, tby, blocks)."""
+        v = [C.c_int() for _ in range(4)]
+        check(_lib.lib().zq3d_ens_get_sweep(self._h, *[C.byref(x) for x in v]), "zq3d_ens_get_sweep")
+        return (_lib.ENS_SWEEP_KINDS[v[0].value],) + tuple(x.value for x in v[1:])
