@@ -398,8 +398,8 @@ int zq3d_get_coarse_sweep(zq3d_sim* sim, int* k, int* zc);
  * with min(sor.iters, region cells) iterations; that branch never adds the guide, so coeff and the
  * arrays' values are not read.  Host work per projection: the level map and faces cross PCIe. */
 int zq3d_set_guide(zq3d_sim* sim, float coeff, const float* gu, const float* gv, const float* gw);
-/* name of the sweep kernel the current shape runs ("k_sor_quad", "k_sor_split_rb", "k_sor_split_rb2",
- * "k_sor_split", "k_sor_fused" or "k_sor_half") */
+/* name of the sweep kernel the current shape runs ("k_sor_quad", "k_sor_block", "k_sor_split_rb",
+ * "k_sor_split_rb2", "k_sor_split" or "k_sor_fused") */
 const char* zq3d_sor_kernel(zq3d_sim* sim);
 
 /* ====================== Part 4: host-side scene set-up (no GPU) ====================== */

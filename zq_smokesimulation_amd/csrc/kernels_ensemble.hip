@@ -205,7 +205,7 @@ __global__ __launch_bounds__(NTH) void ke_sor_quad(const EnsMember* __restrict__
     if ((int)threadIdx.x >= 64 * c.nw) return;  // a wave that this member's tiles do not need
     const int from = K == 1 ? 0 : (odd + at) & 1;
     const float* src = K == 1 || (at == 0 && !odd) ? nullptr : m.qp[from];
-    sor_quad_tile<K, CX, QUAD_R, true, 1, NTH>(m.qn, m.qb, *m.mean32, src, m.qp[1 - from], m.d, c, t.bx, t.by, t.bz,
+    sor_quad_tile<K, CX, QUAD_R, true, NTH>(m.qn, m.qb, *m.mean32, src, m.qp[1 - from], m.d, c, t.bx, t.by, t.bz,
                                               m.omega, m.omw, quad_lds);
 }
 

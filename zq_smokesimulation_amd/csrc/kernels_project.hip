@@ -443,7 +443,7 @@ __global__ __launch_bounds__(NT) void k_sor_quad(const uint8_t* __restrict__ n, 
     if (tile >= c.nx * c.ny * c.nz) return;  // spare block (the grid is a multiple of 8): uniform exit
     const int rest = quad_div(tile, c.mnx), bx = tile - rest * c.nx;
     const int bz = quad_div(rest, c.mny), by = rest - bz * c.ny;
-    sor_quad_tile<K, CX, QUAD_R, MASK, 1, NT>(n, b, *mean32, src, dst, d, c, bx, by, bz, omega, omw, quad_lds);
+    sor_quad_tile<K, CX, QUAD_R, MASK, NT>(n, b, *mean32, src, dst, d, c, bx, by, bz, omega, omw, quad_lds);
 }
 
 // `iters` red-black iterations of a box per workgroup (sor_block_tile), tiles numbered as k_sor_quad's.
@@ -1354,6 +1354,7 @@ float* launch_sor(const Dims& d, const uint8_t* nc, const float* b, const float*
         if (ev1) (void)hipEventRecord(ev1, s);
         return src;
     }
+    // rows too long for the fused ring: only from the entry point without scratch for the quad layout
     const dim3 g = grid_for((d.W + 1) / 2, d.H, d.D);
     for (int it = 0; it < iters; it++) {
         hipLaunchKernelGGL(k_sor_half, g, dim3(BX, BY), 0, s, nc, b, mean32, p_pad, d, omega, omw, 0);
@@ -1369,7 +1370,7 @@ const char* sor_kernel_name(const Dims& d, SorShape shape) {
     if (shape.ty == SOR_SPLIT) return "k_sor_split";
     if (shape.ty <= -SOR_TWO) return "k_sor_split_rb2";
     if (is_split(shape)) return "k_sor_split_rb";
-    return fused_shape(d, shape).nblocks > 0 ? "k_sor_fused" : "k_sor_half";
+    return "k_sor_fused";
 }
 
 long long sor_launches(const Dims& d, SorShape shape, int iters) {
@@ -1382,7 +1383,7 @@ long long sor_launches(const Dims& d, SorShape shape, int iters) {
     if (shape.ty == SOR_SPLIT) return 2LL * iters;
     if (shape.ty <= -SOR_TWO) return (iters + 1) / 2;
     if (is_split(shape)) return iters;
-    return (fused_shape(d, shape).nblocks > 0 ? 1LL : 2LL) * iters;
+    return iters;
 }
 
 bool split_buffers_fit(const Dims& d) {

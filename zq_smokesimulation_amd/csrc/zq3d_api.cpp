@@ -52,8 +52,8 @@ int check_dims(int W, int H, int D, const char* where) {
 namespace {
 
 // ---------------- grow-only workspace for the host-pointer entry points ----------------
-enum Slot { S_U, S_V, S_W, S_OCC, S_T, S_R, S_T2, S_R2, S_VEL4, S_SCR, S_NC, S_B, S_P, S_P2, S_B64, S_P64, S_PART, S_SCAL,
-            S_BFECC, S_SPLIT, S_QUAD, S_COUNT };
+enum Slot { S_U, S_V, S_W, S_OCC, S_T, S_R, S_T2, S_R2, S_VEL4, S_SCR, S_NC, S_B64, S_P64, S_PART, S_SCAL, S_BFECC,
+            S_SPLIT, S_QUAD, S_COUNT };
 
 struct Workspace {
     void* ptr[S_COUNT] = {};

@@ -158,10 +158,10 @@ struct ProjBufs {
 int read_result(const ProjBufs& B, int slot, const unsigned long long* dev_scalar, double* out, hipStream_t s,
                 const char* where);
 
-// launch_sor, timed when pf is set (the sweeps are the only work between the two events)
 // the FP64 mean of a projection whose last divergence check (with mean_slot()) the stream has been waited for
 int read_mean(const ProjBufs& B, double* out, hipStream_t s, const char* where);
 
+// launch_sor, timed when pf is set (the sweeps are the only work between the two events)
 hipError_t timed_sor(const Dims& d, const uint8_t* nc, const float* b, const float* mean32, float* p, float* p_alt,
                      float omega, int iters, hipStream_t s, SorProf* pf, float** result, SorShape shape,
                      const SplitBufs* split);

@@ -194,7 +194,7 @@ int launch_split_sweeps(const Dims& d, const SplitBufs& sp, int from, const floa
                         bool zero_start = false);
 // split counts n_0 / n_1 from the interleaved counts
 void launch_split_counts(const Dims& d, const uint8_t* nc, const SplitBufs& sp, hipStream_t s);
-// name of the sweep kernel a shape runs
+// name of the sweep kernel a simulation's shape runs
 const char* sor_kernel_name(const Dims& d, SorShape shape);
 // sweep-kernel launches of `iters` SOR iterations
 long long sor_launches(const Dims& d, SorShape shape, int iters);

@@ -32,7 +32,7 @@
 
 namespace zq3d {
 
-template <int K, int CX, int R, bool MASK, int PF, int NT>
+template <int K, int CX, int R, bool MASK, int NT>
 struct QuadTile {
     static_assert(CX == 2 || CX == 4, "");
     static_assert(R % 2 == 0, "a row's parity must not depend on the thread");
@@ -43,8 +43,9 @@ struct QuadTile {
     static constexpr int M = CX / 2;  // cells of one colour in a row
     static constexpr int J = 2 * K;   // sweeps a step
     // ring slots: planes modulo RS, an even number (a slot's parity is its plane's) that holds the planes of B
-    // in use, t-J+1 .. t+PF
-    static constexpr int RS = J + PF <= 6 ? 6 : (J + PF + 1) & ~1;
+    // in use, t-J+1 .. t+1
+    static constexpr int RS = 6;
+    static_assert(J + 1 <= RS, "");
 
     float P[RS][R][CX];        // pressures as loaded
     float B[RS][R][CX];        // right-hand sides minus the mean
@@ -53,7 +54,7 @@ struct QuadTile {
     // fixed per thread
     uint32_t off[R], soff[R];  // byte offset of the row's cells in a plane of floats; the same where stored, else SPLIT_NONE
     bool lo, hi;               // first / last lane of a row group
-    // plane t + 1 + PF of the source, t + PF of b and n, t - J + 1 of the destination, and a plane's bytes
+    // plane t + 2 of the source, t + 1 of b and n, t - J + 1 of the destination, and a plane's bytes
     const char *src, *b, *n;
     char* dst;
     uint32_t sbytes, bytes, nbytes;
@@ -179,7 +180,7 @@ struct QuadTile {
     __device__ __forceinline__ void share_all() {
         // V_j's newest plane t-j+1 is the next step's centre plane; the parity of row 0's cells of V_j's
         // colour there is that of sweep j's output in this step (j >= 1), black at plane t+1 for j = 0
-        share<j>((PH - j + 2 * RS + 1) % RS, (PH + 1) & 1, j ? (PH & 1) : (PH & 1));
+        share<j>((PH - j + 2 * RS + 1) % RS, (PH + 1) & 1, PH & 1);
         if constexpr (j + 1 < J) share_all<PH, j + 1>();
     }
 
@@ -193,8 +194,8 @@ struct QuadTile {
                 u[j][mm] = up(j, PH & 1, mm);
                 d[j][mm] = dn(j, PH & 1, mm);
             }
-        load_p<(PH + 1 + PF) % RS>(t + 1 + PF);
-        load_bn<(PH + PF) % RS>(t + PF);
+        load_p<(PH + 2) % RS>(t + 2);
+        load_bn<(PH + 1) % RS>(t + 1);
 #pragma unroll
         for (int r = 0; r < R; r++)
 #pragma unroll
@@ -228,11 +229,11 @@ struct QuadTile {
 
 // One tile: workgroup of c.nw waves, tile (bx, by, bz) of the cut.  src == nullptr: the source is all
 // zeros.  m: the mean subtracted from b.  lds: quad_lds_floats(K, CX, NT) floats, NT >= 64 c.nw.
-template <int K, int CX, int R, bool MASK, int PF, int NT>
+template <int K, int CX, int R, bool MASK, int NT>
 __device__ __forceinline__ void sor_quad_tile(const uint8_t* n, const float* b, float m, const float* src, float* dst,
                                               const Dims& d, const QuadCut& c, int bx, int by, int bz, float omega,
                                               float omw, float* lds) {
-    using T = QuadTile<K, CX, R, MASK, PF, NT>;
+    using T = QuadTile<K, CX, R, MASK, NT>;
     constexpr int J = 2 * K;
     T q;
     const int S = quad_stride(d.W);
@@ -297,14 +298,6 @@ __device__ __forceinline__ void sor_quad_tile(const uint8_t* n, const float* b, 
     q.template load_p<0>(t);
     q.template load_p<1>(t + 1);
     q.template load_bn<0>(t);
-    if constexpr (PF > 1) {
-        q.template load_p<2>(t + 2);
-        q.template load_bn<1>(t + 1);
-    }
-    if constexpr (PF > 2) {
-        q.template load_p<3>(t + 3);
-        q.template load_bn<2>(t + 2);
-    }
     __syncthreads();  // the zeros above before the rows below
     q.template share<0>(0, 0, 1);  // black at plane t: odd cells of row 0
     __syncthreads();
@@ -321,18 +314,6 @@ __device__ __forceinline__ void sor_quad_tile(const uint8_t* n, const float* b, 
         if (++t > te) break;
         q.template step<5>(t, z0);
         if (++t > te) break;
-        if constexpr (T::RS > 6) {
-            q.template step<6 % T::RS>(t, z0);
-            if (++t > te) break;
-            q.template step<7 % T::RS>(t, z0);
-            if (++t > te) break;
-        }
-        if constexpr (T::RS > 8) {
-            q.template step<8 % T::RS>(t, z0);
-            if (++t > te) break;
-            q.template step<9 % T::RS>(t, z0);
-            if (++t > te) break;
-        }
     }
 }
 
