@@ -229,14 +229,15 @@ def test_checkpoint_spacing_does_not_change_gradient():
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_sweep_shape_does_not_change_rollout_or_gradient(dtype):
     """Every projection of the rollout (forward, recomputation, adjoint) runs the sweep algorithm set
-    by set_sor_shape; single-colour split sweeps and one-launch iterations give the same forward
-    bits.  The gradient is compared to a tolerance: the advection adjoint accumulates with atomics,
+    by set_sor_shape; the default, explicit register tiles and boxes, the interleaved fused sweeps,
+    single-colour split sweeps and one-launch iterations give the same forward bits.  The gradient is compared to a tolerance: the advection adjoint accumulates with atomics,
     so its last bits depend on the order in which the GPU retires them, whatever the shape."""
     W, H, D, nsteps = 40, 36, 28, 4
     out = []
-    for shape in ((-1, 0), (-16, 16), (-32, 8)):
+    for shape in ((-1, 0), (-16, 16), (-32, 8), None, (4, 16), (-1208, 8), (-1404, 6), (-130804, 2)):
         eng, _ = make_engine(W, H, D, nsteps, 2, dtype, closed=True, obstacle=True)
-        eng.set_sor_shape(*shape)
+        if shape:
+            eng.set_sor_shape(*shape)
         gen = torch.Generator(device="cpu").manual_seed(9)
         ctrl = (0.5 * torch.randn(eng.controls_shape(), generator=gen, dtype=dtype)).to(DEV)
         target = torch.rand((D, H, W), generator=gen, dtype=dtype).to(DEV)

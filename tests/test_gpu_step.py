@@ -177,20 +177,24 @@ def test_one_launch_iteration_multi_tile(ty):
         sim.close()
 
 
-def test_one_launch_iteration_mixed_precision_same_bits():
+@pytest.mark.parametrize("dims", [(96, 64, 48), (61, 43, 39)], ids=str)
+def test_one_launch_iteration_mixed_precision_same_bits(dims):
     """Mixed-precision steps (FP64 residual, FP32 correction sweeps, several refinement passes) give
-    the same bits -- fields and FP64 pressure -- with the interleaved fused sweeps as with
-    single-colour and one-launch sweeps on colour-split storage (the correction kept in split
-    storage between passes), and reach the divergence bound."""
+    the same bits -- fields and FP64 pressure -- with every family of sweeps: the default and
+    explicit register tiles and boxes (the correction in the quad layout), the interleaved fused
+    sweeps, and single-colour and one-launch sweeps on colour-split storage; and reach the divergence
+    bound.  Rows that are and are not a multiple of four cells."""
     import zq_smokesimulation_amd._lib as L
-    W, H, D = 96, 64, 48
+    W, H, D = dims
     p = oracle_params(W, mixed=1, sor_iters=15, max_outer=400, tol=1e-6, open_mask=O.OPEN_YHI, closed_mean=0)
     shell = O.ALL_FACES & ~O.OPEN_YHI
     out = []
-    for shape in ((0, 0), (-1, 0), (-8, 8)):
+    for shape, kernel in (((0, 0), None), ((-1, 0), "k_sor_split"), ((-8, 8), "k_sor_split_rb"), ((4, 16), "k_sor_fused"),
+                          ((-1208, 8), "k_sor_quad"), ((-1408, 12), "k_sor_quad"), ((-130804, 2), "k_sor_block")):
         occ, u, v, w, T, R = initial_state(W, H, D, shell)
         sim = make_sim(W, H, D, p, SRC)
         sim.set_sor_shape(*shape)
+        assert kernel in (None, sim.sor_kernel())
         sim.set_state(u=u, v=v, w=w, T=T, rho=R, occ=occ)
         sts = []
         for s in range(3):
