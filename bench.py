@@ -37,7 +37,8 @@ hipGraph after the launch-shape autotuner; value = all members' voxels * steps /
 Prints one JSON line.  value = voxels * steps / wall time (Mvoxel-steps/s).  roofline: the
 red-black SOR sweep kernel the autotuner picked (the dominant kernel), algorithmic bytes 13 B/voxel
 per launch (a kernel that runs two iterations a launch reads and writes the grid once for both;
-6.5 B/voxel for a single-colour launch) over its event-timed mean launch time; step_frac: the whole step's algorithmic bytes over the step time.  cpu_baseline: the
+6.5 B/voxel for a single-colour launch) over its event-timed mean launch time; step_frac: the whole
+step's algorithmic bytes over the step time.  cpu_baseline: the
 CPU oracle on a bounded sample of the same step (see --help).
 """
 import argparse
@@ -582,7 +583,8 @@ def main():
                                    for q in (0, 50, 90, 100)},
         "max_div": float(max(s["max_div"] for s in full_stats)),
         "every_step_within_tol": all(s["converged"] == 1 and s["max_div"] <= args.tol for s in full_stats),
-        "step_frac": round(step_bytes(N, grid_passes * full_sweeps, full_passes + 1.0) / (full_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
+        "step_frac": round(step_bytes(N, grid_passes * full_sweeps, full_passes + 1.0) / (full_ms * 1e-3) / 1e9 /
+                           HBM_PEAK_GBS, 4),
         "note": "steps 0..%d of the workload from rest on one clock (the timed steps included)" % (nfull - 1),
     }
     out = {

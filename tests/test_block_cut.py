@@ -33,7 +33,8 @@ static int check(int W, int H, int D, const BlockCut& c) {
         div = div && r == i / c.nx && quad_div(r, c.mny) == r / c.ny;
     }
     if (a || b || e || !fits || !div)
-        return std::printf("%dx%dx%d lx %d ty %d tz %d K %d: %d %d %d %d %d\n", W, H, D, c.lx, c.ty, c.tz, c.K, a, b, e, fits, div), 1;
+        return std::printf("%dx%dx%d lx %d ty %d tz %d K %d: %d %d %d %d %d\n", W, H, D, c.lx, c.ty, c.tz, c.K, a, b, e,
+                           fits, div), 1;
     return 0;
 }
 int main() {

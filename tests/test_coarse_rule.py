@@ -12,7 +12,9 @@ SRC = r"""
 #include <cstdio>
 #include <cstdlib>
 using namespace zq3d;
-static BlockCut rule(int W, int H, int D, double* us) { return block_best_cut(W, H, D, 40, 512, us, block_cost_weighted); }
+static BlockCut rule(int W, int H, int D, double* us) {
+    return block_best_cut(W, H, D, 40, 512, us, block_cost_weighted);
+}
 int main(int argc, char** argv) {
     double us = 0.0;
     if (argc == 4) {
@@ -34,7 +36,8 @@ int main(int argc, char** argv) {
                                 const BlockCut o = block_cut(W, H, D, lx, ty, tz, K);
                                 if (!o.nx || block_threads(o) > 512 || (!o.halo && K > 1)) continue;
                                 const int k = o.halo ? K : 40;
-                                if (block_cost_weighted(o, k) / k < us) return std::printf("%d %d %d: %d %d %d %d\n", W, H, D, lx, ty, tz, K), 1;
+                                if (block_cost_weighted(o, k) / k < us)
+                                    return std::printf("%d %d %d: %d %d %d %d\n", W, H, D, lx, ty, tz, K), 1;
                             }
             }
     std::printf("ok\n");
@@ -50,7 +53,7 @@ def rule(tmp_path):
     exe = str(tmp_path / "rule")
     inc = os.path.join(ROOT, "zq_smokesimulation_amd", "csrc")
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-I", inc, str(src), "-o", exe], check=True)
-    return lambda *dims: subprocess.run([exe, *map(str, dims)], capture_output=True, text=True, check=False).stdout.strip()
+    return lambda *dims: subprocess.run([exe, *map(str, dims)], capture_output=True, text=True).stdout.strip()
 
 
 def test_every_grid_gets_its_cheapest_boxes(rule):
@@ -58,7 +61,8 @@ def test_every_grid_gets_its_cheapest_boxes(rule):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dims,sub", [((64, 64, 64), 2), ((80, 80, 80), 1), ((24, 40, 12), 1), ((96, 80, 64), 8)], ids=str)
+@pytest.mark.parametrize("dims,sub", [((64, 64, 64), 2), ((80, 80, 80), 1), ((24, 40, 12), 1), ((96, 80, 64), 8)],
+                         ids=str)
 def test_a_simulation_takes_the_rules_schedule(rule, dims, sub):
     from zq_smokesimulation_amd.sim import SmokeSim3D
     want = tuple(map(int, rule(*[n // sub for n in dims]).split()))

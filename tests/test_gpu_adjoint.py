@@ -230,8 +230,9 @@ def test_checkpoint_spacing_does_not_change_gradient():
 def test_sweep_shape_does_not_change_rollout_or_gradient(dtype):
     """Every projection of the rollout (forward, recomputation, adjoint) runs the sweep algorithm set
     by set_sor_shape; the default, explicit register tiles and boxes, the interleaved fused sweeps,
-    single-colour split sweeps and one-launch iterations give the same forward bits.  The gradient is compared to a tolerance: the advection adjoint accumulates with atomics,
-    so its last bits depend on the order in which the GPU retires them, whatever the shape."""
+    single-colour split sweeps and one-launch iterations give the same forward bits.  The gradient
+    is compared to a tolerance: the advection adjoint accumulates with atomics, so its last bits
+    depend on the order in which the GPU retires them, whatever the shape."""
     W, H, D, nsteps = 40, 36, 28, 4
     out = []
     for shape in ((-1, 0), (-16, 16), (-32, 8), None, (4, 16), (-1208, 8), (-1404, 6), (-130804, 2)):

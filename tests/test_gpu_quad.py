@@ -31,7 +31,8 @@ def project(W, H, D, shapes, iters, mask, closed, seed=3):
 
 # W: 2 and 3 cells; 4-cell padding 0..3; one full wave of lanes (128 and 256 cells) and one cell more (two
 # tiles with halo lanes); H and D around a tile's rows and a chunk's planes
-@pytest.mark.parametrize("dims", [(2, 3, 2), (3, 2, 5), (16, 9, 7), (17, 20, 9), (18, 33, 8), (19, 12, 31), (64, 17, 13),
+@pytest.mark.parametrize("dims", [(2, 3, 2), (3, 2, 5), (16, 9, 7), (17, 20, 9), (18, 33, 8), (19, 12, 31),
+                                  (64, 17, 13),
                                   (127, 18, 10), (128, 11, 9), (129, 16, 12), (256, 19, 6), (257, 9, 9), (300, 25, 7),
                                   (521, 7, 5)])
 @pytest.mark.parametrize("iters", [0, 1, 2, 5])

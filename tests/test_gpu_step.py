@@ -189,8 +189,9 @@ def test_one_launch_iteration_mixed_precision_same_bits(dims):
     p = oracle_params(W, mixed=1, sor_iters=15, max_outer=400, tol=1e-6, open_mask=O.OPEN_YHI, closed_mean=0)
     shell = O.ALL_FACES & ~O.OPEN_YHI
     out = []
-    for shape, kernel in (((0, 0), None), ((-1, 0), "k_sor_split"), ((-8, 8), "k_sor_split_rb"), ((4, 16), "k_sor_fused"),
-                          ((-1208, 8), "k_sor_quad"), ((-1408, 12), "k_sor_quad"), ((-130804, 2), "k_sor_block")):
+    for shape, kernel in (((0, 0), None), ((-1, 0), "k_sor_split"), ((-8, 8), "k_sor_split_rb"),
+                          ((4, 16), "k_sor_fused"), ((-1208, 8), "k_sor_quad"), ((-1408, 12), "k_sor_quad"),
+                          ((-130804, 2), "k_sor_block")):
         occ, u, v, w, T, R = initial_state(W, H, D, shell)
         sim = make_sim(W, H, D, p, SRC)
         sim.set_sor_shape(*shape)

@@ -42,7 +42,9 @@ struct Fake {
 };
 inline Fake fake;
 inline thread_local hipError_t fake_last = hipSuccess;
-inline bool within(const void* p, const char* b, size_t n) { return b && (const char*)p >= b && (const char*)p < b + n; }
+inline bool within(const void* p, const char* b, size_t n) {
+    return b && (const char*)p >= b && (const char*)p < b + n;
+}
 inline void* resolve(const void* p) {
     return within(p, fake.opaque, fake.opaque_n) ? fake.behind + ((const char*)p - fake.opaque) : (void*)p;
 }
@@ -103,7 +105,10 @@ static std::vector<char> array(int seed) {
     for (size_t i = 0; i < N; i++) v[i] = (char)(i * 31 + i / 4093 + seed);
     return v;
 }
-#define CHECK(c) do { if (!(c)) return std::printf("line %d: %s (direct %zu staged %zu)\n", __LINE__, #c, fake.direct, fake.staged), 1; } while (0)
+static int failed(int line, const char* what) {
+    return std::printf("line %d: %s (direct %zu staged %zu)\n", line, what, fake.direct, fake.staged), 1;
+}
+#define CHECK(c) do { if (!(c)) return failed(__LINE__, #c); } while (0)
 int main() {
     HostCopy h;
     BODY
@@ -140,7 +145,8 @@ SHARED = r"""
     CHECK(h.to_host({{first.data(), host.data(), N}, {second.data(), host.data(), N}}) == hipSuccess);
     CHECK(std::memcmp(host.data(), second.data(), N) == 0);
     CHECK(h.to_host({{first.data(), host.data() + N / 2, N}, {second.data(), host.data(), N}}) == hipSuccess);
-    CHECK(std::memcmp(host.data(), second.data(), N) == 0 && std::memcmp(host.data() + N, first.data() + N / 2, N / 2) == 0);
+    CHECK(std::memcmp(host.data(), second.data(), N) == 0);
+    CHECK(std::memcmp(host.data() + N, first.data() + N / 2, N / 2) == 0);
 """
 # a kernel launch that failed before the copies is still reported when they find no pinned memory
 FAILED_LAUNCH = r"""
@@ -162,8 +168,8 @@ def run(tmp_path, body):
     src.write_text(MAIN.replace("BODY", body))
     exe = str(tmp_path / "copy")
     inc = os.path.join(ROOT, "zq_smokesimulation_amd", "csrc")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-pthread", "-I", str(tmp_path), "-I", inc, str(src), "-o", exe],
-                   check=True)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-pthread", "-I", str(tmp_path), "-I", inc, str(src), "-o",
+                    exe], check=True)
     out = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0 and out.stdout.strip() == "ok", (out.returncode, out.stdout)
 

@@ -53,7 +53,8 @@ def test_each_device_is_asked(tmp_path):
     src = tmp_path / "lds.cpp"
     src.write_text(MAIN)
     exe = str(tmp_path / "lds")
-    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", str(tmp_path), "-I", CSRC, str(src), "-o", exe], check=True)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", str(tmp_path), "-I", CSRC, str(src), "-o", exe],
+                   check=True)
     out = subprocess.run([exe], capture_output=True, text=True)
     assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout
 

@@ -45,7 +45,8 @@ int main() {
                         for (int i = 0; i < iters; i++)
                             for (int j = 0; j < iters; j++)
                                 if (i * OCT_LISTS + a < j * OCT_LISTS + b && at[a][i] >= at[b][j])
-                                    return std::printf("order: adj %d list %d pass %d, list %d pass %d\n", adj, a, i, b, j), 1;
+                                    return std::printf("order: adj %d list %d pass %d, list %d pass %d\n", adj, a, i, b,
+                                                       j), 1;
                     }
                 if (!empty && iters && (int)plan.size() > OCT_LISTS * iters) return std::printf("too many\n"), 1;
                 // leaves stepping one level at a time: four launches a pass once the first has come through

@@ -24,7 +24,8 @@ static int check(int W, int H, int D, int K, int cx, const QuadCut& c) {
     if (c.rows != c.nw * c.g * QUAD_R || c.g * c.lx > 64 || zc % 2) return fail("shape", W, H, D, K, cx, nw, zc);
     if (c.g > 1 && !c.mask && S == W) return fail("unmasked group edge", W, H, D, K, cx, nw, zc);
     // the LDS of a tile: row groups plus one zero group on either side
-    if ((c.nw * c.g + 2) * c.lx * (cx / 2) > quad_edge_floats(cx, 64 * c.nw)) return fail("lds", W, H, D, K, cx, nw, zc);
+    if ((c.nw * c.g + 2) * c.lx * (cx / 2) > quad_edge_floats(cx, 64 * c.nw))
+        return fail("lds", W, H, D, K, cx, nw, zc);
     for (int b = 0; b < c.nx; b++) {
         const int o0 = quad_x_begin(c, K, cx, b, S), o1 = quad_x_begin(c, K, cx, b + 1, S);
         const int x0 = o0 - (b ? cx * hl : 0), x1 = x0 + cx * c.lx;
@@ -44,7 +45,8 @@ static int check(int W, int H, int D, int K, int cx, const QuadCut& c) {
     }
     if (quad_z_begin(c, K, 0, D) != 0 || quad_z_begin(c, K, c.nz, D) != D || quad_x_begin(c, K, cx, c.nx, S) != S ||
         quad_y_begin(c, K, c.ny, H) != H) return fail("cover", W, H, D, K, cx, nw, zc);
-    for (int l = 0; l < 64; l++) if (quad_div(l, c.mlx) != l / c.lx) return fail("lane division", W, H, D, K, cx, nw, zc);
+    for (int l = 0; l < 64; l++)
+        if (quad_div(l, c.mlx) != l / c.lx) return fail("lane division", W, H, D, K, cx, nw, zc);
     const long long tiles = (long long)c.nx * c.ny * c.nz;
     for (long long t = 0; t < tiles; t += 1 + tiles / 997)
         if (quad_div((int)t, c.mnx) != t / c.nx || quad_div((int)(t / c.nx), c.mny) != t / c.nx / c.ny)

@@ -256,7 +256,8 @@ void advect_velocity_bfecc(const Dims& d, R* u, R* v, R* w, const uint8_t* occ, 
         increment<R>(u, F2, K, u, Nu, s);
         increment<R>(v, F2 + Nu, K + Nu, v, Nv, s);
         increment<R>(w, F2 + Nu + Nv, K + Nu + Nv, w, Nw, s);
-        faces_in<R>(d, MacVelCached<R>{K, K + Nu, K + Nu + Nv, d, {}, {}, {}}, MacVel<R>{u, v, w, d}, occ, ou, ov, ow, ap, s);
+        const MacVelCached<R> Vk{K, K + Nu, K + Nu + Nv, d, {}, {}, {}};
+        faces_in<R>(d, Vk, MacVel<R>{u, v, w, d}, occ, ou, ov, ow, ap, s);
     } else {  // mode 5, inReg_outMAC: F = adv(phi; v); C = cells(F); F = adv(C; -v); C = cells(F); C = phi~; F = adv(C; v)
         V4* C = (V4*)bf;
         launch_mac_to_cell4<R>(d, u, v, w, vel4, s, occ);
@@ -307,12 +308,12 @@ void launch_advect_velocity(const Dims& d, R* u, R* v, R* w, const uint8_t* occ,
                            ow, d, h, ap.steps, dtt);
     } else {  // mode 2: inMAC_outMAC
         const MacVelCached<R> V{u, v, w, d, {}, {}, {}};
-        hipLaunchKernelGGL((k_advect_faces<R, 0, MacVelCached<R>>), grid_for(d.W + 1, d.H, d.D), blk, 0, s, V, occ, ou, d,
-                           h, ap.steps, dtt);
-        hipLaunchKernelGGL((k_advect_faces<R, 1, MacVelCached<R>>), grid_for(d.W, d.H + 1, d.D), blk, 0, s, V, occ, ov, d,
-                           h, ap.steps, dtt);
-        hipLaunchKernelGGL((k_advect_faces<R, 2, MacVelCached<R>>), grid_for(d.W, d.H, d.D + 1), blk, 0, s, V, occ, ow, d,
-                           h, ap.steps, dtt);
+        hipLaunchKernelGGL((k_advect_faces<R, 0, MacVelCached<R>>), grid_for(d.W + 1, d.H, d.D), blk, 0, s, V, occ,
+                           ou, d, h, ap.steps, dtt);
+        hipLaunchKernelGGL((k_advect_faces<R, 1, MacVelCached<R>>), grid_for(d.W, d.H + 1, d.D), blk, 0, s, V, occ,
+                           ov, d, h, ap.steps, dtt);
+        hipLaunchKernelGGL((k_advect_faces<R, 2, MacVelCached<R>>), grid_for(d.W, d.H, d.D + 1), blk, 0, s, V, occ,
+                           ow, d, h, ap.steps, dtt);
     }
     hipLaunchKernelGGL((k_apply_faces<R, 0>), grid_for(d.W + 1, d.H, d.D), blk, 0, s, ou, occ, u, d, is_open);
     hipLaunchKernelGGL((k_apply_faces<R, 1>), grid_for(d.W, d.H + 1, d.D), blk, 0, s, ov, occ, v, d, is_open);
@@ -328,8 +329,8 @@ void launch_advect_scalar(const Dims& d, const R* u, const R* v, const R* w, con
     const R dtt = (R)ap.dtt;
     if (mac) {
         const MacVelCached<R> V{u, v, w, d, {}, {}, {}};
-        hipLaunchKernelGGL((k_advect_scalar<R, MacVelCached<R>>), grid_for(d.W, d.H, d.D), blk, 0, s, V, occ, Tin, Rin, Tout,
-                           Rout, d, h, ap.steps, dtt);
+        hipLaunchKernelGGL((k_advect_scalar<R, MacVelCached<R>>), grid_for(d.W, d.H, d.D), blk, 0, s, V, occ, Tin, Rin,
+                           Tout, Rout, d, h, ap.steps, dtt);
     } else {
         launch_mac_to_cell4<R>(d, u, v, w, vel4, s, occ);
         const RegularVelCached<R> V{vel4, d, {}};

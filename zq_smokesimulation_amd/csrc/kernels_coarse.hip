@@ -387,18 +387,19 @@ __global__ __launch_bounds__(256) void k_coarse_unpack(CG g, const float* __rest
 
 // `iters` iterations of a box per workgroup (sor_block_tile with the face weights).  The slabs above
 // spend a launch on staging seven arrays through LDS and read every operand of an update from it; here
-// the operands are registers: at 32^3 coarse cells an iteration takes
-// 2.45 us (slabs 5.8, a launch a colour 6.4), at 64^3 4.3 (6.5).
+// the operands are registers: an iteration takes 2.6 us at 32^3 coarse cells (a launch a colour 6.5) and
+// 4.5 at 64^3 (7.1); other grids at coarse_sweep_default.
 __global__ __launch_bounds__(512) void k_coarse_block(CG g, BlockWeights w, const float* __restrict__ div,
-                                                      const float* __restrict__ src, float* __restrict__ dst, BlockCut c,
-                                                      int iters, float omega, float omw) {
+                                                      const float* __restrict__ src, float* __restrict__ dst,
+                                                      BlockCut c, int iters, float omega, float omw) {
     extern __shared__ float lds[];
     const int per = gridDim.x >> 3;
     const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (tile >= c.nx * c.ny * c.nz) return;  // spare block (the grid is a multiple of 8): uniform exit
     const int rest = quad_div(tile, c.mnx), bx = tile - rest * c.nx;
     const int bz = quad_div(rest, c.mny), by = rest - bz * c.ny;
-    sor_block_tile<true>(nullptr, w, div, 0.0f, src, dst, Dims{g.Wc, g.Hc, g.Dc}, c, bx, by, bz, iters, omega, omw, lds);
+    sor_block_tile<true>(nullptr, w, div, 0.0f, src, dst, Dims{g.Wc, g.Hc, g.Dc}, c, bx, by, bz, iters, omega, omw,
+                         lds);
 }
 
 // ------------------------------------------------------------------------------ coarse delta
@@ -747,8 +748,10 @@ __device__ __forceinline__ double block_sum(double x, double* red) {
 // x plus the value OFF lanes away (lane ^ OFF), without a trip through LDS
 template <int OFF>
 __device__ __forceinline__ unsigned lane_xor(unsigned x) {
-    if constexpr (OFF == 1) return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, true);  // quad [1,0,3,2]
-    if constexpr (OFF == 2) return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, true);  // quad [2,3,0,1]
+    if constexpr (OFF == 1)  // quad [1,0,3,2]
+        return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xf, 0xf, true);
+    if constexpr (OFF == 2)  // quad [2,3,0,1]
+        return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xf, 0xf, true);
     if constexpr (OFF == 4) {  // lanes 0-3, 8-11 of a row from four above, the others from four below
         const int up = __builtin_amdgcn_update_dpp(0, (int)x, 0x104, 0xf, 0x5, true);
         return (unsigned)__builtin_amdgcn_update_dpp(up, (int)x, 0x114, 0xf, 0xa, true);

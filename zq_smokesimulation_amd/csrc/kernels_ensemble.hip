@@ -25,8 +25,9 @@ namespace {
 constexpr int NT = 256;
 
 // the tiles of a table, one a thread; the member by binary search over the members' first tiles
-__global__ __launch_bounds__(NT) void ke_tiles(const EnsMember* __restrict__ M, int count, const int* __restrict__ first,
-                                               int total, EnsTiling t, EnsTile* __restrict__ out) {
+__global__ __launch_bounds__(NT) void ke_tiles(const EnsMember* __restrict__ M, int count,
+                                               const int* __restrict__ first, int total, EnsTiling t,
+                                               EnsTile* __restrict__ out) {
     const int tile = blockIdx.x * NT + threadIdx.x;
     if (tile >= total) return;
     int lo = 0, hi = count - 1;
@@ -99,9 +100,15 @@ __global__ __launch_bounds__(NT) void ke_force_faces(const EnsMember* __restrict
     for_cells(T, M, [&](const EnsMember& m, int i, int j, int k) {
         cell_faces(
             m.d, i, j, k,
-            [&](int x, int y, int z) { st_force_face<float, 0, true>(m.u, m.occ, m.scratch, m.d, m.dt, m.dth, m.aV, x, y, z); },
-            [&](int x, int y, int z) { st_force_face<float, 1, true>(m.v, m.occ, m.scratch, m.d, m.dt, m.dth, m.aV, x, y, z); },
-            [&](int x, int y, int z) { st_force_face<float, 2, true>(m.w, m.occ, m.scratch, m.d, m.dt, m.dth, m.aV, x, y, z); });
+            [&](int x, int y, int z) {
+                st_force_face<float, 0, true>(m.u, m.occ, m.scratch, m.d, m.dt, m.dth, m.aV, x, y, z);
+            },
+            [&](int x, int y, int z) {
+                st_force_face<float, 1, true>(m.v, m.occ, m.scratch, m.d, m.dt, m.dth, m.aV, x, y, z);
+            },
+            [&](int x, int y, int z) {
+                st_force_face<float, 2, true>(m.w, m.occ, m.scratch, m.d, m.dt, m.dth, m.aV, x, y, z);
+            });
     });
 }
 
@@ -122,7 +129,8 @@ __global__ __launch_bounds__(NT) void ke_advect_cells(const EnsMember* __restric
 __global__ __launch_bounds__(NT) void ke_cells_to_faces(const EnsMember* __restrict__ M, EnsTable T) {
     for_cells(T, M, [&](const EnsMember& m, int i, int j, int k) {
         cell_faces(
-            m.d, i, j, k, [&](int x, int y, int z) { st_cells_to_face<float, 0>(m.scratch, m.occ, m.u, m.d, 1, x, y, z); },
+            m.d, i, j, k,
+            [&](int x, int y, int z) { st_cells_to_face<float, 0>(m.scratch, m.occ, m.u, m.d, 1, x, y, z); },
             [&](int x, int y, int z) { st_cells_to_face<float, 1>(m.scratch, m.occ, m.v, m.d, 1, x, y, z); },
             [&](int x, int y, int z) { st_cells_to_face<float, 2>(m.scratch, m.occ, m.w, m.d, 1, x, y, z); });
     });
@@ -191,9 +199,9 @@ __global__ __launch_bounds__(NT) void ke_sor_half(const EnsMember* __restrict__ 
     });
 }
 
-// K iterations of every member's SOR in one launch (sor_quad_tile, each member cut by itself).  Members with an odd count run one iteration
-// first (K == 1, which takes only those, from zero); launch `at` of the pairs then takes every member
-// that still has two to do.
+// K iterations of every member's SOR in one launch (sor_quad_tile, each member cut by itself).  Members
+// with an odd count run one iteration first (K == 1, which takes only those, from zero); launch `at` of
+// the pairs then takes every member that still has two to do.
 template <int K, int CX, int NTH>
 __global__ __launch_bounds__(NTH) void ke_sor_quad(const EnsMember* __restrict__ M, EnsQuadTable T, int at) {
     extern __shared__ float quad_lds[];
@@ -240,8 +248,8 @@ const int kEnsSweepShapes[kEnsSweepShapeCount][2] = {{64, 4}, {32, 8}, {16, 16}}
 
 hipError_t ens_launch_tiles(const EnsMember* members, int count, const int* first, int total, EnsTiling t, EnsTile* out,
                             hipStream_t s) {
-    hipLaunchKernelGGL(ke_tiles, dim3((unsigned)((total + NT - 1) / NT)), dim3(NT), 0, s, members, count, first, total, t,
-                       out);
+    hipLaunchKernelGGL(ke_tiles, dim3((unsigned)((total + NT - 1) / NT)), dim3(NT), 0, s, members, count, first, total,
+                       t, out);
     return hipGetLastError();
 }
 

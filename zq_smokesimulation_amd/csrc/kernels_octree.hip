@@ -269,7 +269,8 @@ __device__ __forceinline__ uint32_t oct_entry(const OG& g, int m, int x, int y, 
 // fine cells in interleaved order (slower axis high), one entry per leaf met (its run of 4^m
 // positions skipped), solid cells skipped.
 template <class Put>
-__device__ __forceinline__ void oct_walk(const OG& g, const uint8_t* __restrict__ lev, int L, int x, int y, int z, Put put) {
+__device__ __forceinline__ void oct_walk(const OG& g, const uint8_t* __restrict__ lev, int L, int x, int y, int z,
+                                         Put put) {
     const int S = 1 << L;
     const int cl[3] = {x, y, z}, dims[3] = {ow(g, L), oh(g, L), od(g, L)}, base[3] = {x * S, y * S, z * S};
 #pragma unroll

@@ -760,9 +760,10 @@ __global__ __launch_bounds__(BX* BY) void k_residual64(const uint8_t* __restrict
 }
 
 // k_residual64 marching z (QUAD: r32 into the quad layout's right-hand side r0, else into the split
-// ones): each thread owns one (i, j) column of a chunk of rz planes and keeps the pressures of planes k-1, k, k+1 in registers, so each padded FP64 pressure is read once
-// (the per-plane kernel reads every plane for three neighbouring planes' blocks).  The same operations
-// per cell in the same order; the block maxima are over the chunk (a maximum is order-free).
+// ones): each thread owns one (i, j) column of a chunk of rz planes and keeps the pressures of planes
+// k-1, k, k+1 in registers, so each padded FP64 pressure is read once (the per-plane kernel reads every
+// plane for three neighbouring planes' blocks).  The same operations per cell in the same order; the
+// block maxima are over the chunk (a maximum is order-free).
 template <bool QUAD>
 __global__ __launch_bounds__(BX* BY) void k_residual64_z(const uint8_t* __restrict__ nc, const double* __restrict__ b64,
                                                          const double* __restrict__ mean64,
@@ -1084,7 +1085,8 @@ bool quad_shape_valid(const Dims& d, SorShape s) {
                quad_cells(d) < (1u << 29);
     }
     const QuadShape q = quad_decode(s);
-    if ((q.cx != 2 && q.cx != 4) || q.nw < 1 || q.nw > (q.cx == 4 ? 8 : 16) || q.zc < 2 || q.zc > 64 || q.zc % 2) return false;
+    if ((q.cx != 2 && q.cx != 4) || q.nw < 1 || q.nw > (q.cx == 4 ? 8 : 16)) return false;
+    if (q.zc < 2 || q.zc > 64 || q.zc % 2) return false;
     return quad_cut(d.W, d.H, d.D, 2, q.cx, q.nw, q.zc).ny > 0;
 }
 

@@ -1214,7 +1214,8 @@ extern "C" int zq3d_set_coarse_sweep(zq3d_sim* s, int k, int zc) {
     if (s->cfg.sub_size <= 0) { set_err(where, "the simulation has no coarse grid (sub_size == 0)"); return ZQ3D_ERR_STATE; }
     const CoarseSweep sw{k, zc};
     if (k < 0 || (k > 0 && !coarse_sweep_valid(s->coarse.cd, sw))) {
-        set_err(where, "k must be 0, or k > 0 and zc > 0 with the slab's planes within 160 KiB of LDS, or zc < 0 a valid box");
+        set_err(where, "k must be 0, or k > 0 and zc > 0 with the slab's planes within 160 KiB of LDS, or zc < 0 a "
+                       "valid box");
         return ZQ3D_ERR_ARG;
     }
     s->coarse.sweep = k == 0 ? CoarseSweep{0, 0} : sw;
@@ -1307,7 +1308,10 @@ extern "C" int zq3d_set_profiling(zq3d_sim* s, int on) {
 extern "C" int zq3d_set_sor_shape(zq3d_sim* s, int ty, int zc) {
     if (!s || zc < 0) { set_err("zq3d_set_sor_shape", "bad argument"); return ZQ3D_ERR_ARG; }
     const SorShape want{ty, zc};
-    if (!sor_shape_valid(s->d, want)) { set_err("zq3d_set_sor_shape", "shape not supported for this grid"); return ZQ3D_ERR_ARG; }
+    if (!sor_shape_valid(s->d, want)) {
+        set_err("zq3d_set_sor_shape", "shape not supported for this grid");
+        return ZQ3D_ERR_ARG;
+    }
     if (is_split(want))
         if (int rc = ensure_split(s, "zq3d_set_sor_shape")) return rc;
     s->shape = want;

@@ -70,7 +70,8 @@ inline double block_cost_weighted(const BlockCut& c, int k) {
     const int rounds = (per + holds - 1) / holds;
     const double simd = std::max(1.0, waves * std::min(per, holds) / 4.0);
     const double rows = (double)boxes * (BLOCK_Y * c.ty) * (BLOCK_Z * c.tz);
-    return 2.0 + rounds * (2.2 + 0.55 * simd + 2.0 * k * (0.26 + 0.2 * simd)) + 1e-6 * rows * (0.67 * BLOCK_X * c.lx + 8.7);
+    return 2.0 + rounds * (2.2 + 0.55 * simd + 2.0 * k * (0.26 + 0.2 * simd)) +
+           1e-6 * rows * (0.67 * BLOCK_X * c.lx + 8.7);
 }
 
 // The cheapest cut per iteration of at most `most` threads (iters: of a pass; a single box runs all of

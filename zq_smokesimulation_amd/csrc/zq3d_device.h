@@ -347,7 +347,8 @@ struct MacVelCached {
     __device__ __forceinline__ R3<R> operator()(R px, R py, R pz) const {
         const R qx = px - R(0.5), qy = py - R(0.5), qz = pz - R(0.5);
         R fx = px - at.x, fy = py - at.y, fz = pz - at.z, hx = qx - half.x, hy = qy - half.y, hz = qz - half.z;
-        if (!all_of(all_of(unit_weight(fx), unit_weight(fy), unit_weight(fz)), all_of(unit_weight(hx), unit_weight(hy), unit_weight(hz)), true)) {
+        if (!all_of(all_of(unit_weight(fx), unit_weight(fy), unit_weight(fz)),
+                    all_of(unit_weight(hx), unit_weight(hy), unit_weight(hz)), true)) {
             const int x = axis_floor(px, d.W + 1, fx), xh = axis_floor(qx, d.W, hx);
             const int y = axis_floor(py, d.H + 1, fy), yh = axis_floor(qy, d.H, hy);
             const int z = axis_floor(pz, d.D + 1, fz), zh = axis_floor(qz, d.D, hz);

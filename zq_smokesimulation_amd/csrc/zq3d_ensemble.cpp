@@ -148,7 +148,8 @@ int quad_shapes(const zq3d_ens* e, int (*shapes)[3]) {
     std::vector<QuadColumns> columns;
     for (int k = 0; k < kEnsQuadFixed; k++) {
         const auto& f = kEnsQuadShapes[k];
-        if (!k || f[0] != kEnsQuadShapes[k - 1][0] || f[1] != kEnsQuadShapes[k - 1][1]) columns = quad_columns(e, f[0], f[1]);
+        if (!k || f[0] != kEnsQuadShapes[k - 1][0] || f[1] != kEnsQuadShapes[k - 1][1])
+            columns = quad_columns(e, f[0], f[1]);
         add(f[0], f[1], f[2], quad_us(columns, f[0], f[2]));
     }
     columns = quad_columns(e, 4, 8);
@@ -206,7 +207,8 @@ int make_table(zq3d_ens* e, EnsTiling t, EnsTable* table, const char* where) {
     for (const Dims& d : e->dims) first.push_back(first.back() + ens_tiles_of(d, t));
     EnsTile* tiles = nullptr;
     int* dev = nullptr;
-    if (ens_alloc(e, &tiles, (size_t)first.back() * sizeof(EnsTile)) || ens_alloc(e, &dev, first.size() * sizeof(int))) {
+    if (ens_alloc(e, &tiles, (size_t)first.back() * sizeof(EnsTile)) ||
+        ens_alloc(e, &dev, first.size() * sizeof(int))) {
         set_err(where, "device allocation failed");
         return ZQ3D_ERR_HIP;
     }
@@ -540,9 +542,10 @@ extern "C" int zq3d_ens_autotune(zq3d_ens* e, int iters, zq3d_ens_tune* rep) {
     static const int blocks[] = {0, 256, 1024, 4096};
     const int nb = (int)(sizeof(blocks) / sizeof(blocks[0]));
     // (kept also where tuning fails later on)
-    for (int sh = 0; sh < kEnsSweepShapeCount; sh++)
-        if (int rc = make_table(e, EnsTiling{kEnsSweepShapes[sh][0], kEnsSweepShapes[sh][1], true}, &e->L.half[sh], where))
-            return rc;
+    for (int sh = 0; sh < kEnsSweepShapeCount; sh++) {
+        const EnsTiling t{kEnsSweepShapes[sh][0], kEnsSweepShapes[sh][1], true};
+        if (int rc = make_table(e, t, &e->L.half[sh], where)) return rc;
+    }
     for (int r = 0; r < kEnsQuadShapeCount; r++)
         if (int rc = make_quad_table(e, 2, e->L.quad_shape[r], &e->L.quad[r], where)) return rc;
     if (e->L.any_odd)

@@ -186,8 +186,9 @@ private:
             if (in_slot[o] != none) {
                 const hipError_t r = hipEventSynchronize(l.ev[o]);
                 l.used[o] = false;
+                const Batch& done = batches_[in_slot[o]];
                 if (r == hipSuccess)
-                    for (size_t k = batches_[in_slot[o]].first; k < batches_[in_slot[o]].first + batches_[in_slot[o]].count; k++)
+                    for (size_t k = done.first; k < done.first + done.count; k++)
                         std::memcpy(pieces_[k].host, l.slot[o] + pieces_[k].at, pieces_[k].bytes);
                 else if (e == hipSuccess) e = r;
                 in_slot[o] = none;

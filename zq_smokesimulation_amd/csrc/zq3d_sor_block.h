@@ -49,10 +49,12 @@ struct BlockTile {
     int slots, me, up, dn, be, ab;  // this thread's slot and its neighbours' (rows above / below, planes below / above)
 
     static __device__ __forceinline__ float shr1(float x) {  // the left lane's value (0 for lane 0)
-        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x138, 0xf, 0xf, true));
+        return __builtin_bit_cast(
+            float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x138, 0xf, 0xf, true));
     }
     static __device__ __forceinline__ float shl1(float x) {  // the right lane's value (0 for lane 63)
-        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x130, 0xf, 0xf, true));
+        return __builtin_bit_cast(
+            float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x130, 0xf, 0xf, true));
     }
 
     // publish colour c's values into buffer buf
@@ -86,7 +88,8 @@ struct BlockTile {
                 const float side = (e ? hi : lo) ? 0.0f : next;
                 const float xm = e ? P[r][z][0] : side, xp = e ? side : P[r][z][1];
                 const float ym = r ? P[0][z][e] : u[z], yp = r ? d[z] : P[1][z][e];
-                const float zm = z ? P[r][z ? z - 1 : 0][e] : b[r], zp = z + 1 < NZ ? P[r][z + 1 < NZ ? z + 1 : z][e] : a[r];
+                const float zm = z ? P[r][z ? z - 1 : 0][e] : b[r];
+                const float zp = z + 1 < NZ ? P[r][z + 1 < NZ ? z + 1 : z][e] : a[r];
                 float s;
                 if constexpr (WT)
                     s = wx[r][z][e] * xm + wx[r][z][e + 1] * xp + wy[r][z][e] * ym + wy[r + 1][z][e] * yp +
@@ -114,9 +117,10 @@ __device__ __forceinline__ void sor_block_tile(const uint8_t* n, const BlockWeig
     const int ix = tid & (c.lx - 1), row = tid / c.lx;  // (lx is a power of two)
     const int iz = quad_div(row, c.mty), iy = row - iz * c.ty;
     const bool on = iz < c.tz;
-    const int xo0 = block_begin(bx, c.nx, S, BLOCK_X * c.lx, c.halo), xo1 = block_begin(bx + 1, c.nx, S, BLOCK_X * c.lx, c.halo);
-    const int yo0 = block_begin(by, c.ny, d.H, BLOCK_Y * c.ty, c.halo), yo1 = block_begin(by + 1, c.ny, d.H, BLOCK_Y * c.ty, c.halo);
-    const int zo0 = block_begin(bz, c.nz, d.D, BLOCK_Z * c.tz, c.halo), zo1 = block_begin(bz + 1, c.nz, d.D, BLOCK_Z * c.tz, c.halo);
+    const int rx = BLOCK_X * c.lx, ry = BLOCK_Y * c.ty, rz = BLOCK_Z * c.tz;  // cells of a box
+    const int xo0 = block_begin(bx, c.nx, S, rx, c.halo), xo1 = block_begin(bx + 1, c.nx, S, rx, c.halo);
+    const int yo0 = block_begin(by, c.ny, d.H, ry, c.halo), yo1 = block_begin(by + 1, c.ny, d.H, ry, c.halo);
+    const int zo0 = block_begin(bz, c.nz, d.D, rz, c.halo), zo1 = block_begin(bz + 1, c.nz, d.D, rz, c.halo);
     const int x = xo0 - (bx ? c.halo : 0) + BLOCK_X * ix;
     const int y0 = yo0 - (by ? c.halo : 0) + BLOCK_Y * iy;
     const int z0 = zo0 - (bz ? c.halo : 0) + BLOCK_Z * iz;
@@ -145,8 +149,8 @@ __device__ __forceinline__ void sor_block_tile(const uint8_t* n, const BlockWeig
             pair(rb, o, q.B[r][z]);
         }
     if constexpr (WT) {
-        const __amdgpu_buffer_rsrc_t rx = split_buf(w.x, 4u * cells), ry = split_buf(w.y, 4u * cells),
-                                     rz = split_buf(w.z, 4u * cells);
+        const __amdgpu_buffer_rsrc_t bwx = split_buf(w.x, 4u * cells), bwy = split_buf(w.y, 4u * cells),
+                                     bwz = split_buf(w.z, 4u * cells);
 #pragma unroll
         for (int r = 0; r <= T::NY; r++)
 #pragma unroll
@@ -154,11 +158,11 @@ __device__ __forceinline__ void sor_block_tile(const uint8_t* n, const BlockWeig
                 const uint32_t o = at(r, z);
                 if (r < T::NY && z < T::NZ) {
                     float t[2];
-                    pair(rx, o, t);
+                    pair(bwx, o, t);
                     q.wx[r][z][0] = t[0], q.wx[r][z][1] = t[1];
                 }
-                if (z < T::NZ) pair(ry, o, q.wy[r][z]);
-                if (r < T::NY) pair(rz, o, q.wz[r][z]);
+                if (z < T::NZ) pair(bwy, o, q.wy[r][z]);
+                if (r < T::NY) pair(bwz, o, q.wz[r][z]);
             }
     }
     q.lo = ix == 0;
@@ -213,7 +217,8 @@ __device__ __forceinline__ void sor_block_tile(const uint8_t* n, const BlockWeig
         for (int z = 0; z < T::NZ; z++) {
             const bool own = xown && y0 + r >= yo0 && y0 + r < yo1 && z0 + z >= zo0 && z0 + z < zo1;
             const uint32_t o = own ? 4u * at(r, z) : SPLIT_NONE;
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(typename T::u2, f2{q.P[r][z][0], q.P[r][z][1]}), rd, (int)o, 0, 0);
+            const f2 t{q.P[r][z][0], q.P[r][z][1]};
+            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(typename T::u2, t), rd, (int)o, 0, 0);
         }
 }
 

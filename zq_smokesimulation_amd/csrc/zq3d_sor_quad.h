@@ -52,7 +52,8 @@ struct QuadTile {
     unsigned N[RS][R];         // CX count bytes
     float V[J][RS][R][M];      // V[j]: values after sweep j (j >= 1)
     // fixed per thread
-    uint32_t off[R], soff[R];  // byte offset of the row's cells in a plane of floats; the same where stored, else SPLIT_NONE
+    // byte offset of the row's cells in a plane of floats; the same where stored, else SPLIT_NONE
+    uint32_t off[R], soff[R];
     bool lo, hi;               // first / last lane of a row group
     // plane t + 2 of the source, t + 1 of b and n, t - J + 1 of the destination, and a plane's bytes
     const char *src, *b, *n;
@@ -72,10 +73,12 @@ struct QuadTile {
     }
 
     static __device__ __forceinline__ float shr1(float x) {  // the left lane's value (0 for lane 0)
-        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x138, 0xf, 0xf, true));
+        return __builtin_bit_cast(
+            float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x138, 0xf, 0xf, true));
     }
     static __device__ __forceinline__ float shl1(float x) {  // the right lane's value (0 for lane 63)
-        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x130, 0xf, 0xf, true));
+        return __builtin_bit_cast(
+            float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x130, 0xf, 0xf, true));
     }
     __device__ __forceinline__ float left(float x) const {
         const float y = shr1(x);
@@ -116,8 +119,9 @@ struct QuadTile {
         for (int r = 0; r < R; r++) {
             load_row(rb, off[r], B[SLOT][r]);
             // a lane with nothing to load has off = SPLIT_NONE; a quarter of it is still past the end
-            if constexpr (CX == 4) N[SLOT][r] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(rn, (int)(off[r] >> 2), 0, 0);
-            else N[SLOT][r] = (unsigned)__builtin_amdgcn_raw_buffer_load_b16(rn, (int)(off[r] >> 2), 0, 0);
+            const int o = (int)(off[r] >> 2);
+            if constexpr (CX == 4) N[SLOT][r] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(rn, o, 0, 0);
+            else N[SLOT][r] = (unsigned)__builtin_amdgcn_raw_buffer_load_b16(rn, o, 0, 0);
         }
     }
 
@@ -218,9 +222,11 @@ struct QuadTile {
                     o[2 * mm + 1 - e] = val<J - 1>(so, r, mm, 1 - e);
                 }
                 if constexpr (CX == 4)
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, f4{o[0], o[1], o[2], o[3]}), rd, (int)soff[r], 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, f4{o[0], o[1], o[2], o[3]}), rd,
+                                                           (int)soff[r], 0, 0);
                 else
-                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, f2{o[0], o[1]}), rd, (int)soff[r], 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, f2{o[0], o[1]}), rd, (int)soff[r], 0,
+                                                          0);
             }
         }
         __syncthreads();
