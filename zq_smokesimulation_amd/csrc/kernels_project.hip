@@ -63,7 +63,8 @@ __global__ __launch_bounds__(BX* BY) void k_proj_setup(const float* __restrict__
 // The mixed-precision set-up: neighbour counts, FP64 divergence b64 (the same sum as the plain
 // set-up, in double), p64 = 0 where the count is 0, per-block FP64 sum/count of the divergence over
 // fluid cells.  One (i, j) column per thread up a chunk of rz planes: the occupancy of planes
-// k-1, k, k+1 and the w face between planes stay in registers, so every input is read once.
+// k-1, k, k+1 and the w face between planes stay in registers, so every input is read once.  The mean's
+// partial sums are per chunk: their grouping, and with it the mean's last FP64 bits, follows rz.
 __global__ __launch_bounds__(BX* BY) void k_proj_setup_z(const float* __restrict__ u, const float* __restrict__ v,
                                                          const float* __restrict__ w, const uint8_t* __restrict__ occ,
                                                          int open_mask, uint8_t* __restrict__ nc,
@@ -1090,12 +1091,14 @@ bool quad_shape_valid(const Dims& d, SorShape s) {
     return quad_cut(d.W, d.H, d.D, 2, q.cx, q.nw, q.zc).ny > 0;
 }
 
-// The sweep shape {0, 0} stands for (computed once per handle): the cheapest marching cut by quad_cost, or
-// the cheapest boxes where block_cost is below it.  What it gives, in microseconds per red-black
-// iteration, beside the shape that was the default (one-pass fused tiles) and the fastest of the older
-// families (single-colour split sweeps up to 160^3, one-launch split iterations above):
-//   marching:  128^3  6.3 (48.8, 10.3)   150x97x61  6.2 (51.5, 8.7)   192^3  11.7 (-, 30.3)   256^3  23.8 (108, 41)
-//   boxes (marching): 20x24x16  1.3 (3.8)   32^3  2.2 (3.6)   64^3  3.3 (3.8)   96^3  5.1 (5.9)   128^3  9.0 (5.9)
+// The sweep shape {0, 0} stands for (searched once per handle, and in a staged solve while the arrays are on
+// their way: 20 to 28 us of host time): the cheapest marching cut by quad_cost, or the cheapest boxes where
+// block_cost is below it.  What it gives, in microseconds per red-black iteration, beside the shape that
+// was the default (one-pass fused tiles) and the fastest of the older families (single-colour split sweeps
+// up to 160^3, one-launch split iterations above); profiles/sweep_shapes.txt has 30 grids, the choice
+// within 5.2 % of the fastest shape on each:
+//   marching:  128^3  6.1 (48.4, 10.8)   160^3  9.3 (59.5, 22.2)   192^3  11.1 (67, 29.8)   256^3  22.7 (77, 41)
+//   boxes (marching): 20x24x16  1.4 (3.9)   32^3  2.3 (3.6)   64^3  3.3 (3.9)   96^3  5.1 (5.7)   128^3  8.9 (6.0)
 // Marching: K = 2 halves the launches and passes; K = 3 and 4 measured slower, their longer pipelines cost
 // what they save.  At 256^3 the iteration moves 13 bytes a cell through the last-level cache, 26 us at the
 // 8.4 TB/s a copy of that size reaches: two iterations a pass go below it.  Boxes have no pipeline and one
@@ -1107,8 +1110,8 @@ QuadPlan quad_plan(const Dims& d) {
     const QuadCut& c = four ? c4 : c2;
     double tb = 0.0;
     const BlockCut cb = block_best_cut(d.W, d.H, d.D, 40, BLOCK_THREADS, &tb);
-    // (predictions that close are in favour of the marching cuts, which lose less when wrong: at 64x64x256
-    // both are 4.8, measured 5.8 against 5.1)
+    // (predictions that close are in favour of the marching cuts, whose choice is nearer their best: at
+    // 64x64x256 both families' best take 4.9, the boxes predicted fastest 5.8)
     if (cb.nx && 2.0 * tb < 0.9 * std::min(t2, t4) && quad_cells(d) < (1u << 29))
         return QuadPlan{block_shape(cb), quad_best_cut(d.W, d.H, d.D, 1, 2, 8)};
     return QuadPlan{SorShape{-(SOR_QUAD + 100 * (four ? 4 : 2) + c.nw), c.zc}, quad_best_cut(d.W, d.H, d.D, 1, 2, 8)};

@@ -52,7 +52,8 @@ inline BlockCut block_cut(int W, int H, int D, int lx, int ty, int tz, int K) {
 // Predicted microseconds of a launch of k iterations: boundary, loads and store, then 2k single-colour
 // sweeps that cost their issue time per wave a SIMD runs.  A CU holds 16 waves of these kernels; boxes
 // beyond what the CUs hold at once run in further rounds.  (Fitted to 2800 launches on 8 grids from
-// 32^3 to 128^3: 10 % rms; its choices are within 4 % of the fastest cut.)
+// 32^3 to 128^3.  On the 24 grids of profiles/sweep_shapes.txt where boxes are chosen, they are within 5.2 %
+// of the fastest cut.)
 inline double block_cost(const BlockCut& c, int k) {
     const int waves = (block_threads(c) + 63) / 64, boxes = c.nx * c.ny * c.nz;
     const int per = (boxes + 255) / 256, holds = std::max(1, 16 / waves);
