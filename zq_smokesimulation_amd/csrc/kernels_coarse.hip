@@ -396,8 +396,8 @@ __global__ __launch_bounds__(512) void k_coarse_block(CG g, BlockWeights w, cons
     const int per = gridDim.x >> 3;
     const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (tile >= c.nx * c.ny * c.nz) return;  // spare block (the grid is a multiple of 8): uniform exit
-    const int rest = quad_div(tile, c.mnx), bx = tile - rest * c.nx;
-    const int bz = quad_div(rest, c.mny), by = rest - bz * c.ny;
+    const int rest = quad_div(tile, c.mnx, c.nx), bx = tile - rest * c.nx;
+    const int bz = quad_div(rest, c.mny, c.ny), by = rest - bz * c.ny;
     sor_block_tile<true>(nullptr, w, div, 0.0f, src, dst, Dims{g.Wc, g.Hc, g.Dc}, c, bx, by, bz, iters, omega, omw,
                          lds);
 }

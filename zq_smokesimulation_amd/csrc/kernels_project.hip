@@ -442,8 +442,8 @@ __global__ __launch_bounds__(NT) void k_sor_quad(const uint8_t* __restrict__ n, 
     const int per = gridDim.x >> 3;
     const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (tile >= c.nx * c.ny * c.nz) return;  // spare block (the grid is a multiple of 8): uniform exit
-    const int rest = quad_div(tile, c.mnx), bx = tile - rest * c.nx;
-    const int bz = quad_div(rest, c.mny), by = rest - bz * c.ny;
+    const int rest = quad_div(tile, c.mnx, c.nx), bx = tile - rest * c.nx;
+    const int bz = quad_div(rest, c.mny, c.ny), by = rest - bz * c.ny;
     sor_quad_tile<K, CX, QUAD_R, MASK, NT>(n, b, *mean32, src, dst, d, c, bx, by, bz, omega, omw, quad_lds);
 }
 
@@ -457,8 +457,8 @@ __global__ __launch_bounds__(NT) void k_sor_block(const uint8_t* __restrict__ n,
     const int per = gridDim.x >> 3;
     const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if (tile >= c.nx * c.ny * c.nz) return;  // spare block (the grid is a multiple of 8): uniform exit
-    const int rest = quad_div(tile, c.mnx), bx = tile - rest * c.nx;
-    const int bz = quad_div(rest, c.mny), by = rest - bz * c.ny;
+    const int rest = quad_div(tile, c.mnx, c.nx), bx = tile - rest * c.nx;
+    const int bz = quad_div(rest, c.mny, c.ny), by = rest - bz * c.ny;
     sor_block_tile<false>(n, BlockWeights{}, b, *mean32, src, dst, d, c, bx, by, bz, iters, omega, omw, block_lds);
 }
 

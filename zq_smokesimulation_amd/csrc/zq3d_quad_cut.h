@@ -31,6 +31,12 @@ struct QuadCut {
 // of small grids, and the compiler's division sequence is long); 0 stands for n = 1
 ZQ_HD inline unsigned quad_magic(int n) { return n > 1 ? (unsigned)(((1ull << 32) + n - 1) / n) : 0u; }
 ZQ_HD inline int quad_div(int i, unsigned magic) { return magic ? (int)(((uint64_t)(unsigned)i * magic) >> 32) : i; }
+// the same for any 0 <= i, n < 2^31 (tile numbers: a grid of millions of cells along one axis has more than
+// 2^16 tiles there): the estimate is at most one too large
+ZQ_HD inline int quad_div(int i, unsigned magic, int n) {
+    const int q = quad_div(i, magic);
+    return q - ((unsigned)q * (unsigned)n > (unsigned)i ? 1 : 0);
+}
 
 // LDS floats of a tile of at most nt threads: the table of reciprocals, then two buffers x 2K arrays x
 // first / last row of every row group (and a zero group on either side, 128 lanes at most), cx/2
