@@ -344,7 +344,7 @@ typedef struct zq3d_timing {
     double ms_sor;              /* red-black sweep launches only */
     double ms_advect_scalar;
     double ms_reinject;
-    long long sor_launches;     /* single-colour sweep kernels timed in ms_sor */
+    long long sor_launches;     /* sweep-kernel launches timed in ms_sor */
     long long steps;
 } zq3d_timing;
 /* on = 0 (off), 1 (stages and sweeps) or 2 (sweeps only); enables and resets the counters */

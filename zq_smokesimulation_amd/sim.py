@@ -164,7 +164,7 @@ class SmokeSim3D:
         return t.as_dict()
 
     def autotune_sor(self, iters=20):
-        """Time every fused-sweep tile shape on this grid and keep the fastest; returns the report."""
+        """Times the sweep shapes that are fastest on some grid and keeps the fastest; returns the report."""
         rep = _lib.TuneReport()
         check(_lib.lib().zq3d_autotune_sor(self._h, int(iters), C.byref(rep)), "autotune_sor")
         return rep.as_dict()
