@@ -1,6 +1,7 @@
 """Tile numbers of the register sweeps on grids that are millions of cells long: the division by the number of
 tiles along an axis (csrc/zq3d_quad_cut.h), compiled with g++, is exact beyond 2^16 tiles, so every tile of a
-launch is somebody's; on the GPU, boxes of four lanes on long thin grids give the oracle's bits."""
+launch is somebody's; on the GPU, boxes of four lanes and marching tiles of one wave on long thin grids
+give the oracle's bits."""
 import os
 import subprocess
 
@@ -51,8 +52,9 @@ def test_the_division_is_exact(tmp_path):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dims", [(410444, 2, 3), (23, 2, 4)], ids=str)
-def test_long_grids_keep_every_tile(dims):
+@pytest.mark.parametrize("dims,shapes", [((410444, 2, 3), [(-120101, 1), (0, 0)]), ((23, 2, 4), [(-120101, 1)]),
+                                         ((8700025, 2, 2), [(-1202, 2)])], ids=str)
+def test_long_grids_keep_every_tile(dims, shapes):
     import zq_oracle as O
     import zq_smokesimulation_amd as z
     from util import faces, occupancy
@@ -65,7 +67,7 @@ def test_long_grids_keep_every_tile(dims):
     O.project(*ref, occ, O.ALL_FACES, 0.0, 1.7, 3)
     sim = z.SmokeSim3D(W, H, D, sor_open_mask=O.ALL_FACES, sor_closed_mean=0, sor_omega=1.7, sor_iters=3)
     try:
-        for shape in ((-120101, 1), (0, 0)):
+        for shape in shapes:
             sim.set_sor_shape(*shape)
             sim.set_state(u=u, v=v, w=w, occ=occ)
             sim.project()

@@ -38,6 +38,11 @@ ZQ_HD inline int quad_div(int i, unsigned magic, int n) {
     return q - ((unsigned)q * (unsigned)n > (unsigned)i ? 1 : 0);
 }
 
+// whether the cut has tiles whose numbers quad_div needs the divisor for
+ZQ_HD inline bool quad_far(const QuadCut& c) {
+    return (long long)c.nx * c.ny * c.nz * (c.nx > c.ny ? c.nx : c.ny) >= 1ll << 32;
+}
+
 // LDS floats of a tile of at most nt threads: the table of reciprocals, then two buffers x 2K arrays x
 // first / last row of every row group (and a zero group on either side, 128 lanes at most), cx/2
 // values a thread.  A block's stride is fixed by nt, so that the accesses have constant offsets.
